@@ -335,13 +335,15 @@ __device__ void lds_fft(cx<T> *buf, int npen, const FftPlan &pl, const cx<T> *__
 #endif
 
 // ---------------------------------------------------------------------------
-// forward z: real comps -> half spectrum, layout B [c][kz][x][y]
+// forward z: real comps -> half spectrum, layout B [c][kz][x][y].  A block takes TY consecutive
+// z rows of the n0 n1 (row (x, y) at x n1 + y, in both layouts), so short z extents fill a block with
+// more rows and a row range may cross x planes: at 256 x 256 x 1 a block of 16 rows had 16 elements
+// to transform (28 us forward, 47 inverse); grid: (ceil(n0 n1 / TY), component pairs)
 // ---------------------------------------------------------------------------
 template <typename T, bool SW>
 __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_fwd_z(const double *__restrict__ in, cx<T> *__restrict__ specB,
                                                      int ncomp, int n0, int n1, int n2, FftPlan pz,
-                                                     const cx<T> *__restrict__ tw, int TY, double m0, double m1,
-                                                     double m2, double m3, double m4, double m5,
+                                                     const cx<T> *__restrict__ tw, int TY,
                                                      const IterCtl *__restrict__ ctl) {
     if (ctl && ctl->done) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -351,24 +353,20 @@ __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_fwd_z(const double
     constexpr bool sw = SW;
     const int P = SW ? n2 + 2 : n2 + 1;   // padded pencil pitch: rows fall on different LDS banks
     cx<T> *stw = buf + TY * P;            // twiddle table staged in LDS
-    const int x = blockIdx.x;
-    const int y0 = blockIdx.y * TY;
-    const int ty = min(TY, n1 - y0);
+    const int rows = n0 * n1, row0 = blockIdx.x * TY;
+    const int ty = min(TY, rows - row0);
     const int H = n2 / 2 + 1;
-    const size_t N = (size_t)n0 * n1 * n2;
-    const size_t HS = (size_t)H * n0 * n1;
-    double mean[6] = {m0, m1, m2, m3, m4, m5};
-    if (ctl)
-        for (int k = 0; k < 6; ++k) mean[k] = ctl->mean6[k];
+    const size_t N = (size_t)rows * n2;
+    const size_t HS = (size_t)H * rows;
     const FastDiv dn2(n2), dty(ty);
     for (int i = threadIdx.x; i < n2; i += FFT_BLOCK) stw[i] = tw[i];
-    // one pair of components per block along grid z
-    for (int ca = 2 * blockIdx.z; ca < ncomp && ca < 2 * blockIdx.z + 2; ca += 2) {
+    // one pair of components per block along grid y
+    for (int ca = 2 * blockIdx.y; ca < ncomp && ca < 2 * blockIdx.y + 2; ca += 2) {
         const int cb = ca + 1;
         const bool two = cb < ncomp;
-        const double ma = ca < 6 ? mean[ca] : 0.0, mb = (two && cb < 6) ? mean[cb] : 0.0;
+        const double ma = ctl && ca < 6 ? ctl->mean6[ca] : 0.0, mb = (ctl && two && cb < 6) ? ctl->mean6[cb] : 0.0;
         const double *ia = in + ca * N, *ib = in + (two ? cb : ca) * N;
-        const size_t g0 = ((size_t)x * n1 + y0) * n2;   // the block's rows are contiguous
+        const size_t g0 = (size_t)row0 * n2;   // the block's rows are contiguous
         chunked_copy<cx<double>>(
             ty * n2, [&](int i) { return cx<double>{ia[g0 + i], ib[g0 + i]}; },
             [&](int i, cx<double> v) {
@@ -383,7 +381,7 @@ __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_fwd_z(const double
             const int e2 = kz == 0 ? 0 : n2 - kz;
             const cx<T> z1 = buf[yy * P + (sw ? lds_swz(kz) : kz)];
             const cx<T> z2 = buf[yy * P + (sw ? lds_swz(e2) : e2)];
-            const size_t o = ((size_t)kz * n0 + x) * n1 + y0 + yy;
+            const size_t o = (size_t)kz * rows + row0 + yy;
             specB[ca * HS + o] = cx<T>{T(0.5) * (z1.x + z2.x), T(0.5) * (z1.y - z2.y)};
             if (two) specB[cb * HS + o] = cx<T>{T(0.5) * (z1.y + z2.y), T(-0.5) * (z1.x - z2.x)};
         }
@@ -456,66 +454,13 @@ __global__ void __launch_bounds__(FFT_BLOCK) k_fft_y(const cx<T> *__restrict__ i
 // ---------------------------------------------------------------------------
 // Green operator at one k point (init.c:542-592 with evolution.c:1169-1183):
 //   Omega = (C0_ijkl n_j n_l)^-1,  du_ij = -Omega_ik (sig_kl n_l) n_j
-// sig: 6 B-basis comps (complex); du: 9 comps (row-major tensor).
+// sig: 6 B-basis comps (complex) -> the strain increment sym(du), 6 B-basis comps.
 // ---------------------------------------------------------------------------
 template <typename A>
 __device__ __forceinline__ void unit_k(int idx, int n, A &t) {
     A v = (A)idx * (A)(1.0 / n);
     v -= round(v);
     t = v * (A)6.28318530718;
-}
-
-__device__ void green_w(const double *__restrict__ C0, const double nv[3], const double sr[9], const double si[9],
-                        double wr[3], double wi[3]) {
-    double A[3][3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            double acc = 0.0;
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-#pragma unroll
-                for (int l = 0; l < 3; ++l) acc += C0[((i * 3 + j) * 3 + k) * 3 + l] * nv[j] * nv[l];
-            A[i][k] = acc;
-        }
-    // M3Inverse (init.c:518-540), cofactors over the determinant
-    const double det = A[0][0] * (A[1][1] * A[2][2] - A[1][2] * A[2][1]) -
-                       A[0][1] * (A[1][0] * A[2][2] - A[1][2] * A[2][0]) +
-                       A[0][2] * (A[1][0] * A[2][1] - A[2][0] * A[1][1]);
-    double om[3][3];
-    om[0][0] = A[1][1] * A[2][2] - A[1][2] * A[2][1];
-    om[0][1] = A[0][2] * A[2][1] - A[0][1] * A[2][2];
-    om[0][2] = A[0][1] * A[1][2] - A[0][2] * A[1][1];
-    om[1][0] = A[1][2] * A[2][0] - A[1][0] * A[2][2];
-    om[1][1] = A[0][0] * A[2][2] - A[0][2] * A[2][0];
-    om[1][2] = A[0][2] * A[1][0] - A[0][0] * A[1][2];
-    om[2][0] = A[1][0] * A[2][1] - A[1][1] * A[2][0];
-    om[2][1] = A[0][1] * A[2][0] - A[0][0] * A[2][1];
-    om[2][2] = A[0][0] * A[1][1] - A[0][1] * A[1][0];
-    const double rdet = 1.0 / det;
-    double tr[3], ti[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        tr[k] = sr[3 * k] * nv[0] + sr[3 * k + 1] * nv[1] + sr[3 * k + 2] * nv[2];
-        ti[k] = si[3 * k] * nv[0] + si[3 * k + 1] * nv[1] + si[3 * k + 2] * nv[2];
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        wr[i] = (om[i][0] * tr[0] + om[i][1] * tr[1] + om[i][2] * tr[2]) * rdet;
-        wi[i] = (om[i][0] * ti[0] + om[i][1] * ti[1] + om[i][2] * ti[2]) * rdet;
-    }
-}
-
-
-template <typename V>
-__device__ __forceinline__ void b6_to_t9(const V v[6], V t[9]) {
-    t[0] = v[0] * V(-SRX_R2) + v[1] * V(-SRX_R6) + v[5] * V(SRX_R3);
-    t[4] = v[0] * V(SRX_R2) + v[1] * V(-SRX_R6) + v[5] * V(SRX_R3);
-    t[8] = v[1] * V(2. * SRX_R6) + v[5] * V(SRX_R3);
-    t[5] = t[7] = v[2] * V(SRX_R2);
-    t[2] = t[6] = v[3] * V(SRX_R2);
-    t[1] = t[3] = v[4] * V(SRX_R2);
 }
 
 // B-basis 6-vector -> symmetric tensor entries (00, 11, 22, 12, 02, 01)
@@ -567,12 +512,176 @@ __device__ __forceinline__ void green_w6(const A *__restrict__ G6, const A n[3],
     wi[2] = (c02 * t0i + c12 * t1i + c22 * t2i) * rdet;
 }
 
+// Symmetric tensor entries (00, 11, 22, 12, 02, 01) -> B basis (chg_basis opt 2), the inverse of b6_to_sym.
+template <typename A>
+__device__ __forceinline__ void sym_to_b6(const A t[6], A v[6]) {
+    v[0] = A(SRX_R2) * (t[1] - t[0]);
+    v[1] = A(SRX_R6) * (A(2) * t[2] - t[0] - t[1]);
+    v[2] = A(2. * SRX_R2) * t[3];
+    v[3] = A(2. * SRX_R2) * t[4];
+    v[4] = A(2. * SRX_R2) * t[5];
+    v[5] = A(SRX_R3) * (t[0] + t[1] + t[2]);
+}
+
+// Unit wave vector of k point (kx, ky, kz) (k != 0).
+template <typename A>
+__device__ __forceinline__ void unit_wave(int kx, int ky, int kz, int n0, int n1, int n2, A n[3]) {
+    unit_k(kx, n0, n[0]);
+    unit_k(ky, n1, n[1]);
+    unit_k(kz, n2, n[2]);
+    const A rg = A(1) / sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+    n[0] *= rg; n[1] *= rg; n[2] *= rg;
+}
+
+// Nyquist accumulator (see green_point): points on a Nyquist plane, kz = n2 / 2 first, then ky = n1 / 2,
+// then kx = n0 / 2; three complex values each, [plane][comp][row][col] with the faster index last.
+__device__ __forceinline__ bool nyq_slot(int kx, int ky, int kz, int n0, int n1, int n2, size_t &at, size_t &pitch) {
+    const int H = n2 / 2 + 1;
+    if (n2 % 2 == 0 && kz == n2 / 2) {
+        at = (size_t)ky * n0 + kx;
+        pitch = (size_t)n0 * n1;
+        return true;
+    }
+    if (n1 % 2 == 0 && ky == n1 / 2) {
+        at = 3 * (size_t)n0 * n1 + (size_t)kz * n0 + kx;
+        pitch = (size_t)H * n0;
+        return true;
+    }
+    if (n0 % 2 == 0 && kx == n0 / 2) {
+        at = 3 * ((size_t)n0 * n1 + (size_t)H * n0) + (size_t)kz * n1 + ky;
+        pitch = (size_t)H * n1;
+        return true;
+    }
+    return false;
+}
+
+// Green operator at one k point (kx, ky, kz): B-basis spectrum q[6] of the stress -> the strain
+// increment sym(du) in the B basis, out[6], computed in the spectrum's precision T (FP32 in the
+// mixed-precision path, whose convolution is FP32 throughout).  The outer iterations need only the
+// strain: the rotation part of du follows from the accumulated strain at the end of the increment
+// (rotation_point), except on the Nyquist planes, where it is summed over the iterations in `nyq`
+// (FP64; null: not kept; `first`: the increment's first iteration stores instead of adding).
+// k = 0: -S0 (sig + dc6) for ElastBC 0, else 0 (init.c:558-569); dc6 is the grid sum of sig that a
+// mean-subtracted (mixed precision) spectrum lacks, B basis.
+// EDGE false: a row away from k = 0 and from the y and z Nyquist planes (NX: nor the x one).
+template <typename T, bool EDGE = true, bool NX = true>
+__device__ __forceinline__ void green_point(const DevConst *__restrict__ cst, const double dc6[6], int kx, int ky,
+                                            int kz, int n0, int n1, int n2, const cx<T> q[6], cx<T> out[6],
+                                            cx<double> *__restrict__ nyq, bool first) {
+    using A = T;
+    const A *G6;
+    if constexpr (sizeof(T) == 4) G6 = cst->G6f;
+    else G6 = cst->G6;
+    if (EDGE && kx == 0 && ky == 0 && kz == 0) {
+        double sr[6], si[6], vr[6], vi[6], br[6] = {0, 0, 0, 0, 0, 0}, bi[6] = {0, 0, 0, 0, 0, 0};
+        if (cst->elast_bc == 0) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) {
+                vr[c] = (double)q[c].x;
+                vi[c] = (double)q[c].y;
+            }
+            b6_to_sym(vr, sr);
+            b6_to_sym(vi, si);
+            double dcs[6], t9r[9], t9i[9], d9[9], er[6], ei[6];
+            b6_to_sym(dc6, dcs);
+            sym_to_t9(sr, t9r);
+            sym_to_t9(si, t9i);
+            sym_to_t9(dcs, d9);
+            const int row[6] = {0, 4, 8, 5, 2, 1};
+#pragma unroll
+            for (int e = 0; e < 6; ++e) {
+                double accr = 0.0, acci = 0.0;
+                for (int r = 0; r < 9; ++r) {
+                    accr += -cst->S0[row[e] * 9 + r] * (t9r[r] + d9[r]);
+                    acci += -cst->S0[row[e] * 9 + r] * t9i[r];
+                }
+                er[e] = accr;
+                ei[e] = acci;
+            }
+            sym_to_b6(er, br);
+            sym_to_b6(ei, bi);
+        }
+#pragma unroll
+        for (int c = 0; c < 6; ++c) out[c] = cx<T>{T(br[c]), T(bi[c])};
+        return;
+    }
+    A nv[3];
+    unit_wave(kx, ky, kz, n0, n1, n2, nv);
+    const bool nyz = EDGE && (n2 % 2 == 0) && (kz == n2 / 2);
+    const bool nyx = NX && (n0 % 2 == 0) && (kx == n0 / 2);
+    const bool nyy = EDGE && (n1 % 2 == 0) && (ky == n1 / 2);
+    A sr[6], si[6];
+    {
+        A vr[6], vi[6];
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+            vr[c] = (A)q[c].x;
+            vi[c] = (A)q[c].y;
+        }
+        b6_to_sym(vr, sr);
+        b6_to_sym(vi, si);
+    }
+    A wr[3], wi[3], er[6], ei[6];
+    green_w6(G6, nv, sr, si, wr, wi);
+    if (!(nyx || nyy || nyz)) {
+        // du_ij = -w_i n_j: entries of sym(du)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const int i = a == 2 ? 0 : a == 1 ? 0 : 1, j = a == 2 ? 1 : 2;   // (1,2), (0,2), (0,1)
+            er[a] = -wr[a] * nv[a];
+            ei[a] = -wi[a] * nv[a];
+            er[3 + a] = A(-0.5) * (wr[i] * nv[j] + wr[j] * nv[i]);
+            ei[3 + a] = A(-0.5) * (wi[i] * nv[j] + wi[j] * nv[i]);
+        }
+    } else {
+        // Taking Re() of the inverse transform (evolution.c:1197) keeps the Hermitian part of du; at
+        // a Nyquist index that part averages Gamma(n) with Gamma(n') where n' has the Nyquist
+        // components negated.
+        const A np[3] = {nyx ? -nv[0] : nv[0], nyy ? -nv[1] : nv[1], nyz ? -nv[2] : nv[2]};
+        A wr2[3], wi2[3];
+        green_w6(G6, np, sr, si, wr2, wi2);
+        size_t at = 0, pitch = 0;
+        nyq_slot(kx, ky, kz, n0, n1, n2, at, pitch);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const int i = a == 2 ? 0 : a == 1 ? 0 : 1, j = a == 2 ? 1 : 2;
+            er[a] = A(-0.5) * (wr[a] * nv[a] + wr2[a] * np[a]);
+            ei[a] = A(-0.5) * (wi[a] * nv[a] + wi2[a] * np[a]);
+            const A rij = A(-0.5) * (wr[i] * nv[j] + wr2[i] * np[j]), rji = A(-0.5) * (wr[j] * nv[i] + wr2[j] * np[i]);
+            const A iij = A(-0.5) * (wi[i] * nv[j] + wi2[i] * np[j]), iji = A(-0.5) * (wi[j] * nv[i] + wi2[j] * np[i]);
+            er[3 + a] = A(0.5) * (rij + rji);
+            ei[3 + a] = A(0.5) * (iij + iji);
+            if (nyq) {
+                // one thread owns the point, so the atomic only spares it the wait for the old sum
+                cx<double> *o = nyq + at + a * pitch;
+                const cx<double> s = {0.5 * ((double)rij - (double)rji), 0.5 * ((double)iij - (double)iji)};
+                if (first) {
+                    *o = s;
+                } else {
+                    atomicAdd(&o->x, s.x);
+                    atomicAdd(&o->y, s.y);
+                }
+            }
+        }
+    }
+    A br[6], bi[6];
+    sym_to_b6(er, br);
+    sym_to_b6(ei, bi);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) out[c] = cx<T>{br[c], bi[c]};
+}
+
+// The nine-component form: mixed precision on grids whose extents are not all powers of two.  There
+// the FP32 wave vector idx * (1/n) - round(..) of a negative index carries a relative error near
+// n / 2^25, so the kz = 0 plane of the strain is Hermitian only to that (3e-6 at n = 96), and the six
+// symmetric components, transformed in other pairs than the nine, differ from them by 1e-5 of the
+// strain after a few increments (2e-7 where the wave vectors are exact).
 // Green operator at one k point (kx, ky, kz): B-basis spectrum q[6] of the stress -> du[9]
 // (row-major), computed in the spectrum's precision T (FP32 in the mixed-precision path, whose
 // convolution is FP32 throughout).  k = 0: -S0 (sig + dc6) for ElastBC 0, else 0 (init.c:558-569);
 // dc6 is the grid sum of sig that a mean-subtracted (mixed precision) spectrum lacks, B basis.
 template <typename T>
-__device__ __forceinline__ void green_point(const DevConst *__restrict__ cst, const double dc6[6], int kx, int ky,
+__device__ __forceinline__ void green_point9(const DevConst *__restrict__ cst, const double dc6[6], int kx, int ky,
                                             int kz, int n0, int n1, int n2, const cx<T> q[6], cx<T> out[9]) {
     using A = T;
     const A *G6;
@@ -661,7 +770,7 @@ __device__ __forceinline__ void green_point(const DevConst *__restrict__ cst, co
 // du_ij = -w_i n_j, the y and z columns are t_y Y_i and t_z Y_i with Y_i = -w_i / |t|, and t_y, t_z
 // are constant along the row, so the row's inverse x transforms of those six components are
 // t_y IFFT(Y_i) and t_z IFFT(Y_i).  X_i is the x column.  At the x Nyquist index the Hermitian
-// average of green_point keeps this form: Y_i = -(w_i + w'_i) / (2 |t|), X_i = -(w_i - w'_i) n_x / 2.
+// average of green_point9 keeps this form: Y_i = -(w_i + w'_i) / (2 |t|), X_i = -(w_i - w'_i) n_x / 2.
 template <typename T>
 __device__ __forceinline__ void green_point_xy(const DevConst *__restrict__ cst, int kx, int ky, int kz, int n0,
                                                int n1, int n2, const cx<T> q[6], cx<T> X[3], cx<T> Y[3]) {
@@ -708,15 +817,53 @@ __device__ __forceinline__ void green_point_xy(const DevConst *__restrict__ cst,
     }
 }
 
-// x pass with the Green operator.  grid: (ceil(n1/TY), H).  LDS: 9 slots of TY*n0.
-// mode 1: forward x of 6 comps, Green, inverse x of 9 comps (the solver pass)
+// Rotation part of the displacement gradient at one k point from the accumulated strain e (B basis).
+// Off the Nyquist planes every iteration's du is u_i n_j, so with g = e n the antisymmetric part
+// (u_i n_j - u_j n_i) / 2 is g_i n_j - g_j n_i (the u.n parts cancel): entries (1,2), (0,2), (0,1).
+// On the Nyquist planes it is the sum kept by green_point; at k = 0 there is none.
+template <typename T>
+__device__ __forceinline__ void rotation_point(int kx, int ky, int kz, int n0, int n1, int n2, const cx<T> q[6],
+                                               const cx<double> *__restrict__ nyq, cx<T> om[3]) {
+    size_t at, pitch;
+    if (kx == 0 && ky == 0 && kz == 0) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) om[a] = cx<T>{T(0), T(0)};
+        return;
+    }
+    if (nyq_slot(kx, ky, kz, n0, n1, n2, at, pitch)) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const cx<double> s = nyq[at + a * pitch];
+            om[a] = cx<T>{T(s.x), T(s.y)};
+        }
+        return;
+    }
+    T n[3], vr[6], vi[6], sr[6], si[6], gr[3], gi[3];
+    unit_wave(kx, ky, kz, n0, n1, n2, n);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+        vr[c] = q[c].x;
+        vi[c] = q[c].y;
+    }
+    b6_to_sym(vr, sr);
+    b6_to_sym(vi, si);
+    gr[0] = sr[0] * n[0] + sr[5] * n[1] + sr[4] * n[2]; gi[0] = si[0] * n[0] + si[5] * n[1] + si[4] * n[2];
+    gr[1] = sr[5] * n[0] + sr[1] * n[1] + sr[3] * n[2]; gi[1] = si[5] * n[0] + si[1] * n[1] + si[3] * n[2];
+    gr[2] = sr[4] * n[0] + sr[3] * n[1] + sr[2] * n[2]; gi[2] = si[4] * n[0] + si[3] * n[1] + si[2] * n[2];
+    om[0] = cx<T>{gr[1] * n[2] - gr[2] * n[1], gi[1] * n[2] - gi[2] * n[1]};
+    om[1] = cx<T>{gr[0] * n[2] - gr[2] * n[0], gi[0] * n[2] - gi[2] * n[0]};
+    om[2] = cx<T>{gr[0] * n[1] - gr[1] * n[0], gi[0] * n[1] - gi[1] * n[0]};
+}
+
+// x pass with the Green operator.  grid: (ceil(n1/TY), H).  LDS: CO slots of TY*n0 (modes 0 and 2: ncomp).
+// mode 1: forward x of 6 comps, Green, inverse x of CO comps (the solver pass)
+// mode 3: forward x of 6 strain comps, rotation_point, inverse x of 3 comps (end of increment)
 // mode 0: forward x only (ncomp comps, testing)   mode 2: inverse x only (testing)
-template <typename T, int MAXB>
+template <typename T, int MAXB, int CO>
 __global__ void __launch_bounds__(FFT_BLOCK) k_green_x(cx<T> *__restrict__ spec, int n0, int n1, int n2, FftPlan px,
                                                        const cx<T> *__restrict__ tw, int TY, int mode, int ncomp,
-                                                       const DevConst *__restrict__ cst, double dc0, double dc1,
-                                                       double dc2, double dc3, double dc4, double dc5,
-                                                       const IterCtl *__restrict__ ctl) {
+                                                       const DevConst *__restrict__ cst,
+                                                       const IterCtl *__restrict__ ctl, cx<double> *__restrict__ nyq) {
     if (ctl && ctl->done) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T> *buf = reinterpret_cast<cx<T> *>(smem_raw);
@@ -726,10 +873,10 @@ __global__ void __launch_bounds__(FFT_BLOCK) k_green_x(cx<T> *__restrict__ spec,
     const int kz = blockIdx.y;
     const size_t plane = (size_t)n0 * n1;
     const int slot = ty * n0;
-    const int cin = mode == 1 ? 6 : ncomp;
-    const int cout = mode == 1 ? 9 : ncomp;
+    const int cin = mode & 1 ? 6 : ncomp;
+    const int cout = mode == 1 ? CO : mode == 3 ? 3 : ncomp;
     const FastDiv dslot(slot), dn0(n0);
-    cx<T> *stw = buf + (mode == 1 ? 9 : ncomp) * slot;
+    cx<T> *stw = buf + (mode & 1 ? CO : ncomp) * slot;
     for (int i = threadIdx.x; i < n0; i += FFT_BLOCK) stw[i] = tw[i];
     // the block's rows of one component are contiguous: y0 * n0 .. (y0 + ty) * n0 of plane kz
     chunked_copy<cx<T>>(
@@ -742,17 +889,30 @@ __global__ void __launch_bounds__(FFT_BLOCK) k_green_x(cx<T> *__restrict__ spec,
     __syncthreads();
     if (mode != 2) lds_fft<T, MAXB, true, false>(buf, cin * ty, px, stw, -1, n0);
     if (mode == 1) {
-        double dc6[6] = {dc0, dc1, dc2, dc3, dc4, dc5};
+        double dc6[6] = {0, 0, 0, 0, 0, 0};
         if (ctl)
             for (int k = 0; k < 6; ++k) dc6[k] = ctl->dcs6[k];
+        const bool first = ctl && ctl->iter == 0;
         for (int i = threadIdx.x; i < slot; i += FFT_BLOCK) {
             const int yy = dn0.div(i), kx = i - yy * n0, ky = y0 + yy;
-            cx<T> q[6], o[9];
+            cx<T> q[6], o[CO];
 #pragma unroll
             for (int c = 0; c < 6; ++c) q[c] = buf[c * slot + i];
-            green_point(cst, dc6, kx, ky, kz, n0, n1, n2, q, o);
+            if constexpr (CO == 9) green_point9(cst, dc6, kx, ky, kz, n0, n1, n2, q, o);
+            else green_point<T>(cst, dc6, kx, ky, kz, n0, n1, n2, q, o, nyq, first);
 #pragma unroll
-            for (int c = 0; c < 9; ++c) buf[c * slot + i] = o[c];
+            for (int c = 0; c < CO; ++c) buf[c * slot + i] = o[c];
+        }
+        __syncthreads();
+    } else if (mode == 3) {
+        for (int i = threadIdx.x; i < slot; i += FFT_BLOCK) {
+            const int yy = dn0.div(i), kx = i - yy * n0, ky = y0 + yy;
+            cx<T> q[6], o[3];
+#pragma unroll
+            for (int c = 0; c < 6; ++c) q[c] = buf[c * slot + i];
+            rotation_point(kx, ky, kz, n0, n1, n2, q, nyq, o);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) buf[c * slot + i] = o[c];
         }
         __syncthreads();
     }
@@ -891,11 +1051,12 @@ __device__ __forceinline__ void wave_fft_inv(cx<T> (&v)[C][NPL], const cx<T> wl[
 #ifndef SRX_GREEN_MIN_BLOCKS
 #define SRX_GREEN_MIN_BLOCKS 1
 #endif
-template <typename T, int NPL>
+// CO = 6: stress -> strain increment; 9: stress -> displacement gradient increment; 3: the
+// end-of-increment pass, strain -> rotation part (rotation_point).
+template <typename T, int NPL, int CO>
 __global__ void __launch_bounds__(256, SRX_GREEN_MIN_BLOCKS) k_green_wave(cx<T> *__restrict__ spec, int n1, int n2,
                                                     const cx<T> *__restrict__ tw, const DevConst *__restrict__ cst,
-                                                    double dc0, double dc1, double dc2, double dc3, double dc4,
-                                                    double dc5, const IterCtl *__restrict__ ctl) {
+                                                    const IterCtl *__restrict__ ctl, cx<double> *__restrict__ nyq) {
     if (ctl && ctl->done) return;
     constexpr int N = 64 * NPL;
     const int lane = threadIdx.x & 63;
@@ -904,9 +1065,12 @@ __global__ void __launch_bounds__(256, SRX_GREEN_MIN_BLOCKS) k_green_wave(cx<T> 
     if (ky >= n1) return;   // the whole wavefront: no barrier follows
     const int H = n2 / 2 + 1;
     const size_t plane = (size_t)N * n1;
-    double dc6[6] = {dc0, dc1, dc2, dc3, dc4, dc5};
-    if (ctl)
+    double dc6[6] = {0, 0, 0, 0, 0, 0};
+    bool first = false;
+    if (ctl) {
         for (int k = 0; k < 6; ++k) dc6[k] = ctl->dcs6[k];
+        first = ctl->iter == 0;
+    }
     // twiddles of this lane: w_N^(l k1) for the four-step split, and W_2h^(l mod h) = w_N^(..) of
     // each cross-lane stage
     cx<T> wl[NPL > 1 ? NPL - 1 : 1];
@@ -927,63 +1091,83 @@ __global__ void __launch_bounds__(256, SRX_GREEN_MIN_BLOCKS) k_green_wave(cx<T> 
         for (int r = 0; r < NPL; ++r) q[c][r] = spec[c * cstride + row + 64 * r];
     wave_fft_fwd<T, NPL, 6>(q, wl, ws, lane);
     const int kb = NPL * brev6(lane);
-    // the row's Green operator in factored form (6 inverse transforms) unless ky or kz is at its
-    // Nyquist index or the row holds k = 0 (wavefront-uniform)
-    const bool factored = !((n1 % 2 == 0 && ky == n1 / 2) || (n2 % 2 == 0 && kz == n2 / 2) || (ky == 0 && kz == 0));
-    if (factored) {
-        cx<T> o[6][NPL];   // X_0..2, Y_0..2
-#pragma unroll
-        for (int r = 0; r < NPL; ++r) {
-            cx<T> qi[6], xi[3], yi[3];
-#pragma unroll
-            for (int c = 0; c < 6; ++c) qi[c] = q[c][r];
-            green_point_xy(cst, r + kb, ky, kz, N, n1, n2, qi, xi, yi);
-#pragma unroll
-            for (int a = 0; a < 3; ++a) { o[a][r] = xi[a]; o[3 + a][r] = yi[a]; }
-        }
-        wave_fft_inv<T, NPL, 6>(o, wl, ws, lane);
-        T ty, tz;
-        unit_k(ky, n1, ty);
-        unit_k(kz, n2, tz);
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
+    if constexpr (CO == 9) {
+        // the row's Green operator in factored form (6 inverse transforms) unless ky or kz is at its
+        // Nyquist index or the row holds k = 0 (wavefront-uniform)
+        const bool factored = !((n1 % 2 == 0 && ky == n1 / 2) || (n2 % 2 == 0 && kz == n2 / 2) || (ky == 0 && kz == 0));
+        if (factored) {
+            cx<T> o[6][NPL];   // X_0..2, Y_0..2
 #pragma unroll
             for (int r = 0; r < NPL; ++r) {
-                const cx<T> y = o[3 + a][r];
-                spec[(3 * a) * cstride + row + 64 * r] = o[a][r];
-                spec[(3 * a + 1) * cstride + row + 64 * r] = cx<T>{ty * y.x, ty * y.y};
-                spec[(3 * a + 2) * cstride + row + 64 * r] = cx<T>{tz * y.x, tz * y.y};
+                cx<T> qi[6], xi[3], yi[3];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) qi[c] = q[c][r];
+                green_point_xy(cst, r + kb, ky, kz, N, n1, n2, qi, xi, yi);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) { o[a][r] = xi[a]; o[3 + a][r] = yi[a]; }
             }
-        return;
+            wave_fft_inv<T, NPL, 6>(o, wl, ws, lane);
+            T ty, tz;
+            unit_k(ky, n1, ty);
+            unit_k(kz, n2, tz);
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+                for (int r = 0; r < NPL; ++r) {
+                    const cx<T> y = o[3 + a][r];
+                    spec[(3 * a) * cstride + row + 64 * r] = o[a][r];
+                    spec[(3 * a + 1) * cstride + row + 64 * r] = cx<T>{ty * y.x, ty * y.y};
+                    spec[(3 * a + 2) * cstride + row + 64 * r] = cx<T>{tz * y.x, tz * y.y};
+                }
+            return;
+        }
     }
-    cx<T> o[9][NPL];
+    cx<T> o[CO][NPL];
+    // a row at the y or z Nyquist index or with k = 0 (wavefront-uniform), about 2% of them at 128^3;
+    // in the others only the lane with kx = N / 2 (lane 1, register 0) takes the averaged form
+    const bool edge = (n1 % 2 == 0 && ky == n1 / 2) || (n2 % 2 == 0 && kz == n2 / 2) || (ky == 0 && kz == 0);
+    auto points = [&](auto point) {
 #pragma unroll
-    for (int r = 0; r < NPL; ++r) {
-        cx<T> qi[6], oi[9];
+        for (int r = 0; r < NPL; ++r) {
+            cx<T> qi[6], oi[CO];
 #pragma unroll
-        for (int c = 0; c < 6; ++c) qi[c] = q[c][r];
-        green_point(cst, dc6, r + kb, ky, kz, N, n1, n2, qi, oi);
+            for (int c = 0; c < 6; ++c) qi[c] = q[c][r];
+            point(r, qi, oi);
 #pragma unroll
-        for (int c = 0; c < 9; ++c) o[c][r] = oi[c];
+            for (int c = 0; c < CO; ++c) o[c][r] = oi[c];
+        }
+    };
+    if constexpr (CO == 9) {
+        points([&](int r, const cx<T> *qi, cx<T> *oi) { green_point9(cst, dc6, r + kb, ky, kz, N, n1, n2, qi, oi); });
+    } else if constexpr (CO == 3) {
+        points([&](int r, const cx<T> *qi, cx<T> *oi) { rotation_point(r + kb, ky, kz, N, n1, n2, qi, nyq, oi); });
+    } else if (edge) {
+        points([&](int r, const cx<T> *qi, cx<T> *oi) {
+            green_point<T>(cst, dc6, r + kb, ky, kz, N, n1, n2, qi, oi, nyq, first);
+        });
+    } else {
+        points([&](int r, const cx<T> *qi, cx<T> *oi) {
+            if (r == 0) green_point<T, false, true>(cst, dc6, r + kb, ky, kz, N, n1, n2, qi, oi, nyq, first);
+            else green_point<T, false, false>(cst, dc6, r + kb, ky, kz, N, n1, n2, qi, oi, nyq, first);
+        });
     }
-    wave_fft_inv<T, NPL, 9>(o, wl, ws, lane);
+    wave_fft_inv<T, NPL, CO>(o, wl, ws, lane);
 #pragma unroll
-    for (int c = 0; c < 9; ++c)
+    for (int c = 0; c < CO; ++c)
 #pragma unroll
         for (int r = 0; r < NPL; ++r) spec[c * cstride + row + 64 * r] = o[c][r];
 }
 
 // ---------------------------------------------------------------------------
-// inverse z (c2r) fused with Eq. 15: dg[c] += ddg[c] + Re(IFFT)/Nxyz
-// grid: (n0, ceil(n1/TY)); `dg` may be an output (scale mode) when accumulate=0
+// inverse z (c2r) fused with Eq. 15: ee[c] += ddg6[c] + Re(IFFT)/Nxyz for the six strain components,
+// or the same for the nine of DisGrad with ddg
+// grid: (ceil(n0 n1 / TY), component pairs); `ee` is an output (scale mode) when accumulate=0
 // ---------------------------------------------------------------------------
 template <typename T, bool SW>
-__global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_inv_z(const cx<T> *__restrict__ specB, double *__restrict__ dg,
+__global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_inv_z(const cx<T> *__restrict__ specB, double *__restrict__ ee,
                                                      int ncomp, int n0, int n1, int n2, FftPlan pz,
                                                      const cx<T> *__restrict__ tw, int TY, int accumulate,
-                                                     double divisor, double a0, double a1, double a2, double a3,
-                                                     double a4, double a5, double a6, double a7, double a8,
-                                                     const IterCtl *__restrict__ ctl) {
+                                                     double divisor, const IterCtl *__restrict__ ctl) {
     if (ctl && ctl->done) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T> *buf = reinterpret_cast<cx<T> *>(smem_raw);
@@ -992,28 +1176,26 @@ __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_inv_z(const cx<T> 
     const int P = SW ? n2 + 2 : n2 + 1;   // padded pencil pitch
     cx<T> *stw = buf + TY * P;
     for (int i = threadIdx.x; i < n2; i += FFT_BLOCK) stw[i] = tw[i];
-    const int x = blockIdx.x;
-    const int y0 = blockIdx.y * TY;
-    const int ty = min(TY, n1 - y0);
+    const int rows = n0 * n1, row0 = blockIdx.x * TY;
+    const int ty = min(TY, rows - row0);
     const int H = n2 / 2 + 1;
-    const size_t N = (size_t)n0 * n1 * n2;
-    const size_t HS = (size_t)H * n0 * n1;
-    double add[9] = {a0, a1, a2, a3, a4, a5, a6, a7, a8};
-    if (ctl)
-        for (int k = 0; k < 9; ++k) add[k] = ctl->ddg[k];
+    const size_t N = (size_t)rows * n2;
+    const size_t HS = (size_t)H * rows;
+    const double *add = ctl ? (ncomp == 9 ? ctl->ddg : ctl->ddg6) : nullptr;
     const FastDiv dn2(n2), dty(ty);
     // 1/Nxyz: a power of two for the usual grids, where the product equals the division
     const double rdiv = 1.0 / divisor;
-    // one pair of components per block along grid z
-    for (int ca = 2 * blockIdx.z; ca < ncomp && ca < 2 * blockIdx.z + 2; ca += 2) {
+    // one pair of components per block along grid y
+    for (int ca = 2 * blockIdx.y; ca < ncomp && ca < 2 * blockIdx.y + 2; ca += 2) {
         const int cb = ca + 1;
         const bool two = cb < ncomp;
         const cx<T> *sa = specB + ca * HS, *sb = specB + (two ? cb : ca) * HS;
+        const double aa = add ? add[ca] : 0.0, ab = add && two ? add[cb] : 0.0;
         chunked_copy<cx2<T>>(
             H * ty,
             [&](int i) {
                 const int kz = dty.div(i), yy = i - kz * ty;
-                const size_t o = ((size_t)kz * n0 + x) * n1 + y0 + yy;
+                const size_t o = (size_t)kz * rows + row0 + yy;
                 return cx2<T>{sa[o], sb[o]};
             },
             [&](int i, cx2<T> v) {
@@ -1024,10 +1206,10 @@ __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_inv_z(const cx<T> 
                 if (kz >= 1 && kz <= n2 - H)
                     buf[yy * P + (sw ? lds_swz(n2 - kz) : n2 - kz)] = cx<T>{A.x + B.y, B.x - A.y};
             });
-        // DisGrad of the block's rows (contiguous): the first chunk of each thread's values is
+        // the strain of the block's rows (contiguous): the first chunk of each thread's values is
         // loaded before the transform, so its round trip to HBM overlaps the LDS work
-        double *da = dg + ca * N, *db = dg + (two ? cb : ca) * N;
-        const size_t g0 = ((size_t)x * n1 + y0) * n2;
+        double *da = ee + ca * N, *db = ee + (two ? cb : ca) * N;
+        const size_t g0 = (size_t)row0 * n2;
         const int tot = ty * n2;
         cx<double> pre[FFT_CHUNK];
         if (accumulate) {
@@ -1055,8 +1237,8 @@ __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_inv_z(const cx<T> 
                     const int yy = dn2.div(i), z = i - yy * n2;
                     const cx<T> v = buf[yy * P + (sw ? lds_swz(z) : z)];
                     if (accumulate) {
-                        da[g0 + i] = pre[e].x + (add[ca] + (double)v.x * rdiv);
-                        if (two) db[g0 + i] = pre[e].y + (add[cb] + (double)v.y * rdiv);
+                        da[g0 + i] = pre[e].x + (aa + (double)v.x * rdiv);
+                        if (two) db[g0 + i] = pre[e].y + (ab + (double)v.y * rdiv);
                     } else {
                         da[g0 + i] = (double)v.x * rdiv;
                         if (two) db[g0 + i] = (double)v.y * rdiv;
@@ -1174,22 +1356,25 @@ static int tile_for(const FftPlan &p, int per_tile_comps, int maxb, int cap, int
     return t;
 }
 
-// Rows (pencils) per block of a z or y pass: `tile` if it is valid, else the largest that fits.
+// Rows (pencils) per block of a z or y pass: `tile` if it is valid, else the largest that fits, up to
+// 16, or up to what makes 1024 elements of short rows (a wavefront's loads then move 64 of them, not a
+// fraction of a row).
 static int zy_tile(const FftPlan &p, int rows, int tile, int prec) {
-    const int t = tile_for(p, 1, 2, rows < 16 ? rows : 16, prec);
+    const int cap = p.n >= 64 ? 16 : 1024 / p.n;
+    const int t = tile_for(p, 1, 2, rows < cap ? rows : cap, prec);
     return tile >= 1 && tile <= t ? tile : t;
 }
 
 // Largest valid tile of pass `pass` (0 forward z, 1 forward y, 2 Green x, 3 inverse y, 4 inverse
 // z); p is the plan of the pass's axis.
-int fft_tile_max(int pass, const int n[3], const FftPlan &p, int prec) {
+int fft_tile_max(int pass, const int n[3], const FftPlan &p, int prec, int comps) {
     switch (pass) {
-    case 0: case 4: return zy_tile(p, n[1], 0, prec);
+    case 0: case 4: return zy_tile(p, n[0] * n[1], 0, prec);
     case 1: case 3: return zy_tile(p, n[0], 0, prec);
-    default: {   // Green x pass: 9 slots of t rows, up to 4 butterflies per thread
-        int t = (4 * FFT_BLOCK * min_radix(p)) / (9 * p.n);
+    default: {   // Green x pass: `comps` slots of t rows, up to 4 butterflies per thread
+        int t = (4 * FFT_BLOCK * min_radix(p)) / (comps * p.n);
         const int csz = prec == 0 ? 16 : 8;
-        const int tl = (FFT_LDS_MAX / csz - p.n) / (9 * p.n);
+        const int tl = (FFT_LDS_MAX / csz - p.n) / (comps * p.n);
         t = t < tl ? t : tl;
         t = t < n[1] ? t : n[1];
         return t < 1 ? 1 : (t > 4 ? 4 : t);
@@ -1197,29 +1382,26 @@ int fft_tile_max(int pass, const int n[3], const FftPlan &p, int prec) {
     }
 }
 
+template <typename T>
+static void launch_fwd_z(hipStream_t s, const double *in, void *specB, int ncomp, const int n[3], const FftPlan &pz,
+                         const void *twz, const IterCtl *ctl, int tile, int prec) {
+    const int rows = n[0] * n[1], TY = zy_tile(pz, rows, tile, prec);
+    const bool sw = plan_swizzled(pz);
+    const dim3 grid((rows + TY - 1) / TY, (ncomp + 1) / 2);
+    const size_t sm = padded_lds(TY, n[2], sizeof(cx<T>), sw);
+    if (sw)
+        SRX_LAUNCH((k_fwd_z<T, true>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<T> *)specB, ncomp, n[0], n[1], n[2], pz,
+                   (const cx<T> *)twz, TY, ctl);
+    else
+        SRX_LAUNCH((k_fwd_z<T, false>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<T> *)specB, ncomp, n[0], n[1], n[2], pz,
+                   (const cx<T> *)twz, TY, ctl);
+    check_launch("fwd_z");
+}
+
 void launch_fft_fwd_z(hipStream_t s, int prec, const double *sig, void *specB, const int n[3], const FftPlan &pz,
                       const void *twz, const IterCtl *ctl, int tile) {
-    const int TY = zy_tile(pz, n[1], tile, prec);
-    const bool sw = plan_swizzled(pz);
-    dim3 grid(n[0], (n[1] + TY - 1) / TY, 3);
-    if (prec == 0) {
-        size_t sm = padded_lds(TY, n[2], sizeof(cx<double>), sw);
-        if (sw)
-            SRX_LAUNCH((k_fwd_z<double, true>), grid, dim3(FFT_BLOCK), sm, s, sig, (cx<double> *)specB, 6, n[0], n[1],
-                           n[2], pz, (const cx<double> *)twz, TY, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, ctl);
-        else
-            SRX_LAUNCH((k_fwd_z<double, false>), grid, dim3(FFT_BLOCK), sm, s, sig, (cx<double> *)specB, 6, n[0], n[1],
-                           n[2], pz, (const cx<double> *)twz, TY, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, ctl);
-    } else {
-        size_t sm = padded_lds(TY, n[2], sizeof(cx<float>), sw);
-        if (sw)
-            SRX_LAUNCH((k_fwd_z<float, true>), grid, dim3(FFT_BLOCK), sm, s, sig, (cx<float> *)specB, 6, n[0], n[1],
-                           n[2], pz, (const cx<float> *)twz, TY, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, ctl);
-        else
-            SRX_LAUNCH((k_fwd_z<float, false>), grid, dim3(FFT_BLOCK), sm, s, sig, (cx<float> *)specB, 6, n[0], n[1],
-                           n[2], pz, (const cx<float> *)twz, TY, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, ctl);
-    }
-    check_launch("fwd_z");
+    if (prec == 0) launch_fwd_z<double>(s, sig, specB, 6, n, pz, twz, ctl, tile, prec);
+    else launch_fwd_z<float>(s, sig, specB, 6, n, pz, twz, ctl, tile, prec);
 }
 
 void launch_fft_y(hipStream_t s, int prec, const void *in, void *out, int ncomp, int sign, int b_to_c, const int n[3],
@@ -1249,13 +1431,14 @@ void launch_fft_y(hipStream_t s, int prec, const void *in, void *out, int ncomp,
     check_launch("fft_y");
 }
 
+template <typename T, int CO>
 static void launch_green_generic(hipStream_t s, int prec, void *specC, const int n[3], const FftPlan &px,
-                                 const void *twx, const DevConst *cst, const double *dc6, int mode, int ncomp,
-                                 const IterCtl *ctl, int tile = 0) {
-    const int slots = mode == 1 ? 9 : ncomp;
+                                 const void *twx, const DevConst *cst, int mode, int ncomp, const IterCtl *ctl,
+                                 void *nyq, int tile = 0) {
+    const int slots = mode & 1 ? CO : ncomp;
     int TY;
     bool wide;
-    if (mode == 1 && tile >= 1 && tile <= fft_tile_max(2, n, px, prec)) {
+    if (mode == 1 && tile >= 1 && tile <= fft_tile_max(2, n, px, prec, CO)) {
         TY = tile;
         wide = (long)slots * TY * n[0] / min_radix(px) > 2 * FFT_BLOCK;
     } else {
@@ -1264,26 +1447,15 @@ static void launch_green_generic(hipStream_t s, int prec, void *specC, const int
         TY = tile_for(px, slots, wide ? 4 : 2, n[1] < 2 ? n[1] : 2, prec);
     }
     const int H = n[2] / 2 + 1;
-    dim3 grid((n[1] + TY - 1) / TY, H);
-    const double z6[6] = {0, 0, 0, 0, 0, 0};
-    const double *d = dc6 ? dc6 : z6;
-    if (prec == 0) {
-        size_t sm = (size_t)(slots * TY + 1) * n[0] * sizeof(cx<double>);
-        if (wide)
-            SRX_LAUNCH((k_green_x<double, 4>), grid, dim3(FFT_BLOCK), sm, s, (cx<double> *)specC, n[0], n[1], n[2],
-                       px, (const cx<double> *)twx, TY, mode, ncomp, cst, d[0], d[1], d[2], d[3], d[4], d[5], ctl);
-        else
-            SRX_LAUNCH((k_green_x<double, 2>), grid, dim3(FFT_BLOCK), sm, s, (cx<double> *)specC, n[0], n[1], n[2],
-                       px, (const cx<double> *)twx, TY, mode, ncomp, cst, d[0], d[1], d[2], d[3], d[4], d[5], ctl);
-    } else {
-        size_t sm = (size_t)(slots * TY + 1) * n[0] * sizeof(cx<float>);
-        if (wide)
-            SRX_LAUNCH((k_green_x<float, 4>), grid, dim3(FFT_BLOCK), sm, s, (cx<float> *)specC, n[0], n[1], n[2],
-                       px, (const cx<float> *)twx, TY, mode, ncomp, cst, d[0], d[1], d[2], d[3], d[4], d[5], ctl);
-        else
-            SRX_LAUNCH((k_green_x<float, 2>), grid, dim3(FFT_BLOCK), sm, s, (cx<float> *)specC, n[0], n[1], n[2],
-                       px, (const cx<float> *)twx, TY, mode, ncomp, cst, d[0], d[1], d[2], d[3], d[4], d[5], ctl);
-    }
+    const dim3 grid((n[1] + TY - 1) / TY, H);
+    cx<double> *ny = (cx<double> *)nyq;
+    const size_t sm = (size_t)(slots * TY + 1) * n[0] * sizeof(cx<T>);
+    if (wide)
+        SRX_LAUNCH((k_green_x<T, 4, CO>), grid, dim3(FFT_BLOCK), sm, s, (cx<T> *)specC, n[0], n[1], n[2], px,
+                   (const cx<T> *)twx, TY, mode, ncomp, cst, ctl, ny);
+    else
+        SRX_LAUNCH((k_green_x<T, 2, CO>), grid, dim3(FFT_BLOCK), sm, s, (cx<T> *)specC, n[0], n[1], n[2], px,
+                   (const cx<T> *)twx, TY, mode, ncomp, cst, ctl, ny);
     check_launch("green_x");
 }
 
@@ -1291,116 +1463,108 @@ static void launch_green_generic(hipStream_t s, int prec, void *specC, const int
 // other extents, and tiles >= 1, use the LDS kernel.
 bool green_wave_ok(const int n[3]) { return n[0] == 64 || n[0] == 128 || n[0] == 256; }
 
-template <typename T>
+template <typename T, int CO>
 static void launch_green_wave(hipStream_t s, void *specC, const int n[3], const void *twx, const DevConst *cst,
-                              const IterCtl *ctl) {
+                              const IterCtl *ctl, void *nyq) {
     const dim3 grid((n[1] + 3) / 4, n[2] / 2 + 1), block(256);
     cx<T> *sp = (cx<T> *)specC;
+    cx<double> *ny = (cx<double> *)nyq;
     const cx<T> *tw = (const cx<T> *)twx;
-    if (n[0] == 64) SRX_LAUNCH((k_green_wave<T, 1>), grid, block, 0, s, sp, n[1], n[2], tw, cst, 0., 0., 0., 0., 0., 0., ctl);
-    else if (n[0] == 128) SRX_LAUNCH((k_green_wave<T, 2>), grid, block, 0, s, sp, n[1], n[2], tw, cst, 0., 0., 0., 0., 0., 0., ctl);
-    else SRX_LAUNCH((k_green_wave<T, 4>), grid, block, 0, s, sp, n[1], n[2], tw, cst, 0., 0., 0., 0., 0., 0., ctl);
+    if (n[0] == 64) SRX_LAUNCH((k_green_wave<T, 1, CO>), grid, block, 0, s, sp, n[1], n[2], tw, cst, ctl, ny);
+    else if (n[0] == 128) SRX_LAUNCH((k_green_wave<T, 2, CO>), grid, block, 0, s, sp, n[1], n[2], tw, cst, ctl, ny);
+    else SRX_LAUNCH((k_green_wave<T, 4, CO>), grid, block, 0, s, sp, n[1], n[2], tw, cst, ctl, ny);
+}
+
+size_t nyq_elems(const int n[3]) {
+    const size_t H = n[2] / 2 + 1;
+    return 3 * ((size_t)n[0] * n[1] + H * n[0] + H * n[1]);
+}
+
+// Whether the outer iterations carry the six strain components (else DisGrad's nine): always in FP64;
+// in mixed precision where the FP32 wave vectors are exact, i.e. every extent is a power of two.
+bool strain_form(const int n[3], int prec) {
+    auto pow2 = [](int v) { return (v & (v - 1)) == 0; };
+    return prec == 0 || (pow2(n[0]) && pow2(n[1]) && pow2(n[2]));
 }
 
 void launch_green_x(hipStream_t s, int prec, void *specC, const int n[3], const FftPlan &px, const void *twx,
-                    const DevConst *cst, const IterCtl *ctl, int tile) {
+                    const DevConst *cst, const IterCtl *ctl, void *nyq, int tile) {
+    const bool six = strain_form(n, prec);
     if (green_wave_ok(n) && tile <= 0) {
-        if (prec == 0) launch_green_wave<double>(s, specC, n, twx, cst, ctl);
-        else launch_green_wave<float>(s, specC, n, twx, cst, ctl);
+        if (prec == 0) launch_green_wave<double, 6>(s, specC, n, twx, cst, ctl, nyq);
+        else if (six) launch_green_wave<float, 6>(s, specC, n, twx, cst, ctl, nyq);
+        else launch_green_wave<float, 9>(s, specC, n, twx, cst, ctl, nyq);
         check_launch("green_x");
         return;
     }
-    launch_green_generic(s, prec, specC, n, px, twx, cst, nullptr, 1, 9, ctl, tile);
+    if (prec == 0) launch_green_generic<double, 6>(s, prec, specC, n, px, twx, cst, 1, 6, ctl, nyq, tile);
+    else if (six) launch_green_generic<float, 6>(s, prec, specC, n, px, twx, cst, 1, 6, ctl, nyq, tile);
+    else launch_green_generic<float, 9>(s, prec, specC, n, px, twx, cst, 1, 9, ctl, nyq, tile);
 }
 
-void launch_fft_inv_z_update(hipStream_t s, int prec, const void *specB, double *dg, const int n[3], const FftPlan &pz,
-                             const void *twz, const IterCtl *ctl, double divisor, int tile) {
-    const int TY = zy_tile(pz, n[1], tile, prec);
+template <typename T>
+static void launch_inv_z(hipStream_t s, const void *specB, double *out, int ncomp, const int n[3], const FftPlan &pz,
+                         const void *twz, int accumulate, double divisor, const IterCtl *ctl, int tile, int prec) {
+    const int rows = n[0] * n[1], TY = zy_tile(pz, rows, tile, prec);
     const bool sw = plan_swizzled(pz);
-    dim3 grid(n[0], (n[1] + TY - 1) / TY, 5);
-    const double a[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};   // dDisGradAvg comes from ctl
-    if (prec == 0) {
-        size_t sm = padded_lds(TY, n[2], sizeof(cx<double>), sw);
-        if (sw)
-            SRX_LAUNCH((k_inv_z<double, true>), grid, dim3(FFT_BLOCK), sm, s, (const cx<double> *)specB, dg, 9, n[0], n[1],
-                           n[2], pz, (const cx<double> *)twz, TY, 1, divisor, a[0], a[1], a[2], a[3], a[4], a[5],
-                           a[6], a[7], a[8], ctl);
-        else
-            SRX_LAUNCH((k_inv_z<double, false>), grid, dim3(FFT_BLOCK), sm, s, (const cx<double> *)specB, dg, 9, n[0], n[1],
-                           n[2], pz, (const cx<double> *)twz, TY, 1, divisor, a[0], a[1], a[2], a[3], a[4], a[5],
-                           a[6], a[7], a[8], ctl);
-    } else {
-        size_t sm = padded_lds(TY, n[2], sizeof(cx<float>), sw);
-        if (sw)
-            SRX_LAUNCH((k_inv_z<float, true>), grid, dim3(FFT_BLOCK), sm, s, (const cx<float> *)specB, dg, 9, n[0], n[1],
-                           n[2], pz, (const cx<float> *)twz, TY, 1, divisor, a[0], a[1], a[2], a[3], a[4], a[5], a[6],
-                           a[7], a[8], ctl);
-        else
-            SRX_LAUNCH((k_inv_z<float, false>), grid, dim3(FFT_BLOCK), sm, s, (const cx<float> *)specB, dg, 9, n[0], n[1],
-                           n[2], pz, (const cx<float> *)twz, TY, 1, divisor, a[0], a[1], a[2], a[3], a[4], a[5], a[6],
-                           a[7], a[8], ctl);
-    }
+    const dim3 grid((rows + TY - 1) / TY, (ncomp + 1) / 2);
+    const size_t sm = padded_lds(TY, n[2], sizeof(cx<T>), sw);
+    if (sw)
+        SRX_LAUNCH((k_inv_z<T, true>), grid, dim3(FFT_BLOCK), sm, s, (const cx<T> *)specB, out, ncomp, n[0], n[1], n[2],
+                   pz, (const cx<T> *)twz, TY, accumulate, divisor, ctl);
+    else
+        SRX_LAUNCH((k_inv_z<T, false>), grid, dim3(FFT_BLOCK), sm, s, (const cx<T> *)specB, out, ncomp, n[0], n[1], n[2],
+                   pz, (const cx<T> *)twz, TY, accumulate, divisor, ctl);
     check_launch("inv_z");
+}
+
+void launch_fft_inv_z_update(hipStream_t s, int prec, const void *specB, double *ee, const int n[3], const FftPlan &pz,
+                             const void *twz, const IterCtl *ctl, double divisor, int tile) {
+    const int nc = strain_form(n, prec) ? 6 : 9;
+    if (prec == 0) launch_inv_z<double>(s, specB, ee, nc, n, pz, twz, 1, divisor, ctl, tile, prec);
+    else launch_inv_z<float>(s, specB, ee, nc, n, pz, twz, 1, divisor, ctl, tile, prec);
+}
+
+// The rotation part of the increment's displacement gradient from its accumulated strain (in [6][N],
+// B basis), into out [3][N] (entries (1,2), (0,2), (0,1)): forward transforms of the six strain
+// components, rotation_point, inverse transforms of three.  tiles: the solver passes' (launch shapes only).
+void launch_rotation_part(hipStream_t s, int prec, const double *in, double *out, void *specB, void *specC,
+                          const int n[3], const FftPlan pl[3], void *const tw[3], const DevConst *cst, void *nyq,
+                          const int tiles[5]) {
+    launch_fft_fwd_z(s, prec, in, specB, n, pl[2], tw[2], nullptr, tiles[0]);
+    launch_fft_y(s, prec, specB, specC, 6, -1, 1, n, pl[1], tw[1], nullptr, tiles[1]);
+    if (green_wave_ok(n)) {
+        if (prec == 0) launch_green_wave<double, 3>(s, specC, n, tw[0], cst, nullptr, nyq);
+        else launch_green_wave<float, 3>(s, specC, n, tw[0], cst, nullptr, nyq);
+        check_launch("rotation_x");
+    } else {
+        if (prec == 0) launch_green_generic<double, 6>(s, prec, specC, n, pl[0], tw[0], cst, 3, 3, nullptr, nyq);
+        else launch_green_generic<float, 6>(s, prec, specC, n, pl[0], tw[0], cst, 3, 3, nullptr, nyq);
+    }
+    launch_fft_y(s, prec, specC, specB, 3, +1, 0, n, pl[1], tw[1], nullptr, tiles[3]);
+    const double divisor = (double)n[0] * n[1] * n[2];
+    if (prec == 0) launch_inv_z<double>(s, specB, out, 3, n, pl[2], tw[2], 0, divisor, nullptr, tiles[4], prec);
+    else launch_inv_z<float>(s, specB, out, 3, n, pl[2], tw[2], 0, divisor, nullptr, tiles[4], prec);
 }
 
 // test path: forward FFT of ncomp real comps to layout C (x pass done), no Green
 void launch_fft_real_forward_test(hipStream_t s, int prec, const double *in, int ncomp, void *specB, void *specC,
                                   const int n[3], const FftPlan *pl, void *const *tw) {
-    const int TY = tile_for(pl[2], 1, 2, n[1] < 16 ? n[1] : 16, prec);
-    const bool sw = plan_swizzled(pl[2]);
-    dim3 grid(n[0], (n[1] + TY - 1) / TY, (ncomp + 1) / 2);
-    if (prec == 0) {
-        size_t sm = padded_lds(TY, n[2], sizeof(cx<double>), sw);
-        if (sw)
-            SRX_LAUNCH((k_fwd_z<double, true>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<double> *)specB, ncomp, n[0], n[1],
-                           n[2], pl[2], (const cx<double> *)tw[2], TY, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, nullptr);
-        else
-            SRX_LAUNCH((k_fwd_z<double, false>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<double> *)specB, ncomp, n[0], n[1],
-                           n[2], pl[2], (const cx<double> *)tw[2], TY, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, nullptr);
-    } else {
-        size_t sm = padded_lds(TY, n[2], sizeof(cx<float>), sw);
-        if (sw)
-            SRX_LAUNCH((k_fwd_z<float, true>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<float> *)specB, ncomp, n[0], n[1],
-                           n[2], pl[2], (const cx<float> *)tw[2], TY, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, nullptr);
-        else
-            SRX_LAUNCH((k_fwd_z<float, false>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<float> *)specB, ncomp, n[0], n[1],
-                           n[2], pl[2], (const cx<float> *)tw[2], TY, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, nullptr);
-    }
-    check_launch("fwd_z(test)");
+    if (prec == 0) launch_fwd_z<double>(s, in, specB, ncomp, n, pl[2], tw[2], nullptr, 0, prec);
+    else launch_fwd_z<float>(s, in, specB, ncomp, n, pl[2], tw[2], nullptr, 0, prec);
     launch_fft_y(s, prec, specB, specC, ncomp, -1, 1, n, pl[1], tw[1], nullptr);
-    launch_green_generic(s, prec, specC, n, pl[0], tw[0], nullptr, nullptr, 0, ncomp, nullptr);
+    if (prec == 0) launch_green_generic<double, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 0, ncomp, nullptr, nullptr);
+    else launch_green_generic<float, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 0, ncomp, nullptr, nullptr);
 }
 
 // test path: inverse of the above for ncomp comps (layout C in, real out = IFFT * 1/divisor)
 void launch_fft_real_inverse_test(hipStream_t s, int prec, void *specC, void *specB, int ncomp, double *out,
                                   const int n[3], const FftPlan *pl, void *const *tw, double divisor) {
-    launch_green_generic(s, prec, specC, n, pl[0], tw[0], nullptr, nullptr, 2, ncomp, nullptr);
+    if (prec == 0) launch_green_generic<double, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 2, ncomp, nullptr, nullptr);
+    else launch_green_generic<float, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 2, ncomp, nullptr, nullptr);
     launch_fft_y(s, prec, specC, specB, ncomp, +1, 0, n, pl[1], tw[1], nullptr);
-    const int TY = tile_for(pl[2], 1, 2, n[1] < 16 ? n[1] : 16, prec);
-    const bool sw = plan_swizzled(pl[2]);
-    dim3 grid(n[0], (n[1] + TY - 1) / TY, (ncomp + 1) / 2);
-    if (prec == 0) {
-        size_t sm = padded_lds(TY, n[2], sizeof(cx<double>), sw);
-        if (sw)
-            SRX_LAUNCH((k_inv_z<double, true>), grid, dim3(FFT_BLOCK), sm, s, (const cx<double> *)specB, out, ncomp, n[0],
-                           n[1], n[2], pl[2], (const cx<double> *)tw[2], TY, 0, divisor, 0., 0., 0., 0., 0., 0., 0.,
-                           0., 0., nullptr);
-        else
-            SRX_LAUNCH((k_inv_z<double, false>), grid, dim3(FFT_BLOCK), sm, s, (const cx<double> *)specB, out, ncomp, n[0],
-                           n[1], n[2], pl[2], (const cx<double> *)tw[2], TY, 0, divisor, 0., 0., 0., 0., 0., 0., 0.,
-                           0., 0., nullptr);
-    } else {
-        size_t sm = padded_lds(TY, n[2], sizeof(cx<float>), sw);
-        if (sw)
-            SRX_LAUNCH((k_inv_z<float, true>), grid, dim3(FFT_BLOCK), sm, s, (const cx<float> *)specB, out, ncomp, n[0],
-                           n[1], n[2], pl[2], (const cx<float> *)tw[2], TY, 0, divisor, 0., 0., 0., 0., 0., 0., 0., 0.,
-                           0., nullptr);
-        else
-            SRX_LAUNCH((k_inv_z<float, false>), grid, dim3(FFT_BLOCK), sm, s, (const cx<float> *)specB, out, ncomp, n[0],
-                           n[1], n[2], pl[2], (const cx<float> *)tw[2], TY, 0, divisor, 0., 0., 0., 0., 0., 0., 0., 0.,
-                           0., nullptr);
-    }
-    check_launch("inv_z(test)");
+    if (prec == 0) launch_inv_z<double>(s, specB, out, ncomp, n, pl[2], tw[2], 0, divisor, nullptr, 0, prec);
+    else launch_inv_z<float>(s, specB, out, ncomp, n, pl[2], tw[2], 0, divisor, nullptr, 0, prec);
 }
 
 // ---------------------------------------------------------------------------

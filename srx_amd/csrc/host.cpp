@@ -331,6 +331,7 @@ struct srx_ctx {
     DevConst *dc = nullptr;
     Fields f;
     void *specB = nullptr, *specC = nullptr;
+    void *nyq = nullptr;                        // rotation sums of the Nyquist planes (nyq_elems complex doubles)
     void *tw[3] = {nullptr, nullptr, nullptr};
     FftPlan pl[3];
     double *partials = nullptr, *red = nullptr, *hred = nullptr, *redseg = nullptr;
@@ -341,6 +342,7 @@ struct srx_ctx {
     // macro state
     double Udot[9], Udot_s[9], Udot_a[9], Scauchy[9];
     double DisGradAvg[9], DisGradAvg_t[9], dDisGradAvg[9], acum[9], uniform[9];
+    double uniform0[9];   // `uniform` before the increment's first outer iteration
     double SigAvg[9], SigAvg1[9];
     double C066[36], S066[36];
     double e_vm = 0, d_vm = 0, s_vm = 0, s_vm1 = 0, TimeTot = 0, err = 0, Err_e = 0, Err_s = 0;
@@ -368,6 +370,9 @@ struct srx_ctx {
     // rows per block of the five FFT passes (0: the default) and their tuned times
     int tiles[5] = {0, 0, 0, 0, 0};
     double tile_us[5] = {0, 0, 0, 0, 0};
+    // what the inverse passes of an outer iteration return: the strain's 6 components, or DisGrad's 9
+    int comps() const { return f.ee ? 6 : 9; }
+    double *strain() const { return f.ee ? f.ee : f.dg; }
 };
 
 namespace {
@@ -673,7 +678,8 @@ int setup(srx_ctx *c) {
         F.nrcf = c->opt.precision == SRX_PREC_MIXED ? reinterpret_cast<float *>(F.nrc) : nullptr;
     }
     if ((rc = dalloc(&F.sig, 6, 0.0)) || (rc = dalloc(&F.sig_pre, 5, 0.0)) || (rc = dalloc(&F.eps, 5, 0.0)) ||
-        (rc = dalloc(&F.edot, 5, 0.0)) || (rc = dalloc(&F.dg, 9, 0.0)) || (rc = dalloc(&F.dg0, 9, 0.0)) ||
+        (rc = dalloc(&F.edot, 5, 0.0)) || (strain_form(c->n, c->opt.precision) && (rc = dalloc(&F.ee, 6, 0.0))) ||
+        (rc = dalloc(&F.dg, 9, 0.0)) || (rc = dalloc(&F.dg0, 9, 0.0)) ||
         (rc = dalloc(&F.tran, 9, 0.0)) || (rc = dalloc(&F.tran0, 9, 0.0)) ||
         (rc = dalloc(&F.rho_s, 12, d.rho_SSD_initial)) || (rc = dalloc(&F.rho_m, 12, 0.0)) ||
         (rc = dalloc(&F.rho_m_old, 12, 0.0)) || (rc = dalloc(&F.rho_F, 12, 0.0)) || (rc = dalloc(&F.rho_P, 12, 0.0)) ||
@@ -767,10 +773,11 @@ int setup(srx_ctx *c) {
     if (int e = ctx_copy(st, c->dc, &c->hc, sizeof(DevConst), hipMemcpyHostToDevice)) return e;
 
     const size_t H = (size_t)(c->n[2] / 2 + 1);
-    const size_t spec_elems = 9 * H * c->n[0] * c->n[1];
+    const size_t spec_elems = (F.ee ? 6 : 9) * H * c->n[0] * c->n[1];
     const size_t csz = c->opt.precision == SRX_PREC_MIXED ? 2 * sizeof(float) : 2 * sizeof(double);
     HIPCK(hipMalloc(&c->specB, spec_elems * csz));
     HIPCK(hipMalloc(&c->specC, spec_elems * csz));
+    if (F.ee) HIPCK(hipMalloc(&c->nyq, nyq_elems(c->n) * 2 * sizeof(double)));
     for (int ax = 0; ax < 3; ++ax) {
         int r = c->opt.precision == SRX_PREC_MIXED ? upload_twiddles<float>(c->n[ax], &c->tw[ax], st)
                                                    : upload_twiddles<double>(c->n[ax], &c->tw[ax], st);
@@ -894,7 +901,7 @@ const char *srx_strerror(int code) {
 
 // Average time (us) of three launches of FFT pass `pass` (0 forward z, 1 forward y, 2 Green x,
 // 3 inverse y, 4 inverse z) at tile `t`, after one warm-up launch, on the context's own buffers with
-// its current plans (the inverse z pass writes the scratch DisGrad `scratch`).  With a `flush`
+// its current plans (the inverse z pass writes the scratch strain `scratch`).  With a `flush`
 // buffer (2 x FLUSH_BYTES) each launch is timed alone after a streaming copy through it, so the
 // pass reads its input from HBM as it does in the solver, where the Newton kernel's traffic has
 // evicted it from the last-level cache; else the three launches run back to back.
@@ -907,8 +914,8 @@ static int time_pass(srx_ctx *c, int pass, int t, double *scratch, hipEvent_t e0
         switch (pass) {
         case 0: launch_fft_fwd_z(st, prec, c->f.sig, c->specB, c->n, c->pl[2], c->tw[2], nullptr, t); break;
         case 1: launch_fft_y(st, prec, c->specB, c->specC, 6, -1, 1, c->n, c->pl[1], c->tw[1], nullptr, t); break;
-        case 2: launch_green_x(st, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, nullptr, t); break;
-        case 3: launch_fft_y(st, prec, c->specC, c->specB, 9, +1, 0, c->n, c->pl[1], c->tw[1], nullptr, t); break;
+        case 2: launch_green_x(st, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, nullptr, nullptr, t); break;
+        case 3: launch_fft_y(st, prec, c->specC, c->specB, c->comps(), +1, 0, c->n, c->pl[1], c->tw[1], nullptr, t); break;
         default:
             launch_fft_inv_z_update(st, prec, c->specB, scratch, c->n, c->pl[2], c->tw[2], nullptr, (double)c->nvox,
                                     t);
@@ -967,7 +974,7 @@ static std::map<std::array<int, 5>, FftPlan> g_plan_cache;
 static int autotune_fft(srx_ctx *c) {
     const int prec = c->opt.precision;
     double *scratch = nullptr;
-    HIPCK(hipMalloc(&scratch, sizeof(double) * 9 * (size_t)c->nvox));
+    HIPCK(hipMalloc(&scratch, sizeof(double) * c->comps() * (size_t)c->nvox));
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = 0;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) rc = SRX_E_HIP;
@@ -1017,7 +1024,7 @@ static int autotune_fft(srx_ctx *c) {
     }
     for (int pass = 0; pass < 5 && !rc && c->opt.reserved[2] == 0; ++pass) {
         const FftPlan &p = c->pl[pass == 2 ? 0 : (pass == 1 || pass == 3) ? 1 : 2];
-        const int tmax = fft_tile_max(pass, c->n, p, prec);
+        const int tmax = fft_tile_max(pass, c->n, p, prec, c->comps());
         std::vector<int> cand;
         if (pass == 2 && green_wave_ok(c->n)) cand.push_back(-1);   // one wavefront per row
         else {
@@ -1334,7 +1341,7 @@ static int step_begin(srx_ctx *c, EnsIncr *batch = nullptr) {
         ctl.mean6[k] = ctl.mixed ? c->sig_sum6[k] / ctl.nvox : 0.0;
         ctl.dcs6[k] = ctl.mixed ? ctl.mean6[k] * ctl.nvox : 0.0;
     }
-    for (int k = 0; k < 9; ++k) ctl.uniform[k] = c->uniform[k];
+    for (int k = 0; k < 9; ++k) ctl.uniform[k] = c->uniform0[k] = c->uniform[k];
     ctl.done = ctl_stop(ctl);
     HIPCK(hipMemcpyAsync(c->dctl, &ctl, sizeof(IterCtl), hipMemcpyHostToDevice, c->stream));
     return 0;
@@ -1369,9 +1376,9 @@ static int step_iterate(srx_ctx *c) {
             const int *tl = c->tiles;
             { Timer t(c, 0, launched); launch_fft_fwd_z(c->stream, prec, c->f.sig, c->specB, c->n, c->pl[2], c->tw[2], g, tl[0]); }
             { Timer t(c, 1, launched); launch_fft_y(c->stream, prec, c->specB, c->specC, 6, -1, 1, c->n, c->pl[1], c->tw[1], g, tl[1]); }
-            { Timer t(c, 2, launched); launch_green_x(c->stream, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, g, tl[2]); }
-            { Timer t(c, 3, launched); launch_fft_y(c->stream, prec, c->specC, c->specB, 9, +1, 0, c->n, c->pl[1], c->tw[1], g, tl[3]); }
-            { Timer t(c, 4, launched); launch_fft_inv_z_update(c->stream, prec, c->specB, c->f.dg, c->n, c->pl[2], c->tw[2], g, divisor, tl[4]); }
+            { Timer t(c, 2, launched); launch_green_x(c->stream, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, g, c->nyq, tl[2]); }
+            { Timer t(c, 3, launched); launch_fft_y(c->stream, prec, c->specC, c->specB, c->comps(), +1, 0, c->n, c->pl[1], c->tw[1], g, tl[3]); }
+            { Timer t(c, 4, launched); launch_fft_inv_z_update(c->stream, prec, c->specB, c->strain(), c->n, c->pl[2], c->tw[2], g, divisor, tl[4]); }
             const bool rec = c->rec_stride > 0 && launched > 1;
             if (rec)
                 launch_mlp_record(c->stream, c->dc, c->f, N, c->rec_stride, 0, c->rec_x, c->rec_t, c->rec_nd,
@@ -1451,6 +1458,16 @@ static int finish_begin(srx_ctx *c, Finish &F) {
     std::memcpy(c->DisGradAvg_t, act, sizeof(act));
     std::memcpy(r.disgrad_avg_actual, act, sizeof(act));
     std::memcpy(r.velgrad_avg, vga, sizeof(vga));
+    // DisGrad of the voxels from the strain the outer iterations advanced and the uniform part they
+    // applied (not the last dDisGradAvg), on the context's stream ahead of the end-of-increment kernel
+    if (F.iter > 0 && c->f.ee) {
+        double du[9];
+        for (int k = 0; k < 9; ++k) du[k] = c->uniform[k] - c->uniform0[k];
+        launch_rot_in(c->stream, c->f, (int)c->nvox, du);
+        launch_rotation_part(c->stream, c->opt.precision, c->f.ee, c->f.ee, c->specB, c->specC, c->n, c->pl, c->tw, c->dc,
+                             c->nyq, c->tiles);
+        launch_rot_out(c->stream, c->f, (int)c->nvox, du);
+    }
     // Edot/Eps, update_orient (istep>1), DislocationEvolution, averages: the end-of-increment kernel
     F.do_orient = (d.Update_Flag == 1 && c->istep > 1) ? 1 : 0;
     return 0;
@@ -1669,9 +1686,9 @@ static int run_lockstep(const std::vector<int> &members, std::vector<srx_ctx *> 
                     IterCtl *g = c->dctl;
                     launch_fft_fwd_z(st, prec, c->f.sig, c->specB, c->n, c->pl[2], c->tw[2], g, tl[0]);
                     launch_fft_y(st, prec, c->specB, c->specC, 6, -1, 1, c->n, c->pl[1], c->tw[1], g, tl[1]);
-                    launch_green_x(st, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, g, tl[2]);
-                    launch_fft_y(st, prec, c->specC, c->specB, 9, +1, 0, c->n, c->pl[1], c->tw[1], g, tl[3]);
-                    launch_fft_inv_z_update(st, prec, c->specB, c->f.dg, c->n, c->pl[2], c->tw[2], g,
+                    launch_green_x(st, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, g, c->nyq, tl[2]);
+                    launch_fft_y(st, prec, c->specC, c->specB, c->comps(), +1, 0, c->n, c->pl[1], c->tw[1], g, tl[3]);
+                    launch_fft_inv_z_update(st, prec, c->specB, c->strain(), c->n, c->pl[2], c->tw[2], g,
                                             (double)c->nvox, tl[4]);
                 }
                 for (int q = 0; q < NS; ++q) ok(hipEventRecord(ev[q], side[q])) && ok(hipStreamWaitEvent(S, ev[q], 0));
@@ -2032,7 +2049,7 @@ void srx_close(srx_ctx *c) {
     if (c->fdd) std::fclose(c->fdd);
     if (c->fdrx) std::fclose(c->fdrx);
     if (c->ferr) std::fclose(c->ferr);
-    double *ptrs[] = {c->f.sig, c->f.sig_pre, c->f.eps, c->f.edot, c->f.dg, c->f.dg0, c->f.tran, c->f.tran0,
+    double *ptrs[] = {c->f.sig, c->f.sig_pre, c->f.eps, c->f.edot, c->f.ee, c->f.dg, c->f.dg0, c->f.tran, c->f.tran0,
                       c->f.rho_s, c->f.rho_m, c->f.rho_m_old, c->f.rho_F, c->f.rho_P, c->f.gamdot, c->f.gam_acum,
                       c->f.rho_dipole, c->f.rho_forest, c->f.rho_inplane, c->f.rho_tot, c->f.fl0, c->f.acr, c->f.nrc,
                       c->hc.rho_g1, c->hc.rho_g2, c->hc.gnd_fp,
@@ -2050,6 +2067,7 @@ void srx_close(srx_ctx *c) {
     if (c->f.nr_it) (void)hipFree(c->f.nr_it);
     if (c->specB) (void)hipFree(c->specB);
     if (c->specC) (void)hipFree(c->specC);
+    if (c->nyq) (void)hipFree(c->nyq);
     for (int i = 0; i < 3; ++i)
         if (c->tw[i]) (void)hipFree(c->tw[i]);
     if (c->dc) (void)hipFree(c->dc);

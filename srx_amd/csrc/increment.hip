@@ -6,10 +6,24 @@
 
 namespace srx {
 
-// increment prologue (evolution.c:1115-1128): dg0 = dg; dg += Udot dt (or = set9 under creep)
 struct Vec9 {
     double v[9];
 };
+
+// sym(d) in the B basis (chg_basis opt 2), d a row-major tensor
+__device__ __forceinline__ void sym_b6(const double d[9], double e[6]) {
+    const double s00 = d[0], s11 = d[4], s22 = d[8];
+    const double s12 = (d[5] + d[7]) / 2.0, s02 = (d[2] + d[6]) / 2.0, s01 = (d[1] + d[3]) / 2.0;
+    e[0] = s00 * (-SRX_R2) + s11 * SRX_R2;
+    e[1] = s00 * (-SRX_R6) + s11 * (-SRX_R6) + s22 * (2. * SRX_R6);
+    e[2] = s12 * SRX_R2 + s12 * SRX_R2;
+    e[3] = s02 * SRX_R2 + s02 * SRX_R2;
+    e[4] = s01 * SRX_R2 + s01 * SRX_R2;
+    e[5] = s00 * SRX_R3 + s11 * SRX_R3 + s22 * SRX_R3;
+}
+
+// increment prologue (evolution.c:1115-1128): dg0 = dg; dg += Udot dt (or = set9 under creep); and
+// the strain the outer iterations advance, ee = sym(dg) - eps (where they do)
 
 // evolution.c:1115-1128.  In a creep run DisGrad is reset to the macroscopic value; the
 // fluctuation it held (DisGrad minus the uniform part uold) is carried in fl0 so that the
@@ -19,12 +33,71 @@ __device__ __forceinline__ void prologue_voxel(const Fields &f, int nvox, unsign
     const int v = blk * blockDim.x + threadIdx.x;
     if (v >= nvox) return;
     const size_t N = (size_t)nvox;
+    double g[9], e[6];
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
         const double d = f.dg[k * N + v];
         f.dg0[k * N + v] = d;
-        f.dg[k * N + v] = creep ? set[k] : d + add[k];
+        g[k] = creep ? set[k] : d + add[k];
+        f.dg[k * N + v] = g[k];
         if (creep && f.fl0) f.fl0[k * N + v] += d - uold[k];
+    }
+    if (!f.ee) return;
+    sym_b6(g, e);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) f.ee[k * N + v] = k < 5 ? e[k] - f.eps[k * N + v] : e[k];
+}
+
+// End of the outer iterations (with ee): DisGrad from the strain they advanced.  Its change over the
+// increment's iterations is a uniform part du9 (the applied dDisGradAvg) and a fluctuation u_i,j
+// whose strain is known; k_rot_in writes the new symmetric part into dg, keeping the old
+// antisymmetric one, and leaves the fluctuation's strain in ee; launch_rotation_part turns that
+// into the fluctuation's rotation (3 components, in ee), and k_rot_out adds it and the uniform part's.
+// The outer iterations thus transform, store and read 6 components instead of 9: at 128^3 one
+// rotation per increment of about 60 iterations costs less than half of one iteration's 9-component
+// passes.
+__device__ __forceinline__ void anti3(const double d[9], double w[3]) {
+    w[0] = 0.5 * (d[5] - d[7]);
+    w[1] = 0.5 * (d[2] - d[6]);
+    w[2] = 0.5 * (d[1] - d[3]);
+}
+
+__global__ void k_rot_in(Fields f, int nvox, Vec9 du) {
+    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= nvox) return;
+    const size_t N = (size_t)nvox;
+    double g[9], e0[6], e[6], w[3], u6[6];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) g[k] = f.dg[k * N + v];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) e[k] = f.ee[k * N + v];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) e[k] += f.eps[k * N + v];
+    sym_b6(g, e0);
+    sym_b6(du.v, u6);
+    anti3(g, w);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) f.ee[k * N + v] = (e[k] - e0[k]) - u6[k];
+    const double s12 = SRX_R2 * e[2], s02 = SRX_R2 * e[3], s01 = SRX_R2 * e[4];
+    const double h = SRX_R3 * e[5] - SRX_R6 * e[1];
+    const double out[9] = {h - SRX_R2 * e[0], s01 + w[2], s02 + w[1], s01 - w[2], h + SRX_R2 * e[0], s12 + w[0],
+                           s02 - w[1], s12 - w[0], SRX_R3 * e[5] + 2. * SRX_R6 * e[1]};
+#pragma unroll
+    for (int k = 0; k < 9; ++k) f.dg[k * N + v] = out[k];
+}
+
+__global__ void k_rot_out(Fields f, int nvox, Vec9 du) {
+    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= nvox) return;
+    const size_t N = (size_t)nvox;
+    double w[3];
+    anti3(du.v, w);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int up = a == 0 ? 5 : a == 1 ? 2 : 1, lo = a == 0 ? 7 : a == 1 ? 6 : 3;
+        const double x = w[a] + f.ee[a * N + v];
+        f.dg[up * N + v] += x;
+        f.dg[lo * N + v] -= x;
     }
 }
 
@@ -555,6 +628,20 @@ void launch_prologue(hipStream_t s, Fields f, int nvox, const double *a, int cre
     }
     SRX_LAUNCH(k_prologue, dim3(prologue_block_count(nvox)), dim3(PRO_BLOCK), 0, s, f, nvox, add, creep, set, uold);
     check_launch("prologue");
+}
+
+void launch_rot_in(hipStream_t s, const Fields &f, int nvox, const double *du9) {
+    Vec9 du;
+    for (int k = 0; k < 9; ++k) du.v[k] = du9[k];
+    SRX_LAUNCH(k_rot_in, dim3(prologue_block_count(nvox)), dim3(PRO_BLOCK), 0, s, f, nvox, du);
+    check_launch("rot_in");
+}
+
+void launch_rot_out(hipStream_t s, const Fields &f, int nvox, const double *du9) {
+    Vec9 du;
+    for (int k = 0; k < 9; ++k) du.v[k] = du9[k];
+    SRX_LAUNCH(k_rot_out, dim3(prologue_block_count(nvox)), dim3(PRO_BLOCK), 0, s, f, nvox, du);
+    check_launch("rot_out");
 }
 
 int prologue_block_count(int nvox) { return (nvox + PRO_BLOCK - 1) / PRO_BLOCK; }

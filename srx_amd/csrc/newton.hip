@@ -56,10 +56,6 @@ __device__ __forceinline__ void sc_rotate(const double *__restrict__ S, const do
         }
 }
 
-// LDS slots of the per-system constants (tau_pass * inv, inv, gamma_0 dt of 12 systems), also the
-// component order of Fields::nrc
-constexpr int NRC_TP = 0, NRC_INV = NSYS, NRC_G0 = 2 * NSYS, NRC_COMPS = 3 * NSYS;
-
 // eps_c = (DisGrad + DisGrad^T) / 2 in the B basis (chg_basis opt 2), from the 9 row-major components
 __device__ __forceinline__ void ec_from_dg(const double d[9], double ec[6]) {
     const double s00 = d[0], s11 = d[4], s22 = d[8];
@@ -71,6 +67,26 @@ __device__ __forceinline__ void ec_from_dg(const double d[9], double ec[6]) {
     ec[4] = s01 * SRX_R2 + s01 * SRX_R2;
     ec[5] = s00 * SRX_R3 + s11 * SRX_R3 + s22 * SRX_R3;
 }
+
+// The strain a Newton call is driven by, eps_c - eps_p in the B basis: f.ee, or formed from DisGrad and
+// the plastic strain where the outer iterations advance DisGrad itself (uniform branch).
+__device__ __forceinline__ void load_strain(const Fields &f, size_t N, unsigned o8, double e[6]) {
+    if (f.ee) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) e[k] = ldc(f.ee + (size_t)k * N, N, o8);
+    } else {
+        double d[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) d[k] = ldc(f.dg + (size_t)k * N, N, o8);
+        ec_from_dg(d, e);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) e[k] -= ldc(f.eps + (size_t)k * N, N, o8);
+    }
+}
+
+// LDS slots of the per-system constants (tau_pass * inv, inv, gamma_0 dt of 12 systems), also the
+// component order of Fields::nrc
+constexpr int NRC_TP = 0, NRC_INV = NSYS, NRC_G0 = 2 * NSYS, NRC_COMPS = 3 * NSYS;
 
 // Per-voxel values every Newton call of an increment starts from, in the crystal frame of the
 // current orientation: lam' = Q^T lam, q' = Q^T (eps_p - eps_c), the matrix A = Sc + S' (packed),
@@ -99,10 +115,10 @@ __device__ __forceinline__ void pin_prologue(NrPro &p) {
     pin(p.lamh); pin(p.qh); pin(p.rsig2);
 }
 
-// The inputs of a Newton call for one voxel: orientation (TranMat), stress, plastic strain,
-// DisGrad and, after the first call of an increment, the increment's matrix A (packed).
+// The inputs of a Newton call for one voxel: orientation (TranMat), stress, the strain
+// eps_c - eps_p and, after the first call of an increment, the increment's matrix A (packed).
 struct NrIn {
-    double a[9], lam6[6], ep[5], d[9], A[15];
+    double a[9], lam6[6], e[6], A[15];
 };
 template <bool LOAD_A>
 __device__ __forceinline__ void nr_load(const Fields &f, size_t N, unsigned o8, NrIn &in) {
@@ -110,10 +126,7 @@ __device__ __forceinline__ void nr_load(const Fields &f, size_t N, unsigned o8, 
     for (int k = 0; k < 9; ++k) in.a[k] = ldc(f.tran + (size_t)k * N, N, o8);
 #pragma unroll
     for (int k = 0; k < 6; ++k) in.lam6[k] = ldc(f.sig + (size_t)k * N, N, o8);
-#pragma unroll
-    for (int k = 0; k < 5; ++k) in.ep[k] = ldc(f.eps + (size_t)k * N, N, o8);
-#pragma unroll
-    for (int k = 0; k < 9; ++k) in.d[k] = ldc(f.dg + (size_t)k * N, N, o8);
+    load_strain(f, N, o8, in.e);
     if (LOAD_A) {
         if (f.acrf) {
 #pragma unroll
@@ -130,8 +143,8 @@ __device__ __forceinline__ void nr_load(const Fields &f, size_t N, unsigned o8, 
 // Prologue of a Newton call from its inputs `in`.  FIRST (the increment's first call): A assembled
 // from the orientations (Sc = Q^T S066 Q and the rotated grain compliance S') and stored in f.acr
 // for the increment's later calls.  Otherwise A is in.A.
-// KEEP_EC (warm starts): eps_c is also stored in f.ecp where `store` is set, for the next call's
-// learned-start features.
+// KEEP_EC (warm starts): the strain is also stored in f.ecp where `store` is set, for the next
+// call's learned-start features.
 template <bool FIRST, bool ROT, int PH, bool KEEP_EC>
 __device__ __forceinline__ void nr_prologue(const DevConst *__restrict__ cst, const Fields &f, int v, size_t N,
                                             const NrIn &in, NrPro &pro, bool store = true) {
@@ -146,19 +159,15 @@ __device__ __forceinline__ void nr_prologue(const DevConst *__restrict__ cst, co
     q5_from(a, Q);
     double lam6[6], w[5];
     {
-        double ec[6];
-        const double *ep = in.ep;
 #pragma unroll
         for (int k = 0; k < 6; ++k) lam6[k] = in.lam6[k];
-        // strain_aux = (DisGrad + DisGrad^T)/2 -> B basis (chg_basis opt 2)
-        ec_from_dg(in.d, ec);
         if (KEEP_EC && store && f.ecp) {
 #pragma unroll
-            for (int k = 0; k < 6; ++k) stcf(f.ecp + (size_t)k * N, N, 4u * (unsigned)v, (float)ec[k]);
+            for (int k = 0; k < 6; ++k) stcf(f.ecp + (size_t)k * N, N, 4u * (unsigned)v, (float)in.e[k]);
         }
 #pragma unroll
-        for (int k = 0; k < 5; ++k) w[k] = ep[k] - ec[k];
-        pro.qh = -ec[5];
+        for (int k = 0; k < 5; ++k) w[k] = -in.e[k];
+        pro.qh = -in.e[5];
     }
     double sn = 0.0;
 #pragma unroll
@@ -597,7 +606,7 @@ __device__ __forceinline__ void copy_wait() {
 }
 
 // Learned start of the wavefront's voxels (every lane calls; non-crystalline lanes get zero).
-// Features from the Newton call's inputs (orientation, stress, DisGrad), the previous change and
+// Features from the Newton call's inputs (orientation, stress, strain), the previous change and
 // rho_s.
 __device__ __forceinline__ void nr_learned_start(const DevConst *__restrict__ cst, const Fields &f, size_t N, int v,
                                                  bool xt, const NrIn &in, float wsp[6]) {
@@ -607,10 +616,9 @@ __device__ __forceinline__ void nr_learned_start(const DevConst *__restrict__ cs
         const double *a = in.a;
         float d[6];
         crystal_stress(a, in.lam6, lamc);
-        // forcing: eps_c now minus eps_c of the previous call, crystal frame
-        ec_from_dg(in.d, de);
+        // forcing: the strain now minus that of the previous call, crystal frame
 #pragma unroll
-        for (int k = 0; k < 6; ++k) de[k] -= (double)f.ecp[k * N + v];
+        for (int k = 0; k < 6; ++k) de[k] = in.e[k] - (double)f.ecp[k * N + v];
         crystal_stress(a, de, dec);
 #pragma unroll
         for (int k = 0; k < 6; ++k) d[k] = f.dsig[k * N + v];
@@ -916,6 +924,9 @@ __device__ __forceinline__ void control_step(const DevConst *__restrict__ cst, I
         c.mean6[k] = c.mixed ? c.sig_sum6[k] / c.nvox : 0.0;
         c.dcs6[k] = c.mixed ? c.mean6[k] * c.nvox : 0.0;
     }
+    const double s12 = 0.5 * (c.ddg[5] + c.ddg[7]), s02 = 0.5 * (c.ddg[2] + c.ddg[6]), s01 = 0.5 * (c.ddg[1] + c.ddg[3]);
+    const double sym[9] = {c.ddg[0], s01, s02, s01, c.ddg[4], s12, s02, s12, c.ddg[8]};
+    ctl_t9_to_b6(sym, c.ddg6);
     c.done = ctl_stop(c);
 }
 
@@ -938,13 +949,12 @@ __global__ void k_mlp_rec_x(const DevConst *__restrict__ cst, Fields f, int nvox
     const int ph = f.phase[v];
     float x[MLP_IN], nd = 0.0f;
     if (ph >= 1 && ph <= NPH && cst->ph[ph - 1].xtal) {
-        double a[9], lam6[6], lamc[6], dg[9], de[6], dec[6], rho = 0.0;
+        double a[9], lam6[6], lamc[6], de[6], dec[6], rho = 0.0;
         float d[6];
         for (int k = 0; k < 9; ++k) a[k] = f.tran[k * N + v];
         for (int k = 0; k < 6; ++k) lam6[k] = f.sig[k * N + v];
         crystal_stress(a, lam6, lamc);
-        for (int k = 0; k < 9; ++k) dg[k] = f.dg[k * N + v];
-        ec_from_dg(dg, de);
+        load_strain(f, N, 8u * (unsigned)v, de);
         for (int k = 0; k < 6; ++k) de[k] -= (double)f.ecp[k * N + v];
         crystal_stress(a, de, dec);
         for (int k = 0; k < 6; ++k) d[k] = f.dsig[k * N + v];

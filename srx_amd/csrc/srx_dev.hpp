@@ -126,6 +126,7 @@ struct IterCtl {
     double mean6[6];      // their means: subtracted before the FP32 cast (mixed precision)
     double dcs6[6];       // the sums reinjected at k = 0 (mixed precision), else 0
     double ddg[9];        // dDisGradAvg, applied by the next inverse-z pass
+    double ddg6[6];       // its symmetric part in the B basis (what that pass adds to the strain)
     double acum[9], uniform[9];
     double SigAvg[9], SigAvg1[9], s_vm, s_vm1;
 };
@@ -223,7 +224,11 @@ struct Fields {
     double *sig_pre;   // [5][N] last NR pre-update iterate, crystal frame of tran (deviatoric)
     double *eps;       // [5][N] plastic strain, B basis (deviatoric)
     double *edot;      // [5][N] plastic strain rate, B basis
-    double *dg;        // [9][N] displacement gradient DisGrad, row-major tensor comps
+    double *ee;        // [6][N] eps_c - eps_p, B basis: the strain sym(DisGrad) the outer iterations advance
+                       //   minus the plastic strain, which does not change within an increment; null where
+                       //   they advance dg itself (strain_form false)
+    double *dg;        // [9][N] displacement gradient DisGrad, row-major tensor comps; with ee, brought up to
+                       //   date at the end of the increment (k_rot_in, k_rot_out)
     double *dg0;       // [9][N] DisGrad at the start of the increment
     double *tran;      // [9][N] TranMat_xt2sa (crystal -> sample), current
     double *tran0;     // [9][N] TranMat_xt2sa at setup (C_gr is never rotated)
@@ -239,7 +244,7 @@ struct Fields {
     float *nrcf;       // mixed precision: the same constants rounded to FP32, [36][nrcf_pitch(N)] in nrc's memory
                        //   (every Newton call of the increment uses the rounded values); null in FP64
     float *dsig;       // [6][N] last Newton call's stress change, B basis, crystal frame (warm start only)
-    float *ecp;        // [6][N] eps_c = sym(DisGrad) (B basis, sample frame) of the last Newton call (warm start only)
+    float *ecp;        // [6][N] eps_c - eps_p (B basis, sample frame) of the last Newton call (warm start only)
     const MlpPacked *mlp;   // learned Newton start (non-null: the start comes from the network)
     int *phase;        // [N]
     int *nr_it;        // [N]
@@ -293,8 +298,9 @@ void set_launch_events(hipEvent_t start, hipEvent_t stop);
 // With a non-null `ctl` the iteration's scalars (mean stress, k = 0 sums, dDisGradAvg) come from
 // the device control block and the kernels return at once when its `done` is set.
 // `tile`: rows (pencils) per block, 0 for the default; fft_tile_max gives the largest valid one of
-// a pass (0 forward z, 1 forward y, 2 Green x, 3 inverse y, 4 inverse z; p: the pass axis's plan).
-int fft_tile_max(int pass, const int n[3], const FftPlan &p, int prec);
+// a pass (0 forward z, 1 forward y, 2 Green x, 3 inverse y, 4 inverse z; p: the pass axis's plan;
+// comps: the components the Green pass returns).
+int fft_tile_max(int pass, const int n[3], const FftPlan &p, int prec, int comps);
 // The solver's Green x pass can run one wavefront per row (tile -1; the default tile 0 selects it)
 // for n0 = 64, 128, 256.
 bool green_wave_ok(const int n[3]);
@@ -302,10 +308,20 @@ void launch_fft_fwd_z(hipStream_t s, int prec, const double *sig, void *specB, c
                       const FftPlan &pz, const void *twz, const IterCtl *ctl, int tile = 0);
 void launch_fft_y(hipStream_t s, int prec, const void *in, void *out, int ncomp, int sign, int b_to_c,
                   const int n[3], const FftPlan &py, const void *twy, const IterCtl *ctl = nullptr, int tile = 0);
+// strain_form: the iterations advance the strain's six components (Fields::ee) instead of DisGrad's nine
+bool strain_form(const int n[3], int prec);
+// nyq: the Nyquist planes' rotation sums, nyq_elems(n) complex doubles (null: not kept)
+size_t nyq_elems(const int n[3]);
 void launch_green_x(hipStream_t s, int prec, void *specC, const int n[3], const FftPlan &px, const void *twx,
-                    const DevConst *cst, const IterCtl *ctl, int tile = 0);
-void launch_fft_inv_z_update(hipStream_t s, int prec, const void *specB, double *dg, const int n[3],
+                    const DevConst *cst, const IterCtl *ctl, void *nyq, int tile = 0);
+void launch_fft_inv_z_update(hipStream_t s, int prec, const void *specB, double *ee, const int n[3],
                              const FftPlan &pz, const void *twz, const IterCtl *ctl, double scale, int tile = 0);
+// End of increment: the rotation part (3 comps) of the DisGrad change from its strain part (6 comps)
+void launch_rotation_part(hipStream_t s, int prec, const double *in, double *out, void *specB, void *specC,
+                          const int n[3], const FftPlan pl[3], void *const tw[3], const DevConst *cst, void *nyq,
+                          const int tiles[5]);
+void launch_rot_in(hipStream_t s, const Fields &f, int nvox, const double *du9);
+void launch_rot_out(hipStream_t s, const Fields &f, int nvox, const double *du9);
 // ph2: the second phase is crystalline (its Newton path is compiled in only then)
 void launch_nr(hipStream_t s, const DevConst *cst, const Fields &f, int nvox, int first_call, int rotated,
                double *partials, const IterCtl *ctl = nullptr, int gnd = 0, int ph2 = 1);

@@ -328,3 +328,25 @@ def test_device_setup_matches_oracle(tmp_path, oracle_lib, creep):
         assert np.abs(a - b).max() <= 1e-13 * max(np.abs(b).max(), 1.0), name
     g.close()
     o.close()
+
+
+@pytest.mark.parametrize("n,precision", [((6, 4, 10), srx_amd.PREC_FP64), ((5, 15, 12), srx_amd.PREC_FP64),
+                                         ((9, 2, 1), srx_amd.PREC_FP64), ((1, 8, 6), srx_amd.PREC_FP64),
+                                         ((64, 5, 2), srx_amd.PREC_FP64), ((8, 16, 4), srx_amd.PREC_MIXED),
+                                         ((128, 2, 4), srx_amd.PREC_MIXED), ((12, 8, 5), srx_amd.PREC_MIXED),
+                                         ((64, 6, 4), srx_amd.PREC_MIXED)])
+@pytest.mark.parametrize("elast_bc", [0, 1])
+def test_displacement_gradient_matches_oracle(tmp_path, oracle_lib, n, precision, elast_bc):
+    """DisGrad, its rotation part and what follows from them (velocity gradient, orientations) over
+    rotating increments, on even, odd and unit extents: the outer iterations advance the strain and the
+    rotation is recovered from it once per increment, with the Nyquist planes' sums kept apart (mixed
+    precision: only where every extent is a power of two).  FP64 to this file's 1e-9; mixed to its 1e-4."""
+    deck = make(tmp_path, n=n, grains=4, seed=23, nsteps=5, elast_bc=elast_bc)
+    o = oracle_lib.Oracle(deck, fixed_iters=5)
+    g = srx_amd.Solver(deck, fixed_iters=5, precision=precision)
+    tol = 1e-9 if precision == srx_amd.PREC_FP64 else 1e-4
+    for step in range(5):
+        o.step(), g.step()
+        compare_fields(g, o, tol, ("sig", "disgrad", "velgrad", "fluct", "tranmat"))
+    g.close()
+    o.close()
