@@ -209,7 +209,7 @@ class Solver:
 
     def field(self, name: str) -> np.ndarray:
         fid, nc = FIELDS[name]
-        out = np.zeros(self.nxyz * nc)
+        out = np.empty(self.nxyz * nc)
         rc = self.L.srx_get_field(self.h, fid, _dptr(out), out.size)
         if rc:
             raise SrxError(rc, "srx_get_field")

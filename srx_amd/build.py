@@ -15,7 +15,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # Packed-FP32 instructions are disabled for all device code.
 DEV_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-DEV_SOURCES = ["newton.hip", "increment.hip", "fft.hip", "mlp.hip", "noalloc.hip"]
+DEV_SOURCES = ["newton.hip", "increment.hip", "fft.hip", "mlp.hip", "noalloc.hip", "fields.hip"]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-fopenmp", "-Wall", "-Wno-unused-function"]
 
 

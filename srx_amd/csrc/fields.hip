@@ -1,0 +1,68 @@
+// fields.hip -- conversion of the device state to the caller's layout: fields leave the GPU as the
+// reference lays them out (per voxel, 3x3 row-major tensors or 12 values per slip system), spectra
+// as the FFT entry points return them.
+#include "kern_common.hpp"
+
+namespace srx {
+
+// One chunk of a field, voxels [v0, v0 + nv), from component-major state to nc values per voxel at
+// `out`, which srx_get_field points at pinned host memory: the kernel's stores cross PCIe directly.
+// Bound by that link; a block turns its 256 voxels around in LDS so that every wavefront's store is one
+// contiguous run of 512 B (54 GB/s measured into 2 MiB of pinned memory, against 3-4 GB/s for copying
+// the components to pageable memory and interleaving them there: the stress of 128^3, 151 MB, took
+// 57 ms).  The arithmetic is the host formulas' own, without contraction.
+constexpr int GATHER_BLOCK = 256;
+template <int MODE, int NC>
+__global__ void __launch_bounds__(GATHER_BLOCK) k_gather(FieldSrc src, int v0, int nv, double *__restrict__ out) {
+#pragma clang fp contract(off)
+    __shared__ double buf[GATHER_BLOCK * NC];
+    const int b0 = blockIdx.x * GATHER_BLOCK, cnt = min(GATHER_BLOCK, nv - b0);
+    if ((int)threadIdx.x < cnt) {
+        const size_t v = (size_t)v0 + b0 + threadIdx.x, N = src.n;
+        double *o = buf + threadIdx.x * NC;
+        if constexpr (MODE == FIELD_INT) {
+            o[0] = (double)src.i[v];
+        } else if constexpr (MODE == FIELD_B6) {
+            double b6[6];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) b6[k] = k < src.comps ? src.a[k * N + v] : 0.0;
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) s += b6[k] * bbasis(k, r, c);
+                    o[3 * r + c] = s;
+                }
+        } else {
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+                double x = src.a[k * N + v];
+                if constexpr (MODE == FIELD_RATE) x = (x - src.b[k * N + v]) / src.dt;
+                if constexpr (MODE == FIELD_FLUCT) x = (x - src.u[k]) + (src.b ? src.b[k * N + v] : 0.0);
+                o[k] = x;
+            }
+        }
+    }
+    __syncthreads();
+    double *dst = out + (size_t)b0 * NC;
+    for (int i = threadIdx.x; i < cnt * NC; i += GATHER_BLOCK) dst[i] = buf[i];
+}
+
+void launch_gather(hipStream_t s, int mode, int nc, const FieldSrc &src, int v0, int nv, double *out) {
+    const dim3 g((nv + GATHER_BLOCK - 1) / GATHER_BLOCK), b(GATHER_BLOCK);
+    switch (mode) {
+    case FIELD_INT: hipLaunchKernelGGL((k_gather<FIELD_INT, 1>), g, b, 0, s, src, v0, nv, out); break;
+    case FIELD_B6: hipLaunchKernelGGL((k_gather<FIELD_B6, 9>), g, b, 0, s, src, v0, nv, out); break;
+    case FIELD_RATE: hipLaunchKernelGGL((k_gather<FIELD_RATE, 9>), g, b, 0, s, src, v0, nv, out); break;
+    case FIELD_FLUCT: hipLaunchKernelGGL((k_gather<FIELD_FLUCT, 9>), g, b, 0, s, src, v0, nv, out); break;
+    default:
+        if (nc == 12) hipLaunchKernelGGL((k_gather<FIELD_PLAIN, 12>), g, b, 0, s, src, v0, nv, out);
+        else if (nc == 9) hipLaunchKernelGGL((k_gather<FIELD_PLAIN, 9>), g, b, 0, s, src, v0, nv, out);
+        else hipLaunchKernelGGL((k_gather<FIELD_PLAIN, 1>), g, b, 0, s, src, v0, nv, out);
+    }
+    check_launch("gather");
+}
+
+}  // namespace srx

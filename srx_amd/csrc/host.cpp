@@ -364,6 +364,10 @@ struct srx_ctx {
     float *rec_x = nullptr, *rec_t = nullptr, *rec_nd = nullptr;
     int *rec_count = nullptr;
     int rec_stride = 0, rec_cap = 0;
+    // field readback: STAGE_SLOTS pinned slots of stage_bytes each (allocated by the first srx_get_field)
+    char *stage = nullptr;
+    size_t stage_bytes = 0;
+    hipEvent_t stage_ev[4] = {nullptr, nullptr, nullptr, nullptr};
     // outer-iteration batches captured as HIP graphs: [first batch of an increment][rotated]
     hipGraphExec_t gexec[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
     bool graphs = true;
@@ -445,6 +449,27 @@ int ctx_zero(hipStream_t st, void *dst, size_t bytes) {
     HIPCK(hipMemsetAsync(dst, 0, bytes, st));
     HIPCK(hipStreamSynchronize(st));
     return 0;
+}
+
+// job(begin, end) over [0, n) in at most `threads` contiguous ranges of at least 4096, on threads that
+// end with the call: OpenMP's workers go on spinning for 200 ms after a region, next to the solver's own
+// host thread and whatever the caller runs (a float conversion on the caller's OpenMP threads took
+// 30-75 ms instead of 1 beside them).
+template <typename Job>
+void parallel_ranges(long n, int threads, Job job) {
+    const int parts = (int)std::max(1L, std::min((long)threads, n / 4096));
+    std::vector<std::thread> th;
+    long next = 0;   // ranges [0, next) run on a thread of their own
+    try {
+        for (int p = 0; p + 1 < parts; ++p) {
+            const long end = n * (p + 1) / parts;
+            th.emplace_back([&job, next, end]() { job(next, end); });
+            next = end;
+        }
+    } catch (...) {   // no more threads: the caller takes the rest
+    }
+    job(next, n);
+    for (auto &t : th) t.join();
 }
 
 int setup(srx_ctx *c) {
@@ -586,16 +611,17 @@ int setup(srx_ctx *c) {
             phase[v] = jph;
         };
         if (whole_lines) {
-#pragma omp parallel for schedule(static) num_threads(nthr)
-            for (long v = 0; v < N; ++v) {
-                char buf[80];
-                const size_t b0 = start[v];
-                size_t len = (v + 1 < (long)start.size() ? start[v + 1] : text.size()) - b0;
-                if (len > 79) len = 79;
-                std::memcpy(buf, &text[b0], len);
-                buf[len] = 0;
-                parse(buf, v);
-            }
+            parallel_ranges(N, nthr, [&](long v0, long v1) {
+                for (long v = v0; v < v1; ++v) {
+                    char buf[80];
+                    const size_t b0 = start[v];
+                    size_t len = (v + 1 < (long)start.size() ? start[v + 1] : text.size()) - b0;
+                    if (len > 79) len = 79;
+                    std::memcpy(buf, &text[b0], len);
+                    buf[len] = 0;
+                    parse(buf, v);
+                }
+            });
         } else {
             FILE *f2 = std::fopen(ms.c_str(), "r");
             if (!f2) return SRX_E_FILE;
@@ -1904,6 +1930,104 @@ int srx_kernel_times(srx_ctx *c, const char **names, double *ms, int *calls, int
     return 0;
 }
 
+// Reads a field through the context's pinned slots: the gather kernel writes chunk after chunk into them
+// in the caller's layout, and while later chunks cross the link the host copies finished ones into the
+// caller's (pageable) buffer.  Slots of 2 MiB reach the link's rate (kernel stores into 1, 2 and 8 MiB:
+// 52, 54 and 55 GB/s).  Large fields take slots of 8 MiB and helper threads for the copy: a fresh buffer's
+// 2 MiB pages are zeroed on first touch, 18 GB/s with one thread and 61 with four, and only a slot of
+// several pages lets the threads do that side by side.  The helpers live for one call (a pool of
+// OpenMP threads, which go on spinning after their region, slowed the caller's own OpenMP work
+// next to it by 30 ms).
+constexpr int STAGE_SLOTS = 4, STAGE_HELPERS = 3;
+constexpr size_t STAGE_SLOT = (size_t)2 << 20, STAGE_SLOT_MAX = (size_t)8 << 20, STAGE_MT = (size_t)8 << 20;
+
+// Copies of finished chunks by the calling thread and its helpers, each a part of every chunk.
+struct StageCopy {
+    const char *stage;
+    char *out;
+    size_t slot_bytes, chunk_bytes, total;
+    int parts = 1;
+    std::atomic<size_t> ready{0};                     // chunks whose slots hold their data
+    std::atomic<size_t> copied[STAGE_HELPERS] = {};   // chunks each helper has copied its part of
+    std::atomic<bool> stop{false};
+    std::vector<std::thread> helpers;
+
+    void part(size_t j, int p) const {
+        const size_t o = j * chunk_bytes, bytes = std::min(chunk_bytes, total - o);
+        const size_t share = (bytes / parts + 4095) & ~(size_t)4095;
+        const size_t a = std::min(bytes, p * share), b = p + 1 == parts ? bytes : std::min(bytes, a + share);
+        std::memcpy(out + o + a, stage + (j % STAGE_SLOTS) * slot_bytes + a, b - a);
+    }
+    void help(int p, size_t nchunk) {
+        for (size_t j = 0; j < nchunk; ++j) {
+            while (ready.load(std::memory_order_acquire) <= j) {
+                if (stop.load(std::memory_order_relaxed)) return;
+                std::this_thread::yield();
+            }
+            part(j, p + 1);
+            copied[p].store(j + 1, std::memory_order_release);
+        }
+    }
+    void start(int count, size_t nchunk) {
+        // the helpers read `parts` only after `ready` is first raised
+        try {
+            for (int p = 0; p < count; ++p) {
+                helpers.emplace_back([this, p, nchunk]() { help(p, nchunk); });
+                parts = p + 2;
+            }
+        } catch (...) {   // no more threads: the ones that run and the caller share the work
+        }
+    }
+    void wait(size_t chunks) const {
+        for (int p = 0; p + 1 < parts; ++p)
+            while (copied[p].load(std::memory_order_acquire) < chunks) std::this_thread::yield();
+    }
+    ~StageCopy() {
+        stop.store(true);
+        for (auto &t : helpers) t.join();
+    }
+};
+
+static int read_field(srx_ctx *c, int mode, int nc, const FieldSrc &src, double *out) {
+    const size_t row = sizeof(double) * nc, total = row * (size_t)c->nvox;
+    if (!c->stage) {
+        // sized for the largest field (12 values per voxel), whole rows of every field in a slot
+        const size_t most = sizeof(double) * 12 * (size_t)c->nvox;
+        c->stage_bytes = std::min(most, std::max(STAGE_SLOT, std::min(STAGE_SLOT_MAX, most / 16)));
+        for (int k = 0; k < STAGE_SLOTS; ++k)
+            if (!c->stage_ev[k]) HIPCK(hipEventCreateWithFlags(&c->stage_ev[k], hipEventDisableTiming));
+        HIPCK(hipHostMalloc((void **)&c->stage, STAGE_SLOTS * c->stage_bytes, hipHostMallocDefault));
+    }
+    const size_t per = c->stage_bytes / row;   // voxels per chunk
+    const size_t nchunk = ((size_t)c->nvox + per - 1) / per;
+    StageCopy cp;
+    cp.stage = c->stage;
+    cp.out = reinterpret_cast<char *>(out);
+    cp.slot_bytes = c->stage_bytes;
+    cp.chunk_bytes = per * row;
+    cp.total = total;
+    if (total >= STAGE_MT)
+        cp.start(c->opt.nthreads > 0 ? std::min(STAGE_HELPERS, c->opt.nthreads - 1) : STAGE_HELPERS, nchunk);
+    // chunk k is launched STAGE_SLOTS - 1 chunks ahead of the one being copied
+    for (size_t k = 0; k < nchunk + STAGE_SLOTS - 1; ++k) {
+        if (k < nchunk) {
+            const int slot = (int)(k % STAGE_SLOTS);
+            if (k >= STAGE_SLOTS) cp.wait(k - STAGE_SLOTS + 1);
+            const size_t v0 = k * per, nv = std::min(per, (size_t)c->nvox - v0);
+            launch_gather(c->stream, mode, nc, src, (int)v0, (int)nv,
+                          reinterpret_cast<double *>(c->stage + slot * c->stage_bytes));
+            HIPCK(hipEventRecord(c->stage_ev[slot], c->stream));
+        }
+        if (k + 1 < STAGE_SLOTS || k - (STAGE_SLOTS - 1) >= nchunk) continue;
+        const size_t j = k - (STAGE_SLOTS - 1);
+        HIPCK(hipEventSynchronize(c->stage_ev[j % STAGE_SLOTS]));
+        cp.ready.store(j + 1, std::memory_order_release);
+        cp.part(j, 0);
+    }
+    cp.wait(nchunk);
+    return 0;
+}
+
 static int field_info(int id, int &nc) {
     switch (id) {
     case SRX_F_SIG: case SRX_F_EPS: case SRX_F_EDOT: case SRX_F_DISGRAD: case SRX_F_VELGRAD: case SRX_F_TRANMAT:
@@ -1922,67 +2046,42 @@ int srx_get_field(srx_ctx *c, int id, double *out, size_t n) {
     if (field_info(id, nc)) return SRX_E_FIELD;
     const long N = c->nvox;
     if (n < (size_t)nc * N) return SRX_E_SIZE;
-    HIPCK(hipStreamSynchronize(c->stream));
-    auto fetch = [&](const void *src, size_t bytes, void *dst) -> int {
-        if (int e = ctx_copy(c->stream, dst, src, bytes, hipMemcpyDeviceToHost)) return e;
-        return 0;
-    };
-    std::vector<double> tmp;
-    int rc = 0;
-    if (id == SRX_F_SIG || id == SRX_F_EPS || id == SRX_F_EDOT) {
-        const int m = id == SRX_F_SIG ? 6 : 5;
-        const double *src = id == SRX_F_SIG ? c->f.sig : id == SRX_F_EPS ? c->f.eps : c->f.edot;
-        tmp.resize((size_t)m * N);
-        if ((rc = fetch(src, sizeof(double) * m * N, tmp.data()))) return rc;
-        for (long v = 0; v < N; ++v) {
-            double b6[6] = {0, 0, 0, 0, 0, 0};
-            for (int k = 0; k < m; ++k) b6[k] = tmp[k * N + v];
-            b6_to_t9(b6, out + 9 * v, 6);
-        }
-        return 0;
-    }
-    if (id == SRX_F_DISGRAD || id == SRX_F_TRANMAT || id == SRX_F_VELGRAD || id == SRX_F_FLUCT) {
-        tmp.resize((size_t)9 * N);
-        if ((rc = fetch(id == SRX_F_TRANMAT ? c->f.tran : c->f.dg, sizeof(double) * 9 * N, tmp.data()))) return rc;
-        std::vector<double> t0;
-        if (id == SRX_F_VELGRAD || (id == SRX_F_FLUCT && c->f.fl0)) {
-            t0.resize((size_t)9 * N);
-            if ((rc = fetch(id == SRX_F_VELGRAD ? c->f.dg0 : c->f.fl0, sizeof(double) * 9 * N, t0.data()))) return rc;
-        }
-        for (long v = 0; v < N; ++v)
-            for (int k = 0; k < 9; ++k) {
-                double x = tmp[k * N + v];
-                if (id == SRX_F_VELGRAD) x = (x - t0[k * N + v]) / c->dk.TimeStep;
-                if (id == SRX_F_FLUCT) x = (x - c->uniform[k]) + (t0.empty() ? 0.0 : t0[k * N + v]);
-                out[9 * v + k] = x;
-            }
-        return 0;
-    }
-    if (nc == 12) {
-        const double *src = id == SRX_F_RHO_S ? c->f.rho_s : id == SRX_F_RHO_M ? c->f.rho_m : id == SRX_F_RHO_F ? c->f.rho_F
-                          : id == SRX_F_RHO_P ? c->f.rho_P : id == SRX_F_GAMDOT ? c->f.gamdot
-                          : id == SRX_F_RHO_DIPOLE ? c->f.rho_dipole : id == SRX_F_RHO_FOREST ? c->f.rho_forest
-                          : id == SRX_F_RHO_INPLANE ? c->f.rho_inplane : id == SRX_F_RHO_G1 ? c->hc.rho_g1
-                          : id == SRX_F_RHO_G2 ? c->hc.rho_g2 : c->f.gam_acum;
-        if (!src) return SRX_E_FIELD;   // GND densities without the GND option
-        tmp.resize((size_t)12 * N);
-        if ((rc = fetch(src, sizeof(double) * 12 * N, tmp.data()))) return rc;
-        for (long v = 0; v < N; ++v)
-            for (int k = 0; k < 12; ++k) out[12 * v + k] = tmp[k * N + v];
-        return 0;
-    }
-    if (id == SRX_F_NR_ITERS || id == SRX_F_PHASE) {
-        std::vector<int> t(N);
-        if ((rc = fetch(id == SRX_F_NR_ITERS ? c->f.nr_it : c->f.phase, sizeof(int) * N, t.data()))) return rc;
-        for (long v = 0; v < N; ++v) out[v] = t[v];
-        return 0;
-    }
     if (id == SRX_F_GRAIN) {
         for (long v = 0; v < N; ++v) out[v] = c->grain[v];
         return 0;
     }
-    if (id == SRX_F_RHO_TOT) return fetch(c->f.rho_tot, sizeof(double) * N, out);
-    return SRX_E_FIELD;
+    FieldSrc src = {};
+    src.n = (size_t)N;
+    int mode = FIELD_PLAIN;
+    if (id == SRX_F_SIG || id == SRX_F_EPS || id == SRX_F_EDOT) {
+        mode = FIELD_B6;
+        src.comps = id == SRX_F_SIG ? 6 : 5;
+        src.a = id == SRX_F_SIG ? c->f.sig : id == SRX_F_EPS ? c->f.eps : c->f.edot;
+    } else if (id == SRX_F_NR_ITERS || id == SRX_F_PHASE) {
+        mode = FIELD_INT;
+        src.i = id == SRX_F_NR_ITERS ? c->f.nr_it : c->f.phase;
+    } else if (nc == 9) {
+        src.a = id == SRX_F_TRANMAT ? c->f.tran : c->f.dg;
+        if (id == SRX_F_VELGRAD) {
+            mode = FIELD_RATE;
+            src.b = c->f.dg0;
+            src.dt = c->dk.TimeStep;
+        } else if (id == SRX_F_FLUCT) {
+            mode = FIELD_FLUCT;
+            src.b = c->f.fl0;
+            for (int k = 0; k < 9; ++k) src.u[k] = c->uniform[k];
+        }
+    } else if (nc == 12) {
+        src.a = id == SRX_F_RHO_S ? c->f.rho_s : id == SRX_F_RHO_M ? c->f.rho_m : id == SRX_F_RHO_F ? c->f.rho_F
+              : id == SRX_F_RHO_P ? c->f.rho_P : id == SRX_F_GAMDOT ? c->f.gamdot
+              : id == SRX_F_RHO_DIPOLE ? c->f.rho_dipole : id == SRX_F_RHO_FOREST ? c->f.rho_forest
+              : id == SRX_F_RHO_INPLANE ? c->f.rho_inplane : id == SRX_F_RHO_G1 ? c->hc.rho_g1
+              : id == SRX_F_RHO_G2 ? c->hc.rho_g2 : c->f.gam_acum;
+        if (!src.a) return SRX_E_FIELD;   // GND densities without the GND option
+    } else {
+        src.a = c->f.rho_tot;
+    }
+    return read_field(c, mode, nc, src, out);
 }
 
 int srx_set_field(srx_ctx *c, int id, const double *in, size_t n) {
@@ -2074,6 +2173,9 @@ void srx_close(srx_ctx *c) {
     if (c->hred) (void)hipHostFree(c->hred);
     if (c->dctl) (void)hipFree(c->dctl);
     if (c->hctl) (void)hipHostFree(c->hctl);
+    if (c->stage) (void)hipHostFree(c->stage);
+    for (hipEvent_t e : c->stage_ev)
+        if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->evpool) (void)hipEventDestroy(e);
     drop_graphs(c);
     if (c->stream) (void)hipStreamDestroy(c->stream);

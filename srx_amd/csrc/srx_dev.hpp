@@ -375,8 +375,18 @@ int nr_block_count(int nvox);
 // accesses in flight per lane, `blocks` blocks of 256 threads, grid-stride.
 void launch_stream_copy(hipStream_t s, const void *in, void *out, size_t n16, int unroll, int blocks);
 int end_block_count(int nvox);
-// Field conversion helpers used by srx_get_field (device -> AoS tensor on device scratch)
-void launch_b6_to_tensor(hipStream_t s, const double *v, int ncomp, int nvox, double *out9);
+// Field readback (fields.hip): what srx_get_field returns, in chunks of voxels, from the component-major
+// state: FIELD_PLAIN the components themselves, FIELD_B6 the tensor of `comps` B-basis components,
+// FIELD_RATE (a - b) / dt, FIELD_FLUCT (a - u) + b (b may be null), FIELD_INT an int field as doubles.
+enum { FIELD_PLAIN, FIELD_B6, FIELD_RATE, FIELD_FLUCT, FIELD_INT };
+struct FieldSrc {
+    const double *a, *b;
+    const int *i;
+    size_t n;        // voxels: the component pitch
+    int comps;
+    double dt, u[9];
+};
+void launch_gather(hipStream_t s, int mode, int nc, const FieldSrc &src, int v0, int nv, double *out);
 void launch_fft_real_forward_test(hipStream_t s, int prec, const double *in, int ncomp, void *specB, void *specC,
                                   const int n[3], const FftPlan *pl, void *const *tw);
 
