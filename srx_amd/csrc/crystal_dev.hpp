@@ -53,6 +53,33 @@ __device__ __forceinline__ void q5_from(const double a[9], double Q[5][5]) {
 #undef SRX_OUTER
 }
 
+// Unit quaternion (x, y, z, w) of a rotation matrix, from its largest component (Shepperd 1978), and the
+// matrix of one: 4 values instead of 9, both ways accurate to rounding for orthogonal matrices.
+__device__ __forceinline__ void quat_from_rot(const double a[9], double q[4]) {
+    const double t = a[0] + a[4] + a[8];
+    const double d[4] = {1.0 + 2.0 * a[0] - t, 1.0 + 2.0 * a[4] - t, 1.0 + 2.0 * a[8] - t, 1.0 + t};   // 4 x^2 .. 4 w^2
+    const double yz = a[5] + a[7], xz = a[2] + a[6], xy = a[1] + a[3];
+    const double wx = a[7] - a[5], wy = a[2] - a[6], wz = a[3] - a[1];
+    int k = 0;
+#pragma unroll
+    for (int i = 1; i < 4; ++i)
+        if (d[i] > d[k == 0 ? 0 : k == 1 ? 1 : 2]) k = i;
+    const double big = k == 0 ? d[0] : k == 1 ? d[1] : k == 2 ? d[2] : d[3];
+    const double r = 0.5 / sqrt(big);
+    q[0] = r * (k == 0 ? big : k == 1 ? xy : k == 2 ? xz : wx);
+    q[1] = r * (k == 0 ? xy : k == 1 ? big : k == 2 ? yz : wy);
+    q[2] = r * (k == 0 ? xz : k == 1 ? yz : k == 2 ? big : wz);
+    q[3] = r * (k == 0 ? wx : k == 1 ? wy : k == 2 ? wz : big);
+}
+__device__ __forceinline__ void rot_from_quat(const double q[4], double a[9]) {
+    const double x2 = 2.0 * q[0], y2 = 2.0 * q[1], z2 = 2.0 * q[2];
+    const double xx = x2 * q[0], yy = y2 * q[1], zz = z2 * q[2], xy = x2 * q[1], xz = x2 * q[2], yz = y2 * q[2];
+    const double wx = x2 * q[3], wy = y2 * q[3], wz = z2 * q[3];
+    a[0] = 1.0 - (yy + zz); a[1] = xy - wz; a[2] = xz + wy;
+    a[3] = xy + wz; a[4] = 1.0 - (xx + zz); a[5] = yz - wx;
+    a[6] = xz - wy; a[7] = yz + wx; a[8] = 1.0 - (xx + yy);
+}
+
 // sample-frame stress (B basis) -> crystal frame of a: deviatoric part Q^T lam, hydrostatic unchanged
 __device__ __forceinline__ void crystal_stress(const double a[9], const double lam6[6], double lamc[6]) {
     double Q[5][5];

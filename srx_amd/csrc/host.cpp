@@ -331,6 +331,7 @@ struct srx_ctx {
     DevConst *dc = nullptr;
     Fields f;
     void *specB = nullptr, *specC = nullptr;
+    double *quat = nullptr;                     // Fields::quat's memory (also while f.quat is null)
     void *nyq = nullptr;                        // rotation sums of the Nyquist planes (nyq_elems complex doubles)
     void *tw[3] = {nullptr, nullptr, nullptr};
     FftPlan pl[3];
@@ -706,15 +707,16 @@ int setup(srx_ctx *c) {
     if ((rc = dalloc(&F.sig, 6, 0.0)) || (rc = dalloc(&F.sig_pre, 5, 0.0)) || (rc = dalloc(&F.eps, 5, 0.0)) ||
         (rc = dalloc(&F.edot, 5, 0.0)) || (strain_form(c->n, c->opt.precision) && (rc = dalloc(&F.ee, 6, 0.0))) ||
         (rc = dalloc(&F.dg, 9, 0.0)) || (rc = dalloc(&F.dg0, 9, 0.0)) ||
-        (rc = dalloc(&F.tran, 9, 0.0)) || (rc = dalloc(&F.tran0, 9, 0.0)) ||
+        (rc = dalloc(&F.tran, 9, 0.0)) || (rc = dalloc(&c->quat, 4, 0.0)) || (rc = dalloc(&F.tran0, 9, 0.0)) ||
         (rc = dalloc(&F.rho_s, 12, d.rho_SSD_initial)) || (rc = dalloc(&F.rho_m, 12, 0.0)) ||
         (rc = dalloc(&F.rho_m_old, 12, 0.0)) || (rc = dalloc(&F.rho_F, 12, 0.0)) || (rc = dalloc(&F.rho_P, 12, 0.0)) ||
         (rc = dalloc(&F.gamdot, 12, 0.0)) || (rc = dalloc(&F.gam_acum, 12, 0.0)) ||
         (rc = dalloc(&F.rho_dipole, 12, 0.0)) || (rc = dalloc(&F.rho_forest, 12, 0.0)) ||
         (rc = dalloc(&F.rho_inplane, 12, 0.0)) || (rc = dalloc(&F.rho_tot, 1, 0.0)) ||
-        (rc = dalloc(&F.acr, 15, 0.0)) ||
+        (rc = dalloc(&F.acr, N < 4 ? 60 : 15, 0.0)) ||   // 15 nrcf_pitch(N) floats must fit too
         (c->creep == 1 && (rc = dalloc(&F.fl0, 9, 0.0))))
         return rc;
+    F.quat = c->quat;
     F.acrf = c->opt.precision == SRX_PREC_MIXED ? reinterpret_cast<float *>(F.acr) : nullptr;
     if (c->opt.gnd) {
         // GND densities start at zero (init.c:1077-1087); same-grain flags of Gradient_ExchangeGrainID
@@ -1695,8 +1697,11 @@ static int run_lockstep(const std::vector<int> &members, std::vector<srx_ctx *> 
             break;
         launch_prologue_ens(S, dinc, nact, pb);
         const srx_options &o = ctx[act[0]]->opt;
-        int ph2 = 0;
-        for (int k : act) ph2 |= ctx[k]->hc.ph[1].xtal;
+        int ph2 = 0, f32 = 1;
+        for (int k : act) {
+            ph2 |= ctx[k]->hc.ph[1].xtal;
+            f32 = f32 && ctx[k]->f.nrcf && ctx[k]->f.quat;
+        }
         int launched = 0;
         bool all_done = false;
         while (!all_done && !rc) {
@@ -1718,7 +1723,7 @@ static int run_lockstep(const std::vector<int> &members, std::vector<srx_ctx *> 
                                             (double)c->nvox, tl[4]);
                 }
                 for (int q = 0; q < NS; ++q) ok(hipEventRecord(ev[q], side[q])) && ok(hipStreamWaitEvent(S, ev[q], 0));
-                launch_nr_ens(S, dtab, nact, nb, launched == 1, rotated, o.warm_start, o.gnd, ph2);
+                launch_nr_ens(S, dtab, nact, nb, launched == 1, rotated, o.warm_start, o.gnd, ph2, f32);
                 launch_reduce_nr_ens(S, dtab, nact);
                 launch_control_ens(S, dtab, nact, ddone);
             }
@@ -2084,6 +2089,35 @@ int srx_get_field(srx_ctx *c, int id, double *out, size_t n) {
     return read_field(c, mode, nc, src, out);
 }
 
+static void drop_graphs(srx_ctx *c);
+// After the caller has set the orientations: the Newton kernel keeps their quaternions where every
+// crystalline voxel's matrix is a rotation to 1e-12 (the quaternion's matrix then equals it to that),
+// and reads the matrices themselves otherwise.
+static int choose_quat(srx_ctx *c, const double *tran) {
+    const long N = c->nvox;
+    std::vector<int> phase(N);
+    if (int e = ctx_copy(c->stream, phase.data(), c->f.phase, sizeof(int) * N, hipMemcpyDeviceToHost)) return e;
+    bool ok = true;
+    for (long v = 0; v < N && ok; ++v) {
+        if (phase[v] < 1 || phase[v] > NPH || !c->ph[phase[v] - 1].xtal) continue;
+        const double *a = tran + 9 * v;
+        for (int i = 0; i < 3; ++i)
+            for (int j = i; j < 3; ++j) {
+                const double d = a[i] * a[j] + a[3 + i] * a[3 + j] + a[6 + i] * a[6 + j] - (double)(i == j);
+                ok = ok && std::fabs(d) <= 1e-12;   // false for NaN
+            }
+        const double det = a[0] * (a[4] * a[8] - a[5] * a[7]) - a[1] * (a[3] * a[8] - a[5] * a[6]) +
+                           a[2] * (a[3] * a[7] - a[4] * a[6]);
+        ok = ok && det > 0.0;
+    }
+    double *q = ok ? c->quat : nullptr;
+    if (q != c->f.quat) {
+        c->f.quat = q;
+        drop_graphs(c);   // captured batches hold the previous kernel arguments
+    }
+    return 0;
+}
+
 int srx_set_field(srx_ctx *c, int id, const double *in, size_t n) {
     if (!c || !in) return SRX_E_ARG;
     int nc = 0;
@@ -2119,6 +2153,7 @@ int srx_set_field(srx_ctx *c, int id, const double *in, size_t n) {
         if (int e = ctx_copy(c->stream, id == SRX_F_DISGRAD ? c->f.dg : c->f.tran, tmp.data(), sizeof(double) * 9 * N,
                              hipMemcpyHostToDevice))
             return e;
+        if (id == SRX_F_TRANMAT) return choose_quat(c, in);
         return 0;
     }
     if (id == SRX_F_RHO_S || id == SRX_F_RHO_M || id == SRX_F_GAM_ACUM) {
@@ -2151,7 +2186,7 @@ void srx_close(srx_ctx *c) {
     double *ptrs[] = {c->f.sig, c->f.sig_pre, c->f.eps, c->f.edot, c->f.ee, c->f.dg, c->f.dg0, c->f.tran, c->f.tran0,
                       c->f.rho_s, c->f.rho_m, c->f.rho_m_old, c->f.rho_F, c->f.rho_P, c->f.gamdot, c->f.gam_acum,
                       c->f.rho_dipole, c->f.rho_forest, c->f.rho_inplane, c->f.rho_tot, c->f.fl0, c->f.acr, c->f.nrc,
-                      c->hc.rho_g1, c->hc.rho_g2, c->hc.gnd_fp,
+                      c->quat, c->hc.rho_g1, c->hc.rho_g2, c->hc.gnd_fp,
                       c->partials, c->red, c->redseg};
     for (double *p : ptrs)
         if (p) (void)hipFree(p);

@@ -87,13 +87,21 @@ __device__ __forceinline__ void load_strain(const Fields &f, size_t N, unsigned 
 // LDS slots of the per-system constants (tau_pass * inv, inv, gamma_0 dt of 12 systems), also the
 // component order of Fields::nrc
 constexpr int NRC_TP = 0, NRC_INV = NSYS, NRC_G0 = 2 * NSYS, NRC_COMPS = 3 * NSYS;
+// after them, the orientation quaternion of the block's voxels: 40 slots of 64 doubles, 20 KB, are
+// exactly an eighth of a compute unit's LDS
+constexpr int NRC_QUAT = NRC_COMPS;
+// The later calls of mixed precision keep their FP32 constants and 14 of the 15 values of A as FP32
+// (widened at each use): 12.5 KB, a twelfth of a compute unit's LDS, so that three wavefronts per
+// SIMD fit where the FP64 layout allows two.
+constexpr int NRF_A = NRC_COMPS, NRF_A_COMPS = 14, NRF_SLOTS = NRC_COMPS + NRF_A_COMPS;
+typedef float __attribute__((may_alias)) float_alias;
 
 // Per-voxel values every Newton call of an increment starts from, in the crystal frame of the
-// current orientation: lam' = Q^T lam, q' = Q^T (eps_p - eps_c), the matrix A = Sc + S' (packed),
-// r0 = q' - Sc lam' (= Q^T (eps_p - eps_c - S066 lam), Q being orthogonal), the hydrostatic parts
-// and 1/||lam||^2.
+// current orientation: lam' = Q^T lam, the matrix A = Sc + S' (packed), r0 = Q^T (eps_p - eps_c -
+// S066 lam) (= Q^T (eps_p - eps_c) - Sc lam', Q being orthogonal), the hydrostatic parts and
+// 1/||lam||^2.
 struct NrPro {
-    double lam[5], q[5], r0[5], A[15];
+    double lam[5], r0[5], A[15];
     double lamh, qh, rsig2;
 };
 // An empty statement that takes x in a register: x is computed before it, and the statement stays
@@ -111,26 +119,44 @@ __device__ __forceinline__ T *fresh(T *p) {
 // them (the compiler would otherwise sink the arithmetic to its first use).
 __device__ __forceinline__ void pin_prologue(NrPro &p) {
 #pragma unroll
-    for (int i = 0; i < 5; ++i) { pin(p.lam[i]); pin(p.q[i]); pin(p.r0[i]); }
+    for (int i = 0; i < 5; ++i) { pin(p.lam[i]); pin(p.r0[i]); }
     pin(p.lamh); pin(p.qh); pin(p.rsig2);
 }
 
-// The inputs of a Newton call for one voxel: orientation (TranMat), stress, the strain
-// eps_c - eps_p and, after the first call of an increment, the increment's matrix A (packed).
+// The inputs of a Newton call for one voxel: orientation, stress, the strain eps_c - eps_p and,
+// after the first call of an increment, the increment's matrix A (packed).  The orientation is TranMat
+// for the first call, and for the later ones its quaternion (in a[0..3] until nr_orient expands it)
+// where the context keeps one: 32 B instead of 72, and the epilogue takes it from LDS instead of
+// reading TranMat again, 112 of 545 B per voxel and launch in mixed precision.
 struct NrIn {
     double a[9], lam6[6], e[6], A[15];
 };
-template <bool LOAD_A>
+__device__ __forceinline__ void nr_orient(const Fields &f, NrIn &in) {
+    if (f.quat) {
+        const double q[4] = {in.a[0], in.a[1], in.a[2], in.a[3]};
+        rot_from_quat(q, in.a);
+    }
+}
+template <bool LOAD_A, bool F32>
 __device__ __forceinline__ void nr_load(const Fields &f, size_t N, unsigned o8, NrIn &in) {
+    if (LOAD_A && f.quat) {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) in.a[k] = ldc(f.tran + (size_t)k * N, N, o8);
+        for (int k = 0; k < 4; ++k) in.a[k] = ldc(f.quat + (size_t)k * N, N, o8);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) in.a[k] = ldc(f.tran + (size_t)k * N, N, o8);
+    }
 #pragma unroll
     for (int k = 0; k < 6; ++k) in.lam6[k] = ldc(f.sig + (size_t)k * N, N, o8);
     load_strain(f, N, o8, in.e);
     if (LOAD_A) {
-        if (f.acrf) {
+        const size_t P = nrcf_pitch(N);
+        if (F32) {
 #pragma unroll
-            for (int k = 0; k < 15; ++k) in.A[k] = (double)ldcf(f.acrf + (size_t)k * N, N, o8 / 2);
+            for (int k = NRF_A_COMPS; k < 15; ++k) in.A[k] = (double)ldcf(f.acrf + (size_t)k * P, P, o8 / 2);
+        } else if (f.acrf) {
+#pragma unroll
+            for (int k = 0; k < 15; ++k) in.A[k] = (double)ldcf(f.acrf + (size_t)k * P, P, o8 / 2);
         } else {
 #pragma unroll
             for (int k = 0; k < 15; ++k) in.A[k] = ldc(f.acr + (size_t)k * N, N, o8);
@@ -145,14 +171,14 @@ __device__ __forceinline__ void nr_load(const Fields &f, size_t N, unsigned o8, 
 // for the increment's later calls.  Otherwise A is in.A.
 // KEEP_EC (warm starts): the strain is also stored in f.ecp where `store` is set, for the next
 // call's learned-start features.
-template <bool FIRST, bool ROT, int PH, bool KEEP_EC>
+template <bool FIRST, bool ROT, int PH, bool KEEP_EC, bool F32>
 __device__ __forceinline__ void nr_prologue(const DevConst *__restrict__ cst, const Fields &f, int v, size_t N,
                                             const NrIn &in, NrPro &pro, bool store = true) {
     const DevPhase &P = cst->ph[PH];
     const unsigned o8 = 8u * (unsigned)v;
     if (!FIRST) {
 #pragma unroll
-        for (int k = 0; k < 15; ++k) pro.A[k] = in.A[k];
+        for (int k = F32 ? NRF_A_COMPS : 0; k < 15; ++k) pro.A[k] = in.A[k];
     }
     const double *a = in.a;
     double Q[5][5];
@@ -183,19 +209,17 @@ __device__ __forceinline__ void nr_prologue(const DevConst *__restrict__ cst, co
         for (int k = 0; k < 5; ++k) acc += cst->S066[i][k] * lam6[k];
         u[i] = acc;
     }
-    // crystal frame: lam' = Q^T lam, q' = Q^T w, r0 = q' - Q^T u
+    // crystal frame: lam' = Q^T lam, r0 = Q^T (w - u)
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
-        double al = 0.0, aq = 0.0, au = 0.0;
+        double al = 0.0, ar = 0.0;
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
             al += Q[k][i] * lam6[k];
-            aq += Q[k][i] * w[k];
-            au += Q[k][i] * u[k];
+            ar += Q[k][i] * (w[k] - u[k]);
         }
         pro.lam[i] = al;
-        pro.q[i] = aq;
-        pro.r0[i] = aq - au;
+        pro.r0[i] = ar;
     }
     if (FIRST) {
         sc_rotate(&cst->S066[0][0], Q, pro.A);
@@ -215,7 +239,7 @@ __device__ __forceinline__ void nr_prologue(const DevConst *__restrict__ cst, co
             for (int k = 0; k < 15; ++k) {
                 const float a32 = (float)pro.A[k];
                 pro.A[k] = (double)a32;
-                stcf(f.acrf + (size_t)(k) * N, N, 4u * (unsigned)v, a32);
+                stcf(f.acrf + (size_t)(k) * nrcf_pitch(N), nrcf_pitch(N), 4u * (unsigned)v, a32);
             }
         } else {
 #pragma unroll
@@ -228,7 +252,8 @@ __device__ __forceinline__ void nr_prologue(const DevConst *__restrict__ cst, co
 // 2 = lam + the learned prediction `wsp` (crystal frame).  FIRST: the call computes its prologue
 // and per-system constants and stores them for the increment; otherwise the caller has put the
 // prologue in `pro` and the constants in the LDS slots NRC_*.
-template <bool FIRST, bool ROT, int PH, int WS, bool GND>
+// F32: the FP32 LDS layout (later calls of mixed precision).
+template <bool FIRST, bool ROT, int PH, int WS, bool GND, bool F32>
 __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const Fields &f, int v, size_t N,
                                          double *lds, NrPro &pro, const float *wsp, NrResult &res) {
     // compile-time phase index: every material constant is a scalar load at a fixed offset
@@ -237,11 +262,19 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
     const unsigned o8 = 8u * (unsigned)v;
     if (FIRST) {
         NrIn in;
-        nr_load<false>(f, N, o8, in);
-        nr_prologue<true, ROT, PH, (WS != 0)>(cst, f, v, N, in, pro);
+        nr_load<false, false>(f, N, o8, in);
+        nr_prologue<true, ROT, PH, (WS != 0), false>(cst, f, v, N, in, pro);
+        if (f.quat) {
+            double q[4];
+            quat_from_rot(in.a, q);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                stc(f.quat + (size_t)k * N, N, o8, q[k]);
+                lds[(NRC_QUAT + k) * NR_BLOCK + threadIdx.x] = q[k];
+            }
+        }
     }
     double (&lam)[5] = pro.lam;
-    double (&q)[5] = pro.q;
     double (&A)[15] = pro.A;
     double (&r0)[5] = pro.r0;
     const double lamh = pro.lamh, qh = pro.qh, rsig2 = pro.rsig2;
@@ -259,6 +292,10 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
     // increment's from f.nrc (this lane's own stores).
     double *tp = lds + NRC_TP * NR_BLOCK + threadIdx.x, *inv = lds + NRC_INV * NR_BLOCK + threadIdx.x;
     double *g0 = lds + NRC_G0 * NR_BLOCK + threadIdx.x;
+    const float_alias *ldf = reinterpret_cast<const float_alias *>(lds) + threadIdx.x;
+    // value of LDS slot `slot` of this lane, and of A
+    auto slot = [&](int k) { return F32 ? (double)ldf[k * NR_BLOCK] : lds[k * NR_BLOCK + threadIdx.x]; };
+    auto Aat = [&](int k) { return F32 && k < NRF_A_COMPS ? (double)ldf[(NRF_A + k) * NR_BLOCK] : A[k]; };
     // mixed precision: the constants are stored in FP32 (f.nrcf), and this call iterates with the
     // rounded values too, so that every call of the increment solves with the same constants
     const size_t fpitch = nrcf_pitch(N);
@@ -317,9 +354,9 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
         for (int i = 0; i < 5; ++i) ws[i] = (double)wsp[i];
         wsh = (double)wsp[5];
     }
-    double sg[5], sh = lamh + wsh, pre[5], preh = sh, ed[5];   // ed: edot dt of the iterate
+    double sg[5], sh = lamh + wsh, pre[5], preh = sh, R[5];   // R: residual of the iterate `pre`
 #pragma unroll
-    for (int i = 0; i < 5; ++i) { sg[i] = lam[i] + ws[i]; pre[i] = sg[i]; ed[i] = 0.0; }
+    for (int i = 0; i < 5; ++i) { sg[i] = lam[i] + ws[i]; pre[i] = sg[i]; R[i] = 0.0; }
     int it = 0, itot = 0;
     // stopping rule ||d sig|| / ||lam|| <= 1e-10, compared squared (no square root per iteration)
     double err2 = 1E-18;
@@ -340,11 +377,17 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
     while (it < 500 && err2 > 1E-20) {
         ++it;
         ++itot;
+        // K = A and R = r0 + A sg, to which the slip systems add
         double K[15];
 #pragma unroll
-        for (int k = 0; k < 15; ++k) K[k] = A[k];
+        for (int k = 0; k < 15; ++k) K[k] = Aat(k);
 #pragma unroll
-        for (int k = 0; k < 5; ++k) ed[k] = 0.0;
+        for (int i = 0; i < 5; ++i) {
+            double acc = r0[i];
+#pragma unroll
+            for (int j = 0; j < 5; ++j) acc += K[ps(i, j)] * sg[j];
+            R[i] = acc;
+        }
         if (FIRST && it == 2) {
             if (f.nrcf) {
                 const float *nc = fresh(f.nrcf);
@@ -358,7 +401,6 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
                     tp[s * NR_BLOCK] = ldc(nc + (size_t)(NRC_TP + s) * nrc_pitch(N), nrc_pitch(N), o8);
             }
         }
-        const double *tpu = tp;
         // SRX_NR_GROUP systems per trip, under one wavefront-uniform branch: their slip-rate
         // evaluations are independent dependency chains the scheduler interleaves (an inactive
         // system of the group evaluates at 0 and adds exact zeros)
@@ -372,34 +414,26 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
             for (int u = 0; u < NG; ++u) {
                 const double *p = P.p[s0 + u];
                 rss[u] = p[0] * sg[0] + p[1] * sg[1] + p[2] * sg[2] + p[3] * sg[3] + p[4] * sg[4];
-                ivs[u] = inv[(s0 + u) * NR_BLOCK];
-                e[u] = fma(fabs(rss[u]), ivs[u], -tpu[(s0 + u) * NR_BLOCK]);
+                ivs[u] = slot(NRC_INV + s0 + u);
+                e[u] = fma(fabs(rss[u]), ivs[u], -slot(NRC_TP + s0 + u));
                 act |= e[u] > 0.0;
             }
             if (__any(act)) {
                 double g[NG], g2dt[NG];
 #pragma unroll
-                for (int u = 0; u < NG; ++u) slip_rate(rss[u], e[u], ivs[u], g0[(s0 + u) * NR_BLOCK], g[u], g2dt[u]);
+                for (int u = 0; u < NG; ++u) slip_rate(rss[u], e[u], ivs[u], slot(NRC_G0 + s0 + u), g[u], g2dt[u]);
 #pragma unroll
                 for (int u = 0; u < NG; ++u) {
                     const double *p = P.p[s0 + u];
 #pragma unroll
                     for (int i = 0; i < 5; ++i) {
-                        ed[i] += p[i] * g[u];
+                        R[i] += p[i] * g[u];
                         const double gp = g2dt[u] * p[i];
 #pragma unroll
                         for (int j = i; j < 5; ++j) K[ps(i, j)] += gp * p[j];
                     }
                 }
             }
-        }
-        double R[5];
-#pragma unroll
-        for (int i = 0; i < 5; ++i) {
-            double acc = r0[i] + ed[i];
-#pragma unroll
-            for (int j = 0; j < 5; ++j) acc += A[ps(i, j)] * sg[j];
-            R[i] = acc;
         }
         // LDL^T in place: K[ps(j,j)] <- 1/D_j, K[ps(i,j)] <- L_ij (i > j)
 #pragma unroll
@@ -452,70 +486,62 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
         for (int i = 0; i < 5; ++i) stcf(f.dsig + (size_t)i * N, N, 4u * (unsigned)v, (float)(sg[i] - lam[i]));
         stcf(f.dsig + 5 * N, N, 4u * (unsigned)v, (float)(sh - lamh));
     }
-    // errors of evolution.c:381-391 (rotation invariant)
-    double cs2 = (sh - lamh) * (sh - lamh);
-#pragma unroll
-    for (int i = 0; i < 5; ++i) cs2 += (sg[i] - lam[i]) * (sg[i] - lam[i]);
-    res.cs = sqrt(cs2);
+    // errors of evolution.c:381-391 and the stress back in the sample frame.  The strain error at the
+    // pre-update iterate, eps_p + edot dt + S' pre - eps_c, is R - Sc (pre - lam') (R the residual there),
+    // in the sample frame Q R - S066 (Q pre - lam).  The orientation comes back from LDS, or from memory
+    // where it does not fit beside the FP32 layout's three wavefronts (the registers that held it were
+    // released for the Newton loop); so does lam.
     {
-        // the orientation again (the registers that held it were released for the Newton loop and
-        // the LDS holds the per-system constants)
-        double a[9];
-        const double *tr = fresh(f.tran);
+        double a[9], qu[4];
+        if (f.quat) {
+            const double *qp = fresh(f.quat);
 #pragma unroll
-        for (int k = 0; k < 9; ++k) a[k] = ldc(tr + (size_t)(k) * N, N, o8);
+            for (int k = 0; k < 4; ++k)
+                qu[k] = F32 ? ldc(qp + (size_t)k * N, N, o8) : lds[(NRC_QUAT + k) * NR_BLOCK + threadIdx.x];
+        }
+        double l5[5];
+        if (F32) {
+            const double *sp = fresh(f.sig);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) l5[k] = ldc(sp + (size_t)k * N, N, o8);
+        }
+        if (f.quat) {
+            rot_from_quat(qu, a);
+        } else {
+            const double *tr = fresh(f.tran);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) a[k] = ldc(tr + (size_t)(k) * N, N, o8);
+        }
         double Q[5][5];
         q5_from(a, Q);
-        // eps_tot - eps_c at the pre-update iterate: q + edot dt + S' pre.  With the texture
-        // rotating, S' pre = A pre - Sc pre (A = Sc + S' is still in registers, Sc = Q^T S066 Q), so
-        // the initial orientation S' was built from is not read again.
-        double spp[5];
-        if (ROT) {
-            double u[5], w[5];
+        double d[5], e[5], cs2 = (sh - lamh) * (sh - lamh);
 #pragma unroll
-            for (int i = 0; i < 5; ++i) {
-                double acc = 0.0;
+        for (int i = 0; i < 5; ++i) {
+            double as = 0.0, ad = 0.0, ar = 0.0;
 #pragma unroll
-                for (int k = 0; k < 5; ++k) acc += Q[i][k] * pre[k];
-                u[i] = acc;
+            for (int k = 0; k < 5; ++k) {
+                as += Q[i][k] * sg[k];
+                ad += Q[i][k] * (F32 ? pre[k] : pre[k] - lam[k]);
+                ar += Q[i][k] * R[k];
             }
-#pragma unroll
-            for (int i = 0; i < 5; ++i) {
-                double acc = 0.0;
-#pragma unroll
-                for (int k = 0; k < 5; ++k) acc += cst->S066[i][k] * u[k];
-                w[i] = acc;
-            }
-#pragma unroll
-            for (int i = 0; i < 5; ++i) {
-                double acc = 0.0;
-#pragma unroll
-                for (int j = 0; j < 5; ++j) acc += A[ps(i, j)] * pre[j];
-#pragma unroll
-                for (int k = 0; k < 5; ++k) acc -= Q[k][i] * w[k];
-                spp[i] = acc;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 5; ++i) spp[i] = P.sinv[i] * pre[i];
+            res.sig[i] = as;
+            d[i] = F32 ? ad - l5[i] : ad;
+            e[i] = ar;
+            const double ds = F32 ? as - l5[i] : sg[i] - lam[i];
+            cs2 += ds * ds;
         }
+        res.cs = sqrt(cs2);
         double ce2 = 0.0;
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
-            const double acc = q[i] + ed[i] + spp[i];
+            double acc = e[i];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) acc -= cst->S066[i][k] * d[k];
             ce2 += acc * acc;
         }
         const double eh = qh + P.sinv[5] * preh;
         ce2 += eh * eh;
         res.ce = sqrt(ce2);
-        // stress back to the sample frame
-#pragma unroll
-        for (int i = 0; i < 5; ++i) {
-            double acc = 0.0;
-#pragma unroll
-            for (int k = 0; k < 5; ++k) acc += Q[i][k] * sg[k];
-            res.sig[i] = acc;
-        }
     }
     res.sig[5] = sh;
 #pragma unroll
@@ -534,6 +560,9 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
 // fit two without spills.
 #ifndef SRX_NR_WAVES_PER_EU
 #define SRX_NR_WAVES_PER_EU 2
+#endif
+#ifndef SRX_NR_F32_WAVES_PER_EU
+#define SRX_NR_F32_WAVES_PER_EU 3
 #endif
 #ifndef SRX_NR_FIRST_WAVES_PER_EU
 #define SRX_NR_FIRST_WAVES_PER_EU 2
@@ -566,29 +595,29 @@ __device__ __forceinline__ void copy_field(const double *base, size_t P, double 
 }
 // The same for constants stored in FP32 at pitch P (a multiple of 4): one 16-byte load per lane moves
 // four components (lanes 16 q .. 16 q + 15 component c + q, four voxels each) into the upper half of
-// the NC FP64 slots: FP32 slot k at float offset (NC + k) 64 from their start (NC a multiple of 4);
-// widen_slots then converts them in place.
-template <int NC>
+// the NC FP64 slots: FP32 slot k at float offset (NC + k) 64 from their start; widen_slots then
+// converts them in place.  (The FP32 layout copies to its own first slot SLOT0 and does not widen.)
+template <int NC, int SLOT0 = NC>
 __device__ __forceinline__ void copy_field_f32(const float *base, size_t P, double *lds, int blk) {
-    static_assert(NC % 4 == 0, "four components per load");
 #if __HIP_DEVICE_COMPILE__
     const int lane = threadIdx.x;
     const int v0 = blk * NR_BLOCK;
     const unsigned pb = 4u * (unsigned)min((size_t)(v0 + 4 * (lane & 15)), P - 4);
     const unsigned q = 4u * (unsigned)P * (unsigned)(lane >> 4);
-    float *half = reinterpret_cast<float *>(lds + NC / 2 * NR_BLOCK);
+    float *half = reinterpret_cast<float *>(lds) + SLOT0 * NR_BLOCK;
 #pragma unroll
-    for (int c = 0; c < NC; c += 4)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base + (size_t)c * P), (short)0,
-                                              rsrc_bytes(4 * P * 4u), 0x00020000),
-            (lds_void *)(half + c * NR_BLOCK), 16, pb + q, 0, 0, 0);
+    for (int c = 0; c < NC; c += 4) {
+        if (c + 4 <= NC || lane < (NC - c) * 16)   // a remainder of components: their lanes only
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base + (size_t)c * P), (short)0,
+                                                  rsrc_bytes((NC - c < 4 ? NC - c : 4) * P * 4u), 0x00020000),
+                (lds_void *)(half + c * NR_BLOCK), 16, pb + q, 0, 0, 0);
+    }
 #endif
 }
 // After copy_field_f32 and copy_wait: FP32 slot k -> FP64 slot k of the lane's voxel.  Every FP32
 // value of the lane is read before the first FP64 slot is written (the FP64 slots overlay the FP32
 // ones; a block is one wavefront, whose LDS accesses complete in program order).
-typedef float __attribute__((may_alias)) float_alias;
 template <int NC>
 __device__ __forceinline__ void widen_slots(double *lds) {
     static_assert(NR_BLOCK == 64, "one wavefront per block");
@@ -645,7 +674,7 @@ __device__ __forceinline__ void nr_learned_start(const DevConst *__restrict__ cs
 // One 64-voxel block of the Newton kernel: block `blk` of the `nblk` blocks of a grid of nvox
 // voxels (partials: NR_NPART x nblk block partial sums).
 // PH2: the second phase is crystalline (else its voxels are gas and its Newton path is not compiled).
-template <bool FIRST, bool ROT, int WS, bool GND, bool PH2>
+template <bool FIRST, bool ROT, int WS, bool GND, bool PH2, bool F32>
 __device__ __forceinline__ void nr_block(const DevConst *__restrict__ cst, const Fields &f, int nvox,
                                          double *__restrict__ partials, const IterCtl *__restrict__ ctl, int blk,
                                          int nblk) {
@@ -654,9 +683,10 @@ __device__ __forceinline__ void nr_block(const DevConst *__restrict__ cst, const
     const size_t N = (size_t)nvox;
     const bool valid = v < nvox;
     const int ph = valid ? f.phase[v] : 0;
-    // LDS: the 36 per-system constants of the block's 64 voxels (18 KB); the first call of an
-    // increment computes them here, the later ones copy them from f.nrc.
-    constexpr int NSLOT = NRC_COMPS;
+    // LDS: the 36 per-system constants of the block's 64 voxels (18 KB; the first call of an
+    // increment computes them here, the later ones copy them from f.nrc) and the orientation.
+    static_assert(!(F32 && FIRST), "the first call computes its constants in the FP64 layout");
+    constexpr int NSLOT = F32 ? NRF_SLOTS / 2 : NRC_COMPS + 4;
     __shared__ __align__(16) double lds[NSLOT * NR_BLOCK];
     NrPro pro;
     float wsp[6] = {0, 0, 0, 0, 0, 0};
@@ -668,22 +698,36 @@ __device__ __forceinline__ void nr_block(const DevConst *__restrict__ cst, const
         // the last one's inputs).
         const int vv = valid ? v : nvox - 1;
         NrIn in;
-        nr_load<true>(f, N, 8u * (unsigned)vv, in);
+        nr_load<true, F32>(f, N, 8u * (unsigned)vv, in);
         if constexpr (WS == 1) {
 #pragma unroll
             for (int k = 0; k < 6; ++k) wsp[k] = ldcf(f.dsig + (size_t)k * N, N, 4u * (unsigned)vv);
         }
-        if constexpr (WS == 2)
+        if constexpr (WS == 2) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) lds[(NRC_QUAT + k) * NR_BLOCK + threadIdx.x] = in.a[k];
+            nr_orient(f, in);
             nr_learned_start(cst, f, N, v, valid && ph >= 1 && ph <= NPH && cst->ph[ph - 1].xtal, in, wsp);
+        }
         const bool f32 = f.nrcf != nullptr;
-        if (f32)
+        if constexpr (F32) {
+            copy_field_f32<NRC_COMPS, 0>(f.nrcf, nrcf_pitch(N), lds, blk);
+            copy_field_f32<NRF_A_COMPS, NRF_A>(f.acrf, nrcf_pitch(N), lds, blk);
+        } else if (f32) {
             copy_field_f32<NRC_COMPS>(f.nrcf, nrcf_pitch(N), lds, blk);
-        else
+        } else {
             copy_field<NRC_COMPS>(f.nrc, nrc_pitch(N), lds, blk);
-        nr_prologue<false, ROT, 0, (WS != 0)>(cst, f, vv, N, in, pro, valid);
+        }
+        if constexpr (WS != 2) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (!F32) lds[(NRC_QUAT + k) * NR_BLOCK + threadIdx.x] = in.a[k];
+            nr_orient(f, in);
+        }
+        nr_prologue<false, ROT, 0, (WS != 0), F32>(cst, f, vv, N, in, pro, valid);
         pin_prologue(pro);
         copy_wait();
-        if (f32) widen_slots<NRC_COMPS>(lds);
+        if (f32 && !F32) widen_slots<NRC_COMPS>(lds);
     }
     NrResult r;
     r.cs = 0.0; r.ce = 0.0; r.it = 0; r.itot = 0; r.bad = 0;
@@ -697,9 +741,9 @@ __device__ __forceinline__ void nr_block(const DevConst *__restrict__ cst, const
         const bool mine = valid && ph == pu;
         if (mine) {
             if (pu == 1) {
-                if (cst->ph[0].xtal) nr_voxel<FIRST, ROT, 0, WS, GND>(cst, f, v, N, lds, pro, wsp, r);
+                if (cst->ph[0].xtal) nr_voxel<FIRST, ROT, 0, WS, GND, F32>(cst, f, v, N, lds, pro, wsp, r);
             } else if constexpr (PH2) {
-                if (cst->ph[1].xtal) nr_voxel<FIRST, ROT, 1, WS, GND>(cst, f, v, N, lds, pro, wsp, r);
+                if (cst->ph[1].xtal) nr_voxel<FIRST, ROT, 1, WS, GND, F32>(cst, f, v, N, lds, pro, wsp, r);
             }
         }
         todo &= ~__ballot(mine);
@@ -738,24 +782,24 @@ __device__ __forceinline__ void nr_block(const DevConst *__restrict__ cst, const
     }
 }
 
-template <bool FIRST, bool ROT, int WS, bool GND, bool PH2>
+template <bool FIRST, bool ROT, int WS, bool GND, bool PH2, bool F32>
 __global__ void __launch_bounds__(NR_BLOCK)
-__attribute__((amdgpu_waves_per_eu(FIRST ? SRX_NR_FIRST_WAVES_PER_EU : SRX_NR_WAVES_PER_EU, 8)))
+__attribute__((amdgpu_waves_per_eu(FIRST ? SRX_NR_FIRST_WAVES_PER_EU : F32 ? SRX_NR_F32_WAVES_PER_EU : SRX_NR_WAVES_PER_EU, 8)))
 k_nr(const DevConst *__restrict__ cst, Fields f, int nvox, double *__restrict__ partials,
      const IterCtl *__restrict__ ctl) {
-    nr_block<FIRST, ROT, WS, GND, PH2>(cst, f, nvox, partials, ctl, blockIdx.x, gridDim.x);
+    nr_block<FIRST, ROT, WS, GND, PH2, F32>(cst, f, nvox, partials, ctl, blockIdx.x, gridDim.x);
 }
 
 // The Newton kernel over every member of an ensemble in one launch: member m owns the blocks
 // [tab[m].blk0, tab[m].blk0 + tab[m].nblk) of the grid.
-template <bool FIRST, bool ROT, int WS, bool GND, bool PH2>
+template <bool FIRST, bool ROT, int WS, bool GND, bool PH2, bool F32>
 __global__ void __launch_bounds__(NR_BLOCK)
-__attribute__((amdgpu_waves_per_eu(FIRST ? SRX_NR_FIRST_WAVES_PER_EU : SRX_NR_WAVES_PER_EU, 8)))
+__attribute__((amdgpu_waves_per_eu(FIRST ? SRX_NR_FIRST_WAVES_PER_EU : F32 ? SRX_NR_F32_WAVES_PER_EU : SRX_NR_WAVES_PER_EU, 8)))
 k_nr_ens(const EnsMember *__restrict__ tab, int nmem) {
     int m = 0;
     while (m + 1 < nmem && (int)blockIdx.x >= tab[m + 1].blk0) ++m;
     const EnsMember &e = tab[m];
-    nr_block<FIRST, ROT, WS, GND, PH2>(e.cst, e.f, e.nvox, e.partials, e.ctl, blockIdx.x - e.blk0, e.nblk);
+    nr_block<FIRST, ROT, WS, GND, PH2, F32>(e.cst, e.f, e.nvox, e.partials, e.ctl, blockIdx.x - e.blk0, e.nblk);
 }
 
 // fixed-order reduction of block partials stored component-major:
@@ -1007,11 +1051,13 @@ int nr_block_count(int nvox) { return (nvox + NR_BLOCK - 1) / NR_BLOCK; }
 
 // Kernel variant of a Newton call: first call of an increment (F), rotated texture (R), Newton
 // start (W: 0 reference, 1 extrapolated, 2 learned; the first call of an increment starts as 1),
-// GND option (G, reference start only), crystalline second phase (P).
+// GND option (G, reference start only), crystalline second phase (P), and the FP32 LDS layout of the later calls
+// of mixed precision (not with the learned start, whose matrix-core operands need the registers).
 #define SRX_NR_VARIANTS(K, ARGS)                                                                           \
     do {                                                                                                 \
         const int ws_ = first_call && ws == 2 ? 1 : ws;                                                  \
-        const int code_ = (first_call ? 16 : 0) | (rotated ? 8 : 0) | (gnd ? 4 : 0) | (ph2 ? 2 : 0);    \
+        const int code_ = (first_call ? 16 : 0) | (rotated ? 8 : 0) | (gnd ? 4 : 0) | (ph2 ? 2 : 0) |   \
+                          (!first_call && ws_ != 2 && f32 ? 1 : 0);                                      \
         switch (code_ * 4 + ws_) {                                                                       \
         SRX_NR_CASE(K, ARGS, 1, 1, 0) SRX_NR_CASE(K, ARGS, 1, 0, 0) SRX_NR_CASE(K, ARGS, 0, 1, 0)        \
         SRX_NR_CASE(K, ARGS, 0, 0, 0) SRX_NR_CASE(K, ARGS, 1, 1, 1) SRX_NR_CASE(K, ARGS, 1, 0, 1)        \
@@ -1024,7 +1070,11 @@ int nr_block_count(int nvox) { return (nvox + NR_BLOCK - 1) / NR_BLOCK; }
     } while (0)
 #define SRX_NR_ONE(K, ARGS, F, R, W, G, P)                                                              \
     case ((F) * 16 + (R) * 8 + (G) * 4 + (P) * 2) * 4 + (W):                                             \
-        SRX_APPLY(SRX_LAUNCH, (K<(F) != 0, (R) != 0, (W), (G) != 0, (P) != 0>), SRX_UNPACK ARGS);        \
+        SRX_APPLY(SRX_LAUNCH, (K<(F) != 0, (R) != 0, (W), (G) != 0, (P) != 0, false>), SRX_UNPACK ARGS); \
+        break;                                                                                           \
+    case ((F) * 16 + (R) * 8 + (G) * 4 + (P) * 2 + 1) * 4 + (W):                                         \
+        SRX_APPLY(SRX_LAUNCH, (K<(F) != 0, (R) != 0, (W), (G) != 0, (P) != 0, (F) == 0 && (W) != 2>),    \
+                  SRX_UNPACK ARGS);                                                                      \
         break;
 #define SRX_NR_CASE(K, ARGS, F, R, W) SRX_NR_ONE(K, ARGS, F, R, W, 0, 0) SRX_NR_ONE(K, ARGS, F, R, W, 0, 1)
 #define SRX_NR_GCASE(K, ARGS, F, R) SRX_NR_ONE(K, ARGS, F, R, 0, 1, 0) SRX_NR_ONE(K, ARGS, F, R, 0, 1, 1)
@@ -1036,6 +1086,7 @@ void launch_nr(hipStream_t s, const DevConst *cst, const Fields &f, int nvox, in
     const dim3 g(nr_block_count(nvox)), b(NR_BLOCK);
     // the learned start needs the network; with only the previous change it is the extrapolated one
     const int ws = gnd ? 0 : (f.dsig && f.mlp) ? 2 : f.dsig ? 1 : 0;
+    const bool f32 = f.nrcf && f.quat;   // (without the quaternion the epilogue's orientation does not fit)
     SRX_NR_VARIANTS(k_nr, (g, b, 0, s, cst, f, nvox, partials, ctl));
     check_launch("nr");
 }
@@ -1058,7 +1109,7 @@ void launch_reduce_nr(hipStream_t s, const double *partials, int nblocks, double
 }
 
 void launch_nr_ens(hipStream_t s, const EnsMember *tab, int nmem, int nblocks, int first_call, int rotated, int ws,
-                   int gnd, int ph2) {
+                   int gnd, int ph2, int f32) {
     const dim3 g(nblocks), b(NR_BLOCK);
     if (gnd) ws = 0;
     SRX_NR_VARIANTS(k_nr_ens, (g, b, 0, s, tab, nmem));

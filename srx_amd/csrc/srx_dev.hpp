@@ -231,6 +231,8 @@ struct Fields {
                        //   date at the end of the increment (k_rot_in, k_rot_out)
     double *dg0;       // [9][N] DisGrad at the start of the increment
     double *tran;      // [9][N] TranMat_xt2sa (crystal -> sample), current
+    double *quat;      // [4][N] quaternion of tran, written by an increment's first Newton call for the later
+                       //   ones; null where a caller has set orientations that are no rotations
     double *tran0;     // [9][N] TranMat_xt2sa at setup (C_gr is never rotated)
     double *rho_s, *rho_m, *rho_m_old, *rho_F, *rho_P, *gamdot, *gam_acum;   // [12][N]
     double *rho_dipole, *rho_forest, *rho_inplane;                          // [12][N]
@@ -240,7 +242,7 @@ struct Fields {
                        //   increment, written by its first Newton call, read by the later ones
     double *nrc;       // [36][nrc_pitch(N)] per-system Newton constants of the increment, written by its first call:
                        //   tau_pass/(tau_0+tau_cut) [12], 1/(tau_0+tau_cut) [12], gamma_0 dt [12]
-    float *acrf;       // mixed precision: A rounded to FP32, [15][N] in acr's memory; null in FP64
+    float *acrf;       // mixed precision: A rounded to FP32, [15][nrcf_pitch(N)] in acr's memory; null in FP64
     float *nrcf;       // mixed precision: the same constants rounded to FP32, [36][nrcf_pitch(N)] in nrc's memory
                        //   (every Newton call of the increment uses the rounded values); null in FP64
     float *dsig;       // [6][N] last Newton call's stress change, B basis, crystal frame (warm start only)
@@ -335,9 +337,9 @@ void launch_reduce_nr(hipStream_t s, const double *partials, int nblocks, double
 void launch_control(hipStream_t s, const DevConst *cst, const double *seg, IterCtl *ctl);
 // The same three kernels over every member of an ensemble in one launch each (tab: device array of
 // nmem members; nblocks: their Newton blocks in total; ws: the Newton start option; done[m]: each
-// member's stop flag after the iteration).
+// member's stop flag after the iteration; f32: every member runs in mixed precision and keeps quaternions).
 void launch_nr_ens(hipStream_t s, const EnsMember *tab, int nmem, int nblocks, int first_call, int rotated, int ws,
-                   int gnd, int ph2);
+                   int gnd, int ph2, int f32);
 void launch_reduce_nr_ens(hipStream_t s, const EnsMember *tab, int nmem);
 void launch_control_ens(hipStream_t s, const EnsMember *tab, int nmem, int *done);
 void launch_prologue(hipStream_t s, Fields f, int nvox, const double *add9, int creep, const double *set9,

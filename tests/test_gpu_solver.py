@@ -350,3 +350,44 @@ def test_displacement_gradient_matches_oracle(tmp_path, oracle_lib, n, precision
         compare_fields(g, o, tol, ("sig", "disgrad", "velgrad", "fluct", "tranmat"))
     g.close()
     o.close()
+
+
+def _two_routes(tmp_path, n, precision, warm_start):
+    """Three runs of a deck: orientations as opened, one voxel scaled by 1 + 1e-10 (no rotation to
+    1e-12: the matrices are read), and scaled then set back."""
+    deck = make(tmp_path, n=n, grains=3, seed=29, nsteps=4)
+    a, b, c = (srx_amd.Solver(deck, fixed_iters=5, precision=precision, warm_start=warm_start) for _ in range(3))
+    t0 = b.field("tranmat")
+    t = t0.copy()
+    t[0] *= 1.0 + 1e-10
+    b.set_field("tranmat", t)
+    c.set_field("tranmat", t)
+    c.set_field("tranmat", t0)
+    for _ in range(4):
+        a.step(), b.step(), c.step()
+    return a, b, c
+
+
+@pytest.mark.parametrize("n", [(1, 1, 2), (3, 5, 1), (15, 9, 5), (16, 8, 6)])
+@pytest.mark.parametrize("warm_start", [0, 1])
+def test_orientations_kept_as_quaternions_or_as_matrices(tmp_path, n, warm_start):
+    """The Newton kernel keeps orientations as quaternions unless a caller has set one that is no
+    rotation; then it reads the matrices.  The two routes agree to the perturbation that selects the
+    second (1e-10, amplified by the stress exponent of order 100: 1e-7), and setting rotations again
+    returns to the first, bit for bit."""
+    a, b, c = _two_routes(tmp_path, n, srx_amd.PREC_FP64, warm_start)
+    for f in ("sig", "edot", "disgrad", "rho_s", "tranmat"):
+        assert rel(b.field(f), a.field(f)) < 1e-7, f
+        np.testing.assert_array_equal(c.field(f), a.field(f))
+
+
+@pytest.mark.parametrize("n", [(1, 1, 2), (3, 5, 1), (15, 9, 5), (16, 8, 8)])
+@pytest.mark.parametrize("warm_start", [0, 1])
+def test_mixed_newton_layouts_agree(tmp_path, n, warm_start):
+    """Mixed precision with quaternions keeps the Newton constants as FP32 in LDS, with matrices it widens
+    them there.  Besides the perturbation the FP32 transforms round differently (6e-8, amplified by
+    the stress exponent): this file's 1e-4 for mixed fields."""
+    a, b, c = _two_routes(tmp_path, n, srx_amd.PREC_MIXED, warm_start)
+    for f in ("sig", "edot", "disgrad", "rho_s", "tranmat"):
+        assert rel(b.field(f), a.field(f)) < 1e-4, f
+        np.testing.assert_array_equal(c.field(f), a.field(f))
