@@ -339,6 +339,7 @@ struct srx_ctx {
     IterCtl *dctl = nullptr, *hctl = nullptr;   // outer-iteration control block (device, pinned host copy)
     int iters_last = 0;                        // outer iterations of the last increment
     int nr_blocks = 0, end_blocks = 0;
+    bool fcc = false;                          // the slip systems have the FCC zero structure (nr_fcc)
     hipStream_t stream = nullptr;
     // macro state
     double Udot[9], Udot_s[9], Udot_a[9], Scauchy[9];
@@ -560,6 +561,7 @@ int setup(srx_ctx *c) {
                 D.sin_g2[i][j] = std::fabs(std::sqrt(std::fabs(1.0 - c2g * c2g)));
             }
     }
+    c->fcc = nr_fcc(c->hc);
     c->hc.dt = d.TimeStep;
     c->hc.nu = d.ElastConst_PhaseI[3];
     c->hc.T = d.T__K;
@@ -1411,7 +1413,7 @@ static int step_iterate(srx_ctx *c) {
             if (rec)
                 launch_mlp_record(c->stream, c->dc, c->f, N, c->rec_stride, 0, c->rec_x, c->rec_t, c->rec_nd,
                                   c->rec_count, c->rec_cap, g);
-            { Timer t(c, 5, launched); launch_nr(c->stream, c->dc, c->f, N, launched == 1, rotated, c->partials, g, c->opt.gnd, c->hc.ph[1].xtal); }
+            { Timer t(c, 5, launched); launch_nr(c->stream, c->dc, c->f, N, launched == 1, rotated, c->partials, g, c->opt.gnd, c->hc.ph[1].xtal, c->fcc); }
             if (rec)
                 launch_mlp_record(c->stream, c->dc, c->f, N, c->rec_stride, 1, c->rec_x, c->rec_t, c->rec_nd,
                                   c->rec_count, c->rec_cap, g);
@@ -1697,10 +1699,11 @@ static int run_lockstep(const std::vector<int> &members, std::vector<srx_ctx *> 
             break;
         launch_prologue_ens(S, dinc, nact, pb);
         const srx_options &o = ctx[act[0]]->opt;
-        int ph2 = 0, f32 = 1;
+        int ph2 = 0, f32 = 1, fcc = 1;
         for (int k : act) {
             ph2 |= ctx[k]->hc.ph[1].xtal;
             f32 = f32 && ctx[k]->f.nrcf && ctx[k]->f.quat;
+            fcc = fcc && ctx[k]->fcc;
         }
         int launched = 0;
         bool all_done = false;
@@ -1723,7 +1726,7 @@ static int run_lockstep(const std::vector<int> &members, std::vector<srx_ctx *> 
                                             (double)c->nvox, tl[4]);
                 }
                 for (int q = 0; q < NS; ++q) ok(hipEventRecord(ev[q], side[q])) && ok(hipStreamWaitEvent(S, ev[q], 0));
-                launch_nr_ens(S, dtab, nact, nb, launched == 1, rotated, o.warm_start, o.gnd, ph2, f32);
+                launch_nr_ens(S, dtab, nact, nb, launched == 1, rotated, o.warm_start, o.gnd, ph2, f32, fcc);
                 launch_reduce_nr_ens(S, dtab, nact);
                 launch_control_ens(S, dtab, nact, ddone);
             }

@@ -7,6 +7,8 @@
 #include "crystal_dev.hpp"
 #include "mlp_dev.hpp"
 
+#include <type_traits>
+
 namespace srx {
 
 // ---------------------------------------------------------------------------
@@ -20,10 +22,21 @@ namespace srx {
 // used for Edot and the errors are the reference's.
 // ---------------------------------------------------------------------------
 constexpr int NR_BLOCK = 64;
-// slip systems evaluated together per trip of the Newton kernel's system loop (divides 12)
-#ifndef SRX_NR_GROUP
-#define SRX_NR_GROUP 2
-#endif
+// Zero components of the 12 {111}<110> Schmid vectors in the crystal frame's B basis, bit i for
+// component i, by system modulo 3 (the order of the reference's slip-mode file and interaction table):
+// a system whose Burgers vector lies in the plane of two axes has no shear in that plane, and with the
+// third axis normal to it (modulo 3: 2) no second normal component either.
+constexpr int fcc_zero(int s) { return s % 3 == 0 ? 1 << 2 : s % 3 == 1 ? 1 << 3 : (1 << 4) | (1 << 1); }
+bool nr_fcc(const DevConst &hc) {
+    for (int p = 0; p < NPH; ++p) {
+        if (!hc.ph[p].xtal) continue;
+        if (p != 0 || hc.ph[p].nsys != NSYS) return false;
+        for (int s = 0; s < NSYS; ++s)
+            for (int i = 0; i < 5; ++i)
+                if ((fcc_zero(s) >> i & 1) && hc.ph[p].p[s][i] != 0.0) return false;
+    }
+    return hc.ph[0].xtal;
+}
 
 struct NrResult {
     double cs, ce;
@@ -252,8 +265,9 @@ __device__ __forceinline__ void nr_prologue(const DevConst *__restrict__ cst, co
 // 2 = lam + the learned prediction `wsp` (crystal frame).  FIRST: the call computes its prologue
 // and per-system constants and stores them for the increment; otherwise the caller has put the
 // prologue in `pro` and the constants in the LDS slots NRC_*.
-// F32: the FP32 LDS layout (later calls of mixed precision).
-template <bool FIRST, bool ROT, int PH, int WS, bool GND, bool F32>
+// F32: the FP32 LDS layout (later calls of mixed precision).  FCC: the Schmid vectors have fcc_zero's zeros,
+// which leaves out 10 of about 70 instructions per active system.
+template <bool FIRST, bool ROT, int PH, int WS, bool GND, bool F32, bool FCC>
 __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const Fields &f, int v, size_t N,
                                          double *lds, NrPro &pro, const float *wsp, NrResult &res) {
     // compile-time phase index: every material constant is a scalar load at a fixed offset
@@ -281,7 +295,7 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
     double ws[5] = {0, 0, 0, 0, 0}, wsh = 0.0;   // warm start: crystal-frame offset of the first iterate
     const double Shh = cst->S066[5][5];
     const double Ah = Shh + P.sinv[5];
-    const double rAh = 1.0 / Ah;
+    const double rAh = rcp(Ah);
     const double r0h = qh - Shh * lamh;
 
     // per-system constants, kept in LDS (lane-major, conflict free): tau_pass * inv, inv and
@@ -359,7 +373,93 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
     for (int i = 0; i < 5; ++i) { sg[i] = lam[i] + ws[i]; pre[i] = sg[i]; R[i] = 0.0; }
     int it = 0, itot = 0;
     // stopping rule ||d sig|| / ||lam|| <= 1e-10, compared squared (no square root per iteration)
-    double err2 = 1E-18;
+    double err2 = 1E-18, errp2 = 0.0;   // this and the previous step's
+    bool again = false;
+    // the last step without K (see below): not with the FP32 layout, where keeping the factors across
+    // iterations spills (349 us at 128^3 instead of 322), nor in the one first call
+    constexpr bool SHORT_LAST = !F32 && !FIRST;
+    // K: the iteration's matrix, then its factors
+    double K[15];
+    // One iteration's residual R = r0 + A sg + sum_s p_s g_s (and K = A + sum_s g2_s p_s p_s^T).
+    // Two systems per trip, under one wavefront-uniform branch: their slip-rate evaluations are
+    // independent dependency chains the scheduler interleaves (an inactive system of the two
+    // evaluates at 0 and adds exact zeros).  Zp: components of the Schmid vectors of both systems that are
+    // exactly zero, left out of the sums.
+    auto two_systems = [&](auto with_k, auto zero, int sa, int sb) {
+        constexpr bool WK = decltype(with_k)::value;
+        constexpr int Zp = decltype(zero)::value;
+        double rss[2], ivs[2], e[2];
+        bool act = false;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int sys = u ? sb : sa;
+            const double *p = P.p[sys];
+            double acc = 0.0;
+            bool any = false;
+#pragma unroll
+            for (int i = 0; i < 5; ++i)
+                if (!(Zp >> i & 1)) {
+                    acc = any ? acc + p[i] * sg[i] : p[i] * sg[i];
+                    any = true;
+                }
+            rss[u] = acc;
+            ivs[u] = slot(NRC_INV + sys);
+            e[u] = fma(fabs(rss[u]), ivs[u], -slot(NRC_TP + sys));
+            act |= e[u] > 0.0;
+        }
+        if (!__any(act)) return;
+        double g[2], g2dt[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int sys = u ? sb : sa;
+            if (WK) slip_rate(rss[u], e[u], ivs[u], slot(NRC_G0 + sys), g[u], g2dt[u]);
+            else g[u] = slip_rate_only(rss[u], e[u], slot(NRC_G0 + sys));
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const double *p = P.p[u ? sb : sa];
+#pragma unroll
+            for (int i = 0; i < 5; ++i) {
+                if (Zp >> i & 1) continue;
+                R[i] += p[i] * g[u];
+                if (WK) {
+                    const double gp = g2dt[u] * p[i];
+#pragma unroll
+                    for (int j = i; j < 5; ++j)
+                        if (!(Zp >> j & 1)) K[ps(i, j)] += gp * p[j];
+                }
+            }
+        }
+    };
+    auto residual = [&](auto with_k) {
+        constexpr bool WK = decltype(with_k)::value;
+        double M[15];
+#pragma unroll
+        for (int k = 0; k < 15; ++k) M[k] = Aat(k);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            double acc = r0[i];
+#pragma unroll
+            for (int j = 0; j < 5; ++j) acc += M[ps(i, j)] * sg[j];
+            R[i] = acc;
+        }
+        if (WK) {
+#pragma unroll
+            for (int k = 0; k < 15; ++k) K[k] = M[k];
+        }
+        if constexpr (FCC) {
+            // the systems of one residue modulo 3 share their zero components (fcc_zero)
+#pragma unroll 1
+            for (int h = 0; h < NSYS; h += 6) two_systems(with_k, std::integral_constant<int, fcc_zero(0)>{}, h, h + 3);
+#pragma unroll 1
+            for (int h = 1; h < NSYS; h += 6) two_systems(with_k, std::integral_constant<int, fcc_zero(1)>{}, h, h + 3);
+#pragma unroll 1
+            for (int h = 2; h < NSYS; h += 6) two_systems(with_k, std::integral_constant<int, fcc_zero(2)>{}, h, h + 3);
+        } else {
+#pragma unroll 1
+            for (int s0 = 0; s0 < NSYS; s0 += 2) two_systems(with_k, std::integral_constant<int, 0>{}, s0, s0 + 1);
+        }
+    };
     // With the learned start (WS 2), a solve that does not converge (non-finite iterate, or 500
     // iterations) is repeated from lam, the reference's start; `itot` counts both attempts.  (The
     // extrapolated start has not needed it; the second attempt costs it registers.  The first call
@@ -373,21 +473,18 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
         preh = sh;
         it = 0;
         err2 = 1E-18;
+        again = false;
     }
     while (it < 500 && err2 > 1E-20) {
+        // A lane's last step: with two steps taken and the next one predicted from their quadratic
+        // convergence, err (err / errp)^2, a decade below the tolerance, the previous iteration's factors
+        // give it as well (they differ by the last step's size, 1e-5 or less, of a step near 1e-12).
+        // When that holds for every lane still iterating, K and its factorisation are left out, a third
+        // of the iteration's instructions; a lane whose step then is not its last (a slip system became
+        // active) repeats the iteration with its own K, so the iterates are the full iteration's.
+        const bool last = SHORT_LAST && !again && it >= 2 && err2 * err2 * err2 <= 1E-22 * (errp2 * errp2);
         ++it;
         ++itot;
-        // K = A and R = r0 + A sg, to which the slip systems add
-        double K[15];
-#pragma unroll
-        for (int k = 0; k < 15; ++k) K[k] = Aat(k);
-#pragma unroll
-        for (int i = 0; i < 5; ++i) {
-            double acc = r0[i];
-#pragma unroll
-            for (int j = 0; j < 5; ++j) acc += K[ps(i, j)] * sg[j];
-            R[i] = acc;
-        }
         if (FIRST && it == 2) {
             if (f.nrcf) {
                 const float *nc = fresh(f.nrcf);
@@ -401,56 +498,29 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
                     tp[s * NR_BLOCK] = ldc(nc + (size_t)(NRC_TP + s) * nrc_pitch(N), nrc_pitch(N), o8);
             }
         }
-        // SRX_NR_GROUP systems per trip, under one wavefront-uniform branch: their slip-rate
-        // evaluations are independent dependency chains the scheduler interleaves (an inactive
-        // system of the group evaluates at 0 and adds exact zeros)
-        constexpr int NG = SRX_NR_GROUP;
-        static_assert(NSYS % NG == 0, "systems are taken in groups of SRX_NR_GROUP");
-#pragma unroll 1
-        for (int s0 = 0; s0 < NSYS; s0 += NG) {
-            double rss[NG], ivs[NG], e[NG];
-            bool act = false;
+        const bool full = !SHORT_LAST || __any(!last);
+        if (full) {
+            residual(std::true_type{});
+            // LDL^T in place: K[ps(j,j)] <- 1/D_j, K[ps(i,j)] <- L_ij (i > j)
+            double D[5];
 #pragma unroll
-            for (int u = 0; u < NG; ++u) {
-                const double *p = P.p[s0 + u];
-                rss[u] = p[0] * sg[0] + p[1] * sg[1] + p[2] * sg[2] + p[3] * sg[3] + p[4] * sg[4];
-                ivs[u] = slot(NRC_INV + s0 + u);
-                e[u] = fma(fabs(rss[u]), ivs[u], -slot(NRC_TP + s0 + u));
-                act |= e[u] > 0.0;
-            }
-            if (__any(act)) {
-                double g[NG], g2dt[NG];
+            for (int j = 0; j < 5; ++j) {
+                double dj = K[ps(j, j)];
 #pragma unroll
-                for (int u = 0; u < NG; ++u) slip_rate(rss[u], e[u], ivs[u], slot(NRC_G0 + s0 + u), g[u], g2dt[u]);
+                for (int k = 0; k < j; ++k) dj -= K[ps(j, k)] * K[ps(j, k)] * D[k];
+                const double rj = rcp_step(dj);
 #pragma unroll
-                for (int u = 0; u < NG; ++u) {
-                    const double *p = P.p[s0 + u];
+                for (int i = j + 1; i < 5; ++i) {
+                    double acc = K[ps(i, j)];
 #pragma unroll
-                    for (int i = 0; i < 5; ++i) {
-                        R[i] += p[i] * g[u];
-                        const double gp = g2dt[u] * p[i];
-#pragma unroll
-                        for (int j = i; j < 5; ++j) K[ps(i, j)] += gp * p[j];
-                    }
+                    for (int k = 0; k < j; ++k) acc -= K[ps(i, k)] * K[ps(j, k)] * D[k];
+                    K[ps(i, j)] = acc * rj;
                 }
+                D[j] = dj;
+                K[ps(j, j)] = rj;
             }
-        }
-        // LDL^T in place: K[ps(j,j)] <- 1/D_j, K[ps(i,j)] <- L_ij (i > j)
-#pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            double dj = K[ps(j, j)];
-#pragma unroll
-            for (int k = 0; k < j; ++k) dj -= K[ps(j, k)] * K[ps(j, k)] * K[ps(k, k)];
-            // K[ps(k,k)] holds D_k until it is inverted below
-            const double rj = rcp_step(dj);
-#pragma unroll
-            for (int i = j + 1; i < 5; ++i) {
-                double acc = K[ps(i, j)];
-#pragma unroll
-                for (int k = 0; k < j; ++k) acc -= K[ps(i, k)] * K[ps(j, k)] * K[ps(k, k)];
-                K[ps(i, j)] = acc * rj;
-            }
-            K[ps(j, j)] = dj;
+        } else {
+            residual(std::false_type{});
         }
         double y[5];
 #pragma unroll
@@ -461,7 +531,7 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
             y[i] = acc;
         }
 #pragma unroll
-        for (int i = 0; i < 5; ++i) y[i] *= rcp_step(K[ps(i, i)]);
+        for (int i = 0; i < 5; ++i) y[i] *= K[ps(i, i)];
 #pragma unroll
         for (int i = 4; i >= 0; --i) {
 #pragma unroll
@@ -470,14 +540,25 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
         const double dh = (Ah * sh + r0h) * rAh;
         double cnr = dh * dh;
 #pragma unroll
+        for (int i = 0; i < 5; ++i) cnr += y[i] * y[i];
+        const double errn = cnr * rsig2;
+        if (SHORT_LAST) {
+            again = !full && errn > 1E-20;
+            if (again) {
+                --it;
+                --itot;
+                continue;
+            }
+            errp2 = err2;
+        }
+        err2 = errn;
+#pragma unroll
         for (int i = 0; i < 5; ++i) {
             pre[i] = sg[i];
             sg[i] -= y[i];
-            cnr += y[i] * y[i];
         }
         preh = sh;
         sh -= dh;
-        err2 = cnr * rsig2;
     }
     }
     if (WS) {
@@ -674,7 +755,7 @@ __device__ __forceinline__ void nr_learned_start(const DevConst *__restrict__ cs
 // One 64-voxel block of the Newton kernel: block `blk` of the `nblk` blocks of a grid of nvox
 // voxels (partials: NR_NPART x nblk block partial sums).
 // PH2: the second phase is crystalline (else its voxels are gas and its Newton path is not compiled).
-template <bool FIRST, bool ROT, int WS, bool GND, bool PH2, bool F32>
+template <bool FIRST, bool ROT, int WS, bool GND, bool PH2, bool F32, bool FCC>
 __device__ __forceinline__ void nr_block(const DevConst *__restrict__ cst, const Fields &f, int nvox,
                                          double *__restrict__ partials, const IterCtl *__restrict__ ctl, int blk,
                                          int nblk) {
@@ -741,9 +822,9 @@ __device__ __forceinline__ void nr_block(const DevConst *__restrict__ cst, const
         const bool mine = valid && ph == pu;
         if (mine) {
             if (pu == 1) {
-                if (cst->ph[0].xtal) nr_voxel<FIRST, ROT, 0, WS, GND, F32>(cst, f, v, N, lds, pro, wsp, r);
+                if (cst->ph[0].xtal) nr_voxel<FIRST, ROT, 0, WS, GND, F32, FCC>(cst, f, v, N, lds, pro, wsp, r);
             } else if constexpr (PH2) {
-                if (cst->ph[1].xtal) nr_voxel<FIRST, ROT, 1, WS, GND, F32>(cst, f, v, N, lds, pro, wsp, r);
+                if (cst->ph[1].xtal) nr_voxel<FIRST, ROT, 1, WS, GND, F32, false>(cst, f, v, N, lds, pro, wsp, r);
             }
         }
         todo &= ~__ballot(mine);
@@ -782,24 +863,24 @@ __device__ __forceinline__ void nr_block(const DevConst *__restrict__ cst, const
     }
 }
 
-template <bool FIRST, bool ROT, int WS, bool GND, bool PH2, bool F32>
+template <bool FIRST, bool ROT, int WS, bool GND, bool PH2, bool F32, bool FCC>
 __global__ void __launch_bounds__(NR_BLOCK)
 __attribute__((amdgpu_waves_per_eu(FIRST ? SRX_NR_FIRST_WAVES_PER_EU : F32 ? SRX_NR_F32_WAVES_PER_EU : SRX_NR_WAVES_PER_EU, 8)))
 k_nr(const DevConst *__restrict__ cst, Fields f, int nvox, double *__restrict__ partials,
      const IterCtl *__restrict__ ctl) {
-    nr_block<FIRST, ROT, WS, GND, PH2, F32>(cst, f, nvox, partials, ctl, blockIdx.x, gridDim.x);
+    nr_block<FIRST, ROT, WS, GND, PH2, F32, FCC>(cst, f, nvox, partials, ctl, blockIdx.x, gridDim.x);
 }
 
 // The Newton kernel over every member of an ensemble in one launch: member m owns the blocks
 // [tab[m].blk0, tab[m].blk0 + tab[m].nblk) of the grid.
-template <bool FIRST, bool ROT, int WS, bool GND, bool PH2, bool F32>
+template <bool FIRST, bool ROT, int WS, bool GND, bool PH2, bool F32, bool FCC>
 __global__ void __launch_bounds__(NR_BLOCK)
 __attribute__((amdgpu_waves_per_eu(FIRST ? SRX_NR_FIRST_WAVES_PER_EU : F32 ? SRX_NR_F32_WAVES_PER_EU : SRX_NR_WAVES_PER_EU, 8)))
 k_nr_ens(const EnsMember *__restrict__ tab, int nmem) {
     int m = 0;
     while (m + 1 < nmem && (int)blockIdx.x >= tab[m + 1].blk0) ++m;
     const EnsMember &e = tab[m];
-    nr_block<FIRST, ROT, WS, GND, PH2, F32>(e.cst, e.f, e.nvox, e.partials, e.ctl, blockIdx.x - e.blk0, e.nblk);
+    nr_block<FIRST, ROT, WS, GND, PH2, F32, FCC>(e.cst, e.f, e.nvox, e.partials, e.ctl, blockIdx.x - e.blk0, e.nblk);
 }
 
 // fixed-order reduction of block partials stored component-major:
@@ -1049,40 +1130,42 @@ void launch_mlp_record(hipStream_t s, const DevConst *cst, const Fields &f, int 
 
 int nr_block_count(int nvox) { return (nvox + NR_BLOCK - 1) / NR_BLOCK; }
 
-// Kernel variant of a Newton call: first call of an increment (F), rotated texture (R), Newton
-// start (W: 0 reference, 1 extrapolated, 2 learned; the first call of an increment starts as 1),
-// GND option (G, reference start only), crystalline second phase (P), and the FP32 LDS layout of the later calls
-// of mixed precision (not with the learned start, whose matrix-core operands need the registers).
+// Kernel variant of a Newton call: first call of an increment (F), rotated texture (R, which only the
+// first call's matrix A depends on), Newton start (W: 0 reference, 1 extrapolated, 2 learned; the first call
+// of an increment starts as 1), GND option (G, reference start only), crystalline second phase (P); for
+// the later calls also the FP32 LDS layout of mixed precision (not with the learned start, whose
+// matrix-core operands need the registers) and the FCC zeros (not with a second phase or the learned
+// start; the first call, one in about sixty, goes without).
 #define SRX_NR_VARIANTS(K, ARGS)                                                                           \
     do {                                                                                                 \
         const int ws_ = first_call && ws == 2 ? 1 : ws;                                                  \
-        const int code_ = (first_call ? 16 : 0) | (rotated ? 8 : 0) | (gnd ? 4 : 0) | (ph2 ? 2 : 0) |   \
-                          (!first_call && ws_ != 2 && f32 ? 1 : 0);                                      \
+        const bool v_ = !first_call && ws_ != 2;                                                         \
+        const int code_ = (first_call ? 32 : 0) | (first_call && rotated ? 16 : 0) | (gnd ? 8 : 0) |     \
+                          (ph2 ? 4 : 0) | (v_ && f32 ? 2 : 0) | (v_ && fcc && !ph2 ? 1 : 0);             \
         switch (code_ * 4 + ws_) {                                                                       \
-        SRX_NR_CASE(K, ARGS, 1, 1, 0) SRX_NR_CASE(K, ARGS, 1, 0, 0) SRX_NR_CASE(K, ARGS, 0, 1, 0)        \
-        SRX_NR_CASE(K, ARGS, 0, 0, 0) SRX_NR_CASE(K, ARGS, 1, 1, 1) SRX_NR_CASE(K, ARGS, 1, 0, 1)        \
-        SRX_NR_CASE(K, ARGS, 0, 1, 1) SRX_NR_CASE(K, ARGS, 0, 0, 1) SRX_NR_CASE(K, ARGS, 0, 1, 2)        \
-        SRX_NR_CASE(K, ARGS, 0, 0, 2)                                                                    \
-        SRX_NR_GCASE(K, ARGS, 1, 1) SRX_NR_GCASE(K, ARGS, 1, 0) SRX_NR_GCASE(K, ARGS, 0, 1)              \
-        SRX_NR_GCASE(K, ARGS, 0, 0)                                                                      \
+        SRX_NR_FIRST(K, ARGS, 0, 0) SRX_NR_FIRST(K, ARGS, 0, 1) SRX_NR_FIRST(K, ARGS, 1, 0)              \
+        SRX_NR_LATER(K, ARGS, 0, 0) SRX_NR_LATER(K, ARGS, 0, 1) SRX_NR_LATER(K, ARGS, 1, 0)              \
+        SRX_NR_ONE(K, ARGS, 0, 0, 2, 0, 0, 0, 0) SRX_NR_ONE(K, ARGS, 0, 0, 2, 0, 1, 0, 0)                \
         default: break;                                                                                  \
         }                                                                                                \
     } while (0)
-#define SRX_NR_ONE(K, ARGS, F, R, W, G, P)                                                              \
-    case ((F) * 16 + (R) * 8 + (G) * 4 + (P) * 2) * 4 + (W):                                             \
-        SRX_APPLY(SRX_LAUNCH, (K<(F) != 0, (R) != 0, (W), (G) != 0, (P) != 0, false>), SRX_UNPACK ARGS); \
-        break;                                                                                           \
-    case ((F) * 16 + (R) * 8 + (G) * 4 + (P) * 2 + 1) * 4 + (W):                                         \
-        SRX_APPLY(SRX_LAUNCH, (K<(F) != 0, (R) != 0, (W), (G) != 0, (P) != 0, (F) == 0 && (W) != 2>),    \
+#define SRX_NR_ONE(K, ARGS, F, R, W, G, P, S, Z)                                                         \
+    case ((F) * 32 + (R) * 16 + (G) * 8 + (P) * 4 + (S) * 2 + (Z)) * 4 + (W):                            \
+        SRX_APPLY(SRX_LAUNCH, (K<(F) != 0, (R) != 0, (W), (G) != 0, (P) != 0, (S) != 0, (Z) != 0>),      \
                   SRX_UNPACK ARGS);                                                                      \
         break;
-#define SRX_NR_CASE(K, ARGS, F, R, W) SRX_NR_ONE(K, ARGS, F, R, W, 0, 0) SRX_NR_ONE(K, ARGS, F, R, W, 0, 1)
-#define SRX_NR_GCASE(K, ARGS, F, R) SRX_NR_ONE(K, ARGS, F, R, 0, 1, 0) SRX_NR_ONE(K, ARGS, F, R, 0, 1, 1)
+#define SRX_NR_FIRST(K, ARGS, G, W)                                                                      \
+    SRX_NR_ONE(K, ARGS, 1, 0, W, G, 0, 0, 0) SRX_NR_ONE(K, ARGS, 1, 1, W, G, 0, 0, 0)                    \
+    SRX_NR_ONE(K, ARGS, 1, 0, W, G, 1, 0, 0) SRX_NR_ONE(K, ARGS, 1, 1, W, G, 1, 0, 0)
+#define SRX_NR_LATER(K, ARGS, G, W)                                                                      \
+    SRX_NR_ONE(K, ARGS, 0, 0, W, G, 0, 0, 0) SRX_NR_ONE(K, ARGS, 0, 0, W, G, 0, 0, 1)                    \
+    SRX_NR_ONE(K, ARGS, 0, 0, W, G, 0, 1, 0) SRX_NR_ONE(K, ARGS, 0, 0, W, G, 0, 1, 1)                    \
+    SRX_NR_ONE(K, ARGS, 0, 0, W, G, 1, 0, 0) SRX_NR_ONE(K, ARGS, 0, 0, W, G, 1, 1, 0)
 #define SRX_UNPACK(...) __VA_ARGS__
 #define SRX_APPLY(M, ...) M(__VA_ARGS__)
 
 void launch_nr(hipStream_t s, const DevConst *cst, const Fields &f, int nvox, int first_call, int rotated,
-               double *partials, const IterCtl *ctl, int gnd, int ph2) {
+               double *partials, const IterCtl *ctl, int gnd, int ph2, int fcc) {
     const dim3 g(nr_block_count(nvox)), b(NR_BLOCK);
     // the learned start needs the network; with only the previous change it is the extrapolated one
     const int ws = gnd ? 0 : (f.dsig && f.mlp) ? 2 : f.dsig ? 1 : 0;
@@ -1109,7 +1192,7 @@ void launch_reduce_nr(hipStream_t s, const double *partials, int nblocks, double
 }
 
 void launch_nr_ens(hipStream_t s, const EnsMember *tab, int nmem, int nblocks, int first_call, int rotated, int ws,
-                   int gnd, int ph2, int f32) {
+                   int gnd, int ph2, int f32, int fcc) {
     const dim3 g(nblocks), b(NR_BLOCK);
     if (gnd) ws = 0;
     SRX_NR_VARIANTS(k_nr_ens, (g, b, 0, s, tab, nmem));

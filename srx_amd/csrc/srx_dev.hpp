@@ -324,9 +324,10 @@ void launch_rotation_part(hipStream_t s, int prec, const double *in, double *out
                           const int tiles[5]);
 void launch_rot_in(hipStream_t s, const Fields &f, int nvox, const double *du9);
 void launch_rot_out(hipStream_t s, const Fields &f, int nvox, const double *du9);
-// ph2: the second phase is crystalline (its Newton path is compiled in only then)
+// ph2: the second phase is crystalline (its Newton path is compiled in only then); fcc: nr_fcc of the constants
+bool nr_fcc(const DevConst &hc);
 void launch_nr(hipStream_t s, const DevConst *cst, const Fields &f, int nvox, int first_call, int rotated,
-               double *partials, const IterCtl *ctl = nullptr, int gnd = 0, int ph2 = 1);
+               double *partials, const IterCtl *ctl, int gnd, int ph2, int fcc);
 void launch_reduce(hipStream_t s, const double *partials, int nblocks, int nvals, double *out,
                    const IterCtl *ctl = nullptr);
 // The per-iteration reduction of the Newton kernel's block partials in two fixed-order stages:
@@ -337,9 +338,10 @@ void launch_reduce_nr(hipStream_t s, const double *partials, int nblocks, double
 void launch_control(hipStream_t s, const DevConst *cst, const double *seg, IterCtl *ctl);
 // The same three kernels over every member of an ensemble in one launch each (tab: device array of
 // nmem members; nblocks: their Newton blocks in total; ws: the Newton start option; done[m]: each
-// member's stop flag after the iteration; f32: every member runs in mixed precision and keeps quaternions).
+// member's stop flag after the iteration; f32: every member runs in mixed precision and keeps quaternions;
+// fcc: nr_fcc of every member).
 void launch_nr_ens(hipStream_t s, const EnsMember *tab, int nmem, int nblocks, int first_call, int rotated, int ws,
-                   int gnd, int ph2, int f32);
+                   int gnd, int ph2, int f32, int fcc);
 void launch_reduce_nr_ens(hipStream_t s, const EnsMember *tab, int nmem);
 void launch_control_ens(hipStream_t s, const EnsMember *tab, int nmem, int *done);
 void launch_prologue(hipStream_t s, Fields f, int nvox, const double *add9, int creep, const double *set9,
