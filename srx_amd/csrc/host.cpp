@@ -1392,6 +1392,11 @@ static int step_iterate(srx_ctx *c) {
     // batches differ from launch to launch)
     const bool use_graph = c->graphs && batch == ITER_BATCH && !c->timing && c->rec_stride == 0;
     int launched = 0;
+    // Batches enqueued before the control block is first read: increments of one loading path take
+    // similar iteration counts, so all but the last of the previous increment's batches go out without
+    // waiting for the one before (a read-back leaves the GPU idle for 20-40 us, of 54 us x 8
+    // iterations at 16^3).  Iterations past convergence return at once.
+    int ahead = batch == ITER_BATCH ? (c->opt.fixed_iters > 0 ? c->opt.fixed_iters : c->iters_last) / ITER_BATCH : 1;
     while (!ctl.done) {
         if (launched > most) return SRX_E_HIP;   // the control kernel must have stopped the loop
         hipGraphExec_t *gx = use_graph ? &c->gexec[launched == 0 ? 1 : 0][rotated] : nullptr;
@@ -1417,8 +1422,11 @@ static int step_iterate(srx_ctx *c) {
             if (rec)
                 launch_mlp_record(c->stream, c->dc, c->f, N, c->rec_stride, 1, c->rec_x, c->rec_t, c->rec_nd,
                                   c->rec_count, c->rec_cap, g);
-            { Timer t(c, 7, launched); launch_reduce_nr(c->stream, c->partials, c->nr_blocks, c->redseg, g); }
-            launch_control(c->stream, c->dc, c->redseg, g);
+            if (c->nr_blocks > NR_RED_ONE) {
+                Timer t(c, 7, launched);
+                launch_reduce_nr(c->stream, c->partials, c->nr_blocks, c->redseg, g);
+            }
+            launch_control(c->stream, c->dc, c->partials, c->nr_blocks, c->redseg, g);
         }
         if (gx) {
             hipGraph_t graph = nullptr;
@@ -1433,6 +1441,7 @@ static int step_iterate(srx_ctx *c) {
             HIPCK(hipGraphLaunch(*gx, c->stream));
         }
         }
+        if (--ahead > 0 && launched + batch <= most) continue;
         HIPCK(hipMemcpyAsync(&ctl, c->dctl, sizeof(IterCtl), hipMemcpyDeviceToHost, c->stream));
         HIPCK(hipStreamSynchronize(c->stream));
         if (c->opt.verbose) std::printf("iter %d Err_e %e Err_s %e\n", ctl.iter, ctl.Err_e, ctl.Err_s);

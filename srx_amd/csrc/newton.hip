@@ -938,6 +938,7 @@ __global__ void __launch_bounds__(RED_BLOCK) k_reduce_end_ens(const EnsIncr *__r
 // RED_SEGS contiguous ranges of block partials, in a fixed order (strided accumulators, then the
 // wavefronts, then the four wavefront results), into seg[k * RED_SEGS + sg].  k_control finishes.
 constexpr int RED_SEGS = 16, RED_SEG_BLOCK = 256;
+
 static_assert(NR_RED_SEG_DOUBLES == NR_NPART * RED_SEGS, "segment buffer size");
 __device__ __forceinline__ void reduce_seg_block(const double *__restrict__ part, int nblocks,
                                                  unsigned long long maxmask, double *__restrict__ seg,
@@ -978,81 +979,217 @@ __global__ void __launch_bounds__(RED_SEG_BLOCK) k_reduce_seg(const double *__re
 __global__ void __launch_bounds__(RED_SEG_BLOCK) k_reduce_seg_ens(const EnsMember *__restrict__ tab,
                                                                   unsigned long long maxmask) {
     const EnsMember &e = tab[blockIdx.z];
+    if (e.nblk <= NR_RED_ONE) return;   // k_control_ens sums this member's partials itself
     reduce_seg_block(e.partials, e.nblk, maxmask, e.redseg, e.ctl, blockIdx.x, blockIdx.y);
 }
 
-// One outer iteration's bookkeeping on the device (the host loop of evolution.c:1150-1256):
-// the dDisGradAvg this iteration's inverse-z pass applied joins the uniform part, the reduced
-// sums give the errors and get_smacro's averages and correction, and `done` decides whether the
-// next iteration runs.  One thread; the iteration's other kernels have finished (stream order).
-__device__ __forceinline__ void control_step(const DevConst *__restrict__ cst, IterCtl &c, const double *red);
-
-__device__ __forceinline__ void control_block(const DevConst *__restrict__ cst, const double *__restrict__ seg,
-                                              IterCtl *ctl) {
-    if (ctl->done) return;
-    // The control block is copied to LDS by the whole block, worked on there by one thread (no
-    // dependent HBM round trips) and copied back.
-    static_assert(sizeof(IterCtl) % 8 == 0, "IterCtl is copied as 64-bit words");
-    constexpr int NW = sizeof(IterCtl) / 8;
-    __shared__ IterCtl lc;
-    for (int i = threadIdx.x; i < NW; i += blockDim.x)
-        reinterpret_cast<unsigned long long *>(&lc)[i] = reinterpret_cast<const unsigned long long *>(ctl)[i];
-    // second stage of the reduction: the RED_SEGS partial results of each value, in order
-    __shared__ double red[NR_NPART];
-    if (threadIdx.x < NR_NPART) {
-        const int k = threadIdx.x;
-        const bool ismax = k == 15;
-        double r = seg[k * RED_SEGS];
-        for (int sg = 1; sg < RED_SEGS; ++sg) r = ismax ? fmax(r, seg[k * RED_SEGS + sg]) : r + seg[k * RED_SEGS + sg];
-        red[k] = r;
+// One outer iteration's bookkeeping on the device (the host loop of evolution.c:1150-1256): the
+// dDisGradAvg this iteration's inverse-z pass applied joins the uniform part, the reduced sums give the
+// errors and get_smacro's averages and correction, and `done` decides whether the next iteration runs.
+// One block; the iteration's other kernels have finished (stream order).
+// Bound by latency alone: the control block, the compliance S0 and the sums are fetched together, and
+// the first wavefront works the algebra out one tensor component per lane, in LDS (5.6-7.5 us a
+// launch when one thread did it with S0 in memory).  Up to NR_RED_ONE Newton blocks the kernel also sums
+// their partials itself, which saves k_reduce_seg's launch (4.6 us); beyond, one block's loads would
+// take longer than that.
+constexpr int CTL_BLOCK = 1024;
+// One wavefront's sum (and, for the last value, maximum too) of one value's partials, 8 loads per lane
+// in flight.
+__device__ __forceinline__ void sum_partials(const double *__restrict__ row, int nblocks, double &sum, double &mx) {
+    constexpr int U = 8;
+    double acc[U], m = -1e308;
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[u] = 0.0;
+    for (int b0 = threadIdx.x & 63; b0 < nblocks; b0 += U * 64) {
+        double x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = row[min(b0 + u * 64, nblocks - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool in = b0 + u * 64 < nblocks;
+            acc[u] += in ? x[u] : 0.0;
+            m = fmax(m, x[u]);
+        }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) control_step(cst, lc, red);
-    __syncthreads();
-    for (int i = threadIdx.x; i < NW; i += blockDim.x)
-        reinterpret_cast<unsigned long long *>(ctl)[i] = reinterpret_cast<const unsigned long long *>(&lc)[i];
+#pragma unroll
+    for (int st = U / 2; st > 0; st >>= 1)
+#pragma unroll
+        for (int u = 0; u < st; ++u) acc[u] += acc[u + st];
+    sum = wave_sum(acc[0]);
+    mx = m;
 }
 
-__global__ void k_control(const DevConst *__restrict__ cst, const double *__restrict__ seg, IterCtl *ctl) {
-    control_block(cst, seg, ctl);
+// orders one wavefront's LDS writes before its lanes' reads of each other's values
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// the B basis as a table, [6][9], for lanes that hold one component each
+#define SRX_BB(i) bbasis(i, 0, 0), bbasis(i, 0, 1), bbasis(i, 0, 2), bbasis(i, 1, 0), bbasis(i, 1, 1), bbasis(i, 1, 2), \
+                  bbasis(i, 2, 0), bbasis(i, 2, 1), bbasis(i, 2, 2)
+__constant__ double k_bbasis[54] = {SRX_BB(0), SRX_BB(1), SRX_BB(2), SRX_BB(3), SRX_BB(4), SRX_BB(5)};
+#undef SRX_BB
+// get_smacro (evolution.c:590-664) by the first wavefront, one component per lane: volume averages, the
+// strain correction dDisGradAvg of the stress-controlled components (upper-triangle entries only), and
+// the two von Mises measures (the first with the out-of-bounds SigDevAvg[3][3] term of evolution.c:648
+// taken as svm_stray).
+// bcol: column l mod 9 of the B basis (tensor entry l mod 9 of each basis tensor), brow: its row l.
+__device__ __forceinline__ void smacro_wave(IterCtl &c, const double *S0, const double *sum6, const double *sum6_ph1,
+                                            const double bcol[6], const double brow[9], double *sda, double *sda1) {
+    constexpr int UP[6] = {0, 4, 8, 5, 2, 1};   // tensor entries of the six upper-triangle components
+    const int l = threadIdx.x;
+    if (l < 18) {   // the averages: tensor entries of the sums
+        const int k = l < 9 ? l : l - 9;
+        const double *v = l < 9 ? sum6 : sum6_ph1;
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < 6; ++i) t += v[i] * bcol[i];
+        if (l < 9) c.SigAvg[k] = t * c.wgt;
+        else c.SigAvg1[k] = t * (c.wgt / c.wgt_ph1);
+    }
+    wave_sync();
+    if (l < 9) c.ddg[l] = 0.0;   // (lower-triangle entries are never set)
+    wave_sync();
+    if (l < 6) {
+        const int q = UP[l];
+        double acc = 0.0;
+        if (c.vbc[l] == 0) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) acc += S0[q * 9 + UP[k]] * c.sbc[k] * (c.Scauchy[UP[k]] - c.SigAvg[UP[k]]);
+        }
+        c.ddg[q] = acc;
+    }
+    // deviators of the two averages: tensor entries of their five deviatoric B-basis components
+    if (l < 18) {
+        const int k = l < 9 ? l : l - 9;
+        const double *a = l < 9 ? c.SigAvg : c.SigAvg1;
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            double b = 0.0;
+#pragma unroll
+            for (int e = 0; e < 9; ++e) b += a[e] * bbasis(i, e / 3, e % 3);
+            t += b * bcol[i];
+        }
+        (l < 9 ? sda : sda1)[k] = t;
+    }
+    wave_sync();
+    if (l < 9) c.acum[l] += c.ddg[l];
+    if (l < 6) {   // sym(dDisGradAvg) in the B basis
+        double b = 0.0;
+#pragma unroll
+        for (int e = 0; e < 9; ++e) {
+            const int i = e / 3, j = e % 3;
+            b += 0.5 * (c.ddg[e] + c.ddg[3 * j + i]) * brow[e];
+        }
+        c.ddg6[l] = b;
+    }
+    if (l == 0) {
+        const double tr = c.svm_mode == 1 ? (sda[0] + sda[4] + sda[8]) : (sda[4] + sda[8] + c.svm_stray);
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            const double x = sda[k];
+            s += k % 4 ? x * x : (x - tr / 3.0) * (x - tr / 3.0);
+        }
+        c.s_vm = sqrt(3. / 2. * s);
+    }
+    if (l == 1) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) s += sda1[k] * sda1[k];
+        c.s_vm1 = sqrt(3. / 2. * s);
+    }
+    wave_sync();
+}
+
+__device__ __forceinline__ void control_block(const DevConst *__restrict__ cst, const double *__restrict__ part,
+                                              int nblocks, const double *__restrict__ seg, IterCtl *ctl) {
+    static_assert(sizeof(IterCtl) % 8 == 0, "IterCtl is copied as 64-bit words");
+    constexpr int NW = sizeof(IterCtl) / 8;
+    static_assert(NW + 81 <= CTL_BLOCK, "one word per thread");
+    __shared__ IterCtl c;
+    __shared__ double S0[81], red[NR_NPART], sda[9], sda1[9];
+    const int t = threadIdx.x, nt = blockDim.x;
+    for (int i = t; i < NW; i += nt)
+        reinterpret_cast<unsigned long long *>(&c)[i] = reinterpret_cast<const unsigned long long *>(ctl)[i];
+    for (int i = t; i < 81; i += nt) S0[i] = cst->S0[i];
+    double bcol[6], brow[9];
+    if (t < 64) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) bcol[i] = k_bbasis[i * 9 + t % 9];
+#pragma unroll
+        for (int e = 0; e < 9; ++e) brow[e] = k_bbasis[t % 6 * 9 + e];
+    }
+    if (nblocks <= NR_RED_ONE) {
+        // wavefront w: value w, the last two also 16 (a flag) and 17 (the sum of what 15 is the maximum of)
+        static_assert(NR_NPART == 18 && CTL_BLOCK == 16 * 64, "18 values over 16 wavefronts");
+        const int w = t >> 6;
+        double r, m;
+        sum_partials(part + (size_t)w * nblocks, nblocks, r, m);
+        if (w == 15) m = wave_max(m);
+        if ((t & 63) == 0) {
+            red[w] = w == 15 ? m : r;
+            if (w == 15) red[17] = r;
+        }
+        if (w == 14) {
+            sum_partials(part + (size_t)16 * nblocks, nblocks, r, m);
+            if ((t & 63) == 0) red[16] = r;
+        }
+    } else if (t < NR_NPART) {
+        // second stage of the reduction: the RED_SEGS partial results of each value, in order
+        double r = seg[t * RED_SEGS];
+#pragma unroll
+        for (int sg = 1; sg < RED_SEGS; ++sg) r = t == 15 ? fmax(r, seg[t * RED_SEGS + sg]) : r + seg[t * RED_SEGS + sg];
+        red[t] = r;
+    }
+    __syncthreads();
+    if (c.done) return;
+    if (t < 64) {
+        const bool bad = red[16] > 0;   // a non-finite stress (the reference asserts, constitutive.c:683)
+        if (t < 9) c.uniform[t] += c.ddg[t];
+        if (t < 6 && !bad) c.sig_sum6[t] = red[2 + t];
+        wave_sync();
+        if (!bad) smacro_wave(c, S0, red + 2, red + 8, bcol, brow, sda, sda1);
+        if (t < 6 && !bad) {
+            const double m = c.mixed ? red[2 + t] / c.nvox : 0.0;
+            c.mean6[t] = m;
+            c.dcs6[t] = c.mixed ? m * c.nvox : 0.0;
+        }
+        if (t == 0) {
+            c.iter += 1;
+            if (bad) {
+                c.nan = 1;
+                c.done = 1;
+            } else {
+                c.nrtot += (long long)red[14];
+                c.nrmax = max(c.nrmax, (int)red[15]);
+                c.nrwave += red[17];
+                const double ee = red[1] * c.wgt;
+                c.Err_e = fabs(c.e_vm_prev) < 1E-5 ? 0.0 : ee / c.e_vm_prev;
+                c.Err_s = red[0] * c.wgt / c.s_vm;
+                c.done = ctl_stop(c);
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = t; i < NW; i += nt)
+        reinterpret_cast<unsigned long long *>(ctl)[i] = reinterpret_cast<const unsigned long long *>(&c)[i];
+}
+
+__global__ void __launch_bounds__(CTL_BLOCK) k_control(const DevConst *__restrict__ cst, const double *__restrict__ part,
+                                                       int nblocks, const double *__restrict__ seg, IterCtl *ctl) {
+    control_block(cst, part, nblocks, seg, ctl);
 }
 
 // the same for every member of an ensemble (one block each); done[m] receives the member's stop
 // flag, the only value the host reads between batches of iterations
-__global__ void k_control_ens(const EnsMember *__restrict__ tab, int *__restrict__ done) {
+__global__ void __launch_bounds__(CTL_BLOCK) k_control_ens(const EnsMember *__restrict__ tab, int *__restrict__ done) {
     const EnsMember &e = tab[blockIdx.x];
-    control_block(e.cst, e.redseg, e.ctl);
+    control_block(e.cst, e.partials, e.nblk, e.redseg, e.ctl);
     __syncthreads();
     if (threadIdx.x == 0) done[blockIdx.x] = e.ctl->done;
-}
-
-// one outer iteration's bookkeeping on the reduced values red[] (thread 0 of k_control)
-__device__ __forceinline__ void control_step(const DevConst *__restrict__ cst, IterCtl &c, const double *red) {
-    for (int k = 0; k < 9; ++k) c.uniform[k] += c.ddg[k];
-    c.iter += 1;
-    if (red[16] > 0) {   // a non-finite stress (the reference asserts, constitutive.c:683)
-        c.nan = 1;
-        c.done = 1;
-        return;
-    }
-    for (int k = 0; k < 6; ++k) c.sig_sum6[k] = red[2 + k];
-    c.nrtot += (long long)red[14];
-    c.nrmax = max(c.nrmax, (int)red[15]);
-    c.nrwave += red[17];
-    c.Err_e = red[1] * c.wgt;
-    c.Err_s = red[0] * c.wgt;
-    smacro_update(c, cst->S0, red + 2, red + 8);
-    if (fabs(c.e_vm_prev) < 1E-5) c.Err_e = 0.0;
-    else c.Err_e /= c.e_vm_prev;
-    c.Err_s /= c.s_vm;
-    for (int k = 0; k < 6; ++k) {
-        c.mean6[k] = c.mixed ? c.sig_sum6[k] / c.nvox : 0.0;
-        c.dcs6[k] = c.mixed ? c.mean6[k] * c.nvox : 0.0;
-    }
-    const double s12 = 0.5 * (c.ddg[5] + c.ddg[7]), s02 = 0.5 * (c.ddg[2] + c.ddg[6]), s01 = 0.5 * (c.ddg[1] + c.ddg[3]);
-    const double sym[9] = {c.ddg[0], s01, s02, s01, c.ddg[4], s12, s02, s12, c.ddg[8]};
-    ctl_t9_to_b6(sym, c.ddg6);
-    c.done = ctl_stop(c);
 }
 
 // ---------------------------------------------------------------------------
@@ -1186,6 +1323,7 @@ void launch_reduce_end_ens(hipStream_t s, const EnsIncr *tab, int nmem) {
 }
 
 void launch_reduce_nr(hipStream_t s, const double *partials, int nblocks, double *seg, const IterCtl *ctl) {
+    if (nblocks <= NR_RED_ONE) return;   // left to k_control
     SRX_LAUNCH(k_reduce_seg, dim3(NR_NPART, RED_SEGS), dim3(RED_SEG_BLOCK), 0, s, partials, nblocks, 1ull << 15, seg,
                ctl);
     check_launch("reduce");
@@ -1205,12 +1343,13 @@ void launch_reduce_nr_ens(hipStream_t s, const EnsMember *tab, int nmem) {
 }
 
 void launch_control_ens(hipStream_t s, const EnsMember *tab, int nmem, int *done) {
-    SRX_LAUNCH(k_control_ens, dim3(nmem), dim3(64), 0, s, tab, done);
+    SRX_LAUNCH(k_control_ens, dim3(nmem), dim3(CTL_BLOCK), 0, s, tab, done);
     check_launch("control_ens");
 }
 
-void launch_control(hipStream_t s, const DevConst *cst, const double *seg, IterCtl *ctl) {
-    SRX_LAUNCH(k_control, dim3(1), dim3(64), 0, s, cst, seg, ctl);
+void launch_control(hipStream_t s, const DevConst *cst, const double *partials, int nblocks, const double *seg,
+                    IterCtl *ctl) {
+    SRX_LAUNCH(k_control, dim3(1), dim3(nblocks <= NR_RED_ONE ? CTL_BLOCK : 256), 0, s, cst, partials, nblocks, seg, ctl);
     check_launch("control");
 }
 

@@ -107,7 +107,7 @@ struct DevConst {
 
 // Outer fixed-point control kept on the device.  The mixed boundary-condition algebra
 // (get_smacro, evolution.c:590-664) and the convergence test (evolution.c:1150, 1246-1252) run in
-// a one-thread kernel after each iteration's reduction, so the host enqueues several iterations
+// a one-block kernel after each iteration's reduction, so the host enqueues several iterations
 // without reading anything back in between; every kernel of an iteration returns at once when
 // `done` is set.
 struct IterCtl {
@@ -143,66 +143,6 @@ __host__ __device__ constexpr double bbasis(int i, int a, int b) {
     default: return a == b ? R3 : 0.0;
     }
 }
-__host__ __device__ inline void ctl_b6_to_t9(const double v[6], double t[9], int dim) {
-    for (int a = 0; a < 3; ++a)
-        for (int b = 0; b < 3; ++b) {
-            double s = 0.0;
-            for (int i = 0; i < dim; ++i) s += v[i] * bbasis(i, a, b);
-            t[3 * a + b] = s;
-        }
-}
-__host__ __device__ inline void ctl_t9_to_b6(const double t[9], double v[6]) {
-    for (int i = 0; i < 6; ++i) {
-        double s = 0.0;
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b) s += t[3 * a + b] * bbasis(i, a, b);
-        v[i] = s;
-    }
-}
-
-// get_smacro (evolution.c:590-664): volume averages, the strain correction dDisGradAvg of the
-// stress-controlled components (upper-triangle entries only), and the two von Mises measures
-// (the first with the out-of-bounds SigDevAvg[3][3] term of evolution.c:648 taken as svm_stray).
-__host__ __device__ inline void smacro_update(IterCtl &c, const double *S0, const double sum6[6],
-                                              const double sum6_ph1[6]) {
-    const int IJV[2][6] = {{0, 1, 2, 1, 0, 0}, {0, 1, 2, 2, 2, 1}};
-    double t[9], t1[9];
-    ctl_b6_to_t9(sum6, t, 6);
-    ctl_b6_to_t9(sum6_ph1, t1, 6);
-    for (int k = 0; k < 9; ++k) {
-        c.SigAvg[k] = t[k] * c.wgt;
-        c.SigAvg1[k] = t1[k] * (c.wgt / c.wgt_ph1);
-    }
-    for (int i = 0; i < 6; ++i) {
-        const int ii = IJV[0][i], jj = IJV[1][i];
-        double acc = 0.0;
-        if (c.vbc[i] == 0) {
-            for (int k = 0; k < 6; ++k) {
-                const int kk = IJV[0][k], ll = IJV[1][k];
-                acc += S0[((ii * 3 + jj) * 3 + kk) * 3 + ll] * c.sbc[k] * (c.Scauchy[3 * kk + ll] - c.SigAvg[3 * kk + ll]);
-            }
-        }
-        c.ddg[3 * ii + jj] = acc;
-    }
-    for (int k = 0; k < 9; ++k) c.acum[k] += c.ddg[k];
-    double sav6[6], sda[9];
-    ctl_t9_to_b6(c.SigAvg, sav6);
-    ctl_b6_to_t9(sav6, sda, 5);
-    const double tr = c.svm_mode == 1 ? (sda[0] + sda[4] + sda[8]) : (sda[4] + sda[8] + c.svm_stray);
-    double s = 0.0;
-    for (int i = 0; i < 3; ++i)
-        for (int j = 0; j < 3; ++j) {
-            const double x = sda[3 * i + j];
-            s += i != j ? x * x : (x - tr / 3.0) * (x - tr / 3.0);
-        }
-    c.s_vm = sqrt(3. / 2. * s);
-    ctl_t9_to_b6(c.SigAvg1, sav6);
-    ctl_b6_to_t9(sav6, sda, 5);
-    s = 0.0;
-    for (int k = 0; k < 9; ++k) s += sda[k] * sda[k];
-    c.s_vm1 = sqrt(3. / 2. * s);
-}
-
 // whether the outer loop stops before iteration c.iter + 1 (evolution.c:1150; fixed_iters > 0:
 // exactly that many iterations)
 __host__ __device__ inline int ctl_stop(const IterCtl &c) {
@@ -331,11 +271,14 @@ void launch_nr(hipStream_t s, const DevConst *cst, const Fields &f, int nvox, in
 void launch_reduce(hipStream_t s, const double *partials, int nblocks, int nvals, double *out,
                    const IterCtl *ctl = nullptr);
 // The per-iteration reduction of the Newton kernel's block partials in two fixed-order stages:
-// launch_reduce_nr writes NR_NPART x 16 segment results to seg, launch_control sums them and does
-// the iteration's bookkeeping (get_smacro and the convergence test).
+// launch_reduce_nr writes NR_NPART x 16 segment results to seg, launch_control sums them (of few blocks
+// it sums the partials itself, and launch_reduce_nr launches nothing) and does the iteration's
+// bookkeeping (get_smacro and the convergence test).
 constexpr int NR_RED_SEG_DOUBLES = NR_NPART * 16;
+constexpr int NR_RED_ONE = 512;   // up to so many Newton blocks launch_control sums their partials itself
 void launch_reduce_nr(hipStream_t s, const double *partials, int nblocks, double *seg, const IterCtl *ctl);
-void launch_control(hipStream_t s, const DevConst *cst, const double *seg, IterCtl *ctl);
+void launch_control(hipStream_t s, const DevConst *cst, const double *partials, int nblocks, const double *seg,
+                    IterCtl *ctl);
 // The same three kernels over every member of an ensemble in one launch each (tab: device array of
 // nmem members; nblocks: their Newton blocks in total; ws: the Newton start option; done[m]: each
 // member's stop flag after the iteration; f32: every member runs in mixed precision and keeps quaternions;
