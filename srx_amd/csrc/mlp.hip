@@ -79,130 +79,197 @@ __global__ void __launch_bounds__(64) k_mlp_infer(const MlpPacked *__restrict__ 
         for (int k = 0; k < MLP_OUT; ++k) y[(size_t)j * MLP_OUT + k] = o[k] * M->ts[k] + M->tm[k];
 }
 
-// One training wavefront: forward for its 64 samples (indices idx[base + ...], or base + ... when
-// idx is null), loss sum((y - t')^2) over normalised targets t' = (t - mean) / spread, and the
-// gradient of scale * loss, written to part[block][0, MLP_NPARAM) with the loss at MLP_NPARAM.
-// Straight-through bf16: the backward pass uses the same rounded weights, inputs and hidden
-// values as the forward pass, in FP32 arithmetic.
-constexpr int MLP_P = MLP_H + 1;   // LDS pitch of the [sample][unit] arrays
-__global__ void __launch_bounds__(64) k_mlp_fwdbwd(const MlpPacked *__restrict__ M, const float *__restrict__ x,
-                                                   const float *__restrict__ t, const int *__restrict__ idx,
-                                                   int base, int nb, float scale, float *__restrict__ part) {
-    __shared__ float h1l[64 * MLP_P], h2l[64 * MLP_P], d2l[64 * MLP_P];
-    __shared__ float xq[64 * (MLP_IN + 1)], dyl[64 * (MLP_OUT + 1)];
-    float *d1l = h2l;   // dz1 replaces h2 once the W3 gradient has been taken
-    const int lane = threadIdx.x;
-    const int j = blockIdx.x * 64 + lane;
-    const bool valid = j < nb;
-    const size_t si = valid ? (size_t)(idx ? idx[base + j] : base + j) : 0;
-    float xn[MLP_IN], y[MLP_OUT];
+// One training block: the 64 samples of sample block blk (indices idx[base + ...], or base + ... when
+// idx is null) and the MLP_HS hidden units of layer 1 from MLP_HS * sp on.  The first wavefront runs
+// the forward pass; loss sum((y - t')^2) over normalised targets t' = (t - mean) / spread, and the
+// gradient of scale * loss, go to part[blk][0, MLP_NPARAM) with the loss at MLP_NPARAM.  Straight-through
+// bf16: the backward pass uses the same rounded weights, inputs and hidden values as the forward
+// pass, in FP32 arithmetic, every sum over samples or units in ascending order.
+//
+// Bound by the length of one block's chain, not by the chip: a batch of 4096 is 64 blocks of samples
+// and 43 MFLOP backward.  dW2's rows, dz1 and dW1's columns of different layer-1 units are
+// independent, so MLP_SPLIT blocks share a block of samples (each repeats the forward pass and dz2,
+// a tenth of the work) and eight wavefronts share a block's units: one wavefront for all of it took
+// 70 us at a batch of 4096, this takes 14 us.  The LDS rows of 68 floats keep both orders free of bank
+// conflicts: 16-byte reads along a sample's row by 64 samples, and 64 units of one sample.
+constexpr int MLP_SPLIT = 4, MLP_HS = MLP_H / MLP_SPLIT, MLP_TB = 512, MLP_WV = MLP_TB / 64;
+constexpr int MLP_P = MLP_H + 4;    // pitch of [sample][unit of layer 2]
+constexpr int MLP_P1 = MLP_HS + 4;  // pitch of [sample][own unit of layer 1]
+static_assert(MLP_H == 64 && MLP_H / MLP_WV == 8 && MLP_HS / MLP_WV == 2 && MLP_HS * (MLP_IN + 1) <= MLP_TB, "");
+__global__ void __launch_bounds__(MLP_TB) k_mlp_fwdbwd(const MlpPacked *__restrict__ M, const float *__restrict__ x,
+                                                       const float *__restrict__ t, const int *__restrict__ idx,
+                                                       int base, int blk0, int nb, float scale,
+                                                       float *__restrict__ part) {
+    __shared__ __attribute__((aligned(16))) float h1l[64 * MLP_P1], h2l[64 * MLP_P], d2l[64 * MLP_P];
+    __shared__ __attribute__((aligned(16))) float w2l[MLP_HS * MLP_H], w3l[MLP_H * MLP_OUT];
+    __shared__ float d1l[64 * (MLP_HS + 1)], xq[64 * (MLP_IN + 1)], dyl[64 * (MLP_OUT + 1)];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int sp = blockIdx.x % MLP_SPLIT, blk = blk0 + blockIdx.x / MLP_SPLIT;
+    float *out = part + (size_t)blk * (MLP_NPARAM + 1);
+    if (wv == 0) {
+        const int j = blk * 64 + lane;
+        const bool valid = j < nb;
+        const size_t si = valid ? (size_t)(idx ? idx[base + j] : base + j) : 0;
+        float xn[MLP_IN], y[MLP_OUT];
 #pragma unroll
-    for (int k = 0; k < MLP_IN; ++k) xn[k] = valid ? x[si * MLP_IN + k] : 0.0f;
-    mlp_normalise(M, xn);
-    MlpAcc z;
-    mlp_forward_wave<true>(M, xn, y, z);
-    const int g = lane >> 5;
+        for (int k = 0; k < MLP_IN; ++k) xn[k] = valid ? x[si * MLP_IN + k] : 0.0f;
+        mlp_normalise(M, xn);
+        MlpAcc z;
+        mlp_forward_wave<true>(M, xn, y, z);
+        const int g = lane >> 5;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+        for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
+            for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int s = 32 * cb + (lane & 31), u = mlp_acc_unit(rb, g, r);
-                h1l[s * MLP_P + u] = bf16r(fmaxf(z.z1[rb][cb][r], 0.0f));
-                h2l[s * MLP_P + u] = bf16r(fmaxf(z.z2[rb][cb][r], 0.0f));
-            }
+                for (int r = 0; r < 16; ++r) {
+                    const int s = 32 * cb + (lane & 31), u = mlp_acc_unit(rb, g, r);
+                    if (2 * rb + r / 8 == sp) h1l[s * MLP_P1 + u % MLP_HS] = bf16r(fmaxf(z.z1[rb][cb][r], 0.0f));
+                    h2l[s * MLP_P + u] = bf16r(fmaxf(z.z2[rb][cb][r], 0.0f));
+                }
 #pragma unroll
-    for (int k = 0; k < MLP_IN; ++k) xq[lane * (MLP_IN + 1) + k] = bf16r(xn[k]);
-    float dy[MLP_OUT], loss = 0.0f;
+        for (int k = 0; k < MLP_IN; ++k) xq[lane * (MLP_IN + 1) + k] = bf16r(xn[k]);
+        float loss = 0.0f;
 #pragma unroll
-    for (int o = 0; o < MLP_OUT; ++o) {
-        const float tn = valid ? (t[si * MLP_OUT + o] - M->tm[o]) / M->ts[o] : 0.0f;
-        const float e = y[o] - tn;
-        dy[o] = valid ? scale * e : 0.0f;
-        loss += valid ? e * e : 0.0f;
-        dyl[lane * (MLP_OUT + 1) + o] = dy[o];
+        for (int o = 0; o < MLP_OUT; ++o) {
+            const float tn = valid ? (t[si * MLP_OUT + o] - M->tm[o]) / M->ts[o] : 0.0f;
+            const float e = y[o] - tn;
+            loss += valid ? e * e : 0.0f;
+            dyl[lane * (MLP_OUT + 1) + o] = valid ? scale * e : 0.0f;
+        }
+        if (sp == 0) {
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o, 64);
+            if (lane == 0) out[MLP_NPARAM] = loss;
+        }
+    } else {
+        for (int k = tid - 64; k < MLP_HS * MLP_H; k += MLP_TB - 64) w2l[k] = M->wq[MLP_OFF_W2 + sp * MLP_HS * MLP_H + k];
+        for (int k = tid - 64; k < MLP_H * MLP_OUT; k += MLP_TB - 64) w3l[k] = M->wq[MLP_OFF_W3 + k];
     }
     __syncthreads();
-    float *out = part + (size_t)blockIdx.x * (MLP_NPARAM + 1);
-    const float *wq = M->wq;
-    {   // W3 [u][o] and b3, lane = hidden unit u of layer 2
-        float acc[MLP_OUT] = {0, 0, 0, 0, 0, 0};
-        for (int s = 0; s < 64; ++s) {
-            const float h = h2l[s * MLP_P + lane];
+    {   // lane = sample: dz2 = (W3 dy) o [z2 > 0], eight units a wavefront
+        float dy[MLP_OUT];
 #pragma unroll
-            for (int o = 0; o < MLP_OUT; ++o) acc[o] += h * dyl[s * (MLP_OUT + 1) + o];
+        for (int o = 0; o < MLP_OUT; ++o) dy[o] = dyl[lane * (MLP_OUT + 1) + o];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int u = 8 * wv + q;
+            float a = 0.0f;
+#pragma unroll
+            for (int o = 0; o < MLP_OUT; ++o) a += w3l[u * MLP_OUT + o] * dy[o];
+            d2l[lane * MLP_P + u] = h2l[lane * MLP_P + u] > 0.0f ? a : 0.0f;
         }
-#pragma unroll
-        for (int o = 0; o < MLP_OUT; ++o) out[MLP_OFF_W3 + lane * MLP_OUT + o] = acc[o];
-        if (lane < MLP_OUT) {
-            float b = 0.0f;
-            for (int s = 0; s < 64; ++s) b += dyl[s * (MLP_OUT + 1) + lane];
-            out[MLP_OFF_B3 + lane] = b;
-        }
-    }
-    // lane = sample: dz2 = (W3 dy) o [z2 > 0], dz1 = (W2 dz2) o [z1 > 0]
-    float dz2[MLP_H];
-#pragma unroll
-    for (int u = 0; u < MLP_H; ++u) {
-        float a = 0.0f;
-#pragma unroll
-        for (int o = 0; o < MLP_OUT; ++o) a += wq[MLP_OFF_W3 + u * MLP_OUT + o] * dy[o];
-        dz2[u] = h2l[lane * MLP_P + u] > 0.0f ? a : 0.0f;
-        d2l[lane * MLP_P + u] = dz2[u];
-    }
-    __syncthreads();   // every lane has read h2l before it is overwritten by dz1
-    for (int i = 0; i < MLP_H; ++i) {
-        float a = 0.0f;
-#pragma unroll
-        for (int u = 0; u < MLP_H; ++u) a += wq[MLP_OFF_W2 + i * MLP_H + u] * dz2[u];
-        d1l[lane * MLP_P + i] = h1l[lane * MLP_P + i] > 0.0f ? a : 0.0f;
     }
     __syncthreads();
-    {   // W2 [i][u] and b2, lane = unit u of layer 2
-        float acc[MLP_H];
+    {   // lane = sample: dz1 = (W2 dz2) o [z1 > 0], two units a wavefront
+        float a[2] = {0.0f, 0.0f};
 #pragma unroll
-        for (int i = 0; i < MLP_H; ++i) acc[i] = 0.0f;
-        float b = 0.0f;
+        for (int u = 0; u < MLP_H; ++u)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) a[q] += w2l[(2 * wv + q) * MLP_H + u] * d2l[lane * MLP_P + u];
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            d1l[lane * (MLP_HS + 1) + 2 * wv + q] = h1l[lane * MLP_P1 + 2 * wv + q] > 0.0f ? a[q] : 0.0f;
+    }
+    {   // lane = unit u of layer 2: W2 [i][u], two rows i a wavefront
+        float acc[2] = {0.0f, 0.0f};
+#pragma unroll 16
         for (int s = 0; s < 64; ++s) {
             const float d = d2l[s * MLP_P + lane];
-            b += d;
 #pragma unroll
-            for (int i = 0; i < MLP_H; ++i) acc[i] += h1l[s * MLP_P + i] * d;
+            for (int q = 0; q < 2; ++q) acc[q] += h1l[s * MLP_P1 + 2 * wv + q] * d;
         }
 #pragma unroll
-        for (int i = 0; i < MLP_H; ++i) out[MLP_OFF_W2 + i * MLP_H + lane] = acc[i];
-        out[MLP_OFF_B2 + lane] = b;
+        for (int q = 0; q < 2; ++q) out[MLP_OFF_W2 + (sp * MLP_HS + 2 * wv + q) * MLP_H + lane] = acc[q];
     }
-    {   // W1 [k][u] and b1, lane = unit u of layer 1
-        float acc[MLP_IN];
-#pragma unroll
-        for (int k = 0; k < MLP_IN; ++k) acc[k] = 0.0f;
+    // The sums that no layer-1 unit divides are shared out by block and wavefront: W3 [u][o] with lane
+    // = u, two outputs o in each of the first three blocks; b2 and b3 in the last.
+    if (2 * sp < MLP_OUT) {
+        if (wv < 2) {
+            const int o = 2 * sp + wv;
+            float acc = 0.0f;
+#pragma unroll 16
+            for (int s = 0; s < 64; ++s) acc += h2l[s * MLP_P + lane] * dyl[s * (MLP_OUT + 1) + o];
+            out[MLP_OFF_W3 + lane * MLP_OUT + o] = acc;
+        }
+    } else if (wv == 0) {
         float b = 0.0f;
-        for (int s = 0; s < 64; ++s) {
-            const float d = d1l[s * MLP_P + lane];
-            b += d;
-#pragma unroll
-            for (int k = 0; k < MLP_IN; ++k) acc[k] += xq[s * (MLP_IN + 1) + k] * d;
-        }
-#pragma unroll
-        for (int k = 0; k < MLP_IN; ++k) out[MLP_OFF_W1 + k * MLP_H + lane] = acc[k];
-        out[MLP_OFF_B1 + lane] = b;
+#pragma unroll 16
+        for (int s = 0; s < 64; ++s) b += d2l[s * MLP_P + lane];
+        out[MLP_OFF_B2 + lane] = b;
+    } else if (wv == 1 && lane < MLP_OUT) {
+        float b = 0.0f;
+#pragma unroll 16
+        for (int s = 0; s < 64; ++s) b += dyl[s * (MLP_OUT + 1) + lane];
+        out[MLP_OFF_B3 + lane] = b;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o, 64);
-    if (lane == 0) out[MLP_NPARAM] = loss;
+    __syncthreads();
+    // W1 [k][own unit] and b1: one thread a sum
+    const int i = tid % MLP_HS, k = tid / MLP_HS;
+    if (k < MLP_IN) {
+        float acc = 0.0f;
+#pragma unroll 16
+        for (int s = 0; s < 64; ++s) acc += xq[s * (MLP_IN + 1) + k] * d1l[s * (MLP_HS + 1) + i];
+        out[MLP_OFF_W1 + k * MLP_H + sp * MLP_HS + i] = acc;
+    } else if (k == MLP_IN) {
+        float b = 0.0f;
+#pragma unroll 16
+        for (int s = 0; s < 64; ++s) b += d1l[s * (MLP_HS + 1) + i];
+        out[MLP_OFF_B1 + sp * MLP_HS + i] = b;
+    }
+}
+
+// Writes parameter p's new value v to its places in the packed operands (k_mlp_pack's layout; each
+// weight has one place there, the padding is written by the full packing alone).
+__device__ __forceinline__ void mlp_repack(MlpPacked *__restrict__ M, int p, float v) {
+    // mlp_k_unit and mlp_acc_unit inverted: unit u is in row block u / 32, half (u / 16) % 2, lane half (u / 4) % 2
+    auto lane_half = [](int u) { return (u >> 2) & 1; };
+    auto k_step = [](int u) { return u >> 4; };
+    auto k_elem = [](int u) { return 4 * ((u >> 3) & 1) + (u & 3); };
+    auto acc_reg = [](int u) { return 4 * ((u >> 3) & 3) + (u & 3); };
+    M->wq[p] = mlp_is_weight(p) ? bf16r(v) : v;
+    if (p < MLP_OFF_B1) {
+        const int k = p / MLP_H, m = p % MLP_H;
+        M->a1[m >> 5][k >> 4][(m & 31) + 32 * ((k >> 3) & 1)][k & 7] = (__bf16)v;
+    } else if (p < MLP_OFF_W2) {
+        const int u = p - MLP_OFF_B1;
+        M->b1[u >> 5][lane_half(u)][acc_reg(u)] = v;
+    } else if (p < MLP_OFF_B2) {
+        const int u = (p - MLP_OFF_W2) / MLP_H, m = (p - MLP_OFF_W2) % MLP_H;
+        M->a2[m >> 5][k_step(u)][(m & 31) + 32 * lane_half(u)][k_elem(u)] = (__bf16)v;
+    } else if (p < MLP_OFF_W3) {
+        const int u = p - MLP_OFF_B2;
+        M->b2[u >> 5][lane_half(u)][acc_reg(u)] = v;
+    } else if (p < MLP_OFF_B3) {
+        const int u = (p - MLP_OFF_W3) / MLP_OUT, m = (p - MLP_OFF_W3) % MLP_OUT;
+        M->a3[k_step(u)][m + 32 * lane_half(u)][k_elem(u)] = (__bf16)v;
+    } else {
+        M->b3[p - MLP_OFF_B3] = v;
+    }
 }
 
 // Sum of the block partials in a fixed order (gradient and loss), then optionally one Adam step
-// on the FP32 master weights w (lr > 0).
-__global__ void k_mlp_adam(const float *__restrict__ part, int nparts, float *__restrict__ w, float *__restrict__ m,
-                           float *__restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2,
-                           float *__restrict__ loss_out, float *__restrict__ grad_out) {
+// on the FP32 master weights w (lr > 0), whose new values also go into the packed operands M.
+// Bound by the latency of the partials' loads: sixteen are in flight per thread and the parameters
+// are spread over 97 blocks of one wavefront (one load in flight and 25 blocks: 16.4 us for 64 partials; now 4.0 us).
+__global__ void __launch_bounds__(64) k_mlp_adam(const float *__restrict__ part, int nparts, float *__restrict__ w,
+                                                 float *__restrict__ m, float *__restrict__ v,
+                                                 MlpPacked *__restrict__ M, float lr, float b1, float b2, float eps,
+                                                 float c1, float c2, float *__restrict__ loss_out,
+                                                 float *__restrict__ grad_out) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p > MLP_NPARAM) return;
     float gsum = 0.0f;
-    for (int b = 0; b < nparts; ++b) gsum += part[(size_t)b * (MLP_NPARAM + 1) + p];
+    const float *src = part + p;
+    int b = 0;
+    for (; b + 16 <= nparts; b += 16, src += 16 * (MLP_NPARAM + 1)) {
+        float q[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) q[k] = src[k * (MLP_NPARAM + 1)];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) gsum += q[k];
+    }
+    for (; b < nparts; ++b, src += MLP_NPARAM + 1) gsum += *src;
     if (p == MLP_NPARAM) {
         if (loss_out) *loss_out = gsum;
         return;
@@ -213,7 +280,66 @@ __global__ void k_mlp_adam(const float *__restrict__ part, int nparts, float *__
         const float vv = b2 * v[p] + (1.0f - b2) * gsum * gsum;
         m[p] = mm;
         v[p] = vv;
-        w[p] -= lr * (mm * c1) / (sqrtf(vv * c2) + eps);
+        const float wn = w[p] - lr * (mm * c1) / (sqrtf(vv * c2) + eps);
+        w[p] = wn;
+        mlp_repack(M, p, wn);
+    }
+}
+
+// Column sums of the samples in FP64 (18 us for 65536 samples; on the host, column by column, they took
+// several milliseconds), features then targets: the values themselves, or with mean given
+// the squares of their distances from it.  Thread (row, column) of a block's 240 walks rows of its
+// column (reads are contiguous over the block); part [block][30].
+constexpr int MLP_COLS = MLP_IN + MLP_OUT, MLP_ST = 240, MLP_STAT_BLOCKS = 256;
+template <int NC>
+__device__ __forceinline__ void mlp_column_sums(const float *__restrict__ a, size_t n, const double *__restrict__ mean,
+                                                double *__restrict__ sh, double *__restrict__ out) {
+    constexpr int ROWS = MLP_ST / NC;
+    const int c = threadIdx.x % NC, r = threadIdx.x / NC;
+    const double mu = mean ? mean[c] : 0.0;
+    double sum = 0.0;
+#pragma unroll 8
+    for (size_t i = (size_t)blockIdx.x * ROWS + r; i < n; i += (size_t)gridDim.x * ROWS) {
+        const double d = (double)a[i * NC + c] - mu;
+        sum += mean ? d * d : d;
+    }
+    sh[threadIdx.x] = sum;
+    __syncthreads();
+    if (threadIdx.x < NC) {
+        double s = 0.0;
+        for (int k = 0; k < ROWS; ++k) s += sh[k * NC + threadIdx.x];
+        out[threadIdx.x] = s;
+    }
+    __syncthreads();
+}
+__global__ void __launch_bounds__(MLP_ST) k_mlp_sums(const float *__restrict__ x, const float *__restrict__ t, size_t n,
+                                                     const double *__restrict__ mean, double *__restrict__ part) {
+    __shared__ double sh[MLP_ST];
+    double *out = part + (size_t)blockIdx.x * MLP_COLS;
+    mlp_column_sums<MLP_IN>(x, n, mean, sh, out);
+    mlp_column_sums<MLP_OUT>(t, n, mean ? mean + MLP_IN : nullptr, sh, out + MLP_IN);
+}
+// Sums of the blocks' partials, in a fixed order: the columns' means (w null), or their spreads, with
+// the statistics written to the parameter blob w.
+__global__ void __launch_bounds__(64) k_mlp_stats(const double *__restrict__ part, int nblocks, size_t n,
+                                                  double *__restrict__ mean, float *__restrict__ w) {
+    const int c = threadIdx.x;
+    if (c >= MLP_COLS) return;
+    double s = 0.0;
+#pragma unroll 16
+    for (int b = 0; b < nblocks; ++b) s += part[(size_t)b * MLP_COLS + c];
+    s /= (double)n;
+    if (!w) {
+        mean[c] = s;
+        return;
+    }
+    const double sd = sqrt(s);
+    if (c < MLP_IN) {
+        w[MLP_OFF_XM + c] = (float)mean[c];
+        w[MLP_OFF_XS + c] = sd > 1e-6 ? (float)(1.0 / sd) : 1.0f;
+    } else {
+        w[MLP_OFF_TM + c - MLP_IN] = (float)mean[c];
+        w[MLP_OFF_TS + c - MLP_IN] = sd > 1e-12 ? (float)sd : 1.0f;
     }
 }
 
@@ -256,13 +382,15 @@ int check_blob(const float *blob) {
 }
 
 // one forward/backward over samples [base, base + nb) (or idx[base ...]), summed into grad/loss
-int grad_pass(hipStream_t s, const MlpPacked *M, const float *x, const float *t, const int *idx, int base, int nb,
+int grad_pass(hipStream_t s, MlpPacked *M, const float *x, const float *t, const int *idx, int base, int nb,
               float scale, float *part, float *w, float *m, float *v, float lr, float c1, float c2, float *loss,
               float *grad) {
     const int nblk = (nb + 63) / 64;
-    hipLaunchKernelGGL(k_mlp_fwdbwd, dim3(nblk), dim3(64), 0, s, M, x, t, idx, base, nb, scale, part);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((MLP_NPARAM + 1 + 255) / 256), dim3(256), 0, s, part, nblk, w, m, v, lr,
-                       0.9f, 0.999f, 1e-8f, c1, c2, loss, grad);
+    constexpr int CHUNK = 1 << 18;   // sample blocks of a launch: a grid holds less than 2^32 threads
+    for (int b0 = 0; b0 < nblk; b0 += CHUNK)
+        hipLaunchKernelGGL(k_mlp_fwdbwd, dim3(MLP_SPLIT * std::min(CHUNK, nblk - b0)), dim3(MLP_TB), 0, s, M, x, t, idx,
+                           base, b0, nb, scale, part);
+    hipLaunchKernelGGL(k_mlp_adam, dim3((MLP_NPARAM + 1 + 63) / 64), dim3(64), 0, s, part, nblk, w, m, v, M, lr, 0.9f, 0.999f, 1e-8f, c1, c2, loss, grad);
     return hipGetLastError() == hipSuccess ? 0 : SRX_E_HIP;
 }
 
@@ -337,25 +465,7 @@ int srx_mlp_train(const float *x, const float *t, size_t n, const srx_mlp_train_
         return SRX_E_ARG;
     std::mt19937_64 rng(o.seed);
     if (o.init) {
-        // feature and target statistics, then He-uniform weights and zero biases
-        for (int k = 0; k < MLP_IN; ++k) {
-            double s = 0.0, s2 = 0.0;
-            for (size_t i = 0; i < n; ++i) s += x[i * MLP_IN + k];
-            const double mu = s / (double)n;
-            for (size_t i = 0; i < n; ++i) s2 += (x[i * MLP_IN + k] - mu) * (x[i * MLP_IN + k] - mu);
-            const double sd = std::sqrt(s2 / (double)n);
-            blob[MLP_OFF_XM + k] = (float)mu;
-            blob[MLP_OFF_XS + k] = sd > 1e-6 ? (float)(1.0 / sd) : 1.0f;
-        }
-        for (int k = 0; k < MLP_OUT; ++k) {
-            double s = 0.0, s2 = 0.0;
-            for (size_t i = 0; i < n; ++i) s += t[i * MLP_OUT + k];
-            const double mu = s / (double)n;
-            for (size_t i = 0; i < n; ++i) s2 += (t[i * MLP_OUT + k] - mu) * (t[i * MLP_OUT + k] - mu);
-            const double sd = std::sqrt(s2 / (double)n);
-            blob[MLP_OFF_TM + k] = (float)mu;
-            blob[MLP_OFF_TS + k] = sd > 1e-12 ? (float)sd : 1.0f;
-        }
+        // He-uniform weights and zero biases; the feature and target statistics are taken on the device
         auto fill = [&](int off, int fan_in, int count) {
             const double lim = std::sqrt(6.0 / fan_in);
             std::uniform_real_distribution<double> U(-lim, lim);
@@ -366,16 +476,17 @@ int srx_mlp_train(const float *x, const float *t, size_t n, const srx_mlp_train_
         fill(MLP_OFF_W3, MLP_H, MLP_H * MLP_OUT);
         for (int i = 0; i < MLP_H; ++i) blob[MLP_OFF_B1 + i] = blob[MLP_OFF_B2 + i] = 0.0f;
         for (int i = 0; i < MLP_OUT; ++i) blob[MLP_OFF_B3 + i] = 0.0f;
+    } else if (int rc = check_blob(blob)) {
+        return rc;
     }
-    if (int rc = check_blob(blob)) return rc;
     const int B = o.batch;
     const size_t steps_per_epoch = (n + B - 1) / B;
     const int nblk = B / 64;
-    DevBuf dw, dM, dx, dt, didx, dpart, dm, dv, dl;
+    DevBuf dw, dM, dx, dt, didx, dpart, dm, dv, dst, dl;
     if (alloc(dw, MLP_BLOB * 4) || alloc(dM, sizeof(MlpPacked)) || alloc(dx, n * MLP_IN * 4) ||
         alloc(dt, n * MLP_OUT * 4) || alloc(didx, n * 4) || alloc(dpart, (size_t)nblk * (MLP_NPARAM + 1) * 4) ||
         alloc(dm, MLP_NPARAM * 4) || alloc(dv, MLP_NPARAM * 4) ||
-        alloc(dl, (size_t)o.epochs * steps_per_epoch * 4))
+        alloc(dst, o.init ? (MLP_STAT_BLOCKS + 1) * MLP_COLS * 8 : 0) || alloc(dl, (size_t)o.epochs * steps_per_epoch * 4))
         return SRX_E_NOMEM;
     hipStream_t s;
     MLP_CHK(hipStreamCreate(&s));
@@ -383,21 +494,32 @@ int srx_mlp_train(const float *x, const float *t, size_t n, const srx_mlp_train_
         hipStream_t s;
         ~StreamGuard() { (void)hipStreamDestroy(s); }
     } sg{s};
-    MLP_CHK(hipMemcpyAsync(dw.p, blob, MLP_BLOB * 4, hipMemcpyHostToDevice, s));
+    MLP_CHK(hipMemcpyAsync(dw.p, blob, (o.init ? MLP_NPARAM : MLP_BLOB) * 4, hipMemcpyHostToDevice, s));
     MLP_CHK(hipMemcpyAsync(dx.p, x, n * MLP_IN * 4, hipMemcpyHostToDevice, s));
     MLP_CHK(hipMemcpyAsync(dt.p, t, n * MLP_OUT * 4, hipMemcpyHostToDevice, s));
+    if (o.init) {
+        double *mean = dst.as<double>(), *part = mean + MLP_COLS;
+        for (int pass = 0; pass < 2; ++pass) {
+            hipLaunchKernelGGL(k_mlp_sums, dim3(MLP_STAT_BLOCKS), dim3(MLP_ST), 0, s, dx.as<float>(), dt.as<float>(), n,
+                               pass ? mean : nullptr, part);
+            hipLaunchKernelGGL(k_mlp_stats, dim3(1), dim3(64), 0, s, part, MLP_STAT_BLOCKS, n, mean,
+                               pass ? dw.as<float>() : nullptr);
+        }
+        MLP_CHK(hipGetLastError());
+    }
     MLP_CHK(hipMemsetAsync(dm.p, 0, MLP_NPARAM * 4, s));
     MLP_CHK(hipMemsetAsync(dv.p, 0, MLP_NPARAM * 4, s));
-    std::vector<int> idx(n);
-    std::iota(idx.begin(), idx.end(), 0);
+    // two index orders: the next epoch's is shuffled while the device works through the current one
+    std::vector<int> idx[2] = {std::vector<int>(n), std::vector<int>(o.epochs > 1 ? n : 0)};
+    std::iota(idx[0].begin(), idx[0].end(), 0);
+    std::shuffle(idx[0].begin(), idx[0].end(), rng);
     const size_t total = (size_t)o.epochs * steps_per_epoch;
     size_t step = 0;
     double b1t = 1.0, b2t = 1.0;
     const double lr0 = o.lr, lr1 = o.lr_final > 0.0f ? o.lr_final : o.lr;
     for (int ep = 0; ep < o.epochs; ++ep) {
-        std::shuffle(idx.begin(), idx.end(), rng);
-        // the index upload must complete before the host reshuffles for the next epoch
-        MLP_CHK(hipMemcpyAsync(didx.p, idx.data(), n * 4, hipMemcpyHostToDevice, s));
+        std::vector<int> &cur = idx[ep & 1], &next = idx[1 - (ep & 1)];
+        MLP_CHK(hipMemcpyAsync(didx.p, cur.data(), n * 4, hipMemcpyHostToDevice, s));
         for (size_t b0 = 0; b0 < n; b0 += B, ++step) {
             const int nb = (int)std::min((size_t)B, n - b0);
             if (step == 0) mlp_pack(s, dw.as<float>(), dM.as<MlpPacked>());
@@ -411,11 +533,14 @@ int srx_mlp_train(const float *x, const float *t, size_t n, const srx_mlp_train_
                           dv.as<float>(), lr, (float)(1.0 / (1.0 - b1t)), (float)(1.0 / (1.0 - b2t)),
                           dl.as<float>() + step, nullptr))
                 return SRX_E_HIP;
-            mlp_pack(s, dw.as<float>(), dM.as<MlpPacked>());
+        }
+        if (ep + 1 < o.epochs) {
+            std::copy(cur.begin(), cur.end(), next.begin());
+            std::shuffle(next.begin(), next.end(), rng);
         }
         MLP_CHK(hipStreamSynchronize(s));
     }
-    MLP_CHK(hipMemcpyAsync(blob, dw.p, MLP_NPARAM * 4, hipMemcpyDeviceToHost, s));
+    MLP_CHK(hipMemcpyAsync(blob, dw.p, MLP_BLOB * 4, hipMemcpyDeviceToHost, s));
     if (loss_hist) {
         std::vector<float> lh(total);
         MLP_CHK(hipMemcpyAsync(lh.data(), dl.p, total * 4, hipMemcpyDeviceToHost, s));

@@ -44,6 +44,52 @@ def test_gradient_matches_oracle():
         assert np.linalg.norm(gg[a:b] - go[a:b]) <= 1e-5 * np.linalg.norm(go[a:b]), (a, b)
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 4097])
+def test_gradient_of_partly_filled_sample_blocks(n):
+    """The bound of test_gradient_matches_oracle at the edges of the 64-sample blocks."""
+    rng = np.random.default_rng(n)
+    blob = stats_blob(5)
+    x = rng.normal(0, 1, (n, 24)).astype(np.float32)
+    t = rng.normal(0, 1, (n, 6)).astype(np.float32)
+    gg, lg = srx_amd.mlp_grad(blob, x, t)
+    lo, go = M.loss_grad(blob, x, t)
+    assert abs(lg - lo) <= 1e-5 * lo
+    assert np.linalg.norm(gg - go) <= 1e-5 * np.linalg.norm(go)
+
+
+@pytest.mark.parametrize("n", [64, 201, 30011])
+def test_statistics_and_repacked_weights(n):
+    """Training from scratch: means and spreads of the columns are those of the samples (FP32 rounding,
+    2^-24, and FP64 sums).  Two full-batch steps from given weights are Adam's with the gradients taken
+    at the start and at the weights after the first step, i.e. the operands rewritten by a step are those
+    of a full packing.  A batch's samples are summed in shuffled order: FP32 rounding of the gradient,
+    about 1e-6 of its scale, moves Adam's normalised steps by about 1e-3 in the mean square over
+    parameters (its smallest entries dominate), stale operands move them by more than a tenth."""
+    rng = np.random.default_rng(n)
+    x = (rng.normal(0, 1, (n, 24)) * rng.uniform(.1, 10, 24) + rng.normal(0, 3, 24)).astype(np.float32)
+    t = rng.normal(0, 2, (n, 6)).astype(np.float32)
+    x[:, 3], t[:, 2] = 0.75, -0.5   # no spread: 1 is used
+    got, _ = srx_amd.mlp_train(x, t, epochs=1, batch=64)
+    xd, td = x.astype(np.float64), t.astype(np.float64)
+    xs, ts = xd.std(0), td.std(0)
+    xs[3], ts[2] = 1.0, 1.0
+    want = np.concatenate([xd.mean(0), 1 / xs, td.mean(0), ts])
+    scale = np.concatenate([np.abs(xd).mean(0), 1 / xs, np.abs(td).mean(0), ts])
+    assert (np.abs(got[M.NPARAM:] - want) <= 2.0**-23 * np.abs(want) + 1e-11 * scale).all()
+
+    batch, lr = 64 * ((n + 63) // 64), 0.05
+    blob0 = stats_blob(9)
+    one, _ = srx_amd.mlp_train(x, t, blob=blob0, epochs=1, batch=batch, lr=lr, lr_final=lr)
+    two, hist = srx_amd.mlp_train(x, t, blob=blob0, epochs=2, batch=batch, lr=lr, lr_final=lr)
+    g0, _ = srx_amd.mlp_grad(blob0, x, t)
+    g1, l1 = srx_amd.mlp_grad(one, x, t)
+    assert abs(hist[1] - l1) <= 1e-5 * l1
+    g0, g1 = g0.astype(np.float64) / 2, g1.astype(np.float64) / 2   # the trainer drops the square's factor 2
+    m, v = 0.9 * 0.1 * g0 + 0.1 * g1, 0.999 * 0.001 * g0**2 + 0.001 * g1**2
+    step = -lr * (m / (1 - 0.9**2)) / (np.sqrt(v / (1 - 0.999**2)) + 1e-8)
+    assert np.linalg.norm((two - one)[:M.NPARAM] - step) <= 1e-2 * np.linalg.norm(step)
+
+
 def test_training_fits_a_teacher_network():
     rng = np.random.default_rng(2)
     teacher = M.random_blob(11)
