@@ -2336,36 +2336,17 @@ int srx_fft_forward(const double *in, int ncomp, int n0, int n1, int n2, int pre
     size_t specn = 0;
     int rc = fft_test_common(ncomp, n0, n1, n2, prec, pl, tw, &sB, &sC, specn);
     const size_t N = (size_t)n0 * n1 * n2;
-    double *din = nullptr;
+    double *buf = nullptr;   // the fields, then the spectra in the caller's order (16 bytes a value, never fewer bytes)
     const int n[3] = {n0, n1, n2};
     if (!rc) {
-        HIPCK(hipMalloc(&din, sizeof(double) * ncomp * N));
-        HIPCK(hipMemcpy(din, in, sizeof(double) * ncomp * N, hipMemcpyHostToDevice));
-        launch_fft_real_forward_test(nullptr, prec, din, ncomp, sB, sC, n, pl, tw);
+        HIPCK(hipMalloc(&buf, sizeof(double) * 2 * specn));
+        HIPCK(hipMemcpy(buf, in, sizeof(double) * ncomp * N, hipMemcpyHostToDevice));
+        launch_fft_real_forward_test(nullptr, prec, buf, ncomp, sB, sC, n, pl, tw);
+        launch_spec_turn(nullptr, prec, true, sC, buf, ncomp, n);
         HIPCK(hipDeviceSynchronize());
-        // layout C [c][kz][y][x] -> out [c][x][y][kz]
-        const size_t H = n2 / 2 + 1;
-        const size_t csz = prec == SRX_PREC_MIXED ? 8 : 16;
-        std::vector<char> h(specn * csz);
-        HIPCK(hipMemcpy(h.data(), sC, specn * csz, hipMemcpyDeviceToHost));
-        for (int c = 0; c < ncomp; ++c)
-            for (size_t kz = 0; kz < H; ++kz)
-                for (int y = 0; y < n1; ++y)
-                    for (int x = 0; x < n0; ++x) {
-                        const size_t src = ((c * H + kz) * n1 + y) * n0 + x;
-                        const size_t dst = (((size_t)c * n0 + x) * n1 + y) * H + kz;
-                        if (prec == SRX_PREC_MIXED) {
-                            const float *f = reinterpret_cast<const float *>(h.data()) + 2 * src;
-                            out[2 * dst] = f[0];
-                            out[2 * dst + 1] = f[1];
-                        } else {
-                            const double *f = reinterpret_cast<const double *>(h.data()) + 2 * src;
-                            out[2 * dst] = f[0];
-                            out[2 * dst + 1] = f[1];
-                        }
-                    }
+        HIPCK(hipMemcpy(out, buf, sizeof(double) * 2 * specn, hipMemcpyDeviceToHost));
     }
-    if (din) (void)hipFree(din);
+    if (buf) (void)hipFree(buf);
     if (sB) (void)hipFree(sB);
     if (sC) (void)hipFree(sC);
     for (int i = 0; i < 3; ++i)
@@ -2379,35 +2360,17 @@ int srx_fft_inverse(const double *in, int ncomp, int n0, int n1, int n2, int pre
     size_t specn = 0;
     int rc = fft_test_common(ncomp, n0, n1, n2, prec, pl, tw, &sB, &sC, specn);
     const size_t N = (size_t)n0 * n1 * n2;
-    double *dout = nullptr;
+    double *buf = nullptr;   // the spectra in the caller's order, then the fields
     const int n[3] = {n0, n1, n2};
     if (!rc) {
-        const size_t H = n2 / 2 + 1;
-        const size_t csz = prec == SRX_PREC_MIXED ? 8 : 16;
-        std::vector<char> h(specn * csz);
-        for (int c = 0; c < ncomp; ++c)
-            for (size_t kz = 0; kz < H; ++kz)
-                for (int y = 0; y < n1; ++y)
-                    for (int x = 0; x < n0; ++x) {
-                        const size_t dst = ((c * H + kz) * n1 + y) * n0 + x;
-                        const size_t src = (((size_t)c * n0 + x) * n1 + y) * H + kz;
-                        if (prec == SRX_PREC_MIXED) {
-                            float *f = reinterpret_cast<float *>(h.data()) + 2 * dst;
-                            f[0] = (float)in[2 * src];
-                            f[1] = (float)in[2 * src + 1];
-                        } else {
-                            double *f = reinterpret_cast<double *>(h.data()) + 2 * dst;
-                            f[0] = in[2 * src];
-                            f[1] = in[2 * src + 1];
-                        }
-                    }
-        HIPCK(hipMemcpy(sC, h.data(), specn * csz, hipMemcpyHostToDevice));
-        HIPCK(hipMalloc(&dout, sizeof(double) * ncomp * N));
-        launch_fft_real_inverse_test(nullptr, prec, sC, sB, ncomp, dout, n, pl, tw, 1.0 / scale);
+        HIPCK(hipMalloc(&buf, sizeof(double) * 2 * specn));
+        HIPCK(hipMemcpy(buf, in, sizeof(double) * 2 * specn, hipMemcpyHostToDevice));
+        launch_spec_turn(nullptr, prec, false, sC, buf, ncomp, n);
+        launch_fft_real_inverse_test(nullptr, prec, sC, sB, ncomp, buf, n, pl, tw, 1.0 / scale);
         HIPCK(hipDeviceSynchronize());
-        HIPCK(hipMemcpy(out, dout, sizeof(double) * ncomp * N, hipMemcpyDeviceToHost));
+        HIPCK(hipMemcpy(out, buf, sizeof(double) * ncomp * N, hipMemcpyDeviceToHost));
     }
-    if (dout) (void)hipFree(dout);
+    if (buf) (void)hipFree(buf);
     if (sB) (void)hipFree(sB);
     if (sC) (void)hipFree(sC);
     for (int i = 0; i < 3; ++i)

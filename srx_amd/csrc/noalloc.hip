@@ -54,22 +54,6 @@ __global__ void k_twiddles(T *tw, int n) {
     tw[2 * m + 1] = (T)s;
 }
 
-// layout C [c][kz][y][x] (complex T) -> out [c][x][y][kz] (complex double), the order of
-// srx_fft_forward's output
-template <typename T>
-__global__ void k_spec_out(const T *__restrict__ specC, double *__restrict__ out, int ncomp, int n0, int n1, int H) {
-    const size_t total = (size_t)ncomp * n0 * n1 * H;
-    for (size_t d = blockIdx.x * (size_t)blockDim.x + threadIdx.x; d < total; d += (size_t)gridDim.x * blockDim.x) {
-        const size_t kz = d % H;
-        const size_t y = (d / H) % n1;
-        const size_t x = (d / ((size_t)H * n1)) % n0;
-        const size_t c = d / ((size_t)H * n1 * n0);
-        const size_t src = ((c * H + kz) * n1 + y) * n0 + x;
-        out[2 * d] = (double)specC[2 * src];
-        out[2 * d + 1] = (double)specC[2 * src + 1];
-    }
-}
-
 }  // namespace
 
 }  // namespace srx
@@ -107,12 +91,7 @@ extern "C" int srx_fft_forward_noalloc(const double *d_in, int ncomp, int n0, in
     }
     void *sB = b + offB, *sC = b + offC;
     launch_fft_real_forward_test(nullptr, precision, d_in, ncomp, sB, sC, n, pl, tw);
-    const size_t total = (size_t)ncomp * n0 * n1 * H;
-    const dim3 grid((unsigned)std::min<size_t>((total + 255) / 256, 4096));
-    if (precision == SRX_PREC_MIXED)
-        hipLaunchKernelGGL(k_spec_out<float>, grid, dim3(256), 0, nullptr, (const float *)sC, d_out, ncomp, n0, n1, (int)H);
-    else
-        hipLaunchKernelGGL(k_spec_out<double>, grid, dim3(256), 0, nullptr, (const double *)sC, d_out, ncomp, n0, n1, (int)H);
+    launch_spec_turn(nullptr, precision, true, sC, d_out, ncomp, n);
     if (hipGetLastError() != hipSuccess) return SRX_E_HIP;
     if (hipStreamSynchronize(nullptr) != hipSuccess) return SRX_E_HIP;
     return 0;

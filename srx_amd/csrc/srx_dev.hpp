@@ -334,6 +334,8 @@ struct FieldSrc {
     double dt, u[9];
 };
 void launch_gather(hipStream_t s, int mode, int nc, const FieldSrc &src, int v0, int nv, double *out);
+// spectra: layout C to the entry points' [c][x][y][kz] order (out), or back
+void launch_spec_turn(hipStream_t s, int prec, bool out, void *spec, double *user, int ncomp, const int n[3]);
 void launch_fft_real_forward_test(hipStream_t s, int prec, const double *in, int ncomp, void *specB, void *specC,
                                   const int n[3], const FftPlan *pl, void *const *tw);
 

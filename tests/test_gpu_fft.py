@@ -41,3 +41,19 @@ def test_mixed_precision_forward_error_bound():
     ref = np.fft.rfftn(x, axes=(1, 2, 3))
     err = np.abs(got - ref).max() / np.abs(ref).max()
     assert err < 5e-6, err
+
+
+@pytest.mark.parametrize("prec", [srx_amd.PREC_FP64, srx_amd.PREC_MIXED])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (30, 3, 60), (32, 1, 64), (36, 2, 128), (64, 5, 2)])
+def test_orders_of_the_spectrum_at_tile_edges(shape, prec):
+    """The entry points turn spectra around in 32 x 32 pieces of x and kz: both directions at extents
+    around one and two pieces, with the FP64 bounds of the tests above and log2(N) roundings of 2^-23
+    of the largest value in mixed precision."""
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal((2,) + shape)
+    X = np.fft.rfftn(x, axes=(1, 2, 3))
+    tol = 1e-13 if prec == srx_amd.PREC_FP64 else 20 * 2.0**-23
+    got = srx_amd.fft_forward(x, precision=prec)
+    assert np.abs(got - X).max() <= tol * np.abs(X).max()
+    back = srx_amd.fft_inverse(X, shape[2], precision=prec, scale=1.0 / np.prod(shape))
+    assert np.abs(back - x).max() <= 10 * tol * np.abs(x).max()
