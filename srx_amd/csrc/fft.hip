@@ -129,12 +129,43 @@ struct Dft<T, 8> {
 constexpr int FFT_BLOCK = 256;
 
 // n / d for 0 <= n with n * d < 2^32, as one high multiply by ceil(2^32 / d) (exact in that
-// range); replaces the long integer-division sequence in the index arithmetic of the passes.
+// range); replaces the long integer-division sequence in the index arithmetic of the passes.  Built on
+// the host and passed to the kernels: the multiplier is itself a division, and working out a handful of
+// them per stage lengthened the passes' chains.  16^3: 50.5 -> 46.7 us an outer iteration, 96^3 in mixed
+// precision 283 -> 272.
 struct FastDiv {
     unsigned m;
     int d;
-    __device__ __forceinline__ explicit FastDiv(int dd) : m(dd > 1 ? 0xFFFFFFFFu / (unsigned)dd + 1u : 0u), d(dd) {}
+    FastDiv() = default;
+    explicit FastDiv(int dd) : m(dd > 1 ? 0xFFFFFFFFu / (unsigned)dd + 1u : 0u), d(dd) {}
     __device__ __forceinline__ int div(int n) const { return d > 1 ? (int)__umulhi((unsigned)n, m) : n; }
+};
+// rows of a block's tile (the last tile of a pass may be short), times a row's length `per`
+struct TileDiv {
+    FastDiv full, last;
+    TileDiv(int rows, int tile, int per) : full(tile * per), last((rows - (rows - 1) / tile * tile) * per) {}
+    __device__ __forceinline__ FastDiv of(bool whole) const {
+        FastDiv f;
+        f.m = whole ? full.m : last.m;
+        f.d = whole ? full.d : last.d;
+        return f;
+    }
+};
+// A plan with what each of its stages needs: radix, twiddle step and the divisors of its indices (dL: by the span)
+struct FftStages {
+    int n, nst;
+    struct Stage {
+        int R, tstep;
+        FastDiv nb, dL;
+    } st[MAX_RADIX_STAGES];
+    explicit FftStages(const FftPlan &p) : n(p.n), nst(p.nst) {
+        int L = 1;
+        for (int i = 0; i < nst; ++i) {
+            const int R = p.rad[i];
+            st[i] = {R, n / (L * R), FastDiv(n / R), FastDiv(L)};
+            L *= R;
+        }
+    }
 };
 
 // Element loop of a pass's global-memory side: elements [0, tot) dealt to the block's threads,
@@ -171,12 +202,11 @@ __device__ __forceinline__ int lds_swz(int e) {
 // length N stored pencil-major in LDS.  Every butterfly of the stage is held
 // in registers between the load and the store, so the stage runs in place.
 template <typename T, int R, int MAXB>
-__device__ __forceinline__ void stockham_stage(cx<T> *buf, int npen, int N, int L, const cx<T> *__restrict__ tw,
-                                               int sign, int pitch) {
-    const int nb = N / R;
+__device__ __forceinline__ void stockham_stage(cx<T> *buf, int npen, const FftStages::Stage &sg,
+                                               const cx<T> *__restrict__ tw, int sign, int pitch) {
+    const FastDiv dnb = sg.nb, dL = sg.dL;
+    const int nb = dnb.d, L = dL.d, tstep = sg.tstep;
     const int total = npen * nb;
-    const int tstep = N / (L * R);
-    const FastDiv dnb(nb), dL(L);
     cx<T> v[MAXB][R];
 #pragma unroll
     for (int m = 0; m < MAXB; ++m) {
@@ -283,12 +313,12 @@ __device__ __forceinline__ void lds_fft_pow2(cx<T> *buf, int npen, const cx<T> *
 // whether plan pl is make_plan's schedule for the power-of-two length N (the one the compile-time
 // stages run); a tuned or caller-set plan with other radices takes the runtime stages
 template <int N>
-__device__ __forceinline__ bool pow2_default(const FftPlan &pl) {
+__device__ __forceinline__ bool pow2_default(const FftStages &pl) {
     constexpr int ns = pow2_radix(N, 0) == 0 ? 0 : pow2_radix(N, 1) == 0 ? 1 : pow2_radix(N, 2) == 0 ? 2
                      : pow2_radix(N, 3) == 0 ? 3 : 4;
     bool same = pl.nst == ns;
 #pragma unroll
-    for (int st = 0; st < ns; ++st) same = same && pl.rad[st] == pow2_radix(N, st);
+    for (int st = 0; st < ns; ++st) same = same && pl.st[st].R == pow2_radix(N, st);
     return same;
 }
 
@@ -299,7 +329,7 @@ __device__ __forceinline__ bool pow2_default(const FftPlan &pl) {
 // the x, y and z passes; in the z passes they cost an occupancy step, which the swizzled, conflict
 // free stages more than repay).
 template <typename T, int MAXB, bool POW2 = true, bool SWZ = true>
-__device__ void lds_fft(cx<T> *buf, int npen, const FftPlan &pl, const cx<T> *__restrict__ tw, int sign,
+__device__ void lds_fft(cx<T> *buf, int npen, const FftStages &pl, const cx<T> *__restrict__ tw, int sign,
                         int pitch) {
     if constexpr (POW2) {
         switch (pl.n) {
@@ -310,17 +340,15 @@ __device__ void lds_fft(cx<T> *buf, int npen, const FftPlan &pl, const cx<T> *__
         default: break;
         }
     }
-    int L = 1;
     for (int st = 0; st < pl.nst; ++st) {
-        const int R = pl.rad[st];
-        switch (R) {
-        case 8: stockham_stage<T, 8, MAXB>(buf, npen, pl.n, L, tw, sign, pitch); break;
-        case 4: stockham_stage<T, 4, MAXB>(buf, npen, pl.n, L, tw, sign, pitch); break;
-        case 2: stockham_stage<T, 2, MAXB>(buf, npen, pl.n, L, tw, sign, pitch); break;
-        case 3: stockham_stage<T, 3, MAXB>(buf, npen, pl.n, L, tw, sign, pitch); break;
-        default: stockham_stage<T, 5, MAXB>(buf, npen, pl.n, L, tw, sign, pitch); break;
+        const FftStages::Stage sg = pl.st[st];
+        switch (sg.R) {
+        case 8: stockham_stage<T, 8, MAXB>(buf, npen, sg, tw, sign, pitch); break;
+        case 4: stockham_stage<T, 4, MAXB>(buf, npen, sg, tw, sign, pitch); break;
+        case 2: stockham_stage<T, 2, MAXB>(buf, npen, sg, tw, sign, pitch); break;
+        case 3: stockham_stage<T, 3, MAXB>(buf, npen, sg, tw, sign, pitch); break;
+        default: stockham_stage<T, 5, MAXB>(buf, npen, sg, tw, sign, pitch); break;
         }
-        L *= R;
     }
 }
 
@@ -342,8 +370,8 @@ __device__ void lds_fft(cx<T> *buf, int npen, const FftPlan &pl, const cx<T> *__
 // ---------------------------------------------------------------------------
 template <typename T, bool SW>
 __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_fwd_z(const double *__restrict__ in, cx<T> *__restrict__ specB,
-                                                     int ncomp, int n0, int n1, int n2, FftPlan pz,
-                                                     const cx<T> *__restrict__ tw, int TY,
+                                                     int ncomp, int n0, int n1, int n2, FftStages pz,
+                                                     FastDiv dn2, TileDiv dt, const cx<T> *__restrict__ tw, int TY,
                                                      const IterCtl *__restrict__ ctl) {
     if (ctl && ctl->done) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -358,7 +386,7 @@ __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_fwd_z(const double
     const int H = n2 / 2 + 1;
     const size_t N = (size_t)rows * n2;
     const size_t HS = (size_t)H * rows;
-    const FastDiv dn2(n2), dty(ty);
+    const FastDiv dty = dt.of(ty == TY);
     for (int i = threadIdx.x; i < n2; i += FFT_BLOCK) stw[i] = tw[i];
     // one pair of components per block along grid y
     for (int ca = 2 * blockIdx.y; ca < ncomp && ca < 2 * blockIdx.y + 2; ca += 2) {
@@ -396,7 +424,8 @@ __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_fwd_z(const double
 // ---------------------------------------------------------------------------
 template <typename T, bool SW>
 __global__ void __launch_bounds__(FFT_BLOCK) k_fft_y(const cx<T> *__restrict__ in, cx<T> *__restrict__ out,
-                                                     int n0, int n1, int n2, int b_to_c, FftPlan py,
+                                                     int n0, int n1, int n2, int b_to_c, FftStages py,
+                                                     FastDiv dn1, TileDiv dt,
                                                      const cx<T> *__restrict__ tw, int TX,
                                                      const IterCtl *__restrict__ ctl) {
     if (ctl && ctl->done) return;
@@ -414,7 +443,7 @@ __global__ void __launch_bounds__(FFT_BLOCK) k_fft_y(const cx<T> *__restrict__ i
     const int c = blockIdx.z;
     const size_t plane = (size_t)n0 * n1;
     const size_t base = ((size_t)c * H + kz) * plane;
-    const FastDiv dn1(n1), dtx(tx);
+    const FastDiv dtx = dt.of(tx == TX);
     if (b_to_c) {
         // the block's x rows are contiguous in B
         const cx<T> *src = in + base + (size_t)x0 * n1;
@@ -860,7 +889,8 @@ __device__ __forceinline__ void rotation_point(int kx, int ky, int kz, int n0, i
 // mode 3: forward x of 6 strain comps, rotation_point, inverse x of 3 comps (end of increment)
 // mode 0: forward x only (ncomp comps, testing)   mode 2: inverse x only (testing)
 template <typename T, int MAXB, int CO>
-__global__ void __launch_bounds__(FFT_BLOCK) k_green_x(cx<T> *__restrict__ spec, int n0, int n1, int n2, FftPlan px,
+__global__ void __launch_bounds__(FFT_BLOCK) k_green_x(cx<T> *__restrict__ spec, int n0, int n1, int n2, FftStages px,
+                                                       FastDiv dn0, TileDiv dt,
                                                        const cx<T> *__restrict__ tw, int TY, int mode, int ncomp,
                                                        const DevConst *__restrict__ cst,
                                                        const IterCtl *__restrict__ ctl, cx<double> *__restrict__ nyq) {
@@ -875,7 +905,7 @@ __global__ void __launch_bounds__(FFT_BLOCK) k_green_x(cx<T> *__restrict__ spec,
     const int slot = ty * n0;
     const int cin = mode & 1 ? 6 : ncomp;
     const int cout = mode == 1 ? CO : mode == 3 ? 3 : ncomp;
-    const FastDiv dslot(slot), dn0(n0);
+    const FastDiv dslot = dt.of(ty == TY);
     cx<T> *stw = buf + (mode & 1 ? CO : ncomp) * slot;
     for (int i = threadIdx.x; i < n0; i += FFT_BLOCK) stw[i] = tw[i];
     // the block's rows of one component are contiguous: y0 * n0 .. (y0 + ty) * n0 of plane kz
@@ -918,8 +948,8 @@ __global__ void __launch_bounds__(FFT_BLOCK) k_green_x(cx<T> *__restrict__ spec,
     }
     if (mode != 0) lds_fft<T, MAXB, true, false>(buf, cout * ty, px, stw, +1, n0);
     for (int i = threadIdx.x; i < cout * slot; i += FFT_BLOCK) {
-        const int c = dslot.div(i), r = i - c * slot, yy = dn0.div(r), x = r - yy * n0;
-        spec[((size_t)c * H + kz) * plane + (size_t)(y0 + yy) * n0 + x] = buf[c * slot + yy * n0 + x];
+        const int c = dslot.div(i), r = i - c * slot;
+        spec[((size_t)c * H + kz) * plane + (size_t)y0 * n0 + r] = buf[i];
     }
 }
 
@@ -1165,8 +1195,8 @@ __global__ void __launch_bounds__(256, SRX_GREEN_MIN_BLOCKS) k_green_wave(cx<T> 
 // ---------------------------------------------------------------------------
 template <typename T, bool SW>
 __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_inv_z(const cx<T> *__restrict__ specB, double *__restrict__ ee,
-                                                     int ncomp, int n0, int n1, int n2, FftPlan pz,
-                                                     const cx<T> *__restrict__ tw, int TY, int accumulate,
+                                                     int ncomp, int n0, int n1, int n2, FftStages pz,
+                                                     FastDiv dn2, TileDiv dt, const cx<T> *__restrict__ tw, int TY, int accumulate,
                                                      double divisor, const IterCtl *__restrict__ ctl) {
     if (ctl && ctl->done) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -1182,7 +1212,7 @@ __global__ void __launch_bounds__(FFT_BLOCK) SRX_ZPASS_ATTR k_inv_z(const cx<T> 
     const size_t N = (size_t)rows * n2;
     const size_t HS = (size_t)H * rows;
     const double *add = ctl ? (ncomp == 9 ? ctl->ddg : ctl->ddg6) : nullptr;
-    const FastDiv dn2(n2), dty(ty);
+    const FastDiv dty = dt.of(ty == TY);
     // 1/Nxyz: a power of two for the usual grids, where the product equals the division
     const double rdiv = 1.0 / divisor;
     // one pair of components per block along grid y
@@ -1390,11 +1420,11 @@ static void launch_fwd_z(hipStream_t s, const double *in, void *specB, int ncomp
     const dim3 grid((rows + TY - 1) / TY, (ncomp + 1) / 2);
     const size_t sm = padded_lds(TY, n[2], sizeof(cx<T>), sw);
     if (sw)
-        SRX_LAUNCH((k_fwd_z<T, true>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<T> *)specB, ncomp, n[0], n[1], n[2], pz,
-                   (const cx<T> *)twz, TY, ctl);
+        SRX_LAUNCH((k_fwd_z<T, true>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<T> *)specB, ncomp, n[0], n[1], n[2], FftStages(pz),
+                   FastDiv(n[2]), TileDiv(rows, TY, 1), (const cx<T> *)twz, TY, ctl);
     else
-        SRX_LAUNCH((k_fwd_z<T, false>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<T> *)specB, ncomp, n[0], n[1], n[2], pz,
-                   (const cx<T> *)twz, TY, ctl);
+        SRX_LAUNCH((k_fwd_z<T, false>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<T> *)specB, ncomp, n[0], n[1], n[2], FftStages(pz),
+                   FastDiv(n[2]), TileDiv(rows, TY, 1), (const cx<T> *)twz, TY, ctl);
     check_launch("fwd_z");
 }
 
@@ -1415,18 +1445,18 @@ void launch_fft_y(hipStream_t s, int prec, const void *in, void *out, int ncomp,
         size_t sm = padded_lds(TX, n[1], sizeof(cx<double>), sw);
         if (sw)
             SRX_LAUNCH((k_fft_y<double, true>), grid, dim3(FFT_BLOCK), sm, s, (const cx<double> *)in, (cx<double> *)out,
-                           n[0], n[1], n[2], b_to_c, py, (const cx<double> *)twy, TX, ctl);
+                           n[0], n[1], n[2], b_to_c, FftStages(py), FastDiv(n[1]), TileDiv(n[0], TX, 1), (const cx<double> *)twy, TX, ctl);
         else
             SRX_LAUNCH((k_fft_y<double, false>), grid, dim3(FFT_BLOCK), sm, s, (const cx<double> *)in, (cx<double> *)out,
-                           n[0], n[1], n[2], b_to_c, py, (const cx<double> *)twy, TX, ctl);
+                           n[0], n[1], n[2], b_to_c, FftStages(py), FastDiv(n[1]), TileDiv(n[0], TX, 1), (const cx<double> *)twy, TX, ctl);
     } else {
         size_t sm = padded_lds(TX, n[1], sizeof(cx<float>), sw);
         if (sw)
             SRX_LAUNCH((k_fft_y<float, true>), grid, dim3(FFT_BLOCK), sm, s, (const cx<float> *)in, (cx<float> *)out,
-                           n[0], n[1], n[2], b_to_c, py, (const cx<float> *)twy, TX, ctl);
+                           n[0], n[1], n[2], b_to_c, FftStages(py), FastDiv(n[1]), TileDiv(n[0], TX, 1), (const cx<float> *)twy, TX, ctl);
         else
             SRX_LAUNCH((k_fft_y<float, false>), grid, dim3(FFT_BLOCK), sm, s, (const cx<float> *)in, (cx<float> *)out,
-                           n[0], n[1], n[2], b_to_c, py, (const cx<float> *)twy, TX, ctl);
+                           n[0], n[1], n[2], b_to_c, FftStages(py), FastDiv(n[1]), TileDiv(n[0], TX, 1), (const cx<float> *)twy, TX, ctl);
     }
     check_launch("fft_y");
 }
@@ -1451,11 +1481,11 @@ static void launch_green_generic(hipStream_t s, int prec, void *specC, const int
     cx<double> *ny = (cx<double> *)nyq;
     const size_t sm = (size_t)(slots * TY + 1) * n[0] * sizeof(cx<T>);
     if (wide)
-        SRX_LAUNCH((k_green_x<T, 4, CO>), grid, dim3(FFT_BLOCK), sm, s, (cx<T> *)specC, n[0], n[1], n[2], px,
-                   (const cx<T> *)twx, TY, mode, ncomp, cst, ctl, ny);
+        SRX_LAUNCH((k_green_x<T, 4, CO>), grid, dim3(FFT_BLOCK), sm, s, (cx<T> *)specC, n[0], n[1], n[2], FftStages(px),
+                   FastDiv(n[0]), TileDiv(n[1], TY, n[0]), (const cx<T> *)twx, TY, mode, ncomp, cst, ctl, ny);
     else
-        SRX_LAUNCH((k_green_x<T, 2, CO>), grid, dim3(FFT_BLOCK), sm, s, (cx<T> *)specC, n[0], n[1], n[2], px,
-                   (const cx<T> *)twx, TY, mode, ncomp, cst, ctl, ny);
+        SRX_LAUNCH((k_green_x<T, 2, CO>), grid, dim3(FFT_BLOCK), sm, s, (cx<T> *)specC, n[0], n[1], n[2], FftStages(px),
+                   FastDiv(n[0]), TileDiv(n[1], TY, n[0]), (const cx<T> *)twx, TY, mode, ncomp, cst, ctl, ny);
     check_launch("green_x");
 }
 
@@ -1511,10 +1541,10 @@ static void launch_inv_z(hipStream_t s, const void *specB, double *out, int ncom
     const size_t sm = padded_lds(TY, n[2], sizeof(cx<T>), sw);
     if (sw)
         SRX_LAUNCH((k_inv_z<T, true>), grid, dim3(FFT_BLOCK), sm, s, (const cx<T> *)specB, out, ncomp, n[0], n[1], n[2],
-                   pz, (const cx<T> *)twz, TY, accumulate, divisor, ctl);
+                   FftStages(pz), FastDiv(n[2]), TileDiv(rows, TY, 1), (const cx<T> *)twz, TY, accumulate, divisor, ctl);
     else
         SRX_LAUNCH((k_inv_z<T, false>), grid, dim3(FFT_BLOCK), sm, s, (const cx<T> *)specB, out, ncomp, n[0], n[1], n[2],
-                   pz, (const cx<T> *)twz, TY, accumulate, divisor, ctl);
+                   FftStages(pz), FastDiv(n[2]), TileDiv(rows, TY, 1), (const cx<T> *)twz, TY, accumulate, divisor, ctl);
     check_launch("inv_z");
 }
 
