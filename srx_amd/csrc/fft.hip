@@ -1189,6 +1189,131 @@ __global__ void __launch_bounds__(256, SRX_GREEN_MIN_BLOCKS) k_green_wave(cx<T> 
 }
 
 // ---------------------------------------------------------------------------
+// The y, x and Green passes of small planes in one kernel: a block holds the whole plane kz of every
+// component in LDS, laid out as the z passes' B ([x][y]), and runs the y transforms, the x transforms
+// (elements a row apart), the Green operator and both inverses there, stage by stage as stockham_stage.
+// grid: (H), PLANE_BLOCK threads.  LDS: CO slots of n0 rows of n1 | 1, then the two twiddle tables.
+// Bound by the chain of one block's stages.  Against the three passes it saves two launches and the
+// spectra's trips through memory, an outer iteration in FP64: 8^3 44.0 -> 37.7 us, 12^3 45.7 -> 41.6, 16^3
+// 46.3 -> 43.6, 16 x 16 x 256 72.1 -> 63.0.  Beyond 256 points a plane's chain is longer than the three
+// launches (18^3 48.9 -> 50.9, 24^3 49.5 -> 53.4): PLANE_POINTS.
+// ---------------------------------------------------------------------------
+constexpr int PLANE_BLOCK = 512, PLANE_POINTS = 256;
+// One stage of a plane's transforms along one axis: nc components of np pencils, pencil stride ps,
+// element stride es.  In place like stockham_stage.
+template <typename T, int R, int CO>
+__device__ __forceinline__ void plane_stage(cx<T> *buf, int nc, FastDiv dnp, int slot, int ps, int es,
+                                            const FftStages::Stage &sg, const cx<T> *__restrict__ tw, int sign) {
+    constexpr int MB = (CO * PLANE_POINTS + PLANE_BLOCK * R - 1) / (PLANE_BLOCK * R);
+    const FastDiv dnb = sg.nb, dL = sg.dL;
+    const int nb = dnb.d, L = dL.d, tstep = sg.tstep, np = dnp.d;
+    const int total = nc * np * nb;
+    cx<T> v[MB][R];
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+        const int t = threadIdx.x + m * PLANE_BLOCK;
+        if (t < total) {
+            const int p = dnb.div(t), j = t - p * nb;
+            const int c = dnp.div(p);
+            const cx<T> *src = buf + c * slot + (p - c * np) * ps + j * es;
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[m][r] = src[r * nb * es];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+        const int t = threadIdx.x + m * PLANE_BLOCK;
+        if (t < total) {
+            const int p = dnb.div(t), j = t - p * nb;
+            const int c = dnp.div(p);
+            const int jl = dL.div(j), k = j - jl * L;
+            if (k) {
+#pragma unroll
+                for (int r = 1; r < R; ++r) {
+                    cx<T> w = tw[r * k * tstep];
+                    if (sign > 0) w.y = -w.y;
+                    v[m][r] = cmul(v[m][r], w);
+                }
+            }
+            Dft<T, R>::run(v[m], sign);
+            cx<T> *dst = buf + c * slot + (p - c * np) * ps + (jl * L * R + k) * es;
+#pragma unroll
+            for (int r = 0; r < R; ++r) dst[r * L * es] = v[m][r];
+        }
+    }
+    __syncthreads();
+}
+struct PlanePlans {
+    FftStages ax[2];   // x, y
+    FastDiv n[2], plane;
+};
+template <typename T, int CO>
+__global__ void __launch_bounds__(PLANE_BLOCK) k_plane(cx<T> *__restrict__ spec, int n0, int n1, int n2, PlanePlans pl,
+                                                       const cx<T> *__restrict__ twx, const cx<T> *__restrict__ twy,
+                                                       const DevConst *__restrict__ cst,
+                                                       const IterCtl *__restrict__ ctl, cx<double> *__restrict__ nyq) {
+    if (ctl && ctl->done) return;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    cx<T> *buf = reinterpret_cast<cx<T> *>(smem_raw);
+    const int P = n1 | 1, slot = n0 * P, plane = n0 * n1;
+    cx<T> *stw = buf + CO * slot;
+    const int H = n2 / 2 + 1, kz = blockIdx.x;
+    const FastDiv dplane = pl.plane, dn1 = pl.n[1];
+    for (int i = threadIdx.x; i < n0 + n1; i += PLANE_BLOCK) stw[i] = i < n0 ? twx[i] : twy[i - n0];
+    auto at = [&](int c, int r) {   // LDS position of point r = x n1 + y
+        const int x = dn1.div(r);
+        return c * slot + x * P + (r - x * n1);
+    };
+    for (int i = threadIdx.x; i < 6 * plane; i += PLANE_BLOCK) {
+        const int c = dplane.div(i), r = i - c * plane;
+        buf[at(c, r)] = spec[((size_t)c * H + kz) * plane + r];
+    }
+    __syncthreads();
+    // forward y and x, the Green operator, inverse x and y: one copy of the stages' code for the four
+#pragma unroll 1
+    for (int pass = 0; pass < 4; ++pass) {
+        const int ax = pass == 0 || pass == 3, sign = pass < 2 ? -1 : 1;
+        const int nc = pass < 2 ? 6 : CO, ps = ax ? P : 1, es = ax ? 1 : P;
+        const FastDiv np = pl.n[1 - ax];
+        const cx<T> *tw = stw + (ax ? n0 : 0);
+        const FftStages &st = pl.ax[ax];
+#pragma unroll 1
+        for (int s = 0; s < st.nst; ++s) {
+            const FftStages::Stage sg = st.st[s];
+            switch (sg.R) {
+            case 8: plane_stage<T, 8, CO>(buf, nc, np, slot, ps, es, sg, tw, sign); break;
+            case 4: plane_stage<T, 4, CO>(buf, nc, np, slot, ps, es, sg, tw, sign); break;
+            case 2: plane_stage<T, 2, CO>(buf, nc, np, slot, ps, es, sg, tw, sign); break;
+            case 3: plane_stage<T, 3, CO>(buf, nc, np, slot, ps, es, sg, tw, sign); break;
+            default: plane_stage<T, 5, CO>(buf, nc, np, slot, ps, es, sg, tw, sign); break;
+            }
+        }
+        if (pass == 1) {
+            double dc6[6] = {0, 0, 0, 0, 0, 0};
+            if (ctl)
+                for (int k = 0; k < 6; ++k) dc6[k] = ctl->dcs6[k];
+            const bool first = ctl && ctl->iter == 0;
+            for (int i = threadIdx.x; i < plane; i += PLANE_BLOCK) {
+                const int kx = dn1.div(i), ky = i - kx * n1, b = kx * P + ky;
+                cx<T> q[6], o[CO];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) q[c] = buf[c * slot + b];
+                if constexpr (CO == 9) green_point9(cst, dc6, kx, ky, kz, n0, n1, n2, q, o);
+                else green_point<T>(cst, dc6, kx, ky, kz, n0, n1, n2, q, o, nyq, first);
+#pragma unroll
+                for (int c = 0; c < CO; ++c) buf[c * slot + b] = o[c];
+            }
+            __syncthreads();
+        }
+    }
+    for (int i = threadIdx.x; i < CO * plane; i += PLANE_BLOCK) {
+        const int c = dplane.div(i), r = i - c * plane;
+        spec[((size_t)c * H + kz) * plane + r] = buf[at(c, r)];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // inverse z (c2r) fused with Eq. 15: ee[c] += ddg6[c] + Re(IFFT)/Nxyz for the six strain components,
 // or the same for the nine of DisGrad with ddg
 // grid: (ceil(n0 n1 / TY), component pairs); `ee` is an output (scale mode) when accumulate=0
@@ -1530,6 +1655,25 @@ void launch_green_x(hipStream_t s, int prec, void *specC, const int n[3], const 
     if (prec == 0) launch_green_generic<double, 6>(s, prec, specC, n, px, twx, cst, 1, 6, ctl, nyq, tile);
     else if (six) launch_green_generic<float, 6>(s, prec, specC, n, px, twx, cst, 1, 6, ctl, nyq, tile);
     else launch_green_generic<float, 9>(s, prec, specC, n, px, twx, cst, 1, 9, ctl, nyq, tile);
+}
+
+// planes of up to 256 points, where one block's chain is shorter than three launches (k_plane's figures)
+bool plane_pass_ok(const int n[3]) { return n[0] * n[1] <= PLANE_POINTS; }
+
+template <typename T, int CO>
+static void launch_plane_t(hipStream_t s, void *specB, const int n[3], const FftPlan pl[3], void *const tw[3],
+                           const DevConst *cst, const IterCtl *ctl, void *nyq) {
+    const PlanePlans pp = {{FftStages(pl[0]), FftStages(pl[1])}, {FastDiv(n[0]), FastDiv(n[1])}, FastDiv(n[0] * n[1])};
+    const size_t sm = ((size_t)CO * n[0] * (n[1] | 1) + n[0] + n[1]) * sizeof(cx<T>);
+    SRX_LAUNCH((k_plane<T, CO>), dim3(n[2] / 2 + 1), dim3(PLANE_BLOCK), sm, s, (cx<T> *)specB, n[0], n[1], n[2], pp,
+               (const cx<T> *)tw[0], (const cx<T> *)tw[1], cst, ctl, (cx<double> *)nyq);
+}
+void launch_plane(hipStream_t s, int prec, void *specB, const int n[3], const FftPlan pl[3], void *const tw[3],
+                  const DevConst *cst, const IterCtl *ctl, void *nyq) {
+    if (prec == 0) launch_plane_t<double, 6>(s, specB, n, pl, tw, cst, ctl, nyq);
+    else if (strain_form(n, prec)) launch_plane_t<float, 6>(s, specB, n, pl, tw, cst, ctl, nyq);
+    else launch_plane_t<float, 9>(s, specB, n, pl, tw, cst, ctl, nyq);
+    check_launch("plane");
 }
 
 template <typename T>

@@ -1410,9 +1410,14 @@ static int step_iterate(srx_ctx *c) {
             IterCtl *g = c->dctl;
             const int *tl = c->tiles;
             { Timer t(c, 0, launched); launch_fft_fwd_z(c->stream, prec, c->f.sig, c->specB, c->n, c->pl[2], c->tw[2], g, tl[0]); }
-            { Timer t(c, 1, launched); launch_fft_y(c->stream, prec, c->specB, c->specC, 6, -1, 1, c->n, c->pl[1], c->tw[1], g, tl[1]); }
-            { Timer t(c, 2, launched); launch_green_x(c->stream, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, g, c->nyq, tl[2]); }
-            { Timer t(c, 3, launched); launch_fft_y(c->stream, prec, c->specC, c->specB, c->comps(), +1, 0, c->n, c->pl[1], c->tw[1], g, tl[3]); }
+            if (plane_pass_ok(c->n)) {
+                Timer t(c, 2, launched);
+                launch_plane(c->stream, prec, c->specB, c->n, c->pl, c->tw, c->dc, g, c->nyq);
+            } else {
+                { Timer t(c, 1, launched); launch_fft_y(c->stream, prec, c->specB, c->specC, 6, -1, 1, c->n, c->pl[1], c->tw[1], g, tl[1]); }
+                { Timer t(c, 2, launched); launch_green_x(c->stream, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, g, c->nyq, tl[2]); }
+                { Timer t(c, 3, launched); launch_fft_y(c->stream, prec, c->specC, c->specB, c->comps(), +1, 0, c->n, c->pl[1], c->tw[1], g, tl[3]); }
+            }
             { Timer t(c, 4, launched); launch_fft_inv_z_update(c->stream, prec, c->specB, c->strain(), c->n, c->pl[2], c->tw[2], g, divisor, tl[4]); }
             const bool rec = c->rec_stride > 0 && launched > 1;
             if (rec)
@@ -1728,9 +1733,13 @@ static int run_lockstep(const std::vector<int> &members, std::vector<srx_ctx *> 
                     const int *tl = c->tiles;
                     IterCtl *g = c->dctl;
                     launch_fft_fwd_z(st, prec, c->f.sig, c->specB, c->n, c->pl[2], c->tw[2], g, tl[0]);
-                    launch_fft_y(st, prec, c->specB, c->specC, 6, -1, 1, c->n, c->pl[1], c->tw[1], g, tl[1]);
-                    launch_green_x(st, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, g, c->nyq, tl[2]);
-                    launch_fft_y(st, prec, c->specC, c->specB, c->comps(), +1, 0, c->n, c->pl[1], c->tw[1], g, tl[3]);
+                    if (plane_pass_ok(c->n)) {
+                        launch_plane(st, prec, c->specB, c->n, c->pl, c->tw, c->dc, g, c->nyq);
+                    } else {
+                        launch_fft_y(st, prec, c->specB, c->specC, 6, -1, 1, c->n, c->pl[1], c->tw[1], g, tl[1]);
+                        launch_green_x(st, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, g, c->nyq, tl[2]);
+                        launch_fft_y(st, prec, c->specC, c->specB, c->comps(), +1, 0, c->n, c->pl[1], c->tw[1], g, tl[3]);
+                    }
                     launch_fft_inv_z_update(st, prec, c->specB, c->strain(), c->n, c->pl[2], c->tw[2], g,
                                             (double)c->nvox, tl[4]);
                 }

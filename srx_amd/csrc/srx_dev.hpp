@@ -256,6 +256,11 @@ bool strain_form(const int n[3], int prec);
 size_t nyq_elems(const int n[3]);
 void launch_green_x(hipStream_t s, int prec, void *specC, const int n[3], const FftPlan &px, const void *twx,
                     const DevConst *cst, const IterCtl *ctl, void *nyq, int tile = 0);
+// the forward y, Green x and inverse y passes in one launch, on layout B in place (planes of
+// plane_pass_ok's grids)
+bool plane_pass_ok(const int n[3]);
+void launch_plane(hipStream_t s, int prec, void *specB, const int n[3], const FftPlan pl[3], void *const tw[3],
+                  const DevConst *cst, const IterCtl *ctl, void *nyq);
 void launch_fft_inv_z_update(hipStream_t s, int prec, const void *specB, double *ee, const int n[3],
                              const FftPlan &pz, const void *twz, const IterCtl *ctl, double scale, int tile = 0);
 // End of increment: the rotation part (3 comps) of the DisGrad change from its strain part (6 comps)

@@ -352,6 +352,24 @@ def test_displacement_gradient_matches_oracle(tmp_path, oracle_lib, n, precision
     o.close()
 
 
+@pytest.mark.parametrize("n,precision", [((16, 16, 3), srx_amd.PREC_FP64), ((256, 1, 4), srx_amd.PREC_FP64),
+                                         ((2, 125, 2), srx_amd.PREC_FP64), ((1, 250, 3), srx_amd.PREC_MIXED),
+                                         ((18, 15, 5), srx_amd.PREC_FP64), ((5, 54, 4), srx_amd.PREC_FP64),
+                                         ((24, 12, 3), srx_amd.PREC_MIXED), ((32, 16, 2), srx_amd.PREC_MIXED)])
+def test_one_pass_or_three_per_plane_match_oracle(tmp_path, oracle_lib, n, precision):
+    """Planes of up to 256 points take the y, x and Green passes in one launch, larger ones in three: both
+    sides of the limit, with the bounds of test_displacement_gradient_matches_oracle."""
+    deck = make(tmp_path, n=n, grains=4, seed=23, nsteps=3)
+    o = oracle_lib.Oracle(deck, fixed_iters=5)
+    g = srx_amd.Solver(deck, fixed_iters=5, precision=precision)
+    tol = 1e-9 if precision == srx_amd.PREC_FP64 else 1e-4
+    for step in range(3):
+        o.step(), g.step()
+        compare_fields(g, o, tol, ("sig", "disgrad", "velgrad", "fluct", "tranmat"))
+    g.close()
+    o.close()
+
+
 def _two_routes(tmp_path, n, precision, warm_start):
     """Three runs of a deck: orientations as opened, one voxel scaled by 1 + 1e-10 (no rotation to
     1e-12: the matrices are read), and scaled then set back."""
