@@ -42,13 +42,19 @@ F_NR = 2300.0                  # flops per voxel per Newton iteration (algorithm
 # rocprofv3 FETCH_SIZE (x2.0) and WRITE_SIZE (x1.0) runs calibrated on a 1 GiB device copy
 # (profiles/evp_fft_128cubed_pmc.md); mixed precision reads the increment's Newton matrix and
 # per-system constants as FP32
-NR_TRAFFIC_BYTES_PER_VOXEL = {"fp64": 817.2, "mixed": 609.4}
+NR_TRAFFIC_BYTES_PER_VOXEL = {"fp64": 641.5, "mixed": 502.1}
 METRIC = "converged voxel-increments/s at 128³, plain FP64 vs mixed-precision at equal stress error"
 
 
-def fft_green_bytes_per_voxel(real_bytes: int, n2: int, c_out: int = 9) -> float:
-    """Algorithmic HBM bytes per voxel of one FFT + Green + inverse FFT + DisGrad update pass:
-    FP64 stress in (6 x 8 B), DisGrad read+write (c_out x 16 B), and the half-spectrum
+def inverse_components(precision: str, n: int) -> int:
+    """Components the outer iterations transform back: the strain's six, or DisGrad's nine (mixed precision
+    where an extent is no power of two)."""
+    return 6 if precision == "fp64" or n & (n - 1) == 0 else 9
+
+
+def fft_green_bytes_per_voxel(real_bytes: int, n2: int, c_out: int = 6) -> float:
+    """Algorithmic HBM bytes per voxel of one FFT + Green + inverse FFT + strain update pass:
+    FP64 stress in (6 x 8 B), strain or DisGrad read+write (c_out x 16 B), and the half-spectrum
     passes: 6 comps x 4 touches forward, c_out comps x 4 touches inverse, each 2*s*h bytes."""
     h = (n2 // 2 + 1) / n2
     return 48.0 + 16.0 * c_out + (24.0 + 4.0 * c_out) * 2.0 * real_bytes * h
@@ -339,7 +345,7 @@ def main() -> int:
         b_iters = max(brk[name]["iters"], 1)
         nr_ms = e["kernels"].get("nr", (0, 0))[0]
         rb = 4 if name == "mixed" else 8
-        b_fg = fft_green_bytes_per_voxel(rb, n[2]) * nvox
+        b_fg = fft_green_bytes_per_voxel(rb, n[2], inverse_components(name, n[2])) * nvox
         per[name] = {
             "value": args.steps * nvox / r["seconds"], "seconds": r["seconds"],
             "newton_event_run_seconds": e["seconds"], "breakdown_run_seconds": brk[name]["seconds"],
@@ -350,7 +356,7 @@ def main() -> int:
             "fft_green_gbs": b_fg * b_iters / (fg_ms * 1e-3) / 1e9 if fg_ms else None,
             "fft_green_frac_hbm": (b_fg * b_iters / (fg_ms * 1e-3) / 1e9) / HBM_PEAK_GBS if fg_ms else None,
             "nr_tflops": F_NR * e["nr_total"] / (nr_ms * 1e-3) / 1e12 if nr_ms else None,
-            "fft_green_bytes_per_voxel": fft_green_bytes_per_voxel(rb, n[2]),
+            "fft_green_bytes_per_voxel": b_fg / nvox,
         }
         if name in fs:
             f = fs[name]
@@ -385,8 +391,9 @@ def main() -> int:
         kt = bk
         rb = 4 if head == "mixed" else 8
         h = (n[2] // 2 + 1) / n[2]
-        pass_bytes = {"fwd_z": (48 + 6 * 2 * rb * h), "fwd_y": 6 * 2 * 2 * rb * h, "green_x": 15 * 2 * rb * h,
-                      "inv_y": 9 * 2 * 2 * rb * h, "inv_z": 9 * 2 * rb * h + 144}
+        co = inverse_components(head, n[2])
+        pass_bytes = {"fwd_z": (48 + 6 * 2 * rb * h), "fwd_y": 6 * 2 * 2 * rb * h, "green_x": (6 + co) * 2 * rb * h,
+                      "inv_y": co * 2 * 2 * rb * h, "inv_z": co * 2 * rb * h + 16 * co}
         bpv = pass_bytes.get(dom, 0.0)
         ach = bpv * nvox * kt[dom][1] / (kt[dom][0] * 1e-3) / 1e9
         out["roofline"] = {"kernel": dom, "bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",

@@ -1,10 +1,10 @@
 // host.cpp -- libsrx host side: input readers, setup, increment driver, C ABI.
 //
 // Replaces the reference's step driver (evp.c main -> GetNameList, SetupJob,
-// Evolution, DestroyJob).  The grid stays resident on one GPU; the host only
-// holds scalars between kernels (the 20 reduced values of each outer
-// iteration) and does the macro-stress / mixed-boundary-condition algebra of
-// get_smacro (evolution.c:590-664) on them.
+// Evolution, DestroyJob).  The grid stays resident on one GPU; the macro-stress
+// and mixed-boundary-condition algebra of get_smacro (evolution.c:590-664) runs
+// there too (k_control), and the host reads its control block once per batch of
+// outer iterations.
 #include "srx_dev.hpp"
 #include "../../include/srx.h"
 
