@@ -72,21 +72,24 @@ void launch_gather(hipStream_t s, int mode, int nc, const FieldSrc &src, int v0,
 // of 60 x 64 x 75, 4.0 ms with this kernel, most of it the copies over PCIe.
 constexpr int TURN_TILE = 32, TURN_BLOCK = 256;
 template <typename T, bool OUT>
-__global__ void __launch_bounds__(TURN_BLOCK) k_spec_turn(T *__restrict__ spec, double *__restrict__ user, int n0, int n1, int H) {
-    __shared__ double2 tile[TURN_TILE][TURN_TILE + 1];   // [x][kz]
+__global__ void __launch_bounds__(TURN_BLOCK) k_spec_turn(T *__restrict__ spec, double *__restrict__ user, int n0, int n1,
+                                                          int H) {
     typedef T T2 __attribute__((ext_vector_type(2)));
+    // the caller's buffer may be aligned to 8 bytes only
+    typedef double U2 __attribute__((ext_vector_type(2), aligned(8)));
+    __shared__ U2 tile[TURN_TILE][TURN_TILE + 1];   // [x][kz]
     const int c = blockIdx.z / n1, y = blockIdx.z % n1;
     const int x0 = blockIdx.x * TURN_TILE, k0 = blockIdx.y * TURN_TILE;
     const int i = threadIdx.x % TURN_TILE;
     T2 *sp = reinterpret_cast<T2 *>(spec);
-    double2 *us = reinterpret_cast<double2 *>(user);
+    U2 *us = reinterpret_cast<U2 *>(user);
     auto at_spec = [&](int x, int kz) { return (((size_t)c * H + kz) * n1 + y) * n0 + x; };
     auto at_user = [&](int x, int kz) { return (((size_t)c * n0 + x) * n1 + y) * H + kz; };
 #pragma unroll
     for (int j = threadIdx.x / TURN_TILE; j < TURN_TILE; j += TURN_BLOCK / TURN_TILE) {
         if (OUT && x0 + i < n0 && k0 + j < H) {
             const T2 v = sp[at_spec(x0 + i, k0 + j)];
-            tile[i][j] = make_double2((double)v.x, (double)v.y);
+            tile[i][j] = U2{(double)v.x, (double)v.y};
         } else if (!OUT && x0 + j < n0 && k0 + i < H) {
             tile[j][i] = us[at_user(x0 + j, k0 + i)];
         }
@@ -97,7 +100,7 @@ __global__ void __launch_bounds__(TURN_BLOCK) k_spec_turn(T *__restrict__ spec, 
         if (OUT && x0 + j < n0 && k0 + i < H) {
             us[at_user(x0 + j, k0 + i)] = tile[j][i];
         } else if (!OUT && x0 + i < n0 && k0 + j < H) {
-            const double2 v = tile[i][j];
+            const U2 v = tile[i][j];
             T2 o;
             o.x = (T)v.x;
             o.y = (T)v.y;

@@ -85,6 +85,25 @@ def test_noalloc_forward_matches_srx_fft_forward_twice(order):
         assert np.abs(g - ref).max() <= (1e-12 if prec == srx_amd.PREC_FP64 else 1e-5) * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("prec", [srx_amd.PREC_FP64, srx_amd.PREC_MIXED])
+def test_noalloc_output_aligned_to_a_double(prec):
+    """The output may start at any double: the same values, bit for bit, at an odd multiple of 8 bytes."""
+    h = hip()
+    n, ncomp = (12, 5, 36), 2
+    x = np.random.default_rng(11).standard_normal((ncomp,) + n)
+    rc, want = noalloc_forward(h, x, n, prec)
+    assert rc == 0, rc
+    din, dout = DevBuf(h, x.nbytes), DevBuf(h, want.nbytes + 8)
+    din.put(x)
+    at = C.c_void_p(dout.p.value + 8)
+    rc = srx_amd.lib().srx_fft_forward_noalloc(din.p, ncomp, n[0], n[1], n[2], prec, at)
+    got = dout.get((want.size + 1,))[1:].reshape(want.shape) if rc == 0 else None
+    din.free()
+    dout.free()
+    assert rc == 0, rc
+    np.testing.assert_array_equal(got, want)
+
+
 def test_noalloc_rejects_a_problem_beyond_its_scratch():
     h = hip()
     # 9 FP64 components of 96^3: two half spectra of 9*49*96*96*16 B > 32 MiB
