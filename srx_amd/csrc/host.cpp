@@ -1678,14 +1678,19 @@ static int run_lockstep(const std::vector<int> &members, std::vector<srx_ctx *> 
         }
         if (act.empty()) break;
         const int nact = (int)act.size();
+        // Members with the FCC zero structure first: the Newton kernel that leaves the zeros out sums the slip
+        // systems in another order, so each of the two groups runs the kernel its members run alone (a
+        // member's bits must not depend on the company it keeps).
+        const int nfcc = (int)(std::stable_partition(act.begin(), act.end(), [&](int k) { return ctx[k]->fcc; }) - act.begin());
         const int istep = ctx[act[0]]->istep;
         for (int k : act)
             if (ctx[k]->istep != istep) rc = SRX_E_ARG;   // members advance together from istep 0
         if (rc) break;
         const int rotated = istep > 2 ? 1 : 0;
-        int nb = 0, most = 0, pb = 0;
+        int nb[2] = {0, 0}, most = 0, pb = 0;   // Newton blocks of the two groups
         for (int j = 0; j < nact && !rc; ++j) {
             srx_ctx *c = ctx[act[j]];
+            int &blocks = nb[j < nfcc ? 0 : 1];
             EnsIncr &inc = hinc[j];
             if (int e = step_begin(c, &inc)) rc = e;
             inc.cst = c->dc;
@@ -1699,13 +1704,13 @@ static int run_lockstep(const std::vector<int> &members, std::vector<srx_ctx *> 
             htab[j].cst = c->dc;
             htab[j].f = c->f;
             htab[j].nvox = (int)c->nvox;
-            htab[j].blk0 = nb;
+            htab[j].blk0 = blocks;
             htab[j].nblk = c->nr_blocks;
             htab[j].pad = 0;
             htab[j].partials = c->partials;
             htab[j].redseg = c->redseg;
             htab[j].ctl = c->dctl;
-            nb += c->nr_blocks;
+            blocks += c->nr_blocks;
             most = std::max(most, std::max(c->itermax, c->opt.fixed_iters));
         }
         if (rc || !ok(hipMemcpyAsync(dtab, htab, sizeof(EnsMember) * nact, hipMemcpyHostToDevice, S)) ||
@@ -1713,11 +1718,12 @@ static int run_lockstep(const std::vector<int> &members, std::vector<srx_ctx *> 
             break;
         launch_prologue_ens(S, dinc, nact, pb);
         const srx_options &o = ctx[act[0]]->opt;
-        int ph2 = 0, f32 = 1, fcc = 1;
-        for (int k : act) {
-            ph2 |= ctx[k]->hc.ph[1].xtal;
-            f32 = f32 && ctx[k]->f.nrcf && ctx[k]->f.quat;
-            fcc = fcc && ctx[k]->fcc;
+        int ph2[2] = {0, 0}, f32[2] = {1, 1};
+        for (int j = 0; j < nact; ++j) {
+            const srx_ctx *c = ctx[act[j]];
+            const int g = j < nfcc ? 0 : 1;
+            ph2[g] |= c->hc.ph[1].xtal;
+            f32[g] = f32[g] && c->f.nrcf && c->f.quat;
         }
         int launched = 0;
         bool all_done = false;
@@ -1744,7 +1750,10 @@ static int run_lockstep(const std::vector<int> &members, std::vector<srx_ctx *> 
                                             (double)c->nvox, tl[4]);
                 }
                 for (int q = 0; q < NS; ++q) ok(hipEventRecord(ev[q], side[q])) && ok(hipStreamWaitEvent(S, ev[q], 0));
-                launch_nr_ens(S, dtab, nact, nb, launched == 1, rotated, o.warm_start, o.gnd, ph2, f32, fcc);
+                for (int g = 0; g < 2; ++g)
+                    if (nb[g])
+                        launch_nr_ens(S, dtab + (g ? nfcc : 0), g ? nact - nfcc : nfcc, nb[g], launched == 1, rotated,
+                                      o.warm_start, o.gnd, ph2[g], f32[g], g == 0);
                 launch_reduce_nr_ens(S, dtab, nact);
                 launch_control_ens(S, dtab, nact, ddone);
             }

@@ -81,6 +81,25 @@ def test_lockstep_ensemble_matches_members_run_alone(tmp_path, concurrency, prec
         assert a == b
 
 
+@pytest.mark.parametrize("precision", [srx_amd.PREC_FP64, srx_amd.PREC_MIXED])
+def test_lockstep_of_different_slip_systems_matches_members_run_alone(tmp_path, precision):
+    """Members with 12 FCC systems and with nine of them, which run different Newton kernels, and of
+    different increment counts, so that the group's make-up changes on the way: every member's results
+    equal its deck run alone, bit for bit."""
+    members = [((16, 16, 16), 8, 1, 12, 4), ((12, 10, 8), 5, 2, 9, 3), ((8, 8, 8), 4, 3, 12, 3), ((9, 6, 5), 3, 4, 9, 5)]
+    decks = [inputs.make_case(str(tmp_path / ("rve%d" % k)), n=n, grains=g, seed=seed, nsteps=steps, timestep=0.1, nsys=nsys)
+             for k, (n, g, seed, nsys, steps) in enumerate(members)]
+    res = srx_amd.run_ensemble(decks, concurrency=0, precision=precision)
+    for k, deck in enumerate(decks):
+        s = srx_amd.Solver(deck, precision=precision)
+        for _ in range(members[k][4]):
+            last = s.step()
+        s.close()
+        assert res[k]["rc"] == 0 and res[k]["increments"] == members[k][4]
+        for key in ("iters", "nr_iters_total", "s_vm", "e_vm", "evmp", "rho_s_avg", "sig_avg", "eps_avg"):
+            assert res[k]["last"][key] == last[key], (k, key)
+
+
 def test_lockstep_members_with_different_increment_counts(tmp_path):
     """A member with fewer increments leaves the lockstep when it is done; the others go on."""
     decks = make_cases(str(tmp_path / "ens"))[:3]
