@@ -1465,12 +1465,27 @@ struct Finish {
     double nrwave;
 };
 
+// DisGrad of the voxels from the strain the outer iterations advanced and the uniform part they applied
+// (not the last dDisGradAvg), on the context's stream: ahead of the end-of-increment kernel, or, after
+// iterations that failed, so that the fields show the iterate they failed at.
+static void disgrad_from_strain(srx_ctx *c) {
+    const IterCtl &ctl = *c->hctl;
+    if (!c->f.ee || ctl.iter == 0) return;
+    double du[9];
+    for (int k = 0; k < 9; ++k) du[k] = ctl.uniform[k] - c->uniform0[k];
+    launch_rot_in(c->stream, c->f, (int)c->nvox, du);
+    launch_rotation_part(c->stream, c->opt.precision, c->f.ee, c->f.ee, c->specB, c->specC, c->n, c->pl, c->tw, c->dc,
+                         c->nyq, c->tiles);
+    launch_rot_out(c->stream, c->f, (int)c->nvox, du);
+}
+
 static int finish_begin(srx_ctx *c, Finish &F) {
     const Deck &d = c->dk;
     const double dt = d.TimeStep;
     IterCtl &ctl = *c->hctl;
     srx_step_report &r = F.r;
     std::memset(&r, 0, sizeof(r));
+    disgrad_from_strain(c);
     if (ctl.nan) return SRX_E_NAN;
     F.iter = ctl.iter;
     F.nrmax = ctl.nrmax;
@@ -1502,16 +1517,6 @@ static int finish_begin(srx_ctx *c, Finish &F) {
     std::memcpy(c->DisGradAvg_t, act, sizeof(act));
     std::memcpy(r.disgrad_avg_actual, act, sizeof(act));
     std::memcpy(r.velgrad_avg, vga, sizeof(vga));
-    // DisGrad of the voxels from the strain the outer iterations advanced and the uniform part they
-    // applied (not the last dDisGradAvg), on the context's stream ahead of the end-of-increment kernel
-    if (F.iter > 0 && c->f.ee) {
-        double du[9];
-        for (int k = 0; k < 9; ++k) du[k] = c->uniform[k] - c->uniform0[k];
-        launch_rot_in(c->stream, c->f, (int)c->nvox, du);
-        launch_rotation_part(c->stream, c->opt.precision, c->f.ee, c->f.ee, c->specB, c->specC, c->n, c->pl, c->tw, c->dc,
-                             c->nyq, c->tiles);
-        launch_rot_out(c->stream, c->f, (int)c->nvox, du);
-    }
     // Edot/Eps, update_orient (istep>1), DislocationEvolution, averages: the end-of-increment kernel
     F.do_orient = (d.Update_Flag == 1 && c->istep > 1) ? 1 : 0;
     return 0;

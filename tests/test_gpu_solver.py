@@ -268,6 +268,26 @@ def test_nan_is_reported_not_aborted(tmp_path):
     assert e.value.code == 3001
 
 
+@pytest.mark.parametrize("precision,tol", [(srx_amd.PREC_FP64, 1e-9), (srx_amd.PREC_MIXED, 1e-4)])
+def test_fields_after_nan_show_the_failing_iterate(tmp_path, oracle_lib, precision, tol):
+    """After SRX_E_NAN the strain fields are those of the outer iteration that failed, as the oracle's are
+    (this file's 1e-9, mixed 1e-4), not the increment's start: DisGrad, and what is derived from it."""
+    deck = inputs.make_case(str(tmp_path), n=(8, 8, 8), grains=4, seed=1, nsteps=2, timestep=1.0)
+    o = oracle_lib.Oracle(deck)
+    with pytest.raises(RuntimeError):
+        o.step()
+    g = srx_amd.Solver(deck, precision=precision)
+    with pytest.raises(srx_amd.SrxError):
+        g.step()
+    want = o.field("disgrad")
+    fluct = want - want.mean(0)
+    assert np.abs(fluct).max() > 0.1 * np.abs(want).max()   # the iterate is not the uniform start
+    assert rel(g.field("disgrad"), want) < tol
+    assert rel(g.field("velgrad"), want / 1.0) < tol        # DisGrad was zero before this increment of 1 s
+    got = g.field("fluct")
+    assert rel(got - got.mean(0), fluct) < tol
+
+
 def test_warm_start_matches_oracle(tmp_path, oracle_lib):
     """warm_start 1 (extrapolated Newton start, no counterpart in the reference): the GPU and the
     oracle run the same algorithm."""
