@@ -1538,7 +1538,7 @@ int fft_tile_max(int pass, const int n[3], const FftPlan &p, int prec, int comps
 }
 
 template <typename T>
-static void launch_fwd_z(hipStream_t s, const double *in, void *specB, int ncomp, const int n[3], const FftPlan &pz,
+static hipError_t launch_fwd_z(hipStream_t s, const double *in, void *specB, int ncomp, const int n[3], const FftPlan &pz,
                          const void *twz, const IterCtl *ctl, int tile, int prec) {
     const int rows = n[0] * n[1], TY = zy_tile(pz, rows, tile, prec);
     const bool sw = plan_swizzled(pz);
@@ -1550,7 +1550,7 @@ static void launch_fwd_z(hipStream_t s, const double *in, void *specB, int ncomp
     else
         SRX_LAUNCH((k_fwd_z<T, false>), grid, dim3(FFT_BLOCK), sm, s, in, (cx<T> *)specB, ncomp, n[0], n[1], n[2], FftStages(pz),
                    FastDiv(n[2]), TileDiv(rows, TY, 1), (const cx<T> *)twz, TY, ctl);
-    check_launch("fwd_z");
+    return check_launch("fwd_z");
 }
 
 void launch_fft_fwd_z(hipStream_t s, int prec, const double *sig, void *specB, const int n[3], const FftPlan &pz,
@@ -1559,7 +1559,7 @@ void launch_fft_fwd_z(hipStream_t s, int prec, const double *sig, void *specB, c
     else launch_fwd_z<float>(s, sig, specB, 6, n, pz, twz, ctl, tile, prec);
 }
 
-void launch_fft_y(hipStream_t s, int prec, const void *in, void *out, int ncomp, int sign, int b_to_c, const int n[3],
+hipError_t launch_fft_y(hipStream_t s, int prec, const void *in, void *out, int ncomp, int sign, int b_to_c, const int n[3],
                   const FftPlan &py, const void *twy, const IterCtl *ctl, int tile) {
     (void)sign;
     const int TX = zy_tile(py, n[0], tile, prec);
@@ -1583,11 +1583,11 @@ void launch_fft_y(hipStream_t s, int prec, const void *in, void *out, int ncomp,
             SRX_LAUNCH((k_fft_y<float, false>), grid, dim3(FFT_BLOCK), sm, s, (const cx<float> *)in, (cx<float> *)out,
                            n[0], n[1], n[2], b_to_c, FftStages(py), FastDiv(n[1]), TileDiv(n[0], TX, 1), (const cx<float> *)twy, TX, ctl);
     }
-    check_launch("fft_y");
+    return check_launch("fft_y");
 }
 
 template <typename T, int CO>
-static void launch_green_generic(hipStream_t s, int prec, void *specC, const int n[3], const FftPlan &px,
+static hipError_t launch_green_generic(hipStream_t s, int prec, void *specC, const int n[3], const FftPlan &px,
                                  const void *twx, const DevConst *cst, int mode, int ncomp, const IterCtl *ctl,
                                  void *nyq, int tile = 0) {
     const int slots = mode & 1 ? CO : ncomp;
@@ -1611,7 +1611,7 @@ static void launch_green_generic(hipStream_t s, int prec, void *specC, const int
     else
         SRX_LAUNCH((k_green_x<T, 2, CO>), grid, dim3(FFT_BLOCK), sm, s, (cx<T> *)specC, n[0], n[1], n[2], FftStages(px),
                    FastDiv(n[0]), TileDiv(n[1], TY, n[0]), (const cx<T> *)twx, TY, mode, ncomp, cst, ctl, ny);
-    check_launch("green_x");
+    return check_launch("green_x");
 }
 
 // The wavefront-per-row x pass serves n0 = 64, 128, 256 (tile -1, and the default tile 0 there);
@@ -1677,7 +1677,7 @@ void launch_plane(hipStream_t s, int prec, void *specB, const int n[3], const Ff
 }
 
 template <typename T>
-static void launch_inv_z(hipStream_t s, const void *specB, double *out, int ncomp, const int n[3], const FftPlan &pz,
+static hipError_t launch_inv_z(hipStream_t s, const void *specB, double *out, int ncomp, const int n[3], const FftPlan &pz,
                          const void *twz, int accumulate, double divisor, const IterCtl *ctl, int tile, int prec) {
     const int rows = n[0] * n[1], TY = zy_tile(pz, rows, tile, prec);
     const bool sw = plan_swizzled(pz);
@@ -1689,7 +1689,7 @@ static void launch_inv_z(hipStream_t s, const void *specB, double *out, int ncom
     else
         SRX_LAUNCH((k_inv_z<T, false>), grid, dim3(FFT_BLOCK), sm, s, (const cx<T> *)specB, out, ncomp, n[0], n[1], n[2],
                    FftStages(pz), FastDiv(n[2]), TileDiv(rows, TY, 1), (const cx<T> *)twz, TY, accumulate, divisor, ctl);
-    check_launch("inv_z");
+    return check_launch("inv_z");
 }
 
 void launch_fft_inv_z_update(hipStream_t s, int prec, const void *specB, double *ee, const int n[3], const FftPlan &pz,
@@ -1721,24 +1721,28 @@ void launch_rotation_part(hipStream_t s, int prec, const double *in, double *out
     else launch_inv_z<float>(s, specB, out, 3, n, pl[2], tw[2], 0, divisor, nullptr, tiles[4], prec);
 }
 
-// test path: forward FFT of ncomp real comps to layout C (x pass done), no Green
-void launch_fft_real_forward_test(hipStream_t s, int prec, const double *in, int ncomp, void *specB, void *specC,
-                                  const int n[3], const FftPlan *pl, void *const *tw) {
-    if (prec == 0) launch_fwd_z<double>(s, in, specB, ncomp, n, pl[2], tw[2], nullptr, 0, prec);
-    else launch_fwd_z<float>(s, in, specB, ncomp, n, pl[2], tw[2], nullptr, 0, prec);
-    launch_fft_y(s, prec, specB, specC, ncomp, -1, 1, n, pl[1], tw[1], nullptr);
-    if (prec == 0) launch_green_generic<double, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 0, ncomp, nullptr, nullptr);
-    else launch_green_generic<float, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 0, ncomp, nullptr, nullptr);
+// forward FFT of ncomp real comps to layout C (x pass done), no Green: the entry points' transforms
+hipError_t launch_fft_real_forward_test(hipStream_t s, int prec, const double *in, int ncomp, void *specB, void *specC,
+                                        const int n[3], const FftPlan *pl, void *const *tw) {
+    hipError_t e;
+    if (prec == 0) e = launch_fwd_z<double>(s, in, specB, ncomp, n, pl[2], tw[2], nullptr, 0, prec);
+    else e = launch_fwd_z<float>(s, in, specB, ncomp, n, pl[2], tw[2], nullptr, 0, prec);
+    if (e == hipSuccess) e = launch_fft_y(s, prec, specB, specC, ncomp, -1, 1, n, pl[1], tw[1], nullptr);
+    if (e != hipSuccess) return e;
+    if (prec == 0) return launch_green_generic<double, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 0, ncomp, nullptr, nullptr);
+    return launch_green_generic<float, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 0, ncomp, nullptr, nullptr);
 }
 
-// test path: inverse of the above for ncomp comps (layout C in, real out = IFFT * 1/divisor)
-void launch_fft_real_inverse_test(hipStream_t s, int prec, void *specC, void *specB, int ncomp, double *out,
-                                  const int n[3], const FftPlan *pl, void *const *tw, double divisor) {
-    if (prec == 0) launch_green_generic<double, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 2, ncomp, nullptr, nullptr);
-    else launch_green_generic<float, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 2, ncomp, nullptr, nullptr);
-    launch_fft_y(s, prec, specC, specB, ncomp, +1, 0, n, pl[1], tw[1], nullptr);
-    if (prec == 0) launch_inv_z<double>(s, specB, out, ncomp, n, pl[2], tw[2], 0, divisor, nullptr, 0, prec);
-    else launch_inv_z<float>(s, specB, out, ncomp, n, pl[2], tw[2], 0, divisor, nullptr, 0, prec);
+// inverse of the above for ncomp comps (layout C in, real out = IFFT * 1/divisor)
+hipError_t launch_fft_real_inverse_test(hipStream_t s, int prec, void *specC, void *specB, int ncomp, double *out,
+                                        const int n[3], const FftPlan *pl, void *const *tw, double divisor) {
+    hipError_t e;
+    if (prec == 0) e = launch_green_generic<double, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 2, ncomp, nullptr, nullptr);
+    else e = launch_green_generic<float, 6>(s, prec, specC, n, pl[0], tw[0], nullptr, 2, ncomp, nullptr, nullptr);
+    if (e == hipSuccess) e = launch_fft_y(s, prec, specC, specB, ncomp, +1, 0, n, pl[1], tw[1], nullptr);
+    if (e != hipSuccess) return e;
+    if (prec == 0) return launch_inv_z<double>(s, specB, out, ncomp, n, pl[2], tw[2], 0, divisor, nullptr, 0, prec);
+    return launch_inv_z<float>(s, specB, out, ncomp, n, pl[2], tw[2], 0, divisor, nullptr, 0, prec);
 }
 
 // ---------------------------------------------------------------------------

@@ -50,7 +50,7 @@ __global__ void __launch_bounds__(GATHER_BLOCK) k_gather(FieldSrc src, int v0, i
     for (int i = threadIdx.x; i < cnt * NC; i += GATHER_BLOCK) dst[i] = buf[i];
 }
 
-void launch_gather(hipStream_t s, int mode, int nc, const FieldSrc &src, int v0, int nv, double *out) {
+hipError_t launch_gather(hipStream_t s, int mode, int nc, const FieldSrc &src, int v0, int nv, double *out) {
     const dim3 g((nv + GATHER_BLOCK - 1) / GATHER_BLOCK), b(GATHER_BLOCK);
     switch (mode) {
     case FIELD_INT: hipLaunchKernelGGL((k_gather<FIELD_INT, 1>), g, b, 0, s, src, v0, nv, out); break;
@@ -62,7 +62,7 @@ void launch_gather(hipStream_t s, int mode, int nc, const FieldSrc &src, int v0,
         else if (nc == 9) hipLaunchKernelGGL((k_gather<FIELD_PLAIN, 9>), g, b, 0, s, src, v0, nv, out);
         else hipLaunchKernelGGL((k_gather<FIELD_PLAIN, 1>), g, b, 0, s, src, v0, nv, out);
     }
-    check_launch("gather");
+    return check_launch("gather");
 }
 
 // Spectra between the passes' layout C [c][kz][y][x] (complex T) and the entry points' [c][x][y][kz]
@@ -109,7 +109,7 @@ __global__ void __launch_bounds__(TURN_BLOCK) k_spec_turn(T *__restrict__ spec, 
     }
 }
 
-void launch_spec_turn(hipStream_t s, int prec, bool out, void *spec, double *user, int ncomp, const int n[3]) {
+hipError_t launch_spec_turn(hipStream_t s, int prec, bool out, void *spec, double *user, int ncomp, const int n[3]) {
     const int H = n[2] / 2 + 1;
     const dim3 g((n[0] + TURN_TILE - 1) / TURN_TILE, (H + TURN_TILE - 1) / TURN_TILE, ncomp * n[1]), b(TURN_BLOCK);
     if (prec != 0) {
@@ -119,7 +119,7 @@ void launch_spec_turn(hipStream_t s, int prec, bool out, void *spec, double *use
         if (out) hipLaunchKernelGGL((k_spec_turn<double, true>), g, b, 0, s, (double *)spec, user, n[0], n[1], H);
         else hipLaunchKernelGGL((k_spec_turn<double, false>), g, b, 0, s, (double *)spec, user, n[0], n[1], H);
     }
-    check_launch("spec_turn");
+    return check_launch("spec_turn");
 }
 
 }  // namespace srx

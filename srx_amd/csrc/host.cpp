@@ -25,11 +25,6 @@
 #include <thread>
 #include <vector>
 
-namespace srx {
-void launch_fft_real_inverse_test(hipStream_t s, int prec, void *specC, void *specB, int ncomp, double *out,
-                                  const int n[3], const FftPlan *pl, void *const *tw, double divisor);
-}
-
 using namespace srx;
 
 namespace {
@@ -2048,14 +2043,15 @@ static int read_field(srx_ctx *c, int mode, int nc, const FieldSrc &src, double 
     cp.total = total;
     if (total >= STAGE_MT)
         cp.start(c->opt.nthreads > 0 ? std::min(STAGE_HELPERS, c->opt.nthreads - 1) : STAGE_HELPERS, nchunk);
+    (void)hipGetLastError();   // an error the caller's own HIP calls left behind is not this read's
     // chunk k is launched STAGE_SLOTS - 1 chunks ahead of the one being copied
     for (size_t k = 0; k < nchunk + STAGE_SLOTS - 1; ++k) {
         if (k < nchunk) {
             const int slot = (int)(k % STAGE_SLOTS);
             if (k >= STAGE_SLOTS) cp.wait(k - STAGE_SLOTS + 1);
             const size_t v0 = k * per, nv = std::min(per, (size_t)c->nvox - v0);
-            launch_gather(c->stream, mode, nc, src, (int)v0, (int)nv,
-                          reinterpret_cast<double *>(c->stage + slot * c->stage_bytes));
+            HIPCK(launch_gather(c->stream, mode, nc, src, (int)v0, (int)nv,
+                                reinterpret_cast<double *>(c->stage + slot * c->stage_bytes)));
             HIPCK(hipEventRecord(c->stage_ev[slot], c->stream));
         }
         if (k + 1 < STAGE_SLOTS || k - (STAGE_SLOTS - 1) >= nchunk) continue;
@@ -2338,6 +2334,7 @@ int srx_mlp_samples(srx_ctx *c, float *x, float *t, size_t max, size_t *n) {
 static int fft_test_common(int ncomp, int n0, int n1, int n2, int prec, FftPlan pl[3], void *tw[3], void **sB,
                            void **sC, size_t &specn) {
     const int n[3] = {n0, n1, n2};
+    (void)hipGetLastError();   // an error the caller's own HIP calls left behind is not this transform's
     for (int i = 0; i < 3; ++i)
         if (!make_plan(n[i], pl[i])) return SRX_E_GRID;
     if (!grid_supported(pl, n, prec) || ncomp < 1 || ncomp > 9) return SRX_E_GRID;
@@ -2364,8 +2361,8 @@ int srx_fft_forward(const double *in, int ncomp, int n0, int n1, int n2, int pre
     if (!rc) {
         HIPCK(hipMalloc(&buf, sizeof(double) * 2 * specn));
         HIPCK(hipMemcpy(buf, in, sizeof(double) * ncomp * N, hipMemcpyHostToDevice));
-        launch_fft_real_forward_test(nullptr, prec, buf, ncomp, sB, sC, n, pl, tw);
-        launch_spec_turn(nullptr, prec, true, sC, buf, ncomp, n);
+        HIPCK(launch_fft_real_forward_test(nullptr, prec, buf, ncomp, sB, sC, n, pl, tw));
+        HIPCK(launch_spec_turn(nullptr, prec, true, sC, buf, ncomp, n));
         HIPCK(hipDeviceSynchronize());
         HIPCK(hipMemcpy(out, buf, sizeof(double) * 2 * specn, hipMemcpyDeviceToHost));
     }
@@ -2388,8 +2385,8 @@ int srx_fft_inverse(const double *in, int ncomp, int n0, int n1, int n2, int pre
     if (!rc) {
         HIPCK(hipMalloc(&buf, sizeof(double) * 2 * specn));
         HIPCK(hipMemcpy(buf, in, sizeof(double) * 2 * specn, hipMemcpyHostToDevice));
-        launch_spec_turn(nullptr, prec, false, sC, buf, ncomp, n);
-        launch_fft_real_inverse_test(nullptr, prec, sC, sB, ncomp, buf, n, pl, tw, 1.0 / scale);
+        HIPCK(launch_spec_turn(nullptr, prec, false, sC, buf, ncomp, n));
+        HIPCK(launch_fft_real_inverse_test(nullptr, prec, sC, sB, ncomp, buf, n, pl, tw, 1.0 / scale));
         HIPCK(hipDeviceSynchronize());
         HIPCK(hipMemcpy(out, buf, sizeof(double) * ncomp * N, hipMemcpyDeviceToHost));
     }

@@ -25,9 +25,11 @@ extern thread_local hipEvent_t g_ev_start, g_ev_stop;
         }                                                                                                \
     } while (0)
 
-inline void check_launch(const char *name) {
+// Takes the error of the launches since the last call (hipGetLastError clears it) and returns it.
+inline hipError_t check_launch(const char *name) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) fprintf(stderr, "srx: launch of %s failed: %s\n", name, hipGetErrorString(e));
+    return e;
 }
 
 // B-basis constants: 1/sqrt(2), 1/sqrt(3), 1/sqrt(6) (chg_basis, kinematics.c:55-60)

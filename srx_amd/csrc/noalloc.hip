@@ -81,6 +81,7 @@ extern "C" int srx_fft_forward_noalloc(const double *d_in, int ncomp, int n0, in
     if (need > (size_t)SRX_NOALLOC_SCRATCH_BYTES) return SRX_E_SCRATCH;
     void *base = nullptr;
     if (int rc = scratch_ptr(&base)) return rc;
+    (void)hipGetLastError();   // an error the caller's own HIP calls left behind is not this transform's
     unsigned char *b = static_cast<unsigned char *>(base);
     void *tw[3];
     for (int ax = 0; ax < 3; ++ax) {
@@ -90,9 +91,10 @@ extern "C" int srx_fft_forward_noalloc(const double *d_in, int ncomp, int n0, in
         else hipLaunchKernelGGL(k_twiddles<double>, grid, dim3(256), 0, nullptr, (double *)tw[ax], n[ax]);
     }
     void *sB = b + offB, *sC = b + offC;
-    launch_fft_real_forward_test(nullptr, precision, d_in, ncomp, sB, sC, n, pl, tw);
-    launch_spec_turn(nullptr, precision, true, sC, d_out, ncomp, n);
-    if (hipGetLastError() != hipSuccess) return SRX_E_HIP;
+    // (a failed twiddle launch is still pending and reported by the first of these)
+    if (launch_fft_real_forward_test(nullptr, precision, d_in, ncomp, sB, sC, n, pl, tw) != hipSuccess ||
+        launch_spec_turn(nullptr, precision, true, sC, d_out, ncomp, n) != hipSuccess)
+        return SRX_E_HIP;
     if (hipStreamSynchronize(nullptr) != hipSuccess) return SRX_E_HIP;
     return 0;
 }

@@ -248,7 +248,7 @@ int fft_tile_max(int pass, const int n[3], const FftPlan &p, int prec, int comps
 bool green_wave_ok(const int n[3]);
 void launch_fft_fwd_z(hipStream_t s, int prec, const double *sig, void *specB, const int n[3],
                       const FftPlan &pz, const void *twz, const IterCtl *ctl, int tile = 0);
-void launch_fft_y(hipStream_t s, int prec, const void *in, void *out, int ncomp, int sign, int b_to_c,
+hipError_t launch_fft_y(hipStream_t s, int prec, const void *in, void *out, int ncomp, int sign, int b_to_c,
                   const int n[3], const FftPlan &py, const void *twy, const IterCtl *ctl = nullptr, int tile = 0);
 // strain_form: the iterations advance the strain's six components (Fields::ee) instead of DisGrad's nine
 bool strain_form(const int n[3], int prec);
@@ -338,10 +338,13 @@ struct FieldSrc {
     int comps;
     double dt, u[9];
 };
-void launch_gather(hipStream_t s, int mode, int nc, const FieldSrc &src, int v0, int nv, double *out);
+// (launches whose kernels write what an entry point returns report their status; the others print it)
+hipError_t launch_gather(hipStream_t s, int mode, int nc, const FieldSrc &src, int v0, int nv, double *out);
 // spectra: layout C to the entry points' [c][x][y][kz] order (out), or back
-void launch_spec_turn(hipStream_t s, int prec, bool out, void *spec, double *user, int ncomp, const int n[3]);
-void launch_fft_real_forward_test(hipStream_t s, int prec, const double *in, int ncomp, void *specB, void *specC,
-                                  const int n[3], const FftPlan *pl, void *const *tw);
+hipError_t launch_spec_turn(hipStream_t s, int prec, bool out, void *spec, double *user, int ncomp, const int n[3]);
+hipError_t launch_fft_real_forward_test(hipStream_t s, int prec, const double *in, int ncomp, void *specB, void *specC,
+                                        const int n[3], const FftPlan *pl, void *const *tw);
+hipError_t launch_fft_real_inverse_test(hipStream_t s, int prec, void *specC, void *specB, int ncomp, double *out,
+                                        const int n[3], const FftPlan *pl, void *const *tw, double divisor);
 
 }  // namespace srx

@@ -1,0 +1,69 @@
+"""A kernel launch that the runtime refuses is an error of the call that made it, not a result: the entry
+points whose kernels write the caller's data, run on tests/host_runtime.c (no GPU)."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from srx_amd import inputs
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRELUDE = """
+import ctypes as C, sys
+import numpy as np
+rt = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+import srx_amd
+L = srx_amd.lib()
+E_HIP = 2003
+def each_launch_refused(call):
+    rt.host_fail_launch(-1)
+    assert call() == 0
+    n = rt.host_launches()
+    assert n > 0
+    for k in range(n):
+        rt.host_fail_launch(k)
+        assert call() == E_HIP, k
+    rt.host_fail_launch(-1)
+    assert call() == 0
+"""
+FFT = """
+n, nc = (12, 10, 8), 3
+x = np.zeros(nc * 12 * 10 * 8)
+X = np.zeros(nc * 12 * 10 * 5 * 2)
+for prec in (srx_amd.PREC_FP64, srx_amd.PREC_MIXED):
+    each_launch_refused(lambda: L.srx_fft_forward(srx_amd._dptr(x), nc, *n, prec, srx_amd._dptr(X)))
+    each_launch_refused(lambda: L.srx_fft_inverse(srx_amd._dptr(X), nc, *n, prec, 1.0, srx_amd._dptr(x)))
+    L.srx_fft_forward_noalloc.argtypes = L.srx_fft_forward.argtypes
+    each_launch_refused(lambda: L.srx_fft_forward_noalloc(srx_amd._dptr(x), nc, *n, prec, srx_amd._dptr(X)))
+"""
+FIELD = """
+s = srx_amd.Solver(sys.argv[2])
+for name, (fid, nc) in srx_amd.FIELDS.items():
+    if name in ("grain", "rho_g1", "rho_g2"):   # kept on the host; GND option only
+        continue
+    out = np.empty(s.nxyz * nc)
+    each_launch_refused(lambda: L.srx_get_field(s.h, fid, srx_amd._dptr(out), out.size))
+"""
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("rt") / "host_runtime.so")
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-O1", "-o", lib, os.path.join(HERE, "host_runtime.c")])
+    return lib
+
+
+def run(body, *args):
+    p = subprocess.run([sys.executable, "-c", PRELUDE + body, *args], cwd=os.path.dirname(HERE), capture_output=True,
+                       text=True, timeout=110)
+    assert p.returncode == 0, p.stderr[-2000:]
+
+
+def test_transforms_report_a_refused_launch(runtime):
+    run(FFT, runtime)
+
+
+@pytest.mark.parametrize("n", [(6, 5, 4), (48, 40, 60)])   # one chunk; several, some of them in flight
+def test_field_reads_report_a_refused_launch(runtime, tmp_path, n):
+    run(FIELD, runtime, inputs.make_case(str(tmp_path), n=n, grains=3, seed=1, nsteps=1, timestep=0.1))
