@@ -2028,7 +2028,8 @@ static int read_field(srx_ctx *c, int mode, int nc, const FieldSrc &src, double 
     if (!c->stage) {
         // sized for the largest field (12 values per voxel), whole rows of every field in a slot
         const size_t most = sizeof(double) * 12 * (size_t)c->nvox;
-        c->stage_bytes = std::min(most, std::max(STAGE_SLOT, std::min(STAGE_SLOT_MAX, most / 16)));
+        const size_t want = std::min(most, std::max(STAGE_SLOT, std::min(STAGE_SLOT_MAX, most / 16)));
+        c->stage_bytes = (want + 4095) & ~(size_t)4095;   // slots start on page boundaries
         for (int k = 0; k < STAGE_SLOTS; ++k)
             if (!c->stage_ev[k]) HIPCK(hipEventCreateWithFlags(&c->stage_ev[k], hipEventDisableTiming));
         HIPCK(hipHostMalloc((void **)&c->stage, STAGE_SLOTS * c->stage_bytes, hipHostMallocDefault));

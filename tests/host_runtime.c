@@ -2,7 +2,9 @@
    host memory, copies and fills happen at once, kernels are counted and do nothing.  Loaded with
    RTLD_GLOBAL before libsrx.so, it answers the library's calls into the runtime.
    host_fail_launch(k): the k-th launch from now (0: the next) fails, -1: none;
-   host_launches(): launches since the last host_fail_launch. */
+   host_launches(): launches since the last host_fail_launch.
+   host_watch_pointer(i): from now on, note the pointer every launch passes as its argument i (-1: none);
+   host_pointer_offsets(): the bits set in any of their distances from the first. */
 #include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
@@ -14,18 +16,28 @@ static int last_error;
 void host_fail_launch(long k) { launches = 0; fail_at = k; last_error = 0; }
 long host_launches(void) { return launches; }
 
-static int launch(void) {
+static int watched = -1;
+static uintptr_t first_pointer, offsets;
+void host_watch_pointer(int i) { watched = i; first_pointer = offsets = 0; }
+long host_pointer_offsets(void) { return (long)offsets; }
+
+static int launch(void **args) {
+    if (watched >= 0) {
+        const uintptr_t p = *(uintptr_t *)args[watched];
+        if (!first_pointer) first_pointer = p;
+        offsets |= p - first_pointer;
+    }
     if (launches++ == fail_at) last_error = 701; /* hipErrorLaunchOutOfResources */
     else return 0;
     return last_error;
 }
 int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **a, size_t m, void *s) {
-    (void)f; (void)g; (void)b; (void)a; (void)m; (void)s;
-    return launch();
+    (void)f; (void)g; (void)b; (void)m; (void)s;
+    return launch(a);
 }
 int hipExtLaunchKernel(const void *f, dim3_t g, dim3_t b, void **a, size_t m, void *s, void *e0, void *e1, int fl) {
-    (void)f; (void)g; (void)b; (void)a; (void)m; (void)s; (void)e0; (void)e1; (void)fl;
-    return launch();
+    (void)f; (void)g; (void)b; (void)m; (void)s; (void)e0; (void)e1; (void)fl;
+    return launch(a);
 }
 int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t m, void *s) { (void)g; (void)b; (void)m; (void)s; return 0; }
 int __hipPopCallConfiguration(dim3_t *g, dim3_t *b, size_t *m, void **s) {

@@ -128,3 +128,16 @@ def test_fields_read_back_whole(tmp_path, n):
     s.set_field("sig", t.reshape(N, 9))
     assert np.abs(s.field("sig") - t.reshape(N, 9)).max() <= 1e-14 * np.abs(t).max()
     s.close()
+
+
+@pytest.mark.parametrize("n", [(75, 75, 75), (81, 75, 81)])
+def test_fields_of_odd_large_grids_read_back_whole(tmp_path, n):
+    """Chunk sizes that follow from an odd number of voxels: what set_field stored comes back bit for bit."""
+    deck = inputs.make_case(str(tmp_path), n=n, grains=3, seed=5, nsteps=1, timestep=0.1)
+    s = srx_amd.Solver(deck)
+    rng = np.random.default_rng(8)
+    for name, nc in (("disgrad", 9), ("rho_s", 12)):
+        a = rng.normal(size=(n[0] * n[1] * n[2], nc))
+        s.set_field(name, a)
+        np.testing.assert_array_equal(s.field(name), a)
+    s.close()

@@ -45,6 +45,15 @@ for name, (fid, nc) in srx_amd.FIELDS.items():
     out = np.empty(s.nxyz * nc)
     each_launch_refused(lambda: L.srx_get_field(s.h, fid, srx_amd._dptr(out), out.size))
 """
+SLOTS = """
+s = srx_amd.Solver(sys.argv[2])
+for name in ("sig", "rho_s", "rho_tot"):
+    fid, nc = srx_amd.FIELDS[name]
+    out = np.empty(s.nxyz * nc)
+    rt.host_watch_pointer(3)   # where k_gather writes
+    assert L.srx_get_field(s.h, fid, srx_amd._dptr(out), out.size) == 0
+    assert rt.host_pointer_offsets() % 512 == 0, (name, rt.host_pointer_offsets())
+"""
 
 
 @pytest.fixture(scope="module")
@@ -67,3 +76,10 @@ def test_transforms_report_a_refused_launch(runtime):
 @pytest.mark.parametrize("n", [(6, 5, 4), (48, 40, 60)])   # one chunk; several, some of them in flight
 def test_field_reads_report_a_refused_launch(runtime, tmp_path, n):
     run(FIELD, runtime, inputs.make_case(str(tmp_path), n=n, grains=3, seed=1, nsteps=1, timestep=0.1))
+
+
+@pytest.mark.parametrize("n", [(75, 75, 75), (81, 81, 81), (120, 81, 75)])
+def test_field_chunks_start_aligned(runtime, tmp_path, n):
+    """The gather kernel stores 8-byte values in runs of 512 B: every chunk's slot starts at a multiple of
+    that from the first, also where the slots' size follows from the number of voxels."""
+    run(SLOTS, runtime, inputs.make_case(str(tmp_path), n=n, grains=3, seed=1, nsteps=1, timestep=0.1))
