@@ -3,6 +3,7 @@
    RTLD_GLOBAL before libsrx.so, it answers the library's calls into the runtime.
    host_fail_launch(k): the k-th launch from now (0: the next) fails, -1: none;
    host_launches(): launches since the last host_fail_launch.
+   host_pinned_bytes(): pinned memory handed out so far;
    host_watch_pointer(i): from now on, note the pointer every launch passes as its argument i (-1: none);
    host_pointer_offsets(): the bits set in any of their distances from the first. */
 #include <stdint.h>
@@ -58,7 +59,9 @@ int hipMalloc(void **p, size_t n) {
     }
     return 0;
 }
-int hipHostMalloc(void **p, size_t n, unsigned f) { (void)f; return get(p, n); }
+static size_t pinned;
+long host_pinned_bytes(void) { return (long)pinned; }
+int hipHostMalloc(void **p, size_t n, unsigned f) { (void)f; pinned += n; return get(p, n); }
 int hipFree(void *p) { free(p); return 0; }
 int hipHostFree(void *p) { free(p); return 0; }
 int hipMemcpy(void *d, const void *s, size_t n, int k) { (void)k; memmove(d, s, n); return 0; }

@@ -54,6 +54,14 @@ for name in ("sig", "rho_s", "rho_tot"):
     assert L.srx_get_field(s.h, fid, srx_amd._dptr(out), out.size) == 0
     assert rt.host_pointer_offsets() % 512 == 0, (name, rt.host_pointer_offsets())
 """
+PINNED = """
+s = srx_amd.Solver(sys.argv[2])
+before = rt.host_pinned_bytes()
+for name in ("sig", "rho_s", "rho_tot"):   # the first read, and larger and smaller fields after it
+    s.field(name)
+most = s.nxyz * 12 * 8
+assert rt.host_pinned_bytes() - before <= (most + 4096 if most <= 2 << 20 else most // 4 + 4 * 4096)
+"""
 
 
 @pytest.fixture(scope="module")
@@ -83,3 +91,10 @@ def test_field_chunks_start_aligned(runtime, tmp_path, n):
     """The gather kernel stores 8-byte values in runs of 512 B: every chunk's slot starts at a multiple of
     that from the first, also where the slots' size follows from the number of voxels."""
     run(SLOTS, runtime, inputs.make_case(str(tmp_path), n=n, grains=3, seed=1, nsteps=1, timestep=0.1))
+
+
+@pytest.mark.parametrize("n", [(4, 4, 4), (27, 27, 27), (32, 32, 32), (48, 48, 48), (75, 60, 45)])
+def test_first_field_read_pins_a_quarter_of_a_field(runtime, tmp_path, n):
+    """Pinned memory is paid for by a context's first read (its pages are mapped on first touch): no more of it
+    than a quarter of the largest field, or one such field where that is small."""
+    run(PINNED, runtime, inputs.make_case(str(tmp_path), n=n, grains=3, seed=1, nsteps=1, timestep=0.1))
