@@ -364,6 +364,7 @@ struct srx_ctx {
     // field readback: pinned slots of stage_bytes each (allocated by the first srx_get_field)
     char *stage = nullptr;
     size_t stage_bytes = 0;
+    std::mutex stage_mu;   // one reader at a time: the slots are the context's, not the call's
     hipEvent_t stage_ev[4] = {nullptr, nullptr, nullptr, nullptr};
     // outer-iteration batches captured as HIP graphs: [first batch of an increment][rotated]
     hipGraphExec_t gexec[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
@@ -2030,6 +2031,7 @@ struct StageCopy {
 
 static int read_field(srx_ctx *c, int mode, int nc, const FieldSrc &src, double *out) {
     const size_t row = sizeof(double) * nc, total = row * (size_t)c->nvox;
+    std::lock_guard<std::mutex> lk(c->stage_mu);
     if (!c->stage) {
         // sized for the largest field (12 values per voxel), whole rows of every field in a slot
         const size_t most = sizeof(double) * 12 * (size_t)c->nvox;

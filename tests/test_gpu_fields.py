@@ -1,5 +1,6 @@
 """Field dumps (.iout, io.c:322-941 at evolution.c:1456-1483) and the derived fields they use
 (fluctuation, rho_tot), GPU path against the oracle's fields through the C ABI."""
+import concurrent.futures
 import os
 
 import numpy as np
@@ -140,4 +141,22 @@ def test_fields_of_odd_large_grids_read_back_whole(tmp_path, n):
         a = rng.normal(size=(n[0] * n[1] * n[2], nc))
         s.set_field(name, a)
         np.testing.assert_array_equal(s.field(name), a)
+    s.close()
+
+
+def test_fields_read_by_several_threads(tmp_path):
+    """Reads of one context from several host threads (between increments) share its pinned slots, one
+    at a time: each thread's values are those of its own field."""
+    n = (40, 36, 30)   # several chunks a field
+    deck = inputs.make_case(str(tmp_path), n=n, grains=3, seed=5, nsteps=1, timestep=0.1)
+    s = srx_amd.Solver(deck)
+    rng = np.random.default_rng(9)
+    want = {}
+    for name, nc in (("disgrad", 9), ("tranmat", 9), ("rho_s", 12), ("gam_acum", 12)):
+        want[name] = rng.normal(size=(n[0] * n[1] * n[2], nc))
+        s.set_field(name, want[name])
+    with concurrent.futures.ThreadPoolExecutor(4) as ex:
+        reads = [(name, ex.submit(s.field, name)) for _ in range(8) for name in want]
+        for name, r in reads:
+            np.testing.assert_array_equal(r.result(), want[name], err_msg=name)
     s.close()
