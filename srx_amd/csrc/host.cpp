@@ -329,6 +329,7 @@ struct srx_ctx {
     double *quat = nullptr;                     // Fields::quat's memory (also while f.quat is null)
     void *nyq = nullptr;                        // rotation sums of the Nyquist planes (nyq_elems complex doubles)
     void *tw[3] = {nullptr, nullptr, nullptr};
+    void *tw64[3] = {nullptr, nullptr, nullptr};   // mixed precision with the strain form: the rotation pass's
     FftPlan pl[3];
     double *partials = nullptr, *red = nullptr, *hred = nullptr, *redseg = nullptr;
     IterCtl *dctl = nullptr, *hctl = nullptr;   // outer-iteration control block (device, pinned host copy)
@@ -800,13 +801,15 @@ int setup(srx_ctx *c) {
 
     const size_t H = (size_t)(c->n[2] / 2 + 1);
     const size_t spec_elems = (F.ee ? 6 : 9) * H * c->n[0] * c->n[1];
-    const size_t csz = c->opt.precision == SRX_PREC_MIXED ? 2 * sizeof(float) : 2 * sizeof(double);
+    // with the strain form the spectra hold FP64 values in mixed precision too: the rotation pass's
+    const bool mixed = c->opt.precision == SRX_PREC_MIXED;
+    const size_t csz = mixed && !F.ee ? 2 * sizeof(float) : 2 * sizeof(double);
     HIPCK(hipMalloc(&c->specB, spec_elems * csz));
     HIPCK(hipMalloc(&c->specC, spec_elems * csz));
     if (F.ee) HIPCK(hipMalloc(&c->nyq, nyq_elems(c->n) * 2 * sizeof(double)));
     for (int ax = 0; ax < 3; ++ax) {
-        int r = c->opt.precision == SRX_PREC_MIXED ? upload_twiddles<float>(c->n[ax], &c->tw[ax], st)
-                                                   : upload_twiddles<double>(c->n[ax], &c->tw[ax], st);
+        int r = mixed ? upload_twiddles<float>(c->n[ax], &c->tw[ax], st) : upload_twiddles<double>(c->n[ax], &c->tw[ax], st);
+        if (!r && mixed && F.ee) r = upload_twiddles<double>(c->n[ax], &c->tw64[ax], st);
         if (r) return r;
     }
     HIPCK(hipMalloc(&c->dctl, sizeof(IterCtl)));
@@ -1470,8 +1473,8 @@ static void disgrad_from_strain(srx_ctx *c) {
     double du[9];
     for (int k = 0; k < 9; ++k) du[k] = ctl.uniform[k] - c->uniform0[k];
     launch_rot_in(c->stream, c->f, (int)c->nvox, du);
-    launch_rotation_part(c->stream, c->opt.precision, c->f.ee, c->f.ee, c->specB, c->specC, c->n, c->pl, c->tw, c->dc,
-                         c->nyq, c->tiles);
+    launch_rotation_part(c->stream, c->f.ee, c->f.ee, c->specB, c->specC, c->n, c->pl,
+                         c->opt.precision == SRX_PREC_MIXED ? c->tw64 : c->tw, c->dc, c->nyq, c->tiles);
     launch_rot_out(c->stream, c->f, (int)c->nvox, du);
 }
 
@@ -2244,7 +2247,8 @@ void srx_close(srx_ctx *c) {
     if (c->specC) (void)hipFree(c->specC);
     if (c->nyq) (void)hipFree(c->nyq);
     for (int i = 0; i < 3; ++i)
-        if (c->tw[i]) (void)hipFree(c->tw[i]);
+        for (void *t : {c->tw[i], c->tw64[i]})
+            if (t) (void)hipFree(t);
     if (c->dc) (void)hipFree(c->dc);
     if (c->hred) (void)hipHostFree(c->hred);
     if (c->dctl) (void)hipFree(c->dctl);

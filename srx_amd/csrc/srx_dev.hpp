@@ -263,10 +263,9 @@ void launch_plane(hipStream_t s, int prec, void *specB, const int n[3], const Ff
                   const DevConst *cst, const IterCtl *ctl, void *nyq);
 void launch_fft_inv_z_update(hipStream_t s, int prec, const void *specB, double *ee, const int n[3],
                              const FftPlan &pz, const void *twz, const IterCtl *ctl, double scale, int tile = 0);
-// End of increment: the rotation part (3 comps) of the DisGrad change from its strain part (6 comps)
-void launch_rotation_part(hipStream_t s, int prec, const double *in, double *out, void *specB, void *specC,
-                          const int n[3], const FftPlan pl[3], void *const tw[3], const DevConst *cst, void *nyq,
-                          const int tiles[5]);
+// End of increment: the rotation part (3 comps) of the DisGrad change from its strain part (6 comps), in FP64
+void launch_rotation_part(hipStream_t s, const double *in, double *out, void *specB, void *specC, const int n[3],
+                          const FftPlan pl[3], void *const tw[3], const DevConst *cst, void *nyq, const int tiles[5]);
 void launch_rot_in(hipStream_t s, const Fields &f, int nvox, const double *du9);
 void launch_rot_out(hipStream_t s, const Fields &f, int nvox, const double *du9);
 // ph2: the second phase is crystalline (its Newton path is compiled in only then); fcc: nr_fcc of the constants

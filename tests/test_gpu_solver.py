@@ -372,6 +372,40 @@ def test_displacement_gradient_matches_oracle(tmp_path, oracle_lib, n, precision
     o.close()
 
 
+@pytest.mark.parametrize("n,precision", [((12, 10, 9), srx_amd.PREC_FP64), ((64, 5, 4), srx_amd.PREC_FP64),
+                                         ((16, 8, 4), srx_amd.PREC_MIXED), ((32, 32, 2), srx_amd.PREC_MIXED),
+                                         ((64, 8, 4), srx_amd.PREC_MIXED), ((128, 4, 8), srx_amd.PREC_MIXED),
+                                         ((512, 2, 4), srx_amd.PREC_MIXED)])
+def test_rotation_recovered_to_fp64(tmp_path, n, precision):
+    """Off the Nyquist planes and k = 0 the rotation of an increment's displacement gradient follows from its
+    strain e as e n x n.  The pass that recovers it works in FP64 in both precisions: against the same
+    formula in numpy, a few FP64 roundings of DisGrad (2^-52 of 1e-3) in increments of 1e-5, 1e-10 with a
+    margin; in FP32 the two would differ by 1e-7."""
+    deck = make(tmp_path, n=n, grains=6, seed=37, nsteps=3)
+    g = srx_amd.Solver(deck, fixed_iters=6, precision=precision)
+    k = [2.0 * np.pi * np.fft.fftfreq(m) for m in n]
+    k[2] = 2.0 * np.pi * np.fft.rfftfreq(n[2])
+    kv = np.stack(np.meshgrid(*k, indexing="ij"))
+    keep = (kv**2).sum(0) > 0
+    for a in range(3):
+        if n[a] % 2 == 0:
+            keep &= np.abs(kv[a]) < np.pi * (1 - 1e-9)
+    nv = kv / np.sqrt(np.where(keep, (kv**2).sum(0), 1.0))
+    before = g.field("disgrad")
+    for _ in range(3):
+        g.step()
+        after = g.field("disgrad")
+        D = np.fft.rfftn((after - before).reshape(n + (3, 3)), axes=(0, 1, 2))
+        before = after
+        e = 0.5 * (D + D.swapaxes(-1, -2))
+        en = np.einsum("xyzij,jxyz->xyzi", e, nv)
+        for i, j in ((1, 2), (0, 2), (0, 1)):
+            w = 0.5 * (D[..., i, j] - D[..., j, i])
+            want = en[..., i] * nv[j] - en[..., j] * nv[i]
+            assert np.abs((w - want)[keep]).max() <= 1e-10 * np.abs(D[keep]).max(), (i, j)
+    g.close()
+
+
 @pytest.mark.parametrize("n,precision", [((16, 16, 3), srx_amd.PREC_FP64), ((256, 1, 4), srx_amd.PREC_FP64),
                                          ((2, 125, 2), srx_amd.PREC_FP64), ((1, 250, 3), srx_amd.PREC_MIXED),
                                          ((18, 15, 5), srx_amd.PREC_FP64), ((5, 54, 4), srx_amd.PREC_FP64),
