@@ -245,7 +245,8 @@ int srx_mlp_samples(srx_ctx *ctx, float *x, float *t, size_t max, size_t *n);
 /* FFT tiles chosen at srx_open (rows per block of the forward z, forward y, Green x, inverse y
    and inverse z passes; 0: default; -1: the Green x pass runs one wavefront per row, possible for
    n0 = 64, 128 and 256, where it is also the default) and their timed launch durations in
-   microseconds. */
+   microseconds.  Grids with n0 n1 <= 256 run the two y passes and the Green x pass as one launch
+   without tiles: 0 and no duration for these three. */
 int srx_fft_tiles(srx_ctx *ctx, int *tiles, double *us);
 
 /* Most radix stages of one FFT plan. */
@@ -258,7 +259,8 @@ int srx_fft_tiles(srx_ctx *ctx, int *tiles, double *us);
    axis whose passes take a plan (not x where the wavefront Green pass runs) and keeps the fastest,
    the same plan for every context of one grid shape and precision in the process.  Another radix
    order rounds differently: results then differ from the default plans within the FFT's rounding
-   error, not bitwise.  The x pass of n0 = 64, 128 and 256 takes no plan (one wavefront per row). */
+   error, not bitwise.  The x pass of n0 = 64, 128 and 256 takes no plan (one wavefront per row),
+   except on grids with n0 n1 <= 256 (see srx_fft_tiles). */
 int srx_fft_plan(srx_ctx *ctx, int axis, int *radices, int *nstages);
 
 /* Sets the plan of one axis: radices[0..nstages-1] from {2, 3, 4, 5, 8} whose product is the

@@ -1195,7 +1195,10 @@ __global__ void __launch_bounds__(256, SRX_GREEN_MIN_BLOCKS) k_green_wave(cx<T> 
 // grid: (H), PLANE_BLOCK threads.  LDS: CO slots of n0 rows of n1 | 1, then the two twiddle tables.
 // Bound by the chain of one block's stages.  Against the three passes it saves two launches and the
 // spectra's trips through memory, an outer iteration in FP64: 8^3 44.0 -> 37.7 us, 12^3 45.7 -> 41.6, 16^3
-// 46.3 -> 43.6, 16 x 16 x 256 72.1 -> 63.0.  Beyond 256 points a plane's chain is longer than the three
+// 46.3 -> 43.6, 16 x 16 x 256 72.1 -> 63.0.  Long planes, whose x pass would be the wavefront Green pass:
+// 64 x 1 x 4 39.1 -> 36.9, 64 x 4 x 64 46.2 -> 46.6, 128 x 2 x 64 49.0 -> 48.3, 256 x 1 x 128 59.0 -> 50.6,
+// 4 x 64 x 64 51.0 -> 47.5 (the one slower by more than 1%: 64 x 4 x 8, 41.6 -> 42.9; in mixed
+// precision all are faster).  Beyond 256 points a plane's chain is longer than the three
 // launches (18^3 48.9 -> 50.9, 24^3 49.5 -> 53.4): PLANE_POINTS.
 // ---------------------------------------------------------------------------
 constexpr int PLANE_BLOCK = 512, PLANE_POINTS = 256;

@@ -929,12 +929,13 @@ const char *srx_strerror(int code) {
 }
 
 // Average time (us) of three launches of FFT pass `pass` (0 forward z, 1 forward y, 2 Green x,
-// 3 inverse y, 4 inverse z) at tile `t`, after one warm-up launch, on the context's own buffers with
+// 3 inverse y, 4 inverse z; PASS_PLANE: passes 1 to 3 in one launch) at tile `t`, after one warm-up launch, on the context's own buffers with
 // its current plans (the inverse z pass writes the scratch strain `scratch`).  With a `flush`
 // buffer (2 x FLUSH_BYTES) each launch is timed alone after a streaming copy through it, so the
 // pass reads its input from HBM as it does in the solver, where the Newton kernel's traffic has
 // evicted it from the last-level cache; else the three launches run back to back.
 constexpr size_t FLUSH_BYTES = (size_t)320 << 20;
+constexpr int PASS_PLANE = 5;
 static int time_pass(srx_ctx *c, int pass, int t, double *scratch, hipEvent_t e0, hipEvent_t e1, double &us,
                      char *flush = nullptr) {
     const int prec = c->opt.precision;
@@ -945,6 +946,7 @@ static int time_pass(srx_ctx *c, int pass, int t, double *scratch, hipEvent_t e0
         case 1: launch_fft_y(st, prec, c->specB, c->specC, 6, -1, 1, c->n, c->pl[1], c->tw[1], nullptr, t); break;
         case 2: launch_green_x(st, prec, c->specC, c->n, c->pl[0], c->tw[0], c->dc, nullptr, nullptr, t); break;
         case 3: launch_fft_y(st, prec, c->specC, c->specB, c->comps(), +1, 0, c->n, c->pl[1], c->tw[1], nullptr, t); break;
+        case PASS_PLANE: launch_plane(st, prec, c->specB, c->n, c->pl, c->tw, c->dc, nullptr, nullptr); break;
         default:
             launch_fft_inv_z_update(st, prec, c->specB, scratch, c->n, c->pl[2], c->tw[2], nullptr, (double)c->nvox,
                                     t);
@@ -977,8 +979,10 @@ static int time_pass(srx_ctx *c, int pass, int t, double *scratch, hipEvent_t e0
 
 static_assert(SRX_FFT_MAX_STAGES == MAX_RADIX_STAGES, "plan stage count of the ABI");
 
-// FFT passes of each plan axis (x: the Green pass; y and z: forward and inverse)
+// FFT passes of each plan axis (x: the Green pass; y and z: forward and inverse), and where the plane
+// kernel runs them
 static const int AXIS_PASSES[3][2] = {{2, -1}, {1, 3}, {0, 4}};
+static const int PLANE_AXIS_PASSES[3][2] = {{PASS_PLANE, -1}, {PASS_PLANE, -1}, {0, 4}};
 
 // Radix plans chosen by timing (options.reserved[3] = 1), kept per process for the grid shape and
 // precision: every context of one shape, e.g. the members of an ensemble, runs the same plans.
@@ -986,6 +990,8 @@ static std::mutex g_plan_mu;
 static std::map<std::array<int, 5>, FftPlan> g_plan_cache;
 
 // FFT autotuner, at srx_open on the context's own buffers.
+// Small planes (plane_pass_ok) run the y and x transforms and the Green operator in one launch: their x
+// and y plans are timed with that kernel, and the passes it replaces keep their default tiles.
 // Radix plans (opt-in, options.reserved[3] = 1): for each axis whose passes take a plan (not the
 // x axis where the wavefront Green pass runs), every candidate of plan_candidates that the passes
 // accept is timed over that axis's passes at their default tiles, each launch alone after a
@@ -1002,6 +1008,8 @@ static std::map<std::array<int, 5>, FftPlan> g_plan_cache;
 // depend on the tile timings (or on what else the GPU runs meanwhile).
 static int autotune_fft(srx_ctx *c) {
     const int prec = c->opt.precision;
+    const bool plane = plane_pass_ok(c->n);
+    const auto &axis_passes = plane ? PLANE_AXIS_PASSES : AXIS_PASSES;
     double *scratch = nullptr;
     HIPCK(hipMalloc(&scratch, sizeof(double) * c->comps() * (size_t)c->nvox));
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1010,7 +1018,7 @@ static int autotune_fft(srx_ctx *c) {
     char *flush = nullptr;
     if (!rc && c->opt.reserved[3] == 1 && hipMalloc(&flush, 2 * FLUSH_BYTES) != hipSuccess) rc = SRX_E_NOMEM;
     for (int ax = 0; ax < 3 && !rc && c->opt.reserved[3] == 1; ++ax) {
-        if (ax == 0 && green_wave_ok(c->n)) continue;   // the wavefront pass takes no plan
+        if (ax == 0 && green_wave_ok(c->n) && !plane) continue;   // the wavefront pass takes no plan
         const std::array<int, 5> key = {ax, c->n[0], c->n[1], c->n[2], prec};
         {
             std::lock_guard<std::mutex> lk(g_plan_mu);
@@ -1036,7 +1044,7 @@ static int autotune_fft(srx_ctx *c) {
                 double tot = 0.0;
                 for (int k = 0; k < 2 && !rc; ++k) {
                     double us = 0.0;
-                    if (AXIS_PASSES[ax][k] >= 0) rc = time_pass(c, AXIS_PASSES[ax][k], 0, scratch, e0, e1, us, flush);
+                    if (axis_passes[ax][k] >= 0) rc = time_pass(c, axis_passes[ax][k], 0, scratch, e0, e1, us, flush);
                     tot += us;
                 }
                 t_best[i] = std::min(t_best[i], tot);
@@ -1052,6 +1060,7 @@ static int autotune_fft(srx_ctx *c) {
         c->pl[ax] = g_plan_cache.emplace(key, best_plan).first->second;   // a context that tuned first wins
     }
     for (int pass = 0; pass < 5 && !rc && c->opt.reserved[2] == 0; ++pass) {
+        if (plane && pass >= 1 && pass <= 3) continue;
         const FftPlan &p = c->pl[pass == 2 ? 0 : (pass == 1 || pass == 3) ? 1 : 2];
         const int tmax = fft_tile_max(pass, c->n, p, prec, c->comps());
         std::vector<int> cand;

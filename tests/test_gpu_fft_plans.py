@@ -98,3 +98,26 @@ def test_tuned_plans_are_candidates_shared_and_accurate(tmp_path, precision):
     close_fields(a, t, TOL[precision])
     for s in (a, t, u):
         s.close()
+
+
+@pytest.mark.parametrize("precision", [srx_amd.PREC_FP64, srx_amd.PREC_MIXED])
+@pytest.mark.parametrize("n", [(16, 16, 12), (64, 4, 6)])
+def test_small_planes_tune_what_they_run(tmp_path, precision, n):
+    """Planes of up to 256 points run the y passes and the Green pass in one launch: no tiles are reported for
+    the three, and the plans tuned on x and y (64 included, which runs no wavefront pass here) are
+    candidates that give the default plans' fields within the FFT's rounding."""
+    deck = inputs.make_case(str(tmp_path), n=n, grains=4, seed=45, nsteps=2, timestep=0.1)
+    a = srx_amd.Solver(deck, precision=precision, fixed_iters=4)
+    t = srx_amd.Solver(deck, precision=precision, fixed_iters=4, reserved=[0, 0, 0, 1])
+    for s in (a, t):
+        tiles, us = s.fft_tiles()
+        assert tiles[1:4] == [0, 0, 0] and us[1:4] == [0.0, 0.0, 0.0]
+        assert tiles[0] >= 1 and tiles[4] >= 1 and us[0] > 0 and us[4] > 0
+    for ax, extent in enumerate(n):
+        assert t.fft_plan(ax) in srx_amd.fft_plan_candidates(extent)
+    for _ in range(2):
+        a.step()
+        t.step()
+    close_fields(a, t, TOL[precision])
+    a.close()
+    t.close()
