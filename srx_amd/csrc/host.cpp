@@ -333,6 +333,8 @@ struct srx_ctx {
     FftPlan pl[3];
     double *partials = nullptr, *red = nullptr, *hred = nullptr, *redseg = nullptr;
     IterCtl *dctl = nullptr, *hctl = nullptr;   // outer-iteration control block (device, pinned host copy)
+    int *hdone = nullptr;                      // IterCtl::done_host, behind hctl
+    hipEvent_t ahead_ev[2] = {nullptr, nullptr};
     int iters_last = 0;                        // outer iterations of the last increment
     int nr_blocks = 0, end_blocks = 0;
     bool fcc = false;                          // the slip systems have the FCC zero structure (nr_fcc)
@@ -813,7 +815,9 @@ int setup(srx_ctx *c) {
         if (r) return r;
     }
     HIPCK(hipMalloc(&c->dctl, sizeof(IterCtl)));
-    HIPCK(hipHostMalloc((void **)&c->hctl, sizeof(IterCtl), hipHostMallocDefault));
+    HIPCK(hipHostMalloc((void **)&c->hctl, sizeof(IterCtl) + sizeof(int), hipHostMallocDefault));
+    c->hdone = reinterpret_cast<int *>(c->hctl + 1);
+    for (hipEvent_t &e : c->ahead_ev) HIPCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     return 0;
 }
 
@@ -1381,6 +1385,10 @@ static int step_begin(srx_ctx *c, EnsIncr *batch = nullptr) {
     }
     for (int k = 0; k < 9; ++k) ctl.uniform[k] = c->uniform0[k] = c->uniform[k];
     ctl.done = ctl_stop(ctl);
+    if (!batch) {
+        __atomic_store_n(c->hdone, 0, __ATOMIC_RELAXED);
+        ctl.done_host = c->hdone;
+    }
     HIPCK(hipMemcpyAsync(c->dctl, &ctl, sizeof(IterCtl), hipMemcpyHostToDevice, c->stream));
     return 0;
 }
@@ -1402,9 +1410,15 @@ static int step_iterate(srx_ctx *c) {
     int launched = 0;
     // Batches enqueued before the control block is first read: increments of one loading path take
     // similar iteration counts, so all but the last of the previous increment's batches go out without
-    // waiting for the one before (a read-back leaves the GPU idle for 20-40 us, of 54 us x 8
-    // iterations at 16^3).  Iterations past convergence return at once.
+    // reading anything back (a read-back leaves the GPU idle for 20-40 us, of 54 us x 8 iterations at 16^3).
+    // Iterations past convergence return at once, but their launches are not free (20 us an iteration at
+    // 16^3): every AHEAD_LOOK batches the host waits for those it sent AHEAD_LOOK earlier and looks at the flag
+    // that the control kernel raises, so that an increment that needs fewer iterations than the last one
+    // drains at most 2 AHEAD_LOOK batches too many, not the rest of them (after 1000 iterations, 124).
+    // An event after every batch cost 3 us of 350 at 16^3.
+    constexpr int AHEAD_LOOK = 4;
     int ahead = batch == ITER_BATCH ? (c->opt.fixed_iters > 0 ? c->opt.fixed_iters : c->iters_last) / ITER_BATCH : 1;
+    int sent = 0;
     while (!ctl.done) {
         if (launched > most) return SRX_E_HIP;   // the control kernel must have stopped the loop
         hipGraphExec_t *gx = use_graph ? &c->gexec[launched == 0 ? 1 : 0][rotated] : nullptr;
@@ -1454,7 +1468,13 @@ static int step_iterate(srx_ctx *c) {
             HIPCK(hipGraphLaunch(*gx, c->stream));
         }
         }
-        if (--ahead > 0 && launched + batch <= most) continue;
+        if (--ahead > 0 && launched + batch <= most) {
+            if (++sent % AHEAD_LOOK) continue;
+            const int look = sent / AHEAD_LOOK;
+            HIPCK(hipEventRecord(c->ahead_ev[look & 1], c->stream));
+            if (look > 1) HIPCK(hipEventSynchronize(c->ahead_ev[(look - 1) & 1]));
+            if (!__atomic_load_n(c->hdone, __ATOMIC_ACQUIRE)) continue;
+        }
         HIPCK(hipMemcpyAsync(&ctl, c->dctl, sizeof(IterCtl), hipMemcpyDeviceToHost, c->stream));
         HIPCK(hipStreamSynchronize(c->stream));
         if (c->opt.verbose) std::printf("iter %d Err_e %e Err_s %e\n", ctl.iter, ctl.Err_e, ctl.Err_s);
@@ -2264,6 +2284,8 @@ void srx_close(srx_ctx *c) {
     if (c->hctl) (void)hipHostFree(c->hctl);
     if (c->stage) (void)hipHostFree(c->stage);
     for (hipEvent_t e : c->stage_ev)
+        if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t e : c->ahead_ev)
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->evpool) (void)hipEventDestroy(e);
     drop_graphs(c);

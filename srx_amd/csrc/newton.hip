@@ -1171,6 +1171,7 @@ __device__ __forceinline__ void control_block(const DevConst *__restrict__ cst, 
                 c.Err_s = red[0] * c.wgt / c.s_vm;
                 c.done = ctl_stop(c);
             }
+            if (c.done && c.done_host) __hip_atomic_store(c.done_host, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
     __syncthreads();

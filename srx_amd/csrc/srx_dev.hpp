@@ -116,6 +116,7 @@ struct IterCtl {
     double Scauchy[9];
     int vbc[6], sbc[6];
     int svm_mode, itermax, fixed_iters, mixed;
+    int *done_host;       // pinned host memory that learns of `done` while batches are in flight; may be null
     // advanced by the control kernel
     int iter, done, nan, pad0;
     long long nrtot;

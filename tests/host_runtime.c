@@ -4,6 +4,8 @@
    host_fail_launch(k): the k-th launch from now (0: the next) fails, -1: none;
    host_launches(): launches since the last host_fail_launch.
    host_pinned_bytes(): pinned memory handed out so far;
+   host_stop_after(k): increments from now on stop after k outer iterations (host_control.cpp answers for
+   the control and reduction kernels);
    host_watch_pointer(i): from now on, note the pointer every launch passes as its argument i (-1: none);
    host_pointer_offsets(): the bits set in any of their distances from the first. */
 #include <stdint.h>
@@ -22,7 +24,22 @@ static uintptr_t first_pointer, offsets;
 void host_watch_pointer(int i) { watched = i; first_pointer = offsets = 0; }
 long host_pointer_offsets(void) { return (long)offsets; }
 
-static int launch(void **args) {
+static const void *control, *reduce;
+static int stop_after = 1;
+void host_stop_after(int k) { stop_after = k; }
+void host_control(void *block, int stop);
+void host_reduce(int nvals, double *out);
+int __hipRegisterFunction(void **m, const void *host, char *dev, const char *name, unsigned t, void *a, void *b, void *c,
+                          void *d, int *w) {
+    (void)m; (void)dev; (void)t; (void)a; (void)b; (void)c; (void)d; (void)w;
+    if (strstr(name, "9k_controlE")) control = host;
+    if (strstr(name, "8k_reduceE")) reduce = host;
+    return 0;
+}
+
+static int launch(const void *f, void **args) {
+    if (f == control) host_control(*(void **)args[4], stop_after);
+    if (f == reduce) host_reduce(*(int *)args[2], *(double **)args[4]);
     if (watched >= 0) {
         const uintptr_t p = *(uintptr_t *)args[watched];
         if (!first_pointer) first_pointer = p;
@@ -33,12 +50,12 @@ static int launch(void **args) {
     return last_error;
 }
 int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **a, size_t m, void *s) {
-    (void)f; (void)g; (void)b; (void)m; (void)s;
-    return launch(a);
+    (void)g; (void)b; (void)m; (void)s;
+    return launch(f, a);
 }
 int hipExtLaunchKernel(const void *f, dim3_t g, dim3_t b, void **a, size_t m, void *s, void *e0, void *e1, int fl) {
-    (void)f; (void)g; (void)b; (void)m; (void)s; (void)e0; (void)e1; (void)fl;
-    return launch(a);
+    (void)g; (void)b; (void)m; (void)s; (void)e0; (void)e1; (void)fl;
+    return launch(f, a);
 }
 int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t m, void *s) { (void)g; (void)b; (void)m; (void)s; return 0; }
 int __hipPopCallConfiguration(dim3_t *g, dim3_t *b, size_t *m, void **s) {

@@ -62,12 +62,28 @@ for name in ("sig", "rho_s", "rho_tot"):   # the first read, and larger and smal
 most = s.nxyz * 12 * 8
 assert rt.host_pinned_bytes() - before <= (most + 4096 if most <= 2 << 20 else most // 4 + 4 * 4096)
 """
+AHEAD = """
+s = srx_amd.Solver(sys.argv[2], reserved=[0, 1])   # launch by launch
+def launches(iters):
+    rt.host_stop_after(iters)
+    rt.host_fail_launch(-1)
+    assert s.step()["iters"] == iters
+    return rt.host_launches()
+first, again = launches(8), launches(8)    # one batch, with nothing known of the iteration count
+per_batch = launches(16) - again           # two batches
+for few in (3, 8, 20):
+    launches(900)
+    assert launches(few) <= again + (few // 8 + 8) * per_batch, few
+"""
 
 
 @pytest.fixture(scope="module")
 def runtime(tmp_path_factory):
     lib = str(tmp_path_factory.mktemp("rt") / "host_runtime.so")
-    subprocess.check_call(["gcc", "-shared", "-fPIC", "-O1", "-o", lib, os.path.join(HERE, "host_runtime.c")])
+    obj = lib + ".o"
+    subprocess.check_call(["gcc", "-c", "-fPIC", "-O1", "-o", obj, os.path.join(HERE, "host_runtime.c")])
+    subprocess.check_call(["g++", "-shared", "-fPIC", "-O1", "-std=c++17", "-w", "-D__HIP_PLATFORM_AMD__",
+                           "-I/opt/rocm/include", "-o", lib, os.path.join(HERE, "host_control.cpp"), obj])
     return lib
 
 
@@ -98,3 +114,9 @@ def test_first_field_read_pins_a_quarter_of_a_field(runtime, tmp_path, n):
     """Pinned memory is paid for by a context's first read (its pages are mapped on first touch): no more of it
     than a quarter of the largest field, or one such field where that is small."""
     run(PINNED, runtime, inputs.make_case(str(tmp_path), n=n, grains=3, seed=1, nsteps=1, timestep=0.1))
+
+
+def test_a_quick_increment_after_a_long_one(runtime, tmp_path):
+    """Batches of 8 iterations go out ahead by the last increment's count: an increment that needs fewer
+    stops the host within eight batches of its own last one."""
+    run(AHEAD, runtime, inputs.make_case(str(tmp_path), n=(6, 5, 4), grains=3, seed=1, nsteps=20, timestep=0.1))
