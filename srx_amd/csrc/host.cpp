@@ -2000,19 +2000,20 @@ int srx_kernel_times(srx_ctx *c, const char **names, double *ms, int *calls, int
 
 // Reads a field through the context's pinned slots: the gather kernel writes chunk after chunk into them
 // in the caller's layout, and while later chunks cross the link the host copies finished ones into the
-// caller's (pageable) buffer.  The slots together hold a quarter of the largest field: pinned memory costs its
-// first reader 0.37 ms a MiB (the host's page faults; 0.03 once they are in), which a context's first
-// read pays, and smaller chunks cost a repeated read their launches.  With four slots of 2 MiB the first read
-// of 32^3 took 1.4 ms and of 48^3 3.5-4.2 (a pageable copy and a host loop: 0.56 and 1.8-3.0); with a
-// quarter 0.17 and 1.7-2.1, repeated ones 0.12 and 0.28 (before 0.12 and 0.32).  A grid whose fields fit STAGE_ONE
+// caller's (pageable) buffer.  Large fields (STAGE_MT) take helper threads for the copy: a fresh buffer's 2 MiB
+// pages are zeroed on first touch, 18 GB/s with one thread and 61 with four, and only a slot of 2 MiB or
+// more lets the threads do that side by side (slots of 8 MiB at 128^3; slots of 1.6 MiB instead of 2 at 64^3
+// read six fields in 6.2 ms instead of 5.6).  The helpers live for one call (a pool of OpenMP threads, which go
+// on spinning after their region, slowed the caller's own OpenMP work next to it by 30 ms).
+// Without helpers the slots together hold a quarter of the largest field: pinned memory costs its first
+// reader 0.37 ms a MiB (the host's page faults; 0.03 once they are in), which a context's first read pays,
+// and smaller chunks cost a repeated read their launches.  With four slots of 2 MiB the first read of
+// 32^3 took 1.4 ms and of 48^3 3.5-4.2 (a pageable copy and a host loop: 0.56 and 1.8-3.0); with a quarter 0.17
+// and 0.4-2.1, repeated ones 0.12-0.16 and 0.28 (before 0.12 and 0.32).  A grid whose fields fit STAGE_ONE
 // takes one slot for the whole field: below it chunks only add launches (24^3: 0.057 ms repeated, in slots of
-// 128 KiB 0.072).  Large fields take helper threads for the copy: a fresh buffer's 2 MiB pages are zeroed on
-// first touch, 18 GB/s with one thread and 61 with four, and only a slot of several pages lets the
-// threads do that side by side (slots of 8 MiB at 128^3).  The helpers live for one call (a pool of
-// OpenMP threads, which go on spinning after their region, slowed the caller's own OpenMP work
-// next to it by 30 ms).
+// 128 KiB 0.072).
 constexpr int STAGE_SLOTS = 4, STAGE_HELPERS = 3;
-constexpr size_t STAGE_ONE = (size_t)2 << 20, STAGE_SLOT_MAX = (size_t)8 << 20, STAGE_MT = (size_t)8 << 20;
+constexpr size_t STAGE_ONE = (size_t)2 << 20, STAGE_SLOT = (size_t)2 << 20, STAGE_SLOT_MAX = (size_t)8 << 20, STAGE_MT = (size_t)8 << 20;
 
 // Copies of finished chunks by the calling thread and its helpers, each a part of every chunk.
 struct StageCopy {
@@ -2068,7 +2069,9 @@ static int read_field(srx_ctx *c, int mode, int nc, const FieldSrc &src, double 
         // sized for the largest field (12 values per voxel), whole rows of every field in a slot
         const size_t most = sizeof(double) * 12 * (size_t)c->nvox;
         const bool one = most <= STAGE_ONE;
-        const size_t want = one ? most : std::min(STAGE_SLOT_MAX, most / (4 * STAGE_SLOTS));
+        const bool helpers = sizeof(double) * 9 * (size_t)c->nvox >= STAGE_MT;   // its 3 x 3 fields take them
+        const size_t part = std::min(STAGE_SLOT_MAX, most / (4 * STAGE_SLOTS));
+        const size_t want = one ? most : helpers ? std::max(STAGE_SLOT, part) : part;
         const size_t slot = (want + 4095) & ~(size_t)4095;   // slots start on page boundaries
         for (int k = 0; k < STAGE_SLOTS; ++k)
             if (!c->stage_ev[k]) HIPCK(hipEventCreateWithFlags(&c->stage_ev[k], hipEventDisableTiming));

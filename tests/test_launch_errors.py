@@ -60,7 +60,8 @@ before = rt.host_pinned_bytes()
 for name in ("sig", "rho_s", "rho_tot"):   # the first read, and larger and smaller fields after it
     s.field(name)
 most = s.nxyz * 12 * 8
-assert rt.host_pinned_bytes() - before <= (most + 4096 if most <= 2 << 20 else most // 4 + 4 * 4096)
+threads = s.nxyz * 9 * 8 >= 8 << 20   # fields that helper threads copy
+assert rt.host_pinned_bytes() - before <= (most + 4096 if most <= 2 << 20 else max(most // 4, threads * (8 << 20)) + 4 * 4096)
 """
 AHEAD = """
 s = srx_amd.Solver(sys.argv[2], reserved=[0, 1])   # launch by launch
@@ -112,7 +113,8 @@ def test_field_chunks_start_aligned(runtime, tmp_path, n):
 @pytest.mark.parametrize("n", [(4, 4, 4), (27, 27, 27), (32, 32, 32), (48, 48, 48), (75, 60, 45)])
 def test_first_field_read_pins_a_quarter_of_a_field(runtime, tmp_path, n):
     """Pinned memory is paid for by a context's first read (its pages are mapped on first touch): no more of it
-    than a quarter of the largest field, or one such field where that is small."""
+    than a quarter of the largest field, or one such field where that is small, or four slots of 2 MiB
+    where helper threads share the page faults."""
     run(PINNED, runtime, inputs.make_case(str(tmp_path), n=n, grains=3, seed=1, nsteps=1, timestep=0.1))
 
 
