@@ -37,12 +37,18 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, GB/s
 FP64_PEAK_TFLOPS = 78.6        # MI355X FP64 (vector and matrix), TFLOP/s
-F_NR = 2300.0                  # flops per voxel per Newton iteration (algorithmic count)
+# FP64 flops per voxel and Newton iteration that the lanes of the Newton kernel execute, its prologue and
+# epilogue included: 64 x SQ_INSTS_VALU_FLOPS_FP64 over all launches of increments 0-4 (masked lanes count) by
+# the Newton iterations of the same increments (profiles/evp_fft_128cubed_pmc.md)
+NR_FLOPS = {"fp64": 1410.0, "mixed": 1498.0}
+# the same of a plain Newton iteration: every component of 12 Schmid vectors, Jacobian and factorisation in
+# each iteration.  The kernel leaves out the Schmid vectors' zeros and, in FP64, the last iteration's Jacobian.
+NR_FLOPS_PLAIN = 2300.0
 # HBM bytes per voxel per launch of the Newton kernel (after the first of an increment), from
 # rocprofv3 FETCH_SIZE (x2.0) and WRITE_SIZE (x1.0) runs calibrated on a 1 GiB device copy
 # (profiles/evp_fft_128cubed_pmc.md); mixed precision reads the increment's Newton matrix and
 # per-system constants as FP32
-NR_TRAFFIC_BYTES_PER_VOXEL = {"fp64": 641.5, "mixed": 502.1}
+NR_TRAFFIC_BYTES_PER_VOXEL = {"fp64": 641.5, "mixed": 506.5}
 METRIC = "converged voxel-increments/s at 128³, plain FP64 vs mixed-precision at equal stress error"
 
 
@@ -355,7 +361,8 @@ def main() -> int:
             "kernel_ms": {k: v[0] for k, v in kt.items()},
             "fft_green_gbs": b_fg * b_iters / (fg_ms * 1e-3) / 1e9 if fg_ms else None,
             "fft_green_frac_hbm": (b_fg * b_iters / (fg_ms * 1e-3) / 1e9) / HBM_PEAK_GBS if fg_ms else None,
-            "nr_tflops": F_NR * e["nr_total"] / (nr_ms * 1e-3) / 1e12 if nr_ms else None,
+            "nr_tflops": NR_FLOPS[name] * e["nr_total"] / (nr_ms * 1e-3) / 1e12 if nr_ms else None,
+            "nr_tflops_plain_newton": NR_FLOPS_PLAIN * e["nr_total"] / (nr_ms * 1e-3) / 1e12 if nr_ms else None,
             "fft_green_bytes_per_voxel": b_fg / nvox,
         }
         if name in fs:
@@ -380,13 +387,15 @@ def main() -> int:
     if dom == "nr":
         E = nre[head]
         kt = E["kernels"]
-        ach = F_NR * E["nr_total"] / (kt["nr"][0] * 1e-3) / 1e12
+        ach = NR_FLOPS[head] * E["nr_total"] / (kt["nr"][0] * 1e-3) / 1e12
         out["roofline"] = {"kernel": "nr", "bound": "fp64_valu", "peak_kind": "FP64 vector ALU (no MFMA in this kernel)",
                            "achieved": ach, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                            "frac": ach / FP64_PEAK_TFLOPS, "traffic": NR_TRAFFIC_BYTES_PER_VOXEL[head] * nvox,
                            "traffic_unit": "HBM bytes per launch (rocprofv3 PMC, profiles/)",
-                           "algorithmic": "%.0f flop per voxel per Newton iteration x %.3f Newton iterations per voxel "
-                                          "per launch" % (F_NR, E["nr_total"] / nvox / max(E["iters"], 1))}
+                           "achieved_plain_newton": ach * NR_FLOPS_PLAIN / NR_FLOPS[head],
+                           "algorithmic": "%.0f executed flop (%.0f of a plain Newton iteration) per voxel per Newton "
+                                          "iteration x %.3f Newton iterations per voxel per launch"
+                                          % (NR_FLOPS[head], NR_FLOPS_PLAIN, E["nr_total"] / nvox / max(E["iters"], 1))}
     else:
         kt = bk
         rb = 4 if head == "mixed" else 8

@@ -1712,7 +1712,7 @@ void launch_fft_inv_z_update(hipStream_t s, int prec, const void *specB, double 
 // B basis), into out [3][N] (entries (1,2), (0,2), (0,1)): forward transforms of the six strain
 // components, rotation_point, inverse transforms of three.  In FP64 in mixed precision too: the strain is a
 // sum of FP32 increments that is kept in FP64, and casting that sum to FP32 for one more pair of
-// transforms added 1.3e-7 of the rotation to its error (0.3 ms an increment at 128^3 instead of 0.15).
+// transforms added 1.3e-7 of the rotation to its error (0.18 ms an increment at 128^3 instead of 0.15).
 // specB, specC: 6 FP64 half spectra each; tw: FP64 twiddles; tiles: the solver passes' (launch shapes only).
 void launch_rotation_part(hipStream_t s, const double *in, double *out, void *specB, void *specC, const int n[3],
                           const FftPlan pl[3], void *const tw[3], const DevConst *cst, void *nyq, const int tiles[5]) {
