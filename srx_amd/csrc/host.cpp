@@ -452,24 +452,24 @@ int ctx_zero(hipStream_t st, void *dst, size_t bytes) {
     return 0;
 }
 
-// job(begin, end) over [0, n) in at most `threads` contiguous ranges of at least 4096, on threads that
-// end with the call: OpenMP's workers go on spinning for 200 ms after a region, next to the solver's own
-// host thread and whatever the caller runs (a float conversion on the caller's OpenMP threads took
-// 30-75 ms instead of 1 beside them).
+// job(begin, end) over [0, n) in ranges of 4096 that up to `threads` threads take in turn (a thread that starts
+// late or shares its core takes fewer), on threads that end with the call: OpenMP's workers go on spinning
+// for 200 ms after a region, next to the solver's own host thread and whatever the caller runs (a float
+// conversion on the caller's OpenMP threads took 30-75 ms instead of 1 beside them).
 template <typename Job>
 void parallel_ranges(long n, int threads, Job job) {
-    const int parts = (int)std::max(1L, std::min((long)threads, n / 4096));
+    constexpr long RANGE = 4096;
+    std::atomic<long> next{0};
+    auto work = [&]() {
+        for (long v0; (v0 = next.fetch_add(RANGE)) < n;) job(v0, std::min(n, v0 + RANGE));
+    };
+    const int parts = (int)std::max(1L, std::min((long)threads, n / RANGE));
     std::vector<std::thread> th;
-    long next = 0;   // ranges [0, next) run on a thread of their own
     try {
-        for (int p = 0; p + 1 < parts; ++p) {
-            const long end = n * (p + 1) / parts;
-            th.emplace_back([&job, next, end]() { job(next, end); });
-            next = end;
-        }
-    } catch (...) {   // no more threads: the caller takes the rest
+        for (int p = 0; p + 1 < parts; ++p) th.emplace_back(work);
+    } catch (...) {   // no more threads: those that run and the caller share the work
     }
-    job(next, n);
+    work();
     for (auto &t : th) t.join();
 }
 

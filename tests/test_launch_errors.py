@@ -76,6 +76,13 @@ for few in (3, 8, 20):
     launches(900)
     assert launches(few) <= again + (few // 8 + 8) * per_batch, few
 """
+MESH = """
+want = np.array([int(line.split()[6]) for line in open(sys.argv[3])], float)
+for threads in (0, 1, 2, 3, 16):
+    s = srx_amd.Solver(sys.argv[2], nthreads=threads)
+    np.testing.assert_array_equal(s.field("grain"), want)
+    s.close()
+"""
 
 
 @pytest.fixture(scope="module")
@@ -122,3 +129,11 @@ def test_a_quick_increment_after_a_long_one(runtime, tmp_path):
     """Batches of 8 iterations go out ahead by the last increment's count: an increment that needs fewer
     stops the host within eight batches of its own last one."""
     run(AHEAD, runtime, inputs.make_case(str(tmp_path), n=(6, 5, 4), grains=3, seed=1, nsteps=20, timestep=0.1))
+
+
+@pytest.mark.parametrize("n", [(5, 4, 3), (16, 16, 16), (16, 16, 32), (27, 15, 18), (27, 27, 30)])
+def test_mesh_is_read_whole_by_any_number_of_threads(runtime, tmp_path, n):
+    """Threads take ranges of 4096 voxels in turn: fewer than one range, whole ranges, remainders, more
+    threads than ranges."""
+    deck = inputs.make_case(str(tmp_path), n=n, grains=40, seed=6, nsteps=1, timestep=0.1)
+    run(MESH, runtime, deck, str(tmp_path / "mesh.txt"))
