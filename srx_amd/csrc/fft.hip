@@ -4,10 +4,12 @@
 // first wait.
 //   fwd_z   real [c][x][y][z]      -> half spectrum B [c][kz][x][y]   (two real comps per complex FFT)
 //   fft_y   B <-> C [c][kz][y][x]  (the y transform doubles as the pencil transpose)
-//   green   C(6 stress comps) -> forward x -> Green operator -> inverse x -> C(9 comps), in place
-//           (k_green_wave: one wavefront per row, cross-lane butterflies, for x extents 64/128/256;
+//   green   C(6 stress comps) -> forward x -> Green operator -> inverse x -> C(6 strain comps, or DisGrad's 9:
+//           strain_form), in place (k_green_wave: one wavefront per row, cross-lane butterflies, for x extents 64/128/256;
 //           k_green_x: LDS transforms otherwise)
-//   inv_z   B(9 comps) -> c2r along z, fused with the FP64 DisGrad update (Eq. 15)
+//   inv_z   B(6 or 9 comps) -> c2r along z, fused with the FP64 update of the strain or of DisGrad (Eq. 15)
+//   plane   forward y, green and inverse y of small planes in one launch, layout B in place
+// and, once per increment with the six components, DisGrad's rotation part (launch_rotation_part).
 // Also here: the FFT-only test entry points and the streaming copy that measures the HBM ceiling.
 #include "kern_common.hpp"
 

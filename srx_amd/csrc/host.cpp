@@ -835,7 +835,6 @@ void open_files(srx_ctx *c) {
     if (c->ferr) std::fprintf(c->ferr, "IT\tERRE\tERRS\tSVM\n");
 }
 
-// get_smacro (evolution.c:590-664) from the reduced sums
 // event-timed launch helper: events come from a pool that is reused every increment
 struct Timer {
     srx_ctx *c;

@@ -636,8 +636,8 @@ __device__ __forceinline__ void nr_voxel(const DevConst *__restrict__ cst, const
 }
 
 // Waves per SIMD the register allocator targets for the Newton kernel: a second wavefront per
-// SIMD to issue from (measured 31% faster than one), which the LDS of the per-system constants
-// (18 KB per 64-lane block) also allows; both the first call of an increment and the later ones
+// SIMD to issue from (measured 31% faster than one), which the LDS of the per-system constants and the
+// quaternion (20 KB per 64-lane block; 12.5 KB and three in the FP32 layout) also allows; both the first call of an increment and the later ones
 // fit two without spills.
 #ifndef SRX_NR_WAVES_PER_EU
 #define SRX_NR_WAVES_PER_EU 2
@@ -765,7 +765,8 @@ __device__ __forceinline__ void nr_block(const DevConst *__restrict__ cst, const
     const bool valid = v < nvox;
     const int ph = valid ? f.phase[v] : 0;
     // LDS: the 36 per-system constants of the block's 64 voxels (18 KB; the first call of an
-    // increment computes them here, the later ones copy them from f.nrc) and the orientation.
+    // increment computes them here, the later ones copy them from f.nrc) and the orientation (2 KB); the FP32
+    // layout holds the constants and 14 values of A in 12.5 KB.
     static_assert(!(F32 && FIRST), "the first call computes its constants in the FP64 layout");
     constexpr int NSLOT = F32 ? NRF_SLOTS / 2 : NRC_COMPS + 4;
     __shared__ __align__(16) double lds[NSLOT * NR_BLOCK];

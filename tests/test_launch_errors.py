@@ -1,5 +1,6 @@
-"""A kernel launch that the runtime refuses is an error of the call that made it, not a result: the entry
-points whose kernels write the caller's data, run on tests/host_runtime.c (no GPU)."""
+"""The host side on a machine without a GPU, on tests/host_runtime.c: a kernel launch that the runtime refuses
+is an error of the call that made it, not a result (the entry points whose kernels write the caller's
+data); the slots of the field readback; how many batches of iterations go out; the mesh reader's threads."""
 import os
 import subprocess
 import sys
