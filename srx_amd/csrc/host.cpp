@@ -2397,51 +2397,59 @@ static int fft_test_common(int ncomp, int n0, int n1, int n2, int prec, FftPlan 
     return 0;
 }
 
+// The entry points' transforms, over the spectra sB, sC and one more device buffer that the caller frees:
+// [the fields, then the spectra in the caller's order] forwards, the reverse backwards (16 bytes a
+// spectrum value, never fewer bytes than the fields').
+static int fft_forward_on(const double *in, int ncomp, const int n[3], int prec, double *out, const FftPlan pl[3],
+                          void *const tw[3], void *sB, void *sC, size_t specn, double **buf) {
+    const size_t N = (size_t)n[0] * n[1] * n[2];
+    HIPCK(hipMalloc(buf, sizeof(double) * 2 * specn));
+    HIPCK(hipMemcpy(*buf, in, sizeof(double) * ncomp * N, hipMemcpyHostToDevice));
+    HIPCK(launch_fft_real_forward_test(nullptr, prec, *buf, ncomp, sB, sC, n, pl, tw));
+    HIPCK(launch_spec_turn(nullptr, prec, true, sC, *buf, ncomp, n));
+    HIPCK(hipDeviceSynchronize());
+    HIPCK(hipMemcpy(out, *buf, sizeof(double) * 2 * specn, hipMemcpyDeviceToHost));
+    return 0;
+}
+
+static int fft_inverse_on(const double *in, int ncomp, const int n[3], int prec, double scale, double *out,
+                          const FftPlan pl[3], void *const tw[3], void *sB, void *sC, size_t specn, double **buf) {
+    const size_t N = (size_t)n[0] * n[1] * n[2];
+    HIPCK(hipMalloc(buf, sizeof(double) * 2 * specn));
+    HIPCK(hipMemcpy(*buf, in, sizeof(double) * 2 * specn, hipMemcpyHostToDevice));
+    HIPCK(launch_spec_turn(nullptr, prec, false, sC, *buf, ncomp, n));
+    HIPCK(launch_fft_real_inverse_test(nullptr, prec, sC, sB, ncomp, *buf, n, pl, tw, 1.0 / scale));
+    HIPCK(hipDeviceSynchronize());
+    HIPCK(hipMemcpy(out, *buf, sizeof(double) * ncomp * N, hipMemcpyDeviceToHost));
+    return 0;
+}
+
+static void fft_test_free(double *buf, void *sB, void *sC, void *const tw[3]) {
+    for (void *p : {(void *)buf, sB, sC, tw[0], tw[1], tw[2]})
+        if (p) (void)hipFree(p);
+}
+
 int srx_fft_forward(const double *in, int ncomp, int n0, int n1, int n2, int prec, double *out) {
     FftPlan pl[3];
     void *tw[3] = {nullptr, nullptr, nullptr}, *sB = nullptr, *sC = nullptr;
+    double *buf = nullptr;
     size_t specn = 0;
-    int rc = fft_test_common(ncomp, n0, n1, n2, prec, pl, tw, &sB, &sC, specn);
-    const size_t N = (size_t)n0 * n1 * n2;
-    double *buf = nullptr;   // the fields, then the spectra in the caller's order (16 bytes a value, never fewer bytes)
     const int n[3] = {n0, n1, n2};
-    if (!rc) {
-        HIPCK(hipMalloc(&buf, sizeof(double) * 2 * specn));
-        HIPCK(hipMemcpy(buf, in, sizeof(double) * ncomp * N, hipMemcpyHostToDevice));
-        HIPCK(launch_fft_real_forward_test(nullptr, prec, buf, ncomp, sB, sC, n, pl, tw));
-        HIPCK(launch_spec_turn(nullptr, prec, true, sC, buf, ncomp, n));
-        HIPCK(hipDeviceSynchronize());
-        HIPCK(hipMemcpy(out, buf, sizeof(double) * 2 * specn, hipMemcpyDeviceToHost));
-    }
-    if (buf) (void)hipFree(buf);
-    if (sB) (void)hipFree(sB);
-    if (sC) (void)hipFree(sC);
-    for (int i = 0; i < 3; ++i)
-        if (tw[i]) (void)hipFree(tw[i]);
+    int rc = fft_test_common(ncomp, n0, n1, n2, prec, pl, tw, &sB, &sC, specn);
+    if (!rc) rc = fft_forward_on(in, ncomp, n, prec, out, pl, tw, sB, sC, specn, &buf);
+    fft_test_free(buf, sB, sC, tw);
     return rc;
 }
 
 int srx_fft_inverse(const double *in, int ncomp, int n0, int n1, int n2, int prec, double scale, double *out) {
     FftPlan pl[3];
     void *tw[3] = {nullptr, nullptr, nullptr}, *sB = nullptr, *sC = nullptr;
+    double *buf = nullptr;
     size_t specn = 0;
-    int rc = fft_test_common(ncomp, n0, n1, n2, prec, pl, tw, &sB, &sC, specn);
-    const size_t N = (size_t)n0 * n1 * n2;
-    double *buf = nullptr;   // the spectra in the caller's order, then the fields
     const int n[3] = {n0, n1, n2};
-    if (!rc) {
-        HIPCK(hipMalloc(&buf, sizeof(double) * 2 * specn));
-        HIPCK(hipMemcpy(buf, in, sizeof(double) * 2 * specn, hipMemcpyHostToDevice));
-        HIPCK(launch_spec_turn(nullptr, prec, false, sC, buf, ncomp, n));
-        HIPCK(launch_fft_real_inverse_test(nullptr, prec, sC, sB, ncomp, buf, n, pl, tw, 1.0 / scale));
-        HIPCK(hipDeviceSynchronize());
-        HIPCK(hipMemcpy(out, buf, sizeof(double) * ncomp * N, hipMemcpyDeviceToHost));
-    }
-    if (buf) (void)hipFree(buf);
-    if (sB) (void)hipFree(sB);
-    if (sC) (void)hipFree(sC);
-    for (int i = 0; i < 3; ++i)
-        if (tw[i]) (void)hipFree(tw[i]);
+    int rc = fft_test_common(ncomp, n0, n1, n2, prec, pl, tw, &sB, &sC, specn);
+    if (!rc) rc = fft_inverse_on(in, ncomp, n, prec, scale, out, pl, tw, sB, sC, specn, &buf);
+    fft_test_free(buf, sB, sC, tw);
     return rc;
 }
 

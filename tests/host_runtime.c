@@ -3,6 +3,7 @@
    RTLD_GLOBAL before libsrx.so, it answers the library's calls into the runtime.
    host_fail_launch(k): the k-th launch from now (0: the next) fails, -1: none;
    host_launches(): launches since the last host_fail_launch.
+   host_device_blocks(): device allocations not yet freed;
    host_pinned_bytes(): pinned memory handed out so far;
    host_stop_after(k): increments from now on stop after k outer iterations (host_control.cpp answers for
    the control and reduction kernels);
@@ -67,9 +68,12 @@ int hipGetLastError(void) { int e = last_error; last_error = 0; return e; }
 const char *hipGetErrorString(int e) { return e ? "launch refused by the test" : "no error"; }
 static int get(void **p, size_t n) { *p = calloc(1, n ? n : 1); return *p ? 0 : 2; }
 /* numbers in [1, 2) that follow no pattern, so that matrices left uncomputed in it are regular */
+static long blocks;
+long host_device_blocks(void) { return blocks; }
 int hipMalloc(void **p, size_t n) {
     uint64_t r = 88172645463325252u;
     if (get(p, n)) return 2;
+    ++blocks;
     for (size_t i = 0; i < n / 8; ++i) {
         r ^= r << 13; r ^= r >> 7; r ^= r << 17;
         ((uint64_t *)*p)[i] = (r >> 12) | 0x3ff0000000000000u;
@@ -79,7 +83,7 @@ int hipMalloc(void **p, size_t n) {
 static size_t pinned;
 long host_pinned_bytes(void) { return (long)pinned; }
 int hipHostMalloc(void **p, size_t n, unsigned f) { (void)f; pinned += n; return get(p, n); }
-int hipFree(void *p) { free(p); return 0; }
+int hipFree(void *p) { blocks -= p != 0; free(p); return 0; }
 int hipHostFree(void *p) { free(p); return 0; }
 int hipMemcpy(void *d, const void *s, size_t n, int k) { (void)k; memmove(d, s, n); return 0; }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *st) { (void)k; (void)st; memmove(d, s, n); return 0; }

@@ -20,11 +20,12 @@ E_HIP = 2003
 def each_launch_refused(call):
     rt.host_fail_launch(-1)
     assert call() == 0
-    n = rt.host_launches()
+    n, held = rt.host_launches(), rt.host_device_blocks()
     assert n > 0
     for k in range(n):
         rt.host_fail_launch(k)
         assert call() == E_HIP, k
+        assert rt.host_device_blocks() == held, k
     rt.host_fail_launch(-1)
     assert call() == 0
 """
